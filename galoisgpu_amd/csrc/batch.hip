@@ -44,6 +44,67 @@ static_assert(kItems >= 1 && kItems <= kWave, "items per ticket");
 // spill and were slower (42 vs 34 ms on the item-major path).
 constexpr int kMultiWaves = 4;
 
+// ---- edge filter ------------------------------------------------------------
+//
+// Nine of ten edge expansions of a batched run improve no source (RMAT-22 x 64
+// sources: 42 M of 463 M), and each costs a row access, whose rate bounds the
+// kernel.  From a few rounds on, one 4-byte bound per vertex tells most of
+// them apart.  With an offset off[s] per source, let
+//     bound[v] = max over s of (D[v][s] - off[s]).
+// An expansion of u for the sources in A can improve v over an edge of weight
+// w only if  min over s in A of (D[u][s] - off[s]) + w < bound[v].
+// This holds for any offsets and for bounds taken at any earlier time
+// (distances only fall).  The offsets make the test sharp: off[s] = D[h][s]
+// for the vertex h of largest out-degree, because on a skewed graph most
+// shortest paths run through the hubs, so D[v][s] - D[h][s] is nearly the same for every s
+// (a model of the rounds on RMAT-19: 5.67 E expansions, of which 0.58 E
+// improve; 5.1 E pass the test without offsets, 1.54 E with them).
+// A source that has not reached h yet is left out of the bounds, and an
+// expansion for such a source always passes.
+//
+// The bounds come from up to kSweeps sweeps over D inside the launch, each
+// with the offsets of its time and into an array of its own, so that bounds
+// read through the caches are never of other offsets.  A sweep reads V rows
+// in order; it follows once E/2 edges were expanded since the last one.
+constexpr int kSweeps = 3;
+// The test needs a hub that most paths share: it is used where the largest
+// out-degree is at least kHubRatio times the mean.  Without / with the test
+// (ms, 64 sources unless said): RMAT-21, ratio 4035, 13.4 / 10.2; RMAT of 32768
+// vertices 1.44 / 1.42 (2 sources 0.75 / 0.72); 2^20 vertices of skewed
+// degrees, ratio 50, 16.8 / 16.3; uniform degrees, ratio 2.5, 16.8 / 17.3;
+// road-like 700x700 14.2 / 14.6.
+constexpr uint32_t kHubRatio = 16;
+constexpr int32_t kNoBound = 0x7FFFFFFF;         // bound of a vertex that some source has not reached
+constexpr int32_t kPass = -0x7FFFFFFF - 1;       // lowest distance of an item that takes no test
+
+struct Filter {
+  uint64_t incl;        // sources whose offset is set
+  uint64_t last_edges;  // edges expanded when the last sweep was ordered
+  uint32_t hub;         // vertex of largest out-degree
+  uint32_t on;          // the graph has such a hub
+  int32_t off[64];
+};
+
+// Work tickets and round totals are kept per group of blocks (block b: group
+// b % kGroups), each on a line of its own: atomics on one word are performed
+// one at a time, ~12 ns each, and a word that all 4096 wavefronts share
+// bounds the launch (RMAT-22 x 64 sources: 0.44 M tickets, 5 ms).
+constexpr uint32_t kGroups = 16;
+struct alignas(128) TicketGroup {
+  uint32_t ticket;
+};
+// Counters the leader turns into trace records and scheduler features.
+struct alignas(128) MultiCounters {
+  uint64_t lane_items;   // sum over expanded items of active sources
+  uint64_t edges;        // edges expanded (per vertex, shared by its sources)
+  uint64_t improved;     // rows in which at least one lane improved
+};
+// One wavefront's share in a round: lane_items and edges per lane, improved wave-uniform.
+struct RoundCounters {
+  uint32_t lane_items, edges;
+  uint64_t improved;
+};
+
 struct MArgs {
   const uint32_t *row_start;
   const uint32_t *edge_dst;
@@ -67,6 +128,12 @@ struct MArgs {
   uint32_t *fmin;       // [2][64] smallest pending far distance per source, by phase parity
   uint32_t *thr;        // [64] per-source near/far threshold of the current phase (bucket mode)
   uint32_t *qstamp;     // [V] last round whose in-queue holds the vertex
+  Filter *flt;          // edge filter state
+  TicketGroup *tickets; // [kGroups]
+  MultiCounters *tot;   // [kGroups]
+  uint64_t *hubs;       // multi_init's largest (out-degree << 32 | ~vertex) of each block
+  uint32_t ninit;       // blocks of multi_init
+  int32_t *bound[kSweeps];  // [V] each: the vertices' bounds, one array per sweep
 };
 
 // Pushes are staged per wavefront in LDS, kPushBuf items per pile, and
@@ -76,6 +143,14 @@ struct MArgs {
 // faster than 256 (26.0 vs 26.5 ms on RMAT-22 x 64 sources).
 constexpr uint32_t kPushBuf = 512;
 
+// Heavy items are staged the same way (one atomic on the chunk count per
+// heavy item, ~0.4 M on RMAT-22 x 64 sources, cost ~5 ms and kept the chunks large).
+constexpr uint32_t kHeavyBuf = 64;
+struct HeavyItem {
+  uint32_t u, nch;
+  uint64_t mask;
+};
+
 // Per-round, per-lane view of the schedule used by the edge loop.
 struct LaneSched {
   uint32_t thr;   // near/far threshold of this lane's source
@@ -84,6 +159,11 @@ struct LaneSched {
   uint32_t thr32; // threshold of this lane as u32: a candidate nd goes near iff nd <= thr32
   uint32_t *pb;   // this wavefront's LDS push buffers: [0, kPushBuf) near, [kPushBuf, 2 kPushBuf) far
   uint32_t pbn[2];  // items staged per pile (wave-uniform)
+  HeavyItem *hb;    // this wavefront's LDS buffer of heavy items, kHeavyBuf entries
+  uint32_t hn, hchunks;  // staged heavy items and their chunks (wave-uniform)
+  const int32_t *bound;  // the last sweep's bounds, or null (no test)
+  int32_t off;      // this lane's source: offset, and whether the bounds include it
+  bool incl;
 };
 
 // Writes pile `which`'s staged items to its queue (one atomic for all).
@@ -114,13 +194,6 @@ __device__ __forceinline__ void pile_push(const MArgs &a, const Sched &s, LaneSc
   ls.pbn[which] += n;
 }
 
-// Counters the leader turns into trace records and scheduler features.
-struct MultiCounters {
-  uint64_t lane_items;   // sum over expanded items of active sources
-  uint64_t edges;        // edges expanded (per vertex, shared by its sources)
-  uint64_t improved;     // rows in which at least one lane improved
-};
-
 __device__ __forceinline__ uint64_t bcast64(uint64_t x, uint32_t l) {
   uint32_t lo = readlane((uint32_t)x, l), hi = readlane((uint32_t)(x >> 32), l);
   return ((uint64_t)hi << 32) | lo;
@@ -131,6 +204,13 @@ __device__ __forceinline__ uint64_t bcast64(uint64_t x, uint32_t l) {
 // is empty again).
 __device__ __forceinline__ bool near_admit(const MArgs &a, const Sched &s, uint32_t v) {
   return __hip_atomic_fetch_max(glb(a.qstamp + v), s.round + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < s.round + 1;
+}
+
+// Whether v has out-edges.  A vertex without any is never expanded, so an
+// improvement of it needs no mask and no queue (RMAT-22 x 64 sources: 14.0 ->
+// 11.7 M items popped, 13.9 -> 13.5 ms).
+__device__ __forceinline__ bool has_edges(const MArgs &a, uint32_t v) {
+  return glb(a.row_start)[v] != glb(a.row_start)[v + 1];
 }
 
 // Distance rows of the items a wavefront is expanding: dl[slot][lane] is the
@@ -191,6 +271,8 @@ __device__ __forceinline__ void relax_batch(const MArgs &a, const Sched &s, Lane
   }
   // Two edges of a batch may share a destination; only the lane whose OR
   // finds the mask empty queues it.
+  const bool live = has_edges(a, ev);
+  if (!live) my_nb = my_fb = 0;
   bool pn = my_nb != 0 && atomic_or64(a.nmask[s.round & 1] + ev, my_nb) == 0 && near_admit(a, s, ev);
   bool pf = my_fb != 0 && atomic_or64(a.fmask[s.phase & 1] + ev, my_fb) == 0;
   pile_push(a, s, ls, 0, pn, ev);
@@ -209,6 +291,11 @@ __device__ __forceinline__ void relax_batch(const MArgs &a, const Sched &s, Lane
 // collected in a per-wavefront list and the destinations' masks are updated
 // 64 at a time.
 constexpr int kGroup = 8;
+// Heavy chunks taken as one unit hold at most kChunkUnit edges (and kItems
+// chunks): their distance rows are loaded when the unit starts, and a unit
+// that runs for long relaxes from old distances (RMAT-22 x 64 sources, chunks
+// of 256 edges: 14.6 ms at 256 to 512 edges a unit, 15.0 at 1024, 18.3 at 4096).
+constexpr uint32_t kChunkUnit = 512;
 // A work ticket covers kSpan units (28.0 -> 27.2 ms from 1 to 2; 4 was
 // slower, 29.1 ms, from load imbalance).
 constexpr uint32_t kSpan = 2;
@@ -237,7 +324,8 @@ struct Pending {
 // lane whose OR finds the mask empty pushes it).
 __device__ __forceinline__ void flush_pending(const MArgs &a, const Sched &s, LaneSched &ls, Pending &p) {
   if (p.n == 0) return;
-  const bool act = lane_id() < p.n;
+  order_release();
+  const bool act = lane_id() < p.n && has_edges(a, lane_id() < p.n ? p.v : 0u);
   const uint64_t nb = ((uint64_t)p.nb_hi << 32) | p.nb_lo, fb = ((uint64_t)p.fb_hi << 32) | p.fb_lo;
   const bool pn = act && nb != 0 && atomic_or64(a.nmask[s.round & 1] + p.v, nb) == 0 && near_admit(a, s, p.v);
   const bool pf = act && fb != 0 && atomic_or64(a.fmask[s.phase & 1] + p.v, fb) == 0;
@@ -246,57 +334,30 @@ __device__ __forceinline__ void flush_pending(const MArgs &a, const Sched &s, La
   p.n = 0;
 }
 
-// One window of kGroup edges in flight: candidates nd, then the loaded
-// distances, then the atomics' results; dst holds destination k in lane k.
-struct Window {
-  uint32_t nd[kGroup];
-  uint32_t val[kGroup];
-  uint32_t dst;
-};
-
-// Issues the row loads of a window of edges (destinations vv, weights ww)
-// leaving an item whose distance for this lane's source is du (INF: no
-// candidate); the first `skip` edges carry no candidate (relaxed already).
-__device__ __forceinline__ void window_load(const MArgs &a, uint32_t du, const U32xG &vv, const U32xG &ww,
-                                            uint32_t skip, uint32_t col, Window &w) {
-#pragma unroll
-  for (int k = 0; k < kGroup; ++k) {
-    // du + w never wraps (du <= INF, w <= INT_MAX); INF + w and a skipped
-    // slot's du + 2^31 both exceed every stored distance
-    w.nd[k] = du + ((uint32_t)k < skip ? 0x80000000u : ww[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < kGroup; ++k) w.val[k] = ld_coh(a.D + (size_t)vv[k] * a.S + col);
-}
-
-// Issues the atomicMins of the lanes whose candidate beats the loaded distance.
-__device__ __forceinline__ void window_atomics(const MArgs &a, const U32xG &vv, uint32_t col, Window &w) {
-#pragma unroll
-  for (int k = 0; k < kGroup; ++k)
-    w.val[k] = w.nd[k] < w.val[k] ? atomic_min(a.D + (size_t)vv[k] * a.S + col, w.nd[k]) : 0u;
-}
-
-// Takes a window's atomic results (issued earlier, so the wait overlaps the
-// loads issued since) and records its improved edges.
-__device__ __forceinline__ void window_results(const MArgs &a, LaneSched &ls, Window &w, Pending &p,
-                                               uint64_t &improved) {
+// Takes a window of kGroup edges whose row loads are in flight (candidate
+// cand(k) for row v[k], loaded distance val[k]): issues the atomicMins of the
+// lanes whose candidate is lower and lists the improved edges.  Whether a lane
+// improved is decided by the loaded distance, so no atomic returns a value
+// (a lane that loses a race is expanded once more, for nothing); flush_pending
+// waits for the atomics before it publishes their sources.
+template <class Cand>
+__device__ __forceinline__ void window_take(const MArgs &a, LaneSched &ls, const uint32_t (&v)[kGroup],
+                                            const Cand &cand, const uint32_t (&val)[kGroup], uint32_t col, Pending &p,
+                                            uint64_t &improved) {
   const uint32_t lane = lane_id();
-  // Results are taken only here (left to itself the compiler tests each
-  // result inside its atomic's branch, waiting for the whole memory queue).
-#pragma unroll
-  for (int k = 0; k < kGroup; ++k) asm volatile("" : "+v"(w.val[k]));
 #pragma unroll
   for (int k = 0; k < kGroup; ++k) {
-    const bool imp = w.nd[k] < w.val[k];
+    const uint32_t nd = cand(k);
+    const bool imp = nd < val[k];
     const uint64_t im = __ballot(imp);
     if (im == 0) continue;
-    const uint32_t v = readlane(w.dst, k);
-    const bool nearl = imp && w.nd[k] <= ls.thr32;
+    if (imp) atomic_min(a.D + (size_t)v[k] * a.S + col, nd);
+    const bool nearl = imp && nd <= ls.thr32;
     const uint64_t nb = __ballot(nearl), fb = im & ~nb;
-    if (fb && imp && !nearl) ls.fmin = min(ls.fmin, w.nd[k]);
+    if (fb && imp && !nearl) ls.fmin = min(ls.fmin, nd);
     improved += 1;
     if (lane == p.n) {
-      p.v = v;
+      p.v = v[k];
       p.nb_lo = (uint32_t)nb;
       p.nb_hi = (uint32_t)(nb >> 32);
       p.fb_lo = (uint32_t)fb;
@@ -322,72 +383,276 @@ __device__ __forceinline__ void relax_edges(const MArgs &a, const Sched &s, Lane
   // the bounds are wave-uniform; say so, so that they stay in scalar registers
   lo = __builtin_amdgcn_readfirstlane(lo);
   hi = __builtin_amdgcn_readfirstlane(hi);
-  uint32_t e = lo, w0 = min(lo, hi - kGroup);
-  U32xG vv = scalar_window(a.edge_dst, w0), ww = scalar_window(a.edge_data, w0);
-  Window cur, prev;
-  bool have_prev = false;
-  for (;;) {
-    window_load(a, du, vv, ww, e - w0, col, cur);
-    cur.dst = lane < kGroup ? glb(a.edge_dst)[w0 + lane] : 0u;
+  uint32_t v[kGroup], nd[kGroup], val[kGroup], nv[kGroup], nnd[kGroup], nval[kGroup];
+  // window of edges from e on: slots below e (relaxed already) carry no candidate
+  auto load = [&](uint32_t e, uint32_t(&vv)[kGroup], uint32_t(&x)[kGroup], uint32_t(&c)[kGroup]) {
+    const uint32_t w0 = min(e, hi - kGroup);
+    const U32xG dst = scalar_window(a.edge_dst, w0), w = scalar_window(a.edge_data, w0);
+#pragma unroll
+    for (int k = 0; k < kGroup; ++k) {
+      vv[k] = dst[k];
+      c[k] = ld_coh(a.D + (size_t)dst[k] * a.S + col);
+      // du + w never wraps (du <= INF, w <= INT_MAX); INF + w and a skipped
+      // slot's du + 2^31 both exceed every stored distance
+      x[k] = du + (w0 + k < e ? 0x80000000u : w[k]);
+    }
+  };
+  load(lo, v, nd, val);
+  for (uint32_t e = lo;;) {
     const uint32_t en = e + kGroup;
     const bool more = en < hi;
-    const uint32_t wn = more ? min(en, hi - kGroup) : w0;
-    const U32xG vvn = scalar_window(a.edge_dst, wn), wwn = scalar_window(a.edge_data, wn);
-    if (have_prev) window_results(a, ls, prev, p, improved);
+    if (more) load(en, nv, nnd, nval);
     if (p.n > (uint32_t)(kWave - kGroup)) flush_pending(a, s, ls, p);
-    window_atomics(a, vv, col, cur);
-    prev = cur;
-    have_prev = true;
+    window_take(a, ls, v, [&](int k) { return nd[k]; }, val, col, p, improved);
     if (!more) break;
-    vv = vvn;
-    ww = wwn;
     e = en;
-    w0 = wn;
-  }
-  window_results(a, ls, prev, p, improved);
-}
-
-// Queues heavy vertex u (edges [rs, re)) as chunks of heavy_deg edges, each
-// expanded by a wavefront in the next round with the sources active now.
-__device__ __forceinline__ void queue_heavy(const MArgs &a, const Sched &s, uint32_t u, uint32_t rs, uint32_t re,
-                                            uint64_t am) {
-  const uint32_t lane = lane_id();
-  uint32_t nch = (re - rs + a.heavy_deg - 1) / a.heavy_deg;
-  uint32_t hqi = 1u - s.heavy_in;
-  uint32_t base = 0;
-  if (lane == 0) base = atomic_add(&a.ctrl->hcount[hqi], nch);
-  base = readlane(base, 0);
-  for (uint32_t k = lane; k < nch; k += kWave) {
-    uint32_t pos = base + k;
-    if (pos < a.hcap) {
-      st_coh64(a.hq[hqi] + 2ull * pos, ((uint64_t)k << 32) | u);
-      st_coh64(a.hq[hqi] + 2ull * pos + 1, am);
-    } else {
-      st_coh(&a.ctrl->abort, kAbortCapacity);
+#pragma unroll
+    for (int k = 0; k < kGroup; ++k) {
+      v[k] = nv[k];
+      nd[k] = nnd[k];
+      val[k] = nval[k];
     }
   }
 }
 
-// Frontier items [base, base + cnt), cnt <= kItems: lane k consumes item k's
-// mask and loads its row bounds; the distance rows of all the items are then
-// loaded together and parked in dl, and the items' edges are relaxed as one
-// flattened list, 64 per batch.  Heavy items are queued as chunks instead.
-__device__ __forceinline__ void process_items(const MArgs &a, const Sched &s, LaneSched &ls, uint32_t base,
-                                              DistSlots &dl, MultiCounters &mc, Pending &p) {
+// ---- filtered relaxation ----------------------------------------------------
+
+// Minimum / maximum over the wavefront's 64 lanes (DPP row shifts and
+// broadcasts: no LDS round trips).
+template <bool kMax>
+__device__ __forceinline__ int32_t wave_extreme(int32_t x) {
+  constexpr int32_t id = kMax ? -0x7FFFFFFF - 1 : 0x7FFFFFFF;
+#define LSG_DPP_STEP(ctrl, rows)                                                    \
+  {                                                                                 \
+    const int32_t y = __builtin_amdgcn_update_dpp(id, x, ctrl, rows, 0xf, false);   \
+    x = kMax ? max(x, y) : min(x, y);                                               \
+  }
+  LSG_DPP_STEP(0x111, 0xf)  // row_shr:1
+  LSG_DPP_STEP(0x112, 0xf)  // row_shr:2
+  LSG_DPP_STEP(0x114, 0xf)  // row_shr:4
+  LSG_DPP_STEP(0x118, 0xf)  // row_shr:8
+  LSG_DPP_STEP(0x142, 0xa)  // row_bcast:15
+  LSG_DPP_STEP(0x143, 0xc)  // row_bcast:31
+#undef LSG_DPP_STEP
+  return __builtin_amdgcn_readlane(x, kWave - 1);
+}
+
+// Lowest offset distance of an item over the lanes with `act` (distance du).
+__device__ __forceinline__ int32_t item_lowest(const LaneSched &ls, bool act, uint32_t du) {
+  const int32_t x = !act ? kNoBound : ls.incl ? (int32_t)du - ls.off : kPass;
+  return wave_extreme<false>(x);
+}
+
+// The bounds of every vertex with the offsets in a.flt: 64 consecutive rows
+// per wavefront and step, kSweepRows row loads in flight.
+constexpr int kSweepRows = 16;
+__device__ __forceinline__ void sweep_bounds(const MArgs &a, const LaneSched &ls, int32_t *bound, uint32_t wave,
+                                             uint32_t nwaves) {
+  const uint32_t lane = lane_id(), col = min(lane, a.S - 1);
+  for (uint64_t v0 = (uint64_t)wave * kWave; v0 < a.nnodes; v0 += (uint64_t)nwaves * kWave) {
+    int32_t mine = 0;
+    for (uint32_t r0 = 0; r0 < (uint32_t)kWave; r0 += kSweepRows) {
+      uint32_t d[kSweepRows];
+#pragma unroll
+      for (int k = 0; k < kSweepRows; ++k) {
+        const uint64_t v = v0 + r0 + k;
+        d[k] = ld_coh(a.D + (size_t)(v < a.nnodes ? v : a.nnodes - 1) * a.S + col);
+      }
+#pragma unroll
+      for (int k = 0; k < kSweepRows; ++k) {
+        const int32_t x = !ls.incl ? -kNoBound : d[k] == kInf ? kNoBound : (int32_t)d[k] - ls.off;
+        const int32_t m = wave_extreme<true>(x);
+        if (lane == r0 + k) mine = m;
+      }
+    }
+    if (v0 + lane < a.nnodes) st_coh((uint32_t *)bound + v0 + lane, (uint32_t)mine);
+  }
+}
+
+// Relaxes the first n <= 64 listed edges (lane i: destination pv, weight pw,
+// item slot pk), kGroup at a time, software-pipelined as relax_edges.
+__device__ __forceinline__ void relax_listed(const MArgs &a, const Sched &s, LaneSched &ls, const DistSlots &dl,
+                                             uint32_t pv, uint32_t pw, uint32_t pk, uint32_t n, Pending &p,
+                                             uint64_t &improved) {
   const uint32_t lane = lane_id();
-  const uint32_t cnt = min((uint32_t)kItems, s.in_count - base);
-  uint64_t *mp = s.aux[0] ? a.fmask[(s.phase - 1) & 1] : a.nmask[(s.round - 1) & 1];
+  const uint32_t col = min(lane, a.S - 1);
+  uint32_t v[kGroup], val[kGroup], nv[kGroup], nval[kGroup];
+  auto load = [&](uint32_t i, uint32_t(&vv)[kGroup], uint32_t(&x)[kGroup]) {
+#pragma unroll
+    for (int k = 0; k < kGroup; ++k) {
+      vv[k] = readlane(pv, min(i + k, n - 1));  // a slot past the list repeats its last edge, with no candidate
+      x[k] = ld_coh(a.D + (size_t)vv[k] * a.S + col);
+    }
+  };
+  load(0, v, val);
+  for (uint32_t i = 0; i < n; i += kGroup) {
+    if (i + kGroup < n) load(i + kGroup, nv, nval);
+    if (p.n > (uint32_t)(kWave - kGroup)) flush_pending(a, s, ls, p);
+    auto cand = [&](int k) {
+      const uint32_t j = min(i + k, n - 1);
+      return dl[readlane(pk, j)][lane] + (i + k < n ? readlane(pw, j) : 0x80000000u);
+    };
+    window_take(a, ls, v, cand, val, col, p, improved);
+#pragma unroll
+    for (int k = 0; k < kGroup; ++k) {
+      v[k] = nv[k];
+      val[k] = nval[k];
+    }
+  }
+}
+
+// Up to kItems items' edges as one flattened list [0, total): lane k's item
+// owns [end - degree, end), its edge f is CSR edge base + f, and its lowest
+// offset distance is low.
+struct Flat {
+  uint32_t total, end, base;
+  int32_t low;
+};
+
+// 64 edges of a flattened list, one per lane: destination, weight, item slot
+// and the item's lowest offset distance (lanes past the list repeat its last edge).
+struct FlatBatch {
+  uint32_t v, w, k;
+  int32_t low;
+};
+__device__ __forceinline__ void flat_load(const MArgs &a, const Flat &t, uint32_t b0, FlatBatch &x) {
+  const uint32_t f = min(b0 + lane_id(), t.total - 1);
+  uint32_t item = 0;  // the items that end at or before f
+#pragma unroll
+  for (int k = 0; k < kItems - 1; ++k) item += readlane(t.end, k) <= f ? 1u : 0u;
+  const uint32_t e = __shfl(t.base, item) + f;
+  x.v = glb(a.edge_dst)[e];
+  x.w = glb(a.edge_data)[e];
+  x.low = __shfl(t.low, item);
+  x.k = item;
+}
+
+// Relaxes a flattened list (total > 0).  The lanes take one edge each and test
+// it against its destination's bound; the edges that pass are collected in a
+// list of up to 64, one per lane, and relaxed from there.  Three batches of 64
+// are in flight: while one is tested and relaxed, the next one's bounds and
+// the edges of the one after it are being loaded.
+__device__ __forceinline__ void relax_filtered(const MArgs &a, const Sched &s, LaneSched &ls, const DistSlots &dl,
+                                               const Flat &t, Pending &p, uint64_t &improved) {
+  const uint32_t lane = lane_id();
+  uint32_t pv = 0, pw = 0, pk = 0, n = 0;
+  FlatBatch x0, x1, x2;
+  flat_load(a, t, 0, x0);
+  flat_load(a, t, kWave, x1);
+  int32_t bd0 = glb(ls.bound)[x0.v], bd1;
+  for (uint32_t b0 = 0;; b0 += kWave) {
+    uint64_t m = 0;
+    uint32_t c = 0;
+    if (b0 < t.total) {
+      flat_load(a, t, b0 + 2 * kWave, x2);
+      bd1 = glb(ls.bound)[x1.v];
+      // the saturated sum is below a bound exactly when the sum is
+      m = __ballot(b0 + lane < t.total && (x0.low == kPass || bd0 == kNoBound ||
+                                           __builtin_elementwise_add_sat(x0.low, (int32_t)x0.w) < bd0));
+      c = (uint32_t)__builtin_popcountll(m);
+    }
+    if (n && (b0 >= t.total || n + c > (uint32_t)kWave)) {
+      relax_listed(a, s, ls, dl, pv, pw, pk, n, p, improved);
+      n = 0;
+    }
+    if (b0 >= t.total) break;
+    if (c) {
+      // a permutation of the lanes: passing edges to n, n + 1, ..., the others behind them
+      const uint32_t to = ((m >> lane) & 1 ? n + lanes_below(m) : n + c + lanes_below(~m)) % kWave * 4;
+      const uint32_t tv = (uint32_t)__builtin_amdgcn_ds_permute((int)to, (int)x0.v);
+      const uint32_t tw = (uint32_t)__builtin_amdgcn_ds_permute((int)to, (int)x0.w);
+      const uint32_t tk = (uint32_t)__builtin_amdgcn_ds_permute((int)to, (int)x0.k);
+      if (lane >= n && lane < n + c) {
+        pv = tv;
+        pw = tw;
+        pk = tk;
+      }
+      n += c;
+    }
+    x0 = x1;
+    x1 = x2;
+    bd0 = bd1;
+  }
+}
+
+// Writes the staged heavy items' chunks to the next round's chunk queue, from
+// slot `base` on (reserved for ls.hchunks chunks).
+__device__ __forceinline__ void heavy_write(const MArgs &a, const Sched &s, LaneSched &ls, uint32_t base) {
+  uint64_t *const hq = a.hq[1u - s.heavy_in];
+  for (uint32_t i = 0; i < ls.hn; ++i) {
+    const HeavyItem h = ls.hb[i];
+    const uint32_t nch = __builtin_amdgcn_readfirstlane(h.nch);
+    for (uint32_t k = lane_id(); k < nch; k += kWave) {
+      const uint32_t pos = base + k;
+      if (pos < a.hcap) {
+        st_coh64(hq + 2ull * pos, ((uint64_t)k << 32) | h.u);
+        st_coh64(hq + 2ull * pos + 1, h.mask);
+      } else {
+        st_coh(&a.ctrl->abort, kAbortCapacity);
+      }
+    }
+    base += nch;
+  }
+  ls.hn = ls.hchunks = 0;
+}
+
+// Queues heavy vertex u (edges [rs, re)) as chunks of heavy_deg edges, each
+// expanded by a wavefront in the next round with the sources active now.
+__device__ __forceinline__ void queue_heavy(const MArgs &a, const Sched &s, LaneSched &ls, uint32_t u, uint32_t rs,
+                                            uint32_t re, uint64_t am) {
+  if (ls.hn == kHeavyBuf) {
+    uint32_t base = 0;
+    if (lane_id() == 0) base = atomic_add(&a.ctrl->hcount[1u - s.heavy_in], ls.hchunks);
+    heavy_write(a, s, ls, readlane(base, 0));
+  }
+  const uint32_t nch = (re - rs + a.heavy_deg - 1) / a.heavy_deg;
+  if (lane_id() == 0) ls.hb[ls.hn] = HeavyItem{u, nch, am};
+  ls.hn += 1;
+  ls.hchunks += nch;
+}
+
+// One work unit, up to kItems items: frontier items [base, base + cnt), cnt <=
+// per, or, with `chunks`, that many of the round's heavy chunks (heavy_deg
+// edges of a vertex, for the sources recorded with the chunk).  Lane k consumes
+// item k's mask and loads its row bounds; the distance rows of all the items
+// are then loaded together and parked in dl.  Heavy items are queued as
+// chunks for the next round; the others are relaxed (items of kLongDeg edges
+// and more one by one, the rest as one flattened list, 64 edges per batch) or,
+// with kFilter, returned as one flattened list.
+template <bool kFilter>
+__device__ __forceinline__ Flat process_unit(const MArgs &a, const Sched &s, LaneSched &ls, bool chunks, uint32_t base,
+                                             uint32_t per, DistSlots &dl, RoundCounters &mc, Pending &p) {
+  const uint32_t lane = lane_id();
+  const uint32_t cnt = min(per, (chunks ? s.heavy_count : s.in_count) - base);
   uint32_t u = a.nnodes;
-  if (lane < cnt) u = ld_coh(a.q[s.in_q] + base + lane);
   uint64_t m = 0;
   uint32_t rs = 0, re = 0;
-  if (u < a.nnodes) {
-    m = atomic_exch64(mp + u, 0ull);
-    // Gauss-Seidel pop: the bits set for the next round so far are expanded
-    // now, with the distances that set them; u stays queued for the next round.
-    m |= atomic_exch64(a.nmask[s.round & 1] + u, 0ull);
-    rs = glb(a.row_start)[u];
-    re = glb(a.row_start)[u + 1];
+  if (chunks) {
+    uint32_t ck = 0;
+    if (lane < cnt) {
+      const uint64_t *const ent = a.hq[s.heavy_in] + 2ull * (base + lane);
+      const uint64_t uk = ld_coh64(ent);
+      m = ld_coh64(ent + 1);
+      u = (uint32_t)uk;
+      ck = (uint32_t)(uk >> 32);
+    }
+    if (u < a.nnodes) {
+      rs = glb(a.row_start)[u] + ck * a.heavy_deg;
+      re = min(glb(a.row_start)[u + 1], rs + a.heavy_deg);
+    } else {
+      m = 0;
+    }
+  } else {
+    uint64_t *mp = s.aux[0] ? a.fmask[(s.phase - 1) & 1] : a.nmask[(s.round - 1) & 1];
+    if (lane < cnt) u = ld_coh(a.q[s.in_q] + base + lane);
+    if (u < a.nnodes) {
+      m = atomic_exch64(mp + u, 0ull);
+      // Gauss-Seidel pop: the bits set for the next round so far are expanded
+      // now, with the distances that set them; u stays queued for the next round.
+      m |= atomic_exch64(a.nmask[s.round & 1] + u, 0ull);
+      rs = glb(a.row_start)[u];
+      re = glb(a.row_start)[u + 1];
+    }
   }
   // The row loads depend on the exchanged masks, so each reads a distance at
   // least as new as the improvements that set the consumed bits.
@@ -398,42 +663,58 @@ __device__ __forceinline__ void process_items(const MArgs &a, const Sched &s, La
     const uint32_t uk = readlane(u, k);
     du[k] = lane < a.S && ((mk >> lane) & 1) ? ld_coh(a.D + (size_t)uk * a.S + lane) : kInf;
   }
-  const bool split = s.aux[0] && s.aux[1];
-  uint32_t mydeg = 0;  // lane k: edges of item k to relax in the flattened list
-  uint32_t longm = 0;  // items relaxed one by one (degree >= kLongDeg)
+  uint64_t am = 0;         // lane k: sources that expand item k
+  int32_t low = kNoBound;  // lane k: item k's lowest offset distance (filtered rounds)
 #pragma unroll
   for (int k = 0; k < kItems; ++k) {
-    bool act = du[k] != kInf;
-    if (__ballot(act) == 0) continue;
-    if (split) {
-      // Split / bucket far pile: a source whose distance is still above this
-      // phase's threshold (shared, or its own in a bucket phase) waits for a
-      // later phase instead of expanding early.
-      const bool defer = act && (ls.bucket ? du[k] > ls.thr : (int64_t)du[k] > s.curdelta());
+    dl[k][lane] = du[k];
+    const uint64_t b = __ballot(du[k] != kInf);
+    int32_t x = 0;
+    if (kFilter) x = item_lowest(ls, du[k] != kInf, du[k]);
+    if (lane == (uint32_t)k) {
+      am = b;
+      low = x;
+    }
+  }
+  if (s.aux[0] && s.aux[1] && !chunks) {
+    // Split / bucket far pile: a source whose distance is still above this
+    // phase's threshold (shared, or its own in a bucket phase) waits for a
+    // later phase instead of expanding early.
+    for (uint32_t k = 0; k < cnt; ++k) {
+      const uint32_t d = dl[k][lane];
+      const bool defer = d != kInf && (ls.bucket ? d > ls.thr : (int64_t)d > s.curdelta());
       const uint64_t dm = __ballot(defer);
-      if (dm) {
-        const uint32_t uk = readlane(u, k);
-        bool push = false;
-        if (lane == 0) push = atomic_or64(a.fmask[s.phase & 1] + uk, dm) == 0;
-        pile_push(a, s, ls, 1, push, uk);
-        if (defer) ls.fmin = min(ls.fmin, du[k]);
-        act = act && !defer;
+      if (dm == 0) continue;
+      const uint32_t uk = readlane(u, k);
+      bool push = false;
+      if (lane == 0) push = atomic_or64(a.fmask[s.phase & 1] + uk, dm) == 0;
+      pile_push(a, s, ls, 1, push, uk);
+      if (defer) {
+        ls.fmin = min(ls.fmin, d);
+        dl[k][lane] = kInf;
+      }
+      int32_t x = 0;
+      if (kFilter) x = item_lowest(ls, d != kInf && !defer, d);
+      if (lane == k) {
+        am &= ~dm;
+        low = x;
       }
     }
-    const uint64_t am = __ballot(act);
-    if (am == 0) continue;
-    const uint32_t rsk = readlane(rs, k), rek = readlane(re, k);
-    if (rek - rsk >= a.heavy_deg) {
-      queue_heavy(a, s, readlane(u, k), rsk, rek, am);
-      continue;
-    }
-    if (rek == rsk) continue;
-    dl[k][lane] = act ? du[k] : kInf;
-    mc.lane_items += __builtin_popcountll(am);
-    mc.edges += rek - rsk;
-    if (rek - rsk >= kLongDeg) longm |= 1u << k;
-    else if (lane == (uint32_t)k) mydeg = rek - rsk;
   }
+  const uint32_t deg = am ? re - rs : 0u;  // lane k: edges of item k
+  const bool heavy = !chunks && deg >= a.heavy_deg;
+  for (uint64_t hm = __ballot(heavy); hm; hm &= hm - 1) {
+    const uint32_t k = (uint32_t)__builtin_ctzll(hm);
+    queue_heavy(a, s, ls, readlane(u, k), readlane(rs, k), readlane(re, k), bcast64(am, k));
+  }
+  const uint32_t now = heavy ? 0u : deg;  // relaxed in this round
+  if (now) {
+    mc.lane_items += __builtin_popcountll(am);
+    mc.edges += now;
+  }
+  // items relaxed one by one (degree >= kLongDeg); the others as a flattened list
+  const uint32_t longm = kFilter ? 0u : (uint32_t)__ballot(now >= kLongDeg);
+  const uint32_t mydeg = kFilter || now < kLongDeg ? now : 0u;
   // Inclusive prefix of the items' edge counts over lanes 0..kItems-1: item k
   // owns flattened edges [end_k - deg_k, end_k).
   uint32_t end = mydeg;
@@ -444,6 +725,7 @@ __device__ __forceinline__ void process_items(const MArgs &a, const Sched &s, La
   }
   const uint32_t total = readlane(end, kItems - 1);
   const uint32_t first = end - mydeg;
+  if (kFilter) return Flat{total, end, rs - first, low};
   for (uint32_t b0 = 0; b0 < total; b0 += kWave) {
     const uint32_t f = b0 + lane;
     // the item holding flattened edge f is the number of items ending at or before f
@@ -462,28 +744,7 @@ __device__ __forceinline__ void process_items(const MArgs &a, const Sched &s, La
     const uint32_t k = (uint32_t)__builtin_ctz(lm);
     relax_edges(a, s, ls, dl[k][lane], readlane(rs, k), readlane(re, k), p, mc.improved);
   }
-}
-
-// Heavy chunk c: edges [k * heavy_deg, (k + 1) * heavy_deg) of u, for the
-// sources recorded with the chunk.
-__device__ __forceinline__ void process_chunk(const MArgs &a, const Sched &s, LaneSched &ls, uint32_t c,
-                                              MultiCounters &mc, Pending &p) {
-  const uint32_t lane = lane_id();
-  uint64_t ent = ld_coh64(a.hq[s.heavy_in] + 2ull * c);
-  uint64_t m = ld_coh64(a.hq[s.heavy_in] + 2ull * c + 1);
-  uint32_t u = (uint32_t)ent, k = (uint32_t)(ent >> 32);
-  if (u >= a.nnodes) return;
-  uint32_t rs = glb(a.row_start)[u], re = glb(a.row_start)[u + 1];
-  if ((uint64_t)k * a.heavy_deg >= re - rs) return;
-  uint32_t lo = rs + k * a.heavy_deg, hi = min(re, lo + a.heavy_deg);
-  bool act = lane < a.S && ((m >> lane) & 1);
-  uint32_t du = act ? ld_coh(a.D + (size_t)u * a.S + lane) : kInf;
-  act = act && du != kInf;
-  uint64_t am = __ballot(act);
-  if (am == 0) return;
-  mc.lane_items += __builtin_popcountll(am);
-  mc.edges += hi - lo;
-  relax_edges(a, s, ls, act ? du : kInf, lo, hi, p, mc.improved);
+  return Flat{0, 0, 0, 0};
 }
 
 // Leader step, run by every thread of the last block to reach the barrier:
@@ -491,14 +752,19 @@ __device__ __forceinline__ void process_chunk(const MArgs &a, const Sched &s, La
 // plus, at each phase boundary, the learned scheduler's choice of the next
 // phase's delta width and far-pile mode.  Schedule words: aux[0] = the
 // in-queue is the far pile, aux[1] = far mode of this phase (LSG_FAR_*).
-__device__ __forceinline__ void multi_leader(const MArgs &a, MultiCounters *tot) {
+__device__ __forceinline__ void multi_leader(const MArgs &a) {
   __shared__ Sched s;
   __shared__ SchedFeatures f;
   __shared__ MlpScratch sc;
   __shared__ uint32_t phase_end, consumed;
   __shared__ uint64_t phases_seen;
+  __shared__ uint64_t edges_now;
   Ctrl *c = a.ctrl;
   const uint32_t t = threadIdx.x;
+  // the hub's distances, for the filter's offsets (beside the loads below)
+  const uint32_t hub_d = t < a.S && ld_coh(&a.flt->on) ? ld_coh(a.D + (size_t)ld_coh(&a.flt->hub) * a.S + t) : kInf;
+  // every wavefront has left the round's item loops: restart the tickets
+  if (t < kGroups) st_coh(&a.tickets[t].ticket, 0u);
   if (t == 0) {
     // every control word of the step in one batch of loads (the schedule to
     // registers first, so that the other loads need not wait for LDS stores)
@@ -506,11 +772,15 @@ __device__ __forceinline__ void multi_leader(const MArgs &a, MultiCounters *tot)
     sched_load(sr, &c->s);
     CtrlCounts k;
     counts_load(k, c);
-    const uint64_t tot_lane_items = ld_coh64(&tot->lane_items), tot_edges = ld_coh64(&tot->edges);
+    uint64_t tot_lane_items = 0, tot_edges = 0;
+#pragma unroll
+    for (uint32_t g = 0; g < kGroups; ++g) {
+      tot_lane_items += ld_coh64(&a.tot[g].lane_items);
+      tot_edges += ld_coh64(&a.tot[g].edges);
+    }
     s = sr;
-    // every wavefront has left the round's item loops: restart the tickets
-    st_coh(&c->ticket, 0u);
-    st_coh(&c->ticket2, 0u);
+    s.aux[3] = 0;
+    edges_now = tot_edges;
     const uint32_t nnear = k.q(s.near_q), nfar = k.q(s.far_q), nheavy = k.h(1u - s.heavy_in);
     phase_end = 0;
     phases_seen = k.phases;
@@ -566,6 +836,22 @@ __device__ __forceinline__ void multi_leader(const MArgs &a, MultiCounters *tot)
     }
   }
   __syncthreads();
+  // Another sweep, once three quarters of the sources have reached the hub:
+  // the next round begins with it, with the hub's distances as offsets.
+  if (t < (uint32_t)kWave && s.aux[2] < (uint32_t)kSweeps) {
+    const uint64_t fin = __ballot(hub_d != kInf);
+    if (4u * (uint32_t)__builtin_popcountll(fin) >= 3u * a.S &&
+        edges_now - ld_coh64(&a.flt->last_edges) >= a.nedges / 2) {
+      st_coh((uint32_t *)&a.flt->off[t], hub_d != kInf ? hub_d : 0u);
+      if (t == 0) {
+        st_coh64(&a.flt->incl, fin);
+        st_coh64(&a.flt->last_edges, edges_now);
+        s.aux[2] += 1;
+        s.aux[3] = 1;
+      }
+    }
+  }
+  __syncthreads();
   if (!phase_end) {
     if (t == 0) sched_store(&c->s, s);
     return;
@@ -613,15 +899,29 @@ __device__ __forceinline__ void multi_leader(const MArgs &a, MultiCounters *tot)
   }
 }
 
-template <int BS>
+__device__ __forceinline__ uint64_t wave_sum(uint64_t x) {
+#pragma unroll
+  for (int d = kWave / 2; d >= 1; d >>= 1) x += __shfl_xor((unsigned long long)x, d);
+  return x;
+}
+
+// Blocks of group g in a grid of nb.
+__device__ __forceinline__ uint32_t group_blocks(uint32_t nb, uint32_t g) { return (nb + kGroups - 1 - g) / kGroups; }
+
+// kFilter: the rounds from the first sweep on, whose edges are all tested
+// against the bounds; the other variant runs the rounds before, and returns
+// when a sweep has been ordered.  (One kernel with both edge loops spilled
+// 170 VGPRs.)
+template <int BS, bool kFilter>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kMultiWaves, kMultiWaves)))
-void multi_kernel(MArgs a, MultiCounters *tot) {
+void multi_kernel(MArgs a) {
   __shared__ Sched ss;
   __shared__ uint32_t quit;
   __shared__ unsigned long long blk[3];
   __shared__ DistSlots dls[BS / kWave];
   __shared__ uint32_t pushbuf[BS / kWave][2 * kPushBuf];
-  __shared__ uint32_t drain_n[BS / kWave][2], drain_base[2];
+  __shared__ HeavyItem heavybuf[BS / kWave][kHeavyBuf];
+  __shared__ uint32_t drain_n[BS / kWave][3], drain_base[3];  // near, far, heavy chunks
   Ctrl *c = a.ctrl;
   const uint32_t nb = gridDim.x;
   if (!residency_handshake(c, nb, a.residency_limit)) return;
@@ -633,13 +933,13 @@ void multi_kernel(MArgs a, MultiCounters *tot) {
       Sched s;
       sched_load(s, &c->s);
       ss = s;
-      quit = s.done || ld_coh(&c->abort) != kAbortNone;
+      quit = s.done || (!kFilter && s.aux[3]) || ld_coh(&c->abort) != kAbortNone;
       blk[0] = blk[1] = blk[2] = 0;
     }
     __syncthreads();
     if (quit) break;
     const Sched s = ss;
-    MultiCounters mc = {0, 0, 0};
+    RoundCounters mc = {0, 0, 0};
     LaneSched ls;
     ls.bucket = s.aux[1] == LSG_FAR_BUCKET;
     ls.thr = ls.bucket && lane_id() < a.S ? ld_coh(a.thr + lane_id()) : 0u;
@@ -647,49 +947,80 @@ void multi_kernel(MArgs a, MultiCounters *tot) {
     ls.fmin = kInf;
     ls.pb = &pushbuf[threadIdx.x / kWave][0];
     ls.pbn[0] = ls.pbn[1] = 0;
+    ls.hb = heavybuf[threadIdx.x / kWave];
+    ls.hn = ls.hchunks = 0;
+    ls.bound = nullptr;
+    ls.off = 0;
+    ls.incl = false;
+    if (kFilter) {
+      int32_t *const bound = s.aux[2] == 1 ? a.bound[0] : s.aux[2] == 2 ? a.bound[1] : a.bound[2];
+      ls.bound = bound;
+      ls.off = (int32_t)ld_coh((const uint32_t *)&a.flt->off[lane_id()]);
+      ls.incl = (ld_coh64(&a.flt->incl) >> lane_id()) & 1;
+      if (s.aux[3]) {
+        sweep_bounds(a, ls, bound, wave, nwaves);
+        grid_barrier_block(c, nb, a.spin_limit, [] {});
+      }
+    }
     Pending p;
     p.n = 0;
     p.v = p.nb_lo = p.nb_hi = p.fb_lo = p.fb_hi = 0;
     DistSlots &dl = dls[threadIdx.x / kWave];
-    // Static first pass (ticket = wavefront id), then dynamic tickets; the
-    // next ticket is fetched while the current one is processed.
-    const uint32_t nchunks = (s.in_count + kItems - 1) / kItems;
-    // A ticket covers kSpan consecutive work units; the next ticket is taken
-    // when the last unit of the current range starts.
-    for (uint32_t ck = wave, cend = wave + 1; ck < nchunks;) {
-      const bool last = ck + 1 >= cend;
-      uint32_t t = 0;
-      if (last && lane_id() == 0) t = atomic_add(&c->ticket, 1u);
-      process_items(a, s, ls, ck * kItems, dl, mc, p);
-      if (last) {
-        ck = nwaves + readlane(t, 0) * kSpan;
-        cend = ck + kSpan;
-      } else {
-        ++ck;
+    // Work units: first the in-queue's items, `per` at a time (fewer than
+    // kItems where that would leave wavefronts idle), then the heavy chunks.
+    // Unit j * kGroups + g belongs to group g; its wavefronts take one each,
+    // then kSpan per ticket (the next ticket is fetched while the last unit of
+    // the current one is processed), and at the end help other groups.
+    const uint32_t per = min((uint32_t)kItems, max(1u, (s.in_count + nwaves - 1) / nwaves));
+    const uint32_t hper = min(min((uint32_t)kItems, max(1u, kChunkUnit / a.heavy_deg)),
+                              max(1u, (s.heavy_count + nwaves - 1) / nwaves));
+    const uint32_t nitems = (s.in_count + per - 1) / per;
+    const uint32_t nunits = nitems + (s.heavy_count + hper - 1) / hper;
+    uint32_t g = blockIdx.x % kGroups;
+    uint32_t j = blockIdx.x / kGroups * wpb + threadIdx.x / kWave, jend = j + 1;
+    for (;;) {
+      const uint32_t u = j * kGroups + g;
+      if (u < nunits) {
+        const bool last = j + 1 >= jend && nunits > nwaves;
+        uint32_t t = 0;
+        if (last && lane_id() == 0) t = atomic_add(&a.tickets[g].ticket, 1u);
+        const bool chunks = u >= nitems;
+        const Flat f = process_unit<kFilter>(a, s, ls, chunks, chunks ? (u - nitems) * hper : u * per,
+                                             chunks ? hper : per, dl, mc, p);
+        if (kFilter && f.total) relax_filtered(a, s, ls, dl, f, p, mc.improved);
+        if (last) {
+          j = group_blocks(nb, g) * wpb + readlane(t, 0) * kSpan;
+          jend = j + kSpan;
+        } else {
+          ++j;
+          if (nunits <= nwaves) break;
+        }
+        continue;
       }
-    }
-    for (uint32_t ck = wave, cend = wave + 1; ck < s.heavy_count;) {
-      const bool last = ck + 1 >= cend;
+      if (nunits <= nwaves) break;
+      // this group's units are taken: the next group that has some left
+      const uint32_t og = (g + 1 + lane_id()) % kGroups;
+      const uint32_t oj = group_blocks(nb, og) * wpb + ld_coh(&a.tickets[og].ticket) * kSpan;
+      const uint64_t left = __ballot(lane_id() < kGroups && oj * kGroups + og < nunits);
+      if (left == 0) break;
+      g = (g + 1 + (uint32_t)__builtin_ctzll(left)) % kGroups;
       uint32_t t = 0;
-      if (last && lane_id() == 0) t = atomic_add(&c->ticket2, 1u);
-      process_chunk(a, s, ls, ck, mc, p);
-      if (last) {
-        ck = nwaves + readlane(t, 0) * kSpan;
-        cend = ck + kSpan;
-      } else {
-        ++ck;
-      }
+      if (lane_id() == 0) t = atomic_add(&a.tickets[g].ticket, 1u);
+      j = group_blocks(nb, g) * wpb + readlane(t, 0) * kSpan;
+      jend = j + kSpan;
     }
     flush_pending(a, s, ls, p);
     // this wavefront's smallest far push per source -> phase minimum
     if (__ballot(ls.fmin != kInf) && ls.fmin != kInf) atomic_min(a.fmin + (s.phase & 1) * 64 + lane_id(), ls.fmin);
     const uint32_t wv = threadIdx.x / kWave;
+    const uint64_t lane_items = wave_sum(mc.lane_items), edges = wave_sum(mc.edges);
     if (lane_id() == 0) {
       drain_n[wv][0] = ls.pbn[0];
       drain_n[wv][1] = ls.pbn[1];
-      if (mc.lane_items | mc.edges) {
-        atomicAdd(&blk[0], (unsigned long long)mc.lane_items);
-        atomicAdd(&blk[1], (unsigned long long)mc.edges);
+      drain_n[wv][2] = ls.hchunks;
+      if (lane_items | edges) {
+        atomicAdd(&blk[0], (unsigned long long)lane_items);
+        atomicAdd(&blk[1], (unsigned long long)edges);
         atomicAdd(&blk[2], (unsigned long long)mc.improved);
       }
     }
@@ -697,7 +1028,7 @@ void multi_kernel(MArgs a, MultiCounters *tot) {
     // The block's staged pushes get their places with one queue-tail atomic
     // per pile (one per wavefront, 4096 on one tail, serialise for ~50 us at
     // the memory-side atomic unit every round).
-    if (threadIdx.x < 2) {
+    if (threadIdx.x < 3) {
       const uint32_t which = threadIdx.x;
       uint32_t tot_n = 0;
       for (uint32_t w = 0; w < BS / kWave; ++w) {
@@ -705,9 +1036,11 @@ void multi_kernel(MArgs a, MultiCounters *tot) {
         drain_n[w][which] = tot_n;  // becomes the wavefront's offset
         tot_n += n;
       }
-      drain_base[which] = tot_n ? atomic_add(&c->qcount[which ? s.far_q : s.near_q], tot_n) : 0u;
+      uint32_t *const tail = which == 2 ? &c->hcount[1u - s.heavy_in] : &c->qcount[which ? s.far_q : s.near_q];
+      drain_base[which] = tot_n ? atomic_add(tail, tot_n) : 0u;
     }
     if (threadIdx.x == 0 && (blk[0] | blk[1])) {
+      MultiCounters *const tot = a.tot + blockIdx.x % kGroups;
       __hip_atomic_fetch_add(&tot->lane_items, (uint64_t)blk[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_fetch_add(&tot->edges, (uint64_t)blk[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_fetch_add(&tot->improved, (uint64_t)blk[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -726,12 +1059,13 @@ void multi_kernel(MArgs a, MultiCounters *tot) {
         else st_coh(&a.ctrl->abort, kAbortCapacity);
       }
     }
-    grid_barrier_block(c, nb, a.spin_limit, [&] { multi_leader(a, tot); });
+    if (ls.hn) heavy_write(a, s, ls, drain_base[2] + drain_n[wv][2]);
+    grid_barrier_block(c, nb, a.spin_limit, [&] { multi_leader(a); });
   }
 }
 
 // D[v][s] = INF, masks cleared.
-__global__ void multi_init(MArgs a, MultiCounters *tot) {
+__global__ void multi_init(MArgs a) {
   size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
   size_t cells = (size_t)a.nnodes * a.S;
   for (size_t i = tid; i < cells; i += nt) a.D[i] = kInf;
@@ -742,7 +1076,22 @@ __global__ void multi_init(MArgs a, MultiCounters *tot) {
     a.fmask[1][v] = 0;
     a.qstamp[v] = 0;
   }
-  if (tid == 0) *tot = MultiCounters{0, 0, 0};
+  if (tid < kGroups) {
+    a.tot[tid] = MultiCounters{0, 0, 0};
+    a.tickets[tid].ticket = 0;
+  }
+  // the block's vertex of largest out-degree (lowest id on ties)
+  __shared__ unsigned long long best;
+  if (threadIdx.x == 0) best = 0;
+  __syncthreads();
+  uint64_t mine = 0;
+  for (size_t v = tid; v < a.nnodes; v += nt) {
+    const uint64_t x = (uint64_t)(a.row_start[v + 1] - a.row_start[v]) << 32 | (uint32_t)~(uint32_t)v;
+    mine = x > mine ? x : mine;
+  }
+  atomicMax(&best, (unsigned long long)mine);
+  __syncthreads();
+  if (threadIdx.x == 0) a.hubs[blockIdx.x] = best;
 }
 
 // Seeds every source (apps/sssp/kernel.cu:33,476-477) and the control block.
@@ -760,15 +1109,23 @@ __global__ void multi_seed(MArgs a) {
   uint64_t pm = __ballot(push);
   if (push) a.q[0][lanes_below(pm)] = src;
   ctrl_reset_barrier(a.ctrl, lane, kWave);
+  uint64_t hub = 0;
+  for (uint32_t i = lane; i < a.ninit; i += kWave) hub = a.hubs[i] > hub ? a.hubs[i] : hub;
+#pragma unroll
+  for (int d = kWave / 2; d >= 1; d >>= 1) {
+    const uint64_t x = __shfl_xor((unsigned long long)hub, d);
+    hub = x > hub ? x : hub;
+  }
   if (lane == 0) {
+    a.flt->hub = ~(uint32_t)hub;
+    a.flt->on = (hub >> 32) * a.nnodes >= (uint64_t)kHubRatio * a.nedges && a.nedges;
+    a.flt->incl = a.flt->last_edges = 0;
     Ctrl *c = a.ctrl;
     c->qcount[0] = (uint32_t)__builtin_popcountll(pm);
     c->qcount[1] = 0;
     c->qcount[2] = 0;
     c->hcount[0] = 0;
     c->hcount[1] = 0;
-    c->ticket = 0;
-    c->ticket2 = 0;
     c->abort = kAbortNone;
     c->checkin = 0;
     c->resident_seen = 0;
@@ -821,14 +1178,21 @@ __global__ void multi_expand(const uint32_t *Dc, uint32_t Sc, const int32_t *col
     if (lane < S) D[v * S + lane] = c >= 0 ? Dc[v * Sc + (uint32_t)c] : (v == sv ? 0u : kInf);
 }
 
-using MultiFn = void (*)(MArgs, MultiCounters *);
+using MultiFn = void (*)(MArgs);
 
+template <bool kFilter>
 static MultiFn pick_multi(int bs) {
   switch (bs) {
-    case 256: return multi_kernel<256>;
-    case 1024: return multi_kernel<1024>;
-    default: return multi_kernel<512>;
+    case 256: return multi_kernel<256, kFilter>;
+    case 1024: return multi_kernel<1024, kFilter>;
+    default: return multi_kernel<512, kFilter>;
   }
+}
+
+// Between the two kernels: the barrier and residency words start again.
+__global__ void multi_switch(Ctrl *c) {
+  ctrl_reset_barrier(c, threadIdx.x, blockDim.x);
+  if (threadIdx.x == 0) c->checkin = 0;
 }
 
 struct MultiRun {
@@ -843,16 +1207,19 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
   int rc;
   int bs = o.block_size ? o.block_size : 512;
   if (bs != 256 && bs != 512 && bs != 1024) return fail(LSG_ERR_ARG, "block_size must be 256, 512 or 1024");
-  // default chunk size, measured on RMAT-22 x 64 sources: 512 30.0 ms, 256
-  // 34.3, 1024 30.6, 128 63
-  uint32_t heavy_deg = o.heavy_deg > 0 ? (uint32_t)o.heavy_deg : 512u;
+  // Default chunk size: short chunks spread a small graph's edges over the
+  // wavefronts, long ones cost a large graph fewer units (ms at 64 / 256 / 512
+  // edges: RMAT of 131072 vertices x 64 sources 2.2 / 2.6 / 2.8, 2^19 3.6 /
+  // 3.6 / 4.8, 2^20 4.8 / 4.7 / 4.9, 2^21 8.2 / 7.9 / 7.7, 2^22 15.6 / 13.5 / 13.7;
+  // 524288 x 33 at delta 32 14.7 / 16.9 / 23.1).
+  uint32_t heavy_deg = o.heavy_deg > 0 ? (uint32_t)o.heavy_deg : g->nedges < (1u << 24) ? 64u : 256u;
   if (heavy_deg < kLongDeg) return fail(LSG_ERR_ARG, "heavy_deg must be >= %u for batched runs", kLongDeg);
   uint32_t V = g->nnodes;
   uint64_t hcap64 = 2ull * g->nedges / heavy_deg + 64;
   uint32_t hcap = (uint32_t)std::min<uint64_t>(hcap64, UINT32_MAX / 4);
   void *qbuf, *hbuf, *mbuf, *sbuf;
   if ((rc = ws_buffer(w, kBufQueues, 3ull * V * 4, &qbuf)) || (rc = ws_buffer(w, kBufHeavy, 2ull * hcap * 16, &hbuf)) ||
-      (rc = ws_buffer(w, kBufMasks, 4ull * V * 8 + 4ull * V + 256, &mbuf)) || (rc = ws_buffer(w, kBufSeeds, 2048, &sbuf)))
+      (rc = ws_buffer(w, kBufMasks, (4ull * 8 + 4 + 4 * kSweeps) * V + 16ull * w->cus * 8 + 256, &mbuf)) || (rc = ws_buffer(w, kBufSeeds, 2048 + kGroups * (sizeof(TicketGroup) + sizeof(MultiCounters)), &sbuf)))
     return rc;
   MArgs a;
   memset(&a, 0, sizeof a);
@@ -866,6 +1233,9 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
   a.fmask[0] = masks + 2ull * V;
   a.fmask[1] = masks + 3ull * V;
   a.qstamp = (uint32_t *)(masks + 4ull * V);
+  for (int i = 0; i < kSweeps; ++i) a.bound[i] = (int32_t *)(masks + 4ull * V) + (1ull + i) * V;
+  a.hubs = (uint64_t *)(((uintptr_t)(a.bound[kSweeps - 1] + V) + 7) & ~(uintptr_t)7);
+  a.ninit = (uint32_t)std::min<uint64_t>(((uint64_t)V * nsrc + 255) / 256, 16ull * w->cus);
   for (int i = 0; i < 3; ++i) a.q[i] = (uint32_t *)qbuf + (size_t)i * V;
   a.hq[0] = (uint64_t *)hbuf;
   a.hq[1] = (uint64_t *)hbuf + 2ull * hcap;
@@ -880,9 +1250,11 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
   a.spin_limit = spin_limit_ticks(w);
   a.residency_limit = residency_limit_ticks(w);
   a.nedges = g->nedges;
-  MultiCounters *tot = (MultiCounters *)((char *)sbuf + 256);
   a.fmin = (uint32_t *)((char *)sbuf + 512);
   a.thr = (uint32_t *)((char *)sbuf + 1024);
+  a.flt = (Filter *)((char *)sbuf + 1280);
+  a.tickets = (TicketGroup *)((char *)sbuf + 2048);
+  a.tot = (MultiCounters *)(a.tickets + kGroups);
   if (o.sched) {
     a.sched = 1;
     a.mlp = sched_model_device(w->device, LSG_SCHED_BATCHED);
@@ -901,18 +1273,21 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
     a.feat = (float *)((char *)tbuf + tbytes);
   }
   HIPCHK(hipMemcpyAsync(sbuf, srcs_host, nsrc * 4, hipMemcpyHostToDevice, w->stream));
-  MultiFn fn = pick_multi(bs);
-  int grid = 0;
-  if ((rc = resident_grid(w, (const void *)fn, bs, &grid))) return rc;
+  const MultiFn fn = pick_multi<false>(bs), ffn = pick_multi<true>(bs);
+  int grid = 0, fgrid = 0;
+  if ((rc = resident_grid(w, (const void *)fn, bs, &grid)) || (rc = resident_grid(w, (const void *)ffn, bs, &fgrid)))
+    return rc;
+  grid = std::min(grid, fgrid);
   if (o.grid_blocks > 0) grid = std::min(o.grid_blocks, grid);
   Ctrl hc;
   float ms = 0;
   for (int attempt = 0;; ++attempt) {
-    uint32_t init_blocks = (uint32_t)std::min<uint64_t>(((uint64_t)V * nsrc + 255) / 256, 16ull * w->cus);
     auto enqueue = [&]() -> int {
-      hipLaunchKernelGGL(multi_init, dim3(init_blocks), dim3(256), 0, w->stream, a, tot);
+      hipLaunchKernelGGL(multi_init, dim3(a.ninit), dim3(256), 0, w->stream, a);
       hipLaunchKernelGGL(multi_seed, dim3(1), dim3(64), 0, w->stream, a);
-      hipLaunchKernelGGL(fn, dim3(grid), dim3(bs), 0, w->stream, a, tot);
+      hipLaunchKernelGGL(fn, dim3(grid), dim3(bs), 0, w->stream, a);
+      hipLaunchKernelGGL(multi_switch, dim3(1), dim3(128), 0, w->stream, w->ctrl);
+      hipLaunchKernelGGL(ffn, dim3(grid), dim3(bs), 0, w->stream, a);
       HIPCHK(hipGetLastError());
       return LSG_OK;
     };
@@ -920,7 +1295,6 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
     if (o.graph_launch) {
       std::vector<uint8_t> key;
       key_append(key, a);
-      key_append(key, tot);
       key_append(key, grid);
       key_append(key, bs);
       if ((rc = launch_captured(w, key, enqueue))) return rc;
@@ -937,13 +1311,19 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
                   hc.resident_seen);
     grid = (int)hc.resident_seen;
     record_resident_grid(w, (const void *)fn, bs, grid);
+    record_resident_grid(w, (const void *)ffn, bs, grid);
   }
   if (hc.abort == kAbortTimeout)
     return fail(LSG_ERR_TIMEOUT, "grid barrier timed out (grid %d x %d) at round %u; distances are incomplete",
                 grid, bs, hc.s.round);
   if (hc.abort == kAbortCapacity) return fail(LSG_ERR_CAPACITY, "device queue capacity exceeded");
-  MultiCounters ht;
-  HIPCHK(hipMemcpy(&ht, tot, sizeof ht, hipMemcpyDeviceToHost));
+  MultiCounters tg[kGroups], ht = {0, 0, 0};
+  HIPCHK(hipMemcpy(tg, a.tot, sizeof tg, hipMemcpyDeviceToHost));
+  for (const MultiCounters &t : tg) {
+    ht.lane_items += t.lane_items;
+    ht.edges += t.edges;
+    ht.improved += t.improved;
+  }
   if (o.trace) {
     uint32_t n = (uint32_t)std::min<uint64_t>(hc.stat_rounds, a.trace_cap);
     w->last_trace.resize(n);

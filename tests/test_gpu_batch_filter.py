@@ -1,0 +1,75 @@
+"""The batched kernel's edge filter against the oracle's Dijkstra, exact in every column.
+
+The filter tests an edge against a bound per vertex and is used on graphs with
+a hub, once three quarters of the sources have reached it.  The cases are
+where that can go wrong: few and many sources, sources that never reach the
+hub, weights of zero and near INT_MAX (sums that saturate), every far mode,
+chunk sizes at both ends, graphs whose size is no multiple of a wavefront.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from galoisgpu_amd import CSRGraph, Options
+from galoisgpu_amd.batch import sssp_multi
+
+pytestmark = pytest.mark.gpu
+
+INT_MAX = 0x7FFFFFFF
+
+
+def hub_graph(n, seed, whi, wlo=0):
+    """A hub with edges to and from a third of the vertices, random edges besides, and a part cut off from the hub."""
+    rng = np.random.default_rng(seed)
+    core = n - n // 8
+    spokes = rng.choice(core, core // 3, replace=False)
+    src = np.concatenate([np.full(len(spokes), 7), spokes, rng.integers(0, core, 4 * n), rng.integers(core, n, n // 4)])
+    dst = np.concatenate([spokes, np.full(len(spokes), 7), rng.integers(0, core, 4 * n), rng.integers(core, n, n // 4)])
+    order = np.argsort(src, kind="stable")
+    row = np.zeros(n + 1, dtype=np.int64)
+    row[1:] = np.cumsum(np.bincount(src, minlength=n))
+    w = rng.integers(wlo, whi, len(src), endpoint=True)
+    return CSRGraph.from_arrays(row, dst[order], w)
+
+
+def check(g, srcs, **kw):
+    dev = g.copy_to_gpu()
+    try:
+        d, st = sssp_multi(dev, srcs, Options(**kw))
+    finally:
+        dev.close()
+    for i, s in enumerate(srcs):
+        assert np.array_equal(d[:, i], oracle.dijkstra(g.row_start, g.edge_dst, g.edge_data, int(s))), (i, s, kw)
+    return st
+
+
+@pytest.mark.parametrize("n,nsrc,whi", [(1000, 1, 255), (4097, 5, 255), (20011, 33, 1), (20011, 64, 255),
+                                        (3001, 64, INT_MAX), (65537, 17, 1 << 28)])
+def test_hub_graphs(n, nsrc, whi):
+    g = hub_graph(n, n + nsrc, whi)
+    srcs = np.random.default_rng(nsrc).integers(0, n, nsrc)  # about an eighth cannot reach the hub
+    print("filter", n, nsrc, whi, flush=True)
+    check(g, srcs, delta=1 << 30)
+
+
+@pytest.mark.parametrize("far_mode", [0, 1, 2])
+@pytest.mark.parametrize("heavy_deg", [8, 64, 700])
+def test_modes_and_chunks(far_mode, heavy_deg):
+    g = CSRGraph.rmat(13, 12, seed=3)
+    srcs = np.random.default_rng(far_mode).integers(0, g.nnodes, 40)
+    print("filter modes", far_mode, heavy_deg, flush=True)
+    check(g, srcs, delta=64, far_mode=far_mode, heavy_deg=heavy_deg, block_size=256)
+
+
+def test_most_sources_cut_off_from_the_hub():
+    g = hub_graph(8000, 5, 100)
+    cut = np.arange(7000 + 8, 7000 + 40)
+    check(g, np.concatenate([cut, [1, 2, 3]]), delta=1 << 30)
+
+
+def test_more_work_units_than_wavefronts():
+    # rounds of more than 4096 x 16 items: tickets, group helping, staged heavy items
+    g = CSRGraph.rmat(18, 8, seed=9)
+    srcs = np.random.default_rng(1).integers(0, g.nnodes, 12)
+    st = check(g, srcs, delta=1 << 30, block_size=256, heavy_deg=16)
+    assert st["items"] > 4096 * 16
