@@ -14,19 +14,36 @@
 // (every rank is at least 1 - ALPHA; an absolute test would wait on the
 // float rounding of the largest ranks).
 //
-// Layout: rank and contribution arrays f32[V], two of each (current and
-// next); the reverse CSR from lsg_graph_transpose; a list of the vertices
-// with in-degree >= kWaveDeg (the others take one lane each), whose in-edges
-// are cut into chunks of kChunk: one wavefront sums a chunk into a partial
-// (part[]), then one lane per vertex adds its partials in chunk order.  (One
-// wavefront per vertex left the whole sweep waiting on the largest in-degree,
-// ~97 K edges on RMAT-22: ~0.4 ms of a 0.72 ms iteration.)
+// Layout.  The iterations gather one contribution per in-edge from an array of
+// V floats, and at RMAT-22's 16 MB that array, four times an XCD's L2, bounds
+// them.  So a call first renumbers the vertices by in-degree, largest first
+// (a stable counting sort; in-degrees from kHeavyDeg on, or kWideDeg on small
+// graphs, are one class): the
+// contributions read most lie together, and vertices of one in-degree are
+// neighbours.  In that order
+//   positions [0, heavy)     in-degree >= kHeavyDeg: in-edges cut into chunks of
+//     kChunk; one wavefront sums a chunk, and where a vertex has several, one
+//     lane then adds their partials in chunk order (one wavefront per vertex left the
+//     sweep waiting on the largest in-degree, ~97 K edges on RMAT-22);
+//   positions [heavy, live)  the others with in-edges, in slices of 64, one lane
+//     per vertex: a slice's sources are stored transposed, slot k of the 64
+//     lanes consecutive, as many slots as its largest vertex has in-edges;
+//     slots past a vertex's last one name a contribution that is 0;
+//   positions [live, V)      no in-edges: rank 1 - alpha from the start.
+// Without heavy vertices the sort is by in-degree within tiles of kPrTile
+// vertices only (heavy = 0, live = V): there is no hub to bring together, and
+// neighbours of a road network stay near (2048^2 road-like: 60 us per
+// iteration, sorted as a whole 187).
+// Ranks, out-degrees and both contribution arrays are kept in that order and
+// the ranks put back at the end.  Per iteration, against lanes that walked the
+// reverse CSR in vertex order: RMAT-22 513 -> 242 us, 2^20 vertices of uniform
+// degrees 146 -> 88, road-like 73 -> 60; preparing takes 1.0 ms on RMAT-22.
 //
 // The convergence test stays on the device: the host enqueues iterations in
-// batches; after each iteration a one-thread step kernel counts it and sets a
-// done flag when no rank moved by more than epsilon, and every kernel of a
-// later iteration returns at once when it finds the flag set.  The host reads
-// the flag once per batch instead of once per iteration.  Iterations stay
+// batches of one or two launches each; a block in which some rank moved by more than
+// epsilon raises one of kFlags flags, and the iteration's last block
+// counts the iteration and sets a done flag when none was raised; the kernels
+// of later iterations return at once when they find it set.  Iterations stay
 // separate launches: the launch boundary makes one iteration's contributions
 // visible to every XCD's L2 for the next iteration's gathers, which a
 // persistent kernel would have to buy with an L2 invalidate in every block at
@@ -48,204 +65,461 @@
 #include "engine.h"
 #include "lsg_internal.h"
 #include "runtime.h"
+#include "scan_dev.h"
 
 namespace lsg {
 
-constexpr uint32_t kWaveDeg = 32;  // in-degree from which a wavefront sums a vertex
-
-constexpr uint32_t kChunk = 4096;  // in-edges per wavefront-sized partial sum
-constexpr int kUnrollPr = 8;       // in-edges per lane in flight in a partial sum
+constexpr uint32_t kHeavyDeg = 255;  // in-degree from which a vertex is summed in chunks
+constexpr uint32_t kWideDeg = 32;    // slices of at least as many slots take a wavefront each, others kSlices
+constexpr int kSlices = 4;
+// Contributions that pr_sweep_kernel<true> keeps in LDS (one block of kTabBlock
+// threads per CU); it is used on graphs of at least kTabEdges edges of which
+// at least one in kTabShare leaves those vertices.  A CU's L1 has about 64
+// misses in flight, ~290 clocks each from the L2 (counters: 51 M L2 requests
+// in 0.40 ms), so gathers that LDS answers are what makes the sweep faster.
+// us per iteration without / with it: RMAT-22 (56% of the edges) 400 / 261, of
+// ef 8 221 / 141, RMAT-21 179 / 107, RMAT-20 88 / 67, 8 M edges 47 / 49, 4 M 28 / 43.
+// 16384 entries and twice the wavefronts: 320 on RMAT-22; 32768: 273.
+constexpr uint32_t kTabSize = 40448, kTabBlock = 1024, kTabEdges = 10000000, kTabShare = 4;
+// Index arrays of this many edges and more outgrow the memory-side cache
+// (256 MB), which then holds nothing of the last iteration when the next one
+// begins where that one began: odd iterations take the units backwards
+// (RMAT-22, 261 MB: 261 -> 242 us; 197 MB: 172 -> 166; 64 MB: 67 -> 83, the
+// longest units coming last).
+constexpr uint32_t kTurnEdges = 48000000;
+constexpr uint32_t kPrGroups = 16;  // groups of blocks with work tickets of their own
+// Below this many edges vertices of kWideDeg in-edges are heavy already: a wide
+// slice is a chain of up to 32 steps, which a small graph has nothing to hide
+// behind (whole call, kHeavyDeg / kWideDeg: 120 K edges 1.58 / 1.12 ms, 228 K
+// 1.29 / 1.30, 679 K 1.74 / 2.27, 3.9 M 2.8 / 5.5).
+constexpr uint32_t kSmallEdges = 200000;
+constexpr uint32_t kChunk = 4096;    // in-edges per wavefront-sized partial sum
+constexpr int kUnrollPr = 8;         // in-edges per lane in flight
+constexpr uint32_t kPrBlock = 256;
+constexpr uint32_t kPrTile = 4096;   // vertices per block of the counting sort
+// Sweeps of at most this many blocks end the iteration themselves (every block
+// arrives on one word, ~12 ns each); larger ones leave it to pr_finish_kernel's
+// launch, ~5 us (road-like 128^2, whole call: 0.88 -> 0.75 ms).
+constexpr uint32_t kFusedBlocks = 256;
+constexpr uint32_t kFlags = 64;      // "some rank moved" flags, spread over as many words
+constexpr uint32_t kIterBatch = 8;   // iterations enqueued per host check
 
 struct PrArgs {
-  const uint32_t *row_start;         // forward CSR (out-degrees)
-  const uint32_t *in_row, *in_src;   // reverse CSR
-  const float *c_cur;                // contributions of the current ranks
-  float *p_next, *c_next;
-  const uint32_t *heavy;             // vertices with in-degree >= kWaveDeg
-  const uint32_t *hbase;             // heavy vertex i's first partial; its partials are consecutive
-  const uint32_t *chunk;             // partial k belongs to heavy vertex chunk[k] (chunk number k - hbase[.])
-  float *part;                       // partial sums, kChunk in-edges each
-  uint32_t nheavy, nchunks, nnodes;
-  float alpha;
-  uint32_t *maxdiff;                 // bits of the largest |p_next - p_cur| / p_next (non-negative floats order as u32)
-  const float *p_cur;
-  const uint32_t *done;              // set once an earlier iteration converged
+  const uint32_t *row_start;        // forward CSR (out-degrees)
+  const uint32_t *in_row, *in_src;  // reverse CSR
+  uint32_t *hist;                   // [256][tiles] class counts, then places
+  const uint32_t *hist_tiles;       // their scan's tile offsets
+  uint32_t *pos_of;                 // [V] position of a vertex
+  uint32_t *rs, *deg, *od;          // by position: first in-edge, in-degree, out-degree
+  float *p, *c[2];                  // by position; c[.][V] = 0
+  uint32_t *shape;                  // scanned: heavy in-degrees | chunks | slots of a slice (nh + 1, nh + 1, ns + 1 entries)
+  const uint32_t *shape_tiles;
+  uint4 *chunk;                     // a chunk: heavy vertex, in-edges, where they lie in idx (two words)
+  float *part;                      // a chunk's sum
+  uint32_t *hbase;                  // [heavy + 1] a heavy vertex's first chunk
+  uint32_t *slice;                  // [slices + 1] a slice's first slot in idx, past slots, / 64
+  uint32_t *idx;                    // source positions: heavy vertices' edges, then the slices
+  uint32_t *ctl;
+  size_t slots;                     // where the slices begin in idx
+  uint32_t V, tiles, nh, ns;        // nh, ns: bounds of the numbers of heavy vertices and slices
+  uint32_t heavy, live, nchunks, wide, nslices;  // wide: slices taken one per wavefront
+  uint32_t units;                   // of the sweep
+  uint32_t turn;                    // odd iterations take the units backwards
+  uint32_t hdeg;                    // in-degree from which a vertex is heavy
+  uint32_t fused;                   // the sweep also ends the iteration
+  uint32_t local;                   // sorted within tiles
+  float alpha, epsilon;
 };
 
-constexpr uint32_t kIterBatch = 8;  // iterations enqueued per host check
+// control words; the flags of an iteration are those of its parity, so that
+// the next iteration's can be cleared while they are read
+constexpr int kCtlMax = 0, kCtlDone = 1, kCtlIters = 2, kCtlArrive = 3, kCtlHeavy = 4, kCtlWide = 5, kCtlLive = 6,
+              kCtlChunks = 7, kCtlEdges = 8, kCtlHot = 9, kCtlFlags = 16, kCtlTickets = kCtlFlags + 2 * (int)kFlags + 16, kCtlWords = kCtlTickets + 32 * (int)kPrGroups;
 
-// control words; the largest change is kept per iteration parity, so the step
-// kernel can clear the next iteration's word while this one's is read
-constexpr int kCtlHeavy = 0, kCtlMax = 1, kCtlDone = 3, kCtlIters = 4, kCtlChunks = 5;
+__device__ __forceinline__ uint32_t pr_class(const PrArgs &a, uint32_t indeg) { return a.hdeg - min(indeg, a.hdeg); }
 
-// Whether an earlier iteration converged (written by pr_step_kernel in an
-// earlier launch, so a plain load sees it).
-__device__ __forceinline__ bool pr_done(const PrArgs &a) {
-  __shared__ uint32_t s_done;
-  if (threadIdx.x == 0) s_done = *a.done;
+// Entry of class d and tile b in the order of the sort.
+__device__ __forceinline__ size_t pr_entry(const PrArgs &a, uint32_t d, uint32_t b) {
+  return a.local ? (size_t)b * 256 + d : (size_t)d * a.tiles + b;
+}
+
+__global__ void pr_clear_kernel(PrArgs a) {
+  for (uint32_t i = threadIdx.x; i < (uint32_t)kCtlWords; i += blockDim.x) a.ctl[i] = 0;
+}
+
+// The largest in-degree.
+__global__ __launch_bounds__(kPrBlock) void pr_max_kernel(PrArgs a) {
+  __shared__ uint32_t s_m;
+  if (threadIdx.x == 0) s_m = 0;
   __syncthreads();
-  return s_done != 0;
-}
-
-__global__ void pr_init_kernel(const uint32_t *row_start, const uint32_t *in_row, uint32_t V, float alpha, float *p,
-                               float *c, uint32_t *heavy, uint32_t *nheavy) {
-  for (size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < V; v += (size_t)gridDim.x * blockDim.x) {
-    const float p0 = 1.0f - alpha;  // apps/pr/kernel.cu:38
-    const uint32_t od = row_start[v + 1] - row_start[v];
-    p[v] = p0;
-    c[v] = od ? p0 / (float)od : 0.0f;
-    const bool h = in_row[v + 1] - in_row[v] >= kWaveDeg;
-    const uint64_t m = __ballot(h);
-    if (m) {
-      uint32_t base = 0;
-      const uint32_t leader = (uint32_t)__builtin_ctzll(m);
-      if (lane_id() == leader) base = atomic_add(nheavy, (uint32_t)__builtin_popcountll(m));
-      base = readlane(base, leader);
-      if (h) heavy[base + lanes_below(m)] = (uint32_t)v;
-    }
-  }
-}
-
-// After pr_init_kernel: heavy vertex i gets ceil(indeg / kChunk) consecutive
-// partials starting at hbase[i] (where they sit depends on the order of the
-// atomics; the order in which a vertex's partials are added never does).
-__global__ void pr_chunks_kernel(const uint32_t *in_row, const uint32_t *heavy, uint32_t nheavy, uint32_t *hbase,
-                                 uint32_t *chunk, uint32_t *nchunks) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  const uint32_t lane = lane_id();
-  // wavefront-uniform loop: one reservation atomic per wavefront (one per
-  // vertex, ~280 K on one word for RMAT-22, would serialise for milliseconds)
-  for (size_t i0 = blockIdx.x * (size_t)blockDim.x + (threadIdx.x & ~(uint32_t)(kWave - 1)); i0 < nheavy; i0 += stride) {
-    const size_t i = i0 + lane;
-    const bool ok = i < nheavy;
-    const uint32_t v = ok ? heavy[i] : 0u;
-    const uint32_t n = ok ? (in_row[v + 1] - in_row[v] + kChunk - 1) / kChunk : 0u;
-    uint32_t incl = n;
+  uint32_t m = 0;
+  for (size_t v = blockIdx.x * (size_t)kPrBlock + threadIdx.x; v < a.V; v += (size_t)gridDim.x * kPrBlock)
+    m = max(m, a.in_row[v + 1] - a.in_row[v]);
 #pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const uint32_t y = __shfl_up(incl, d);
-      if (lane >= (uint32_t)d) incl += y;
+  for (int d = kWave / 2; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor(m, d));
+  if (lane_id() == 0) atomicMax(&s_m, m);
+  __syncthreads();
+  // (most blocks find a larger one there already)
+  if (threadIdx.x == 0 && s_m > ld_coh(a.ctl + kCtlMax))
+    __hip_atomic_fetch_max(glb(a.ctl + kCtlMax), s_m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// hist: vertices of every class and tile.
+__global__ __launch_bounds__(kPrBlock) void pr_hist_kernel(PrArgs a) {
+  __shared__ uint32_t h[256];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  const uint64_t base = (uint64_t)blockIdx.x * kPrTile;
+  for (uint32_t i = threadIdx.x; i < kPrTile && base + i < a.V; i += kPrBlock)
+    atomicAdd(&h[pr_class(a, a.in_row[base + i + 1] - a.in_row[base + i])], 1u);
+  __syncthreads();
+  a.hist[pr_entry(a, threadIdx.x, blockIdx.x)] = h[threadIdx.x];
+}
+
+// Exclusive prefix over the classes and tiles at entry i.
+__device__ __forceinline__ uint32_t pr_place(const PrArgs &a, size_t i) { return a.hist[i] + a.hist_tiles[i / kScanTile]; }
+
+// Every vertex to its position, stable within a class, with its first rank
+// and contribution (lanes of one class are ranked by ballots over its 8 bits).
+__global__ __launch_bounds__(kPrBlock) void pr_place_kernel(PrArgs a) {
+  constexpr uint32_t NW = kPrBlock / kWave;
+  __shared__ uint32_t run[256], wcnt[NW][256], hot;
+  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  run[threadIdx.x] = pr_place(a, pr_entry(a, threadIdx.x, blockIdx.x));
+  for (uint32_t w = 0; w < NW; ++w) wcnt[w][threadIdx.x] = 0;
+  if (threadIdx.x == 0) hot = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const bool whole = !a.local;
+    a.ctl[kCtlHeavy] = whole ? pr_place(a, (size_t)a.tiles) : 0u;
+    a.ctl[kCtlWide] = whole ? pr_place(a, (size_t)(a.hdeg - kWideDeg + 1) * a.tiles) : 0u;
+    a.ctl[kCtlLive] = whole ? pr_place(a, (size_t)a.hdeg * a.tiles) : a.V;
+    a.c[0][a.V] = a.c[1][a.V] = 0.0f;
+  }
+  __syncthreads();
+  const float p0 = 1.0f - a.alpha;  // apps/pr/kernel.cu:38
+  for (uint32_t it = 0; it < kPrTile / kPrBlock; ++it) {
+    const uint64_t v = (uint64_t)blockIdx.x * kPrTile + it * kPrBlock + threadIdx.x;
+    const bool valid = v < a.V;
+    uint32_t e0 = 0, dg = 0, od = 0, d = 0;
+    if (valid) {
+      e0 = a.in_row[v];
+      dg = a.in_row[v + 1] - e0;
+      od = a.row_start[v + 1] - a.row_start[v];
+      d = pr_class(a, dg);
     }
-    const uint32_t total = readlane(incl, kWave - 1);
-    uint32_t base = 0;
-    if (lane == 0 && total) base = atomic_add(nchunks, total);
-    base = readlane(base, 0) + incl - n;
-    if (ok) {
-      hbase[i] = base;
-      for (uint32_t k = 0; k < n; ++k) chunk[base + k] = (uint32_t)i;
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (uint32_t bit = 0; bit < 8; ++bit) {
+      const uint64_t m = __ballot((d >> bit) & 1u);
+      peers &= ((d >> bit) & 1u) ? m : ~m;
+    }
+    const uint32_t rank = lanes_below(peers);
+    if (valid && rank == 0) wcnt[wv][d] = (uint32_t)__builtin_popcountll(peers);
+    __syncthreads();
+    if (valid) {
+      uint32_t pos = run[d] + rank;
+      for (uint32_t w = 0; w < wv; ++w) pos += wcnt[w][d];
+      a.pos_of[v] = pos;
+      a.rs[pos] = e0;
+      a.deg[pos] = dg;
+      a.od[pos] = od;
+      if (pos < kTabSize) atomicAdd(&hot, od);
+      a.p[pos] = p0;
+      a.c[0][pos] = a.c[1][pos] = od ? p0 / (float)od : 0.0f;
+    }
+    __syncthreads();
+    uint32_t sum = 0;
+    for (uint32_t w = 0; w < NW; ++w) {
+      sum += wcnt[w][threadIdx.x];
+      wcnt[w][threadIdx.x] = 0;
+    }
+    run[threadIdx.x] += sum;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && hot) atomic_add(a.ctl + kCtlHot, hot);
+}
+
+// The unscanned shape: in-degrees and chunk counts of the heavy vertices, slots
+// per lane of the slices (a slice's largest in-degree is its first vertex's,
+// or, where a tile ends in it, the first one of the next tile's).
+__global__ void pr_shape_kernel(PrArgs a) {
+  const uint32_t heavy = a.ctl[kCtlHeavy], live = a.ctl[kCtlLive];
+  const size_t n = 2 * ((size_t)a.nh + 1) + a.ns + 1;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+    uint32_t x = 0;
+    if (i < a.nh + 1) {
+      if (i < heavy) x = a.deg[i];
+    } else if (i < 2 * ((size_t)a.nh + 1)) {
+      const size_t k = i - (a.nh + 1);
+      if (k < heavy) x = (a.deg[k] + kChunk - 1) / kChunk;
+    } else {
+      const uint64_t pos = heavy + (uint64_t)(i - 2 * ((size_t)a.nh + 1)) * kWave;
+      if (pos < live) x = a.deg[pos];  // kPrTile is a multiple of 64: no slice crosses a tile
+    }
+    a.shape[i] = x;
+  }
+}
+
+__device__ __forceinline__ uint32_t pr_shape_at(const PrArgs &a, size_t i) {
+  return a.shape[i] + a.shape_tiles[i / kScanTile];
+}
+// From the shape's scan (each part from 0 on; u32 differences are exact
+// whatever wraps): the heavy vertices' first chunks, the chunks, the slices.
+__global__ void pr_chunks_kernel(PrArgs a) {
+  const uint32_t heavy = a.ctl[kCtlHeavy], live = a.ctl[kCtlLive], lane = lane_id();
+  const size_t c0 = a.nh + 1, s0 = 2 * c0;
+  const uint32_t first = pr_shape_at(a, c0), first_slot = pr_shape_at(a, s0);
+  const size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = tid / kWave; i < heavy; i += nt / kWave) {
+    const uint32_t b = pr_shape_at(a, c0 + i) - first, e = pr_shape_at(a, c0 + i + 1) - first, dg = a.deg[i];
+    const uint64_t at = pr_shape_at(a, i);
+    if (lane == 0) a.hbase[i] = b;
+    for (uint32_t k = b + lane; k < e; k += kWave) {
+      const uint32_t lo = (k - b) * kChunk;
+      a.chunk[k] = make_uint4((uint32_t)i, min(dg - lo, kChunk), (uint32_t)(at + lo), (uint32_t)((at + lo) >> 32));
+    }
+  }
+  const size_t nsl = ((size_t)live - heavy + kWave - 1) / kWave;
+  for (size_t k = tid; k <= nsl; k += nt) a.slice[k] = pr_shape_at(a, s0 + k) - first_slot;
+  if (tid == 0) {
+    a.ctl[kCtlChunks] = a.hbase[heavy] = pr_shape_at(a, c0 + heavy) - first;
+    a.ctl[kCtlEdges] = pr_shape_at(a, heavy);
+  }
+}
+
+// idx: the position of every in-edge's source, one wavefront per chunk or slice.
+__global__ __launch_bounds__(kPrBlock) void pr_layout_kernel(PrArgs a) {
+  const uint32_t lane = lane_id();
+  const uint32_t units = a.nchunks + a.nslices;
+  const uint32_t waves = gridDim.x * (kPrBlock / kWave);
+  for (uint32_t k = blockIdx.x * (kPrBlock / kWave) + threadIdx.x / kWave; k < units; k += waves) {
+    if (k < a.nchunks) {
+      const uint4 x = a.chunk[k];
+      const uint32_t *src = a.in_src + a.rs[x.x] + (size_t)(k - a.hbase[x.x]) * kChunk;
+      uint32_t *const idx = a.idx + ((uint64_t)x.w << 32 | x.z);
+      for (uint32_t e = lane; e < x.y; e += kWave) idx[e] = a.pos_of[src[e]];
+    } else {
+      const uint32_t sl = k - a.nchunks, at = a.slice[sl], w = a.slice[sl + 1] - at;
+      uint32_t *const idx = a.idx + a.slots + (size_t)at * kWave + lane;
+      const uint64_t pos = a.heavy + (uint64_t)sl * kWave + lane;
+      const uint32_t dg = pos < a.live ? a.deg[pos] : 0u;
+      const uint32_t *src = a.in_src + (pos < a.live ? a.rs[pos] : 0u);
+      for (uint32_t q = 0; q < w; ++q) idx[(size_t)q * kWave] = q < dg ? a.pos_of[src[q]] : a.V;
     }
   }
 }
 
-__device__ __forceinline__ void pr_store(const PrArgs &a, uint32_t v, float sum, float &dmax) {
+// Whether an earlier iteration converged (written in an earlier launch, so a plain load sees it).
+__device__ __forceinline__ bool pr_done(const PrArgs &a) { return a.ctl[kCtlDone] != 0; }
+
+// The vertex at `pos`, whose rank was pc: its new rank and contribution from
+// the sum of its in-neighbours' contributions; whether the rank moved.
+__device__ __forceinline__ bool pr_store(const PrArgs &a, float *c_next, size_t pos, float sum, float pc, uint32_t od) {
   const float pn = (1.0f - a.alpha) + a.alpha * sum;
-  const uint32_t od = a.row_start[v + 1] - a.row_start[v];
-  a.p_next[v] = pn;
-  a.c_next[v] = od ? pn / (float)od : 0.0f;
-  dmax = fmaxf(dmax, fabsf(pn - a.p_cur[v]) / pn);  // pn >= 1 - alpha > 0
+  a.p[pos] = pn;
+  c_next[pos] = od ? pn / (float)od : 0.0f;
+  return fabsf(pn - pc) / pn > a.epsilon;  // pn >= 1 - alpha > 0
 }
 
-// The block's largest change goes to maxdiff with one atomic per block (one
-// per wavefront on the same word serialises at the memory-side atomic unit).
-__device__ __forceinline__ void pr_reduce_max(const PrArgs &a, float dmax) {
-  __shared__ uint32_t s_max;
-  if (threadIdx.x == 0) s_max = 0;
-  __syncthreads();
-#pragma unroll
-  for (int d = kWave / 2; d >= 1; d >>= 1) dmax = fmaxf(dmax, __shfl_xor(dmax, d));
-  if (lane_id() == 0 && dmax > 0.0f) atomicMax(&s_max, __float_as_uint(dmax));
-  __syncthreads();
-  if (threadIdx.x == 0 && s_max)
-    __hip_atomic_fetch_max(a.maxdiff, s_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Raises the block's flag if some lane's rank moved.
+__device__ __forceinline__ void pr_raise(const PrArgs &a, uint32_t it, bool moved) {
+  if (__syncthreads_or(moved) && threadIdx.x == 0) st_coh(a.ctl + kCtlFlags + (it & 1) * kFlags + blockIdx.x % kFlags, 1u);
 }
 
-// One lane per vertex of in-degree < kWaveDeg.
-__global__ void pr_light_kernel(PrArgs a) {
-  if (pr_done(a)) return;
-  float dmax = 0.0f;
-  const size_t nt = (size_t)gridDim.x * blockDim.x;
-  for (size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < a.nnodes; v += nt) {
-    const uint32_t e0 = a.in_row[v], e1 = a.in_row[v + 1];
-    if (e1 - e0 >= kWaveDeg) continue;
-    // four in-edges per step, summed in edge order
-    float sum = 0.0f;
-    uint32_t e = e0;
-    for (; e + 4 <= e1; e += 4) {
-      uint32_t u[4];
-      float c[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) u[k] = a.in_src[e + k];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) c[k] = a.c_cur[u[k]];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) sum += c[k];
-    }
-    for (; e < e1; ++e) sum += a.c_cur[a.in_src[e]];
-    pr_store(a, (uint32_t)v, sum, dmax);
+// A contribution.  kTab: those of the first kTabSize positions are in LDS, and
+// their lanes read the 0 at c[V] instead (one line for all of them).
+template <bool kTab>
+__device__ __forceinline__ float pr_c(const PrArgs &a, const float *tab, const float *c, uint32_t u) {
+  if (!kTab) return glb(c)[u];
+  const bool hot = u < kTabSize;
+  return tab[hot ? u : kTabSize] + glb(c)[hot ? a.V : u];
+}
+
+// The iteration's end, called by every thread of every block of its last
+// launch: the last block to get here counts the iteration and decides whether
+// it was the last.
+__device__ __forceinline__ void pr_end(const PrArgs &a, uint32_t it) {
+  __shared__ uint32_t last;
+  if (threadIdx.x == 0) {
+    order_release();
+    last = atomic_add(a.ctl + kCtlArrive, 1u) + 1 == gridDim.x;
   }
-  pr_reduce_max(a, dmax);
+  __syncthreads();
+  if (!last) return;
+  uint32_t *const flags = a.ctl + kCtlFlags;
+  const bool some = threadIdx.x < kFlags && ld_coh(flags + (it & 1) * kFlags + threadIdx.x) != 0;
+  if (threadIdx.x < kFlags) flags[((it + 1) & 1) * kFlags + threadIdx.x] = 0;
+  if (threadIdx.x < kPrGroups) a.ctl[kCtlTickets + threadIdx.x * 32] = 0;
+  const bool go_on = __syncthreads_or(some);
+  if (threadIdx.x == 0) {
+    a.ctl[kCtlIters] = it + 1;
+    a.ctl[kCtlDone] = !go_on;
+    a.ctl[kCtlArrive] = 0;
+  }
 }
 
-// One wavefront per partial: kChunk in-edges of a heavy vertex, 64 per step
-// (four steps' loads in flight), then a butterfly sum -- the same order every
-// iteration.
-__global__ void pr_chunk_kernel(PrArgs a) {
-  if (pr_done(a)) return;
+// One unit of the sweep; whether some rank moved.
+template <bool kTab>
+__device__ __forceinline__ bool pr_unit(const PrArgs &a, const float *tab, const float *c, float *c_next, uint32_t k) {
   const uint32_t lane = lane_id();
-  const size_t waves = (size_t)gridDim.x * blockDim.x / kWave;
-  for (size_t k = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) / kWave; k < a.nchunks; k += waves) {
-    const uint32_t i = a.chunk[k];
-    const uint32_t v = a.heavy[i];
-    const uint32_t e0 = a.in_row[v] + (uint32_t)(k - a.hbase[i]) * kChunk;
-    const uint32_t e1 = min(a.in_row[v + 1], e0 + kChunk);
-    // lane l sums in-edges e0 + l, e0 + l + 64, ... in that order, eight per
-    // step.  Every lane loads (past the chunk's end it reloads the last edge
-    // and adds 0): loads under per-lane conditions make the compiler wait for
-    // the whole memory queue at each, one round trip per load.
+  bool moved = false;
+  if (k < a.nchunks) {
+    const uint4 x = a.chunk[k];
+    const uint32_t n = __builtin_amdgcn_readfirstlane(x.y);
+    const uint32_t *idx = a.idx + ((uint64_t)x.w << 32 | x.z);
+    const bool whole = a.deg[x.x] <= kChunk;  // the vertex has no other chunk
+    const float pc = a.p[x.x];
+    const uint32_t od = a.od[x.x];
+    // Every lane loads (past the chunk's end it reloads the last edge and adds
+    // 0): loads under per-lane conditions make the compiler wait for the whole
+    // memory queue at each, one round trip per load.
     float sum = 0.0f;
-    for (uint32_t b = e0; b < e1; b += kUnrollPr * kWave) {
+    for (uint32_t e = 0; e < n; e += kUnrollPr * kWave) {
       uint32_t u[kUnrollPr];
-      float c[kUnrollPr];
+      float x8[kUnrollPr];
 #pragma unroll
-      for (int q = 0; q < kUnrollPr; ++q) u[q] = a.in_src[min(b + q * kWave + lane, e1 - 1)];
+      for (int q = 0; q < kUnrollPr; ++q) u[q] = glb(idx)[min(e + q * kWave + lane, n - 1)];
 #pragma unroll
-      for (int q = 0; q < kUnrollPr; ++q) c[q] = a.c_cur[u[q]];
+      for (int q = 0; q < kUnrollPr; ++q) x8[q] = pr_c<kTab>(a, tab, c, u[q]);
 #pragma unroll
-      for (int q = 0; q < kUnrollPr; ++q) sum += b + q * kWave + lane < e1 ? c[q] : 0.0f;
+      for (int q = 0; q < kUnrollPr; ++q) sum += e + q * kWave + lane < n ? x8[q] : 0.0f;
     }
 #pragma unroll
     for (int d = kWave / 2; d >= 1; d >>= 1) sum += __shfl_xor(sum, d);
-    if (lane == 0) a.part[k] = sum;
+    if (lane == 0) {
+      if (whole) moved = pr_store(a, c_next, x.x, sum, pc, od);
+      else a.part[k] = sum;
+    }
+  } else if ((k -= a.nchunks) < a.wide) {
+    const uint32_t at = a.slice[k], w = __builtin_amdgcn_readfirstlane(a.slice[k + 1] - at);
+    const uint32_t *idx = a.idx + a.slots + (size_t)at * kWave + lane;
+    const uint64_t pos = min(a.heavy + (uint64_t)k * kWave + lane, (uint64_t)a.live - 1);
+    const float pc = a.p[pos];
+    const uint32_t od = a.od[pos];
+    float sum[kUnrollPr];
+#pragma unroll
+    for (int q = 0; q < kUnrollPr; ++q) sum[q] = 0.0f;
+    for (uint32_t q0 = 0; q0 < w; q0 += kUnrollPr) {
+      uint32_t u[kUnrollPr];
+      float x8[kUnrollPr];
+#pragma unroll
+      for (int q = 0; q < kUnrollPr; ++q) u[q] = glb(idx)[(size_t)min(q0 + q, w - 1) * kWave];
+#pragma unroll
+      for (int q = 0; q < kUnrollPr; ++q) x8[q] = pr_c<kTab>(a, tab, c, u[q]);
+#pragma unroll
+      for (int q = 0; q < kUnrollPr; ++q) sum[q] += q0 + q < w ? x8[q] : 0.0f;
+    }
+    if (a.heavy + (uint64_t)k * kWave + lane < a.live)
+      moved |= pr_store(a, c_next, pos, ((sum[0] + sum[1]) + (sum[2] + sum[3])) + ((sum[4] + sum[5]) + (sum[6] + sum[7])),
+                       pc, od);
+  } else if ((k = a.wide + (k - a.wide) * kSlices) < a.nslices) {
+    uint32_t at[kSlices + 1], w[kSlices], od[kSlices], wmax = 0;
+    float pc[kSlices], sum[kSlices];
+    const uint64_t pos = a.heavy + (uint64_t)k * kWave + lane;
+#pragma unroll
+    for (int j = 0; j <= kSlices; ++j)
+      at[j] = __builtin_amdgcn_readfirstlane(a.slice[min(k + j, a.nslices)]);
+#pragma unroll
+    for (int j = 0; j < kSlices; ++j) {
+      w[j] = at[j + 1] - at[j];
+      wmax = max(wmax, w[j]);
+      const uint64_t x = min(pos + (uint64_t)j * kWave, (uint64_t)a.live - 1);
+      pc[j] = a.p[x];
+      od[j] = a.od[x];
+      sum[j] = 0.0f;
+    }
+    const uint32_t *idx = a.idx + a.slots + lane;
+    constexpr int kSlots = kUnrollPr / kSlices;
+    for (uint32_t q0 = 0; q0 < wmax; q0 += kSlots) {
+      uint32_t u[kSlices][kSlots];
+      float x[kSlices][kSlots];
+#pragma unroll
+      for (int j = 0; j < kSlices; ++j)
+#pragma unroll
+        for (int q = 0; q < kSlots; ++q) u[j][q] = q0 + q < w[j] ? glb(idx)[(at[j] + (size_t)(q0 + q)) * kWave] : a.V;
+#pragma unroll
+      for (int j = 0; j < kSlices; ++j)
+#pragma unroll
+        for (int q = 0; q < kSlots; ++q) x[j][q] = pr_c<kTab>(a, tab, c, u[j][q]);
+#pragma unroll
+      for (int j = 0; j < kSlices; ++j)
+#pragma unroll
+        for (int q = 0; q < kSlots; ++q) sum[j] += x[j][q];
+    }
+#pragma unroll
+    for (int j = 0; j < kSlices; ++j)
+      if (pos + (uint64_t)j * kWave < a.live) moved |= pr_store(a, c_next, pos + j * kWave, sum[j], pc[j], od[j]);
   }
+  return moved;
 }
 
-// One lane per heavy vertex: its partials added in chunk order.
-__global__ void pr_finish_kernel(PrArgs a) {
+// One iteration's sums.  Wavefront units: the chunks, the wide slices, then the
+// others kSlices at a time (few slots each: their loads go out together).
+// Every sum is taken in in-edge order, a wide slice's (32 and more in-edges)
+// in eight sums added pairwise, a chunk's per lane and then over the lanes.
+template <bool kTab>
+__global__ __launch_bounds__(kTab ? kTabBlock : kPrBlock) void pr_sweep_kernel(PrArgs a, uint32_t it) {
   if (pr_done(a)) return;
-  float dmax = 0.0f;
-  const size_t nt = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < a.nheavy; i += nt) {
-    const uint32_t v = a.heavy[i];
-    const uint32_t n = (a.in_row[v + 1] - a.in_row[v] + kChunk - 1) / kChunk;
-    const float *pp = a.part + a.hbase[i];
-    float sum = 0.0f;
-    for (uint32_t k = 0; k < n; ++k) sum += pp[k];
-    pr_store(a, v, sum, dmax);
+  constexpr uint32_t kBlock = kTab ? kTabBlock : kPrBlock;
+  __shared__ float tab[kTab ? kTabSize + 1 : 1];
+  const uint32_t lane = lane_id();
+  const float *const c = a.c[it & 1];
+  if (kTab) {
+    for (uint32_t i = threadIdx.x; i <= kTabSize; i += kBlock) tab[i] = i < kTabSize ? c[i] : 0.0f;
+    __syncthreads();
   }
-  pr_reduce_max(a, dmax);
+  float *const c_next = a.c[(it & 1) ^ 1];
+  const uint32_t wave = threadIdx.x / kWave;
+  uint32_t unit, g = 0;
+  if (kTab) {
+    // Unit j * kPrGroups + g belongs to the blocks b with b % kPrGroups == g: a
+    // wavefront takes one, then one per ticket, fetched a unit ahead.
+    g = blockIdx.x % kPrGroups;
+    unit = (blockIdx.x / kPrGroups * (kBlock / kWave) + wave) * kPrGroups + g;
+  } else {
+    // One unit per wavefront.  Sorted within tiles, neighbours are near: every
+    // XCD takes one contiguous eighth of the units.  (Sorted as a whole the
+    // longest units come first and are dealt to all XCDs.)
+    const uint32_t b = a.local ? blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+    unit = b * (kBlock / kWave) + wave;
+  }
+  bool moved = false;
+  while (unit < a.units) {
+    uint32_t t = 0;
+    if (kTab && lane == 0) t = atomic_add(a.ctl + kCtlTickets + g * 32, 1u);
+    moved |= pr_unit<kTab>(a, tab, c, c_next, a.turn && (it & 1) ? a.units - 1 - unit : unit);
+    if (!kTab) break;
+    const uint32_t first = (gridDim.x + kPrGroups - 1 - g) / kPrGroups * (kBlock / kWave);
+    unit = (first + readlane(t, 0)) * kPrGroups + g;
+  }
+  pr_raise(a, it, moved);
+  if (!kTab && a.fused) pr_end(a, it);
 }
 
-__global__ void pr_clear_kernel(uint32_t *w, uint32_t n) {
-  if (threadIdx.x < n) w[threadIdx.x] = 0;
+// One lane per heavy vertex of several chunks: its partials added in chunk
+// order; the iteration's end.
+__global__ __launch_bounds__(kPrBlock) void pr_finish_kernel(PrArgs a, uint32_t it) {
+  if (pr_done(a)) return;
+  const uint32_t i = blockIdx.x * kPrBlock + threadIdx.x;
+  bool moved = false;
+  if (i < a.heavy) {
+    const uint32_t b = a.hbase[i], e = a.hbase[i + 1];
+    if (e - b > 1) {
+      const float pc = a.p[i];
+      const uint32_t od = a.od[i];
+      float sum = 0.0f;
+      for (uint32_t k = b; k < e; ++k) sum += a.part[k];
+      moved = pr_store(a, a.c[(it & 1) ^ 1], i, sum, pc, od);
+    }
+  }
+  pr_raise(a, it, moved);
+  pr_end(a, it);
 }
 
-// After iteration `it` (one thread): count it, raise done when no rank moved
-// by more than epsilon, and clear the next iteration's change word.
-__global__ void pr_step_kernel(uint32_t *ctl, uint32_t it, float epsilon) {
-  if (ctl[kCtlDone]) return;
-  ctl[kCtlIters] = it + 1;
-  if (__uint_as_float(ctl[kCtlMax + (it & 1)]) <= epsilon) ctl[kCtlDone] = 1;
-  ctl[kCtlMax + ((it + 1) & 1)] = 0;
+// The ranks in vertex order.
+__global__ void pr_ranks_kernel(PrArgs a, float *rank) {
+  for (size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < a.V; v += (size_t)gridDim.x * blockDim.x)
+    rank[v] = a.p[a.pos_of[v]];
 }
 
 }  // namespace lsg
@@ -272,82 +546,111 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
   std::lock_guard<std::mutex> lk(w->mu);
   HIPCHK(hipSetDevice(w->device));
   const uint32_t V = g->nnodes;
-  void *buf, *cbuf;
-  // p[2], c[2] (f32[V] each), the heavy list and its partials' bases (u32[V]
-  // each), and per partial its heavy vertex (u32) and sum (f32): at most
-  // V + E / kChunk partials
-  const uint64_t maxchunks = (uint64_t)V + g->nedges / kChunk + 1;
-  if ((rc = ws_buffer(w, kBufQueues, (6ull * V + 2 * maxchunks) * 4, &buf)) ||
-      (rc = ws_buffer(w, kBufSeeds, 2048, &cbuf)))
-    return rc;
-  float *p[2] = {(float *)buf, (float *)buf + V};
-  float *c[2] = {(float *)buf + 2ull * V, (float *)buf + 3ull * V};
-  uint32_t *heavy = (uint32_t *)buf + 4ull * V;
-  uint32_t *hbase = (uint32_t *)buf + 5ull * V;
-  uint32_t *chunk = (uint32_t *)buf + 6ull * V;
-  float *part = (float *)buf + 6ull * V + maxchunks;
-  uint32_t *ctl = (uint32_t *)cbuf;  // heavy count, max change (x2), done, iterations, partial count
-  const uint32_t vgrid = (uint32_t)std::min<uint64_t>(((uint64_t)V + 255) / 256, 16ull * w->cus);
-  HIPCHK(hipEventRecord(w->ev0, w->stream));
-  hipLaunchKernelGGL(pr_clear_kernel, dim3(1), dim3(64), 0, w->stream, ctl, 6u);
-  hipLaunchKernelGGL(pr_init_kernel, dim3(vgrid), dim3(256), 0, w->stream, g->row_start, gt->row_start, V, alpha,
-                     p[0], c[0], heavy, ctl);
-  HIPCHK(hipGetLastError());
-  uint32_t *hc = w->pinned;
-  HIPCHK(hipMemcpyAsync(hc, ctl, 4, hipMemcpyDeviceToHost, w->stream));
-  HIPCHK(hipStreamSynchronize(w->stream));
-  const uint32_t nheavy = hc[0];
-  const uint32_t fgrid = (uint32_t)std::min<uint64_t>(((uint64_t)nheavy + 255) / 256 + 1, 16ull * w->cus);
-  if (nheavy) {
-    hipLaunchKernelGGL(pr_chunks_kernel, dim3(fgrid), dim3(256), 0, w->stream, gt->row_start, heavy, nheavy, hbase,
-                       chunk, ctl + kCtlChunks);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(hc, ctl + kCtlChunks, 4, hipMemcpyDeviceToHost, w->stream));
-    HIPCHK(hipStreamSynchronize(w->stream));
-  } else {
-    hc[0] = 0;
-  }
-  const uint32_t nchunks = hc[0];
-  if (nchunks > maxchunks) return fail(LSG_ERR_CAPACITY, "pagerank: %u partial sums exceed the buffer", nchunks);
+  const uint64_t E = g->nedges;
+  const uint32_t tiles = (uint32_t)(((uint64_t)V + kPrTile - 1) / kPrTile);
   PrArgs a;
+  memset(&a, 0, sizeof a);
+  a.V = V;
+  a.tiles = tiles;
+  a.nh = (uint32_t)std::min<uint64_t>(V, E / kWideDeg);
+  a.ns = V / kWave + 1;
+  const uint64_t nhist = 256ull * tiles, hscan = (nhist + kScanTile - 1) / kScanTile;
+  const uint64_t nshape = 2 * (a.nh + 1ull) + a.ns + 1, sscan = (nshape + kScanTile - 1) / kScanTile;
+  const uint64_t maxchunks = a.nh + E / kChunk + 1;
+  void *buf, *ibuf;
+  if ((rc = ws_buffer(w, kBufQueues,
+                      (7ull * V + 2 + nhist + hscan + nshape + sscan + (a.nh + 1ull) + (a.ns + 1ull) + 5 * maxchunks +
+                       kCtlWords + 2) * 4 + 16, &buf)))
+    return rc;
+  uint32_t *at = (uint32_t *)buf;
+  auto take = [&](uint64_t n) {
+    uint32_t *const x = at;
+    at += n;
+    return x;
+  };
+  a.pos_of = take(V);
+  a.rs = take(V);
+  a.deg = take(V);
+  a.od = take(V);
+  a.p = (float *)take(V);
+  a.c[0] = (float *)take(V + 1ull);
+  a.c[1] = (float *)take(V + 1ull);
+  a.hist = take(nhist);
+  uint32_t *const hist_tiles = take(hscan);
+  a.hist_tiles = hist_tiles;
+  a.shape = take(nshape);
+  uint32_t *const shape_tiles = take(sscan);
+  a.shape_tiles = shape_tiles;
+  a.hbase = take(a.nh + 1ull);
+  a.slice = take(a.ns + 1ull);
+  a.part = (float *)take(maxchunks);
+  a.ctl = take(kCtlWords);
+  uint32_t *const total = take(2);
+  a.chunk = (uint4 *)(((uintptr_t)at + 15) & ~(uintptr_t)15);
   a.row_start = g->row_start;
   a.in_row = gt->row_start;
   a.in_src = gt->edge_dst;
-  a.heavy = heavy;
-  a.hbase = hbase;
-  a.chunk = chunk;
-  a.part = part;
-  a.nheavy = nheavy;
-  a.nchunks = nchunks;
-  a.nnodes = V;
   a.alpha = alpha;
-  a.done = ctl + kCtlDone;
-  const uint32_t cgrid = (uint32_t)std::min<uint64_t>(((uint64_t)nchunks * kWave + 255) / 256 + 1, 16ull * w->cus);
-  // Iteration `it` reads p[it & 1], c[it & 1] and writes the other pair.
+  a.epsilon = epsilon;
+  const uint32_t vgrid = (uint32_t)std::min<uint64_t>(((uint64_t)V + 255) / 256, 16ull * w->cus);
+  HIPCHK(hipEventRecord(w->ev0, w->stream));
+  uint32_t *hc = w->pinned;
+  hipLaunchKernelGGL(pr_clear_kernel, dim3(1), dim3(256), 0, w->stream, a);
+  hipLaunchKernelGGL(pr_max_kernel, dim3(std::min<uint32_t>(vgrid, 4u * w->cus)), dim3(kPrBlock), 0, w->stream, a);
+  HIPCHK(hipMemcpyAsync(hc, a.ctl, 16 * 4, hipMemcpyDeviceToHost, w->stream));
+  HIPCHK(hipStreamSynchronize(w->stream));
+  const uint32_t maxdeg = hc[kCtlMax];
+  a.local = maxdeg < kWideDeg;
+  a.hdeg = E < kSmallEdges ? kWideDeg : kHeavyDeg;
+  // slots: every in-edge, and empty ones where a slice's vertices differ (the
+  // widths of a tile's slices, or of all, never rise: less than 64 x the first)
+  const uint64_t nidx = E + (uint64_t)kWave * (std::min(maxdeg, kHeavyDeg) + 1ull) * (a.local ? tiles : 1u);
+  if ((rc = ws_buffer(w, kBufUnion, nidx * 4, &ibuf))) return rc;
+  a.idx = (uint32_t *)ibuf;
+  hipLaunchKernelGGL(pr_hist_kernel, dim3(tiles), dim3(kPrBlock), 0, w->stream, a);
+  hipLaunchKernelGGL(scan_tile_kernel, dim3((uint32_t)hscan), dim3(kScanBlock), 0, w->stream, a.hist, (uint32_t)nhist,
+                     a.hist, hist_tiles);
+  hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kScanBlock), 0, w->stream, hist_tiles, (uint32_t)hscan, total);
+  hipLaunchKernelGGL(pr_place_kernel, dim3(tiles), dim3(kPrBlock), 0, w->stream, a);
+  hipLaunchKernelGGL(pr_shape_kernel, dim3(vgrid), dim3(256), 0, w->stream, a);
+  hipLaunchKernelGGL(scan_tile_kernel, dim3((uint32_t)sscan), dim3(kScanBlock), 0, w->stream, a.shape,
+                     (uint32_t)nshape, a.shape, shape_tiles);
+  hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kScanBlock), 0, w->stream, shape_tiles, (uint32_t)sscan, total);
+  hipLaunchKernelGGL(pr_chunks_kernel, dim3(vgrid), dim3(256), 0, w->stream, a);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(hc, a.ctl, 16 * 4, hipMemcpyDeviceToHost, w->stream));
+  HIPCHK(hipStreamSynchronize(w->stream));
+  const uint32_t nheavy = hc[kCtlHeavy];
+  a.heavy = nheavy;
+  a.live = hc[kCtlLive];
+  a.nchunks = hc[kCtlChunks];
+  a.nslices = (a.live - a.heavy + kWave - 1) / kWave;
+  a.wide = std::min(a.nslices, (hc[kCtlWide] - nheavy * (a.local ? 0u : 1u) + kWave - 1) / kWave);
+  a.slots = ((size_t)hc[kCtlEdges] + kWave - 1) / kWave * kWave;
+  if (nheavy > a.nh || a.nchunks > maxchunks || a.nslices > a.ns)
+    return fail(LSG_ERR_CAPACITY, "pagerank: the reverse graph's degrees exceed its edge count");
+  hipLaunchKernelGGL(pr_layout_kernel, dim3(8u * w->cus), dim3(kPrBlock), 0, w->stream, a);
+  a.units = (uint32_t)((uint64_t)a.nchunks + a.wide + (a.nslices - a.wide + kSlices - 1) / kSlices);
+  const bool tab = V >= kTabSize && E >= kTabEdges && hc[kCtlHot] >= E / kTabShare;
+  a.turn = E >= kTurnEdges;
+  const uint32_t sgrid = tab ? (uint32_t)w->cus : ((a.units + kPrBlock / kWave - 1) / (kPrBlock / kWave) + 7) / 8 * 8;
+  a.fused = maxdeg <= kChunk && !tab && sgrid && sgrid <= kFusedBlocks;
+  const uint32_t fgrid = std::max(1u, maxdeg <= kChunk ? 1u : (nheavy + kPrBlock - 1) / kPrBlock);
   for (uint32_t it = 0; it < (uint32_t)max_iterations;) {
     const uint32_t end = std::min<uint32_t>((uint32_t)max_iterations, it + kIterBatch);
     for (; it < end; ++it) {
-      a.p_cur = p[it & 1];
-      a.c_cur = c[it & 1];
-      a.p_next = p[(it & 1) ^ 1];
-      a.c_next = c[(it & 1) ^ 1];
-      a.maxdiff = ctl + kCtlMax + (it & 1);
-      hipLaunchKernelGGL(pr_light_kernel, dim3(vgrid), dim3(256), 0, w->stream, a);
-      if (nheavy) {
-        hipLaunchKernelGGL(pr_chunk_kernel, dim3(cgrid), dim3(256), 0, w->stream, a);
-        hipLaunchKernelGGL(pr_finish_kernel, dim3(fgrid), dim3(256), 0, w->stream, a);
-      }
-      hipLaunchKernelGGL(pr_step_kernel, dim3(1), dim3(1), 0, w->stream, ctl, it, epsilon);
+      if (tab) hipLaunchKernelGGL(pr_sweep_kernel<true>, dim3(sgrid), dim3(kTabBlock), 0, w->stream, a, it);
+      else if (sgrid) hipLaunchKernelGGL(pr_sweep_kernel<false>, dim3(sgrid), dim3(kPrBlock), 0, w->stream, a, it);
+      if (!a.fused) hipLaunchKernelGGL(pr_finish_kernel, dim3(fgrid), dim3(kPrBlock), 0, w->stream, a, it);
     }
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(hc, ctl + kCtlDone, 4, hipMemcpyDeviceToHost, w->stream));
+    HIPCHK(hipMemcpyAsync(hc, a.ctl, 16 * 4, hipMemcpyDeviceToHost, w->stream));
     HIPCHK(hipStreamSynchronize(w->stream));
-    if (hc[0]) break;
+    if (hc[kCtlDone]) break;
   }
-  HIPCHK(hipMemcpyAsync(hc, ctl + kCtlIters, 4, hipMemcpyDeviceToHost, w->stream));
-  HIPCHK(hipStreamSynchronize(w->stream));
-  const int iters = (int)hc[0];
-  HIPCHK(hipMemcpyAsync(rank_dev, p[iters & 1], (size_t)V * 4, hipMemcpyDeviceToDevice, w->stream));
+  const int iters = (int)hc[kCtlIters];
+  hipLaunchKernelGGL(pr_ranks_kernel, dim3(vgrid), dim3(256), 0, w->stream, a, rank_dev);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(w->ev1, w->stream));
   HIPCHK(hipEventSynchronize(w->ev1));
   float ms = 0;
@@ -357,7 +660,7 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
     stats->ms_kernel = ms;
     stats->iterations = (uint64_t)iters;
     stats->items = nheavy;
-    stats->grid_blocks = (int32_t)vgrid;
+    stats->grid_blocks = (int32_t)sgrid;
     stats->block_size = 256;
     stats->ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   }
