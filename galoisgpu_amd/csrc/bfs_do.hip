@@ -32,20 +32,7 @@
 namespace lsg {
 
 constexpr int kDoBlock = 256;
-constexpr uint32_t kScatterRun = 16;  // edges per thread when finding edge sources
 constexpr uint32_t kAlpha = 14, kBeta = 24;
-
-// ---- reverse CSR ------------------------------------------------------------
-
-// Adds each tile's offset; writes the row starts and the scatter cursors.
-__global__ void scan_add_kernel(uint32_t *row, uint32_t n, const uint32_t *tile_off, uint32_t *cursor,
-                                const uint32_t *total) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i <= n; i += (size_t)gridDim.x * blockDim.x) {
-    const uint32_t r = i < n ? row[i] + tile_off[i / kScanTile] : *total;
-    row[i] = r;
-    if (cursor && i < n) cursor[i] = r;
-  }
-}
 
 // ---- reverse CSR by a stable radix sort ------------------------------------------
 //
@@ -53,101 +40,187 @@ __global__ void scan_add_kernel(uint32_t *row, uint32_t n, const uint32_t *tile_
 // weight) triples by destination with a stable sort gives each reverse row
 // in ascending source order: the reverse CSR is the same on every call (a
 // PageRank sum over in-edges has one order) and a bottom-up search meets low
-// source ids first.  LSD radix sort, 8 bits per pass; each pass is a per-tile
-// digit histogram, a prefix sum over (digit, tile), and a stable scatter that
-// ranks equal digits within a wavefront by ballots.  No atomics on global
+// source ids first.  LSD radix sort, at most 8 bits per pass (the destination's
+// bits spread evenly over the passes); each pass is a per-tile digit histogram,
+// a prefix sum over (digit, tile), and a stable scatter.  No atomics on global
 // memory: the atomic-counter version serialised on the in-degree counters of
 // the hubs (RMAT-20: 4.3 ms).
+//
+// The scatter is bound by memory: 24 bytes per edge and pass.  A block ranks
+// its tile's elements by digit (ballots within a wavefront, counters per
+// wavefront), puts them in digit order through LDS and writes each digit's
+// run, kRadixTile / 256 = 32 elements on average, as one (writing every element
+// to its place as it was ranked: 1.27 ms per pass on RMAT-22, now 0.40: 3.9 TB/s).  The
+// first pass finds the sources from the row starts, 64 rows at a time in the
+// wavefront's lanes, instead of reading them from an array written before
+// (0.81 ms).
 
-constexpr uint32_t kRadixTile = 16384;                 // elements per block
-constexpr uint32_t kRadixIters = kRadixTile / kDoBlock;  // elements per thread, strided by the block
+constexpr int kRadixBlock = 512;
+constexpr uint32_t kRadixTile = 8192;                        // elements per block
+constexpr uint32_t kRadixPer = kRadixTile / kRadixBlock;     // per thread
+constexpr uint32_t kRadixWave = kWave * kRadixPer;           // per wavefront, consecutive
 
-// src[e] = the source of edge e; thread t takes edges [16 t, 16 t + 16).
-__global__ void edge_source_kernel(const uint32_t *row_start, uint32_t V, uint32_t E, uint32_t *src) {
-  const size_t nthreads = (size_t)gridDim.x * blockDim.x;
-  for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t * kScatterRun < E; t += nthreads) {
-    const uint32_t e0 = (uint32_t)(t * kScatterRun), e1 = min(E, e0 + kScatterRun);
-    uint32_t lo = 0, hi = V;  // last u with row_start[u] <= e0
-    while (hi - lo > 1) {
-      const uint32_t mid = lo + (hi - lo) / 2;
-      if (row_start[mid] <= e0) lo = mid;
-      else hi = mid;
-    }
-    uint32_t u = lo, next = row_start[u + 1];
-    for (uint32_t e = e0; e < e1; ++e) {
-      while (next <= e) next = row_start[++u + 1];
-      src[e] = u;
-    }
-  }
-}
+struct RadixArgs {
+  const uint32_t *row_start;               // first pass: forward row starts
+  const uint32_t *key, *v1, *v2;           // v1 null: first pass; v2 null: zeros
+  uint32_t *key_out, *v1_out, *v2_out;
+  uint32_t *hist;                          // [256][ntiles] counts, then places within a scan tile
+  const uint32_t *hist_tiles;              // the scan's tile offsets
+  uint32_t n, V, shift, mask, ntiles;
+};
 
 // hist[d * ntiles + b] = elements of tile b whose digit is d.
-__global__ __launch_bounds__(kDoBlock) void radix_hist_kernel(const uint32_t *key, uint32_t n, uint32_t shift,
-                                                              uint32_t ntiles, uint32_t *hist) {
+__global__ __launch_bounds__(kRadixBlock) void radix_hist_kernel(RadixArgs a) {
   __shared__ uint32_t h[256];
-  h[threadIdx.x] = 0;
+  if (threadIdx.x < 256) h[threadIdx.x] = 0;
   __syncthreads();
-  const size_t base = (size_t)blockIdx.x * kRadixTile;
-  for (uint32_t it = 0; it < kRadixIters; ++it) {
-    const size_t e = base + (size_t)it * kDoBlock + threadIdx.x;
-    if (e < n) atomicAdd(&h[(key[e] >> shift) & 255u], 1u);
+  const uint32_t base = blockIdx.x * kRadixTile, count = min(a.n - base, kRadixTile);
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it) {
+    const uint32_t i = it * kRadixBlock + threadIdx.x;
+    if (i < count) atomicAdd(&h[(a.key[base + i] >> a.shift) & a.mask], 1u);
   }
   __syncthreads();
-  hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+  if (threadIdx.x <= a.mask) a.hist[(size_t)threadIdx.x * a.ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter of tile b: element e (in tile order: iteration, wavefront,
-// lane) goes to off[d * ntiles + b] + the number of earlier elements of the
-// tile with the same digit d.
-__global__ __launch_bounds__(kDoBlock) void radix_scatter_kernel(const uint32_t *key, const uint32_t *v1,
-                                                                 const uint32_t *v2, uint32_t n, uint32_t shift,
-                                                                 uint32_t ntiles, const uint32_t *off,
-                                                                 uint32_t *key_out, uint32_t *v1_out,
-                                                                 uint32_t *v2_out) {
-  constexpr uint32_t NW = kDoBlock / kWave;
-  __shared__ uint32_t run[256];      // next position per digit
-  __shared__ uint32_t wcnt[NW][256];  // this iteration's count per wavefront and digit
-  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
-  run[threadIdx.x] = off[(size_t)threadIdx.x * ntiles + blockIdx.x];
-  for (uint32_t k = 0; k < NW; ++k) wcnt[k][threadIdx.x] = 0;
+// Writes the tile's values x[] (element of thread and step) in digit order:
+// LDS place lp[], global place of thread i's p-th element in that order gp[].
+__device__ __forceinline__ void radix_write(uint32_t *buf, const uint32_t (&x)[kRadixPer],
+                                            const uint32_t (&lp)[kRadixPer], const uint32_t (&gp)[kRadixPer],
+                                            uint32_t count, uint32_t *out) {
   __syncthreads();
-  const size_t base = (size_t)blockIdx.x * kRadixTile;
-  for (uint32_t it = 0; it < kRadixIters; ++it) {
-    const size_t e = base + (size_t)it * kDoBlock + threadIdx.x;
-    const bool valid = e < n;
-    uint32_t k = 0, a = 0, b = 0, d = 0;
-    if (valid) {
-      k = key[e];
-      a = v1[e];
-      b = v2 ? v2[e] : 0u;
-      d = (k >> shift) & 255u;
-    }
-    // lanes holding the same digit: AND over the digit's 8 bits of the matching ballots
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it)
+    if (lp[it] < kRadixTile) buf[lp[it]] = x[it];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it) {
+    const uint32_t p = it * kRadixBlock + threadIdx.x;
+    if (p < count) out[gp[it]] = buf[p];
+  }
+}
+
+// Stable scatter of tile b: the elements of digit d go to its place for (d, b)
+// on, in tile order.
+template <bool kFirst>
+__global__ __launch_bounds__(kRadixBlock) void radix_scatter_kernel(RadixArgs a) {
+  constexpr uint32_t NW = kRadixBlock / kWave;
+  __shared__ uint32_t buf[kRadixTile];
+  __shared__ uint32_t wcnt[NW][256];  // per wavefront: count, then LDS place of its first element of the digit
+  __shared__ uint32_t goff[256];      // global place of a digit's run, less its LDS place
+  __shared__ uint32_t wsum[4];
+  const uint32_t lane = lane_id(), wv = threadIdx.x / kWave;
+  const uint32_t base = blockIdx.x * kRadixTile, count = min(a.n - base, kRadixTile);
+  const uint32_t first = wv * kRadixWave;  // this wavefront's elements in the tile
+  for (uint32_t d = lane; d < 256; d += kWave) wcnt[wv][d] = 0;
+  uint32_t k[kRadixPer], lp[kRadixPer], gp[kRadixPer];
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it) {
+    const uint32_t i = first + it * kWave + lane;
+    k[it] = a.key[base + min(i, count - 1)];
+  }
+  // rank within the wavefront's elements of the same digit
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it) {
+    const bool valid = first + it * kWave + lane < count;
+    const uint32_t d = (k[it] >> a.shift) & a.mask;
     uint64_t peers = __ballot(valid);
 #pragma unroll
     for (uint32_t bit = 0; bit < 8; ++bit) {
       const uint64_t m = __ballot((d >> bit) & 1u);
       peers &= ((d >> bit) & 1u) ? m : ~m;
     }
-    const uint32_t rank = (uint32_t)__builtin_popcountll(peers & ((1ull << lane) - 1));
-    if (valid && rank == 0) wcnt[wv][d] = (uint32_t)__builtin_popcountll(peers);
-    __syncthreads();
-    if (valid) {
-      uint32_t pos = run[d] + rank;
-      for (uint32_t w = 0; w < wv; ++w) pos += wcnt[w][d];
-      key_out[pos] = k;
-      v1_out[pos] = a;
-      v2_out[pos] = b;
-    }
-    __syncthreads();
-    uint32_t sum = 0;
-    for (uint32_t w = 0; w < NW; ++w) {
-      sum += wcnt[w][threadIdx.x];
-      wcnt[w][threadIdx.x] = 0;
-    }
-    run[threadIdx.x] += sum;
-    __syncthreads();
+    const uint32_t below = lanes_below(peers), before = wcnt[wv][d];
+    __builtin_amdgcn_wave_barrier();
+    if (valid && below == 0) wcnt[wv][d] = before + (uint32_t)__builtin_popcountll(peers);
+    __builtin_amdgcn_wave_barrier();
+    lp[it] = valid ? before + below : kRadixTile;
   }
+  __syncthreads();
+  // per digit: the wavefronts' counts become offsets, the digits' totals places
+  uint32_t total = 0, incl = 0;
+  if (threadIdx.x < 256) {
+#pragma unroll
+    for (uint32_t w = 0; w < NW; ++w) {
+      const uint32_t c = wcnt[w][threadIdx.x];
+      wcnt[w][threadIdx.x] = total;
+      total += c;
+    }
+    incl = total;
+#pragma unroll
+    for (int s = 1; s < kWave; s <<= 1) {
+      const uint32_t y = __shfl_up(incl, s);
+      if (lane >= (uint32_t)s) incl += y;
+    }
+    if (lane == kWave - 1) wsum[wv] = incl;
+  }
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    uint32_t start = incl - total;
+    for (uint32_t w = 0; w < wv; ++w) start += wsum[w];
+#pragma unroll
+    for (uint32_t w = 0; w < NW; ++w) wcnt[w][threadIdx.x] += start;
+    const size_t e = (size_t)threadIdx.x * a.ntiles + blockIdx.x;
+    if (threadIdx.x <= a.mask) goff[threadIdx.x] = a.hist[e] + a.hist_tiles[e / kScanTile] - start;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it) {
+    if (lp[it] < kRadixTile) {
+      lp[it] += wcnt[wv][(k[it] >> a.shift) & a.mask];
+      buf[lp[it]] = k[it];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it) {
+    const uint32_t p = it * kRadixBlock + threadIdx.x;
+    gp[it] = 0;
+    if (p < count) {
+      const uint32_t x = buf[p];
+      gp[it] = goff[(x >> a.shift) & a.mask] + p;
+      a.key_out[gp[it]] = x;
+    }
+  }
+  uint32_t x[kRadixPer];
+  if (kFirst) {
+    uint32_t u0 = 0, re = 0;  // 64 rows: the first, and the end of each
+#pragma unroll
+    for (uint32_t it = 0; it < kRadixPer; ++it) {
+      const uint32_t i = base + first + it * kWave + lane;
+      bool todo = lp[it] < kRadixTile;
+      x[it] = 0;
+      for (uint64_t m = __ballot(todo); m; m = __ballot(todo)) {
+        const uint32_t e = readlane(i, (uint32_t)__builtin_ctzll(m));
+        if (readlane(re, kWave - 1) <= e) {
+          u0 = wave_row_near(a.row_start, a.V, e);
+          re = glb(a.row_start)[min(u0 + lane, a.V - 1) + 1];
+        }
+        uint32_t pos = 0;  // rows that end at or before edge i
+#pragma unroll
+        for (uint32_t s = kWave / 2; s >= 1; s >>= 1)
+          if (__shfl(re, pos + s - 1) <= i) pos += s;
+        if (todo && i < readlane(re, kWave - 1)) {
+          x[it] = u0 + pos;
+          todo = false;
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (uint32_t it = 0; it < kRadixPer; ++it) {
+      const uint32_t i = first + it * kWave + lane;
+      x[it] = a.v1[base + min(i, count - 1)];
+    }
+  }
+  radix_write(buf, x, lp, gp, count, a.v1_out);
+#pragma unroll
+  for (uint32_t it = 0; it < kRadixPer; ++it) {
+    const uint32_t i = first + it * kWave + lane;
+    x[it] = a.v2 ? a.v2[base + min(i, count - 1)] : 0u;
+  }
+  radix_write(buf, x, lp, gp, count, a.v2_out);
 }
 
 // Row starts of the reverse CSR from the sorted destinations: the first
@@ -456,10 +529,8 @@ int lsg_graph_transpose(const lsg_graph *g, lsg_graph *gt) {
   std::lock_guard<std::mutex> lk(w->mu);
   HIPCHK(hipSetDevice(w->device));
   const uint32_t V = g->nnodes, E = g->nedges;
-  // (destination, source, weight) triples sorted by destination, 8 bits per
-  // pass; pass p writes slot (P - p) & 1, so the last pass lands in slot 1,
-  // the output arrays.  Pass 0 reads the forward arrays and the sources,
-  // which sit in the slot pass 0 does not write.
+  // (destination, source, weight) triples sorted by destination; pass p writes
+  // slot (P - p) & 1, so the last pass lands in slot 1, the output arrays.
   uint32_t bits = 0;
   while (bits < 32 && (V > 1 ? (uint64_t)(V - 1) >> bits : 0) != 0) ++bits;
   const uint32_t P = std::max<uint32_t>(1, (bits + 7) / 8);
@@ -485,27 +556,35 @@ int lsg_graph_transpose(const lsg_graph *g, lsg_graph *gt) {
   uint32_t *vs[2] = {(uint32_t *)((char *)tbuf + 2 * ne4), t.edge_dst};
   uint32_t *vw[2] = {(uint32_t *)((char *)tbuf + 3 * ne4), (uint32_t *)t.edge_data};
   uint32_t *hist = (uint32_t *)hbuf, *htiles = hist + nh + 1, *htotal = htiles + hscan;
-  const uint32_t sgrid = (uint32_t)std::min<uint64_t>(((uint64_t)E / kScatterRun + 256) / 256, 16ull * w->cus);
-  const uint32_t first_out = P & 1;
-  uint32_t *src0 = vs[first_out ^ 1];
   if (E) {
-    hipLaunchKernelGGL(edge_source_kernel, dim3(sgrid), dim3(256), 0, w->stream, g->row_start, V, E, src0);
-    const uint32_t *kin = g->edge_dst, *sin = src0, *win = (const uint32_t *)g->edge_data;
-    // (an unweighted forward graph passes win = null: its reverse weights are 0)
+    RadixArgs a;
+    a.row_start = g->row_start;
+    a.key = g->edge_dst;
+    a.v1 = nullptr;
+    a.v2 = (const uint32_t *)g->edge_data;  // (null for an unweighted graph: its reverse weights are 0)
+    a.hist = hist;
+    a.hist_tiles = htiles;
+    a.n = E;
+    a.V = V;
+    a.shift = 0;
+    a.ntiles = ntiles;
     for (uint32_t p = 0; p < P; ++p) {
-      const uint32_t o = (P - p) & 1, shift = 8 * p;
-      hipLaunchKernelGGL(radix_hist_kernel, dim3(ntiles), dim3(kDoBlock), 0, w->stream, kin, E, shift, ntiles, hist);
-      hipLaunchKernelGGL(scan_tile_kernel, dim3(hscan), dim3(kDoBlock), 0, w->stream, hist, (uint32_t)nh, hist,
-                         htiles);
-      hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kDoBlock), 0, w->stream, htiles, hscan, htotal);
-      const uint32_t agrid = (uint32_t)std::min<uint64_t>((nh + 256) / 256, 16ull * w->cus);
-      hipLaunchKernelGGL(scan_add_kernel, dim3(agrid), dim3(256), 0, w->stream, hist, (uint32_t)nh,
-                         (const uint32_t *)htiles, (uint32_t *)nullptr, (const uint32_t *)htotal);
-      hipLaunchKernelGGL(radix_scatter_kernel, dim3(ntiles), dim3(kDoBlock), 0, w->stream, kin, sin, win, E, shift,
-                         ntiles, (const uint32_t *)hist, key[o], vs[o], vw[o]);
-      kin = key[o];
-      sin = vs[o];
-      win = vw[o];
+      const uint32_t o = (P - p) & 1, width = (bits - a.shift + (P - p) - 1) / (P - p);
+      a.mask = (1u << width) - 1;
+      a.key_out = key[o];
+      a.v1_out = vs[o];
+      a.v2_out = vw[o];
+      const uint64_t n = ((uint64_t)a.mask + 1) * ntiles;
+      const uint32_t nscan = (uint32_t)((n + kScanTile - 1) / kScanTile);
+      hipLaunchKernelGGL(radix_hist_kernel, dim3(ntiles), dim3(kRadixBlock), 0, w->stream, a);
+      hipLaunchKernelGGL(scan_tile_kernel, dim3(nscan), dim3(kScanBlock), 0, w->stream, hist, (uint32_t)n, hist, htiles);
+      hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kScanBlock), 0, w->stream, htiles, nscan, htotal);
+      if (p == 0) hipLaunchKernelGGL(radix_scatter_kernel<true>, dim3(ntiles), dim3(kRadixBlock), 0, w->stream, a);
+      else hipLaunchKernelGGL(radix_scatter_kernel<false>, dim3(ntiles), dim3(kRadixBlock), 0, w->stream, a);
+      a.key = key[o];
+      a.v1 = vs[o];
+      a.v2 = vw[o];
+      a.shift += width;
     }
   }
   const uint32_t rgrid = (uint32_t)std::min<uint64_t>(((uint64_t)E + 256) / 256, 16ull * w->cus);

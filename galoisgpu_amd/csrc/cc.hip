@@ -173,20 +173,6 @@ __device__ __forceinline__ void cc_join(uint32_t *label, uint32_t &a, uint32_t &
   a = hooked ? lo : seen;
 }
 
-// A vertex at most 63 below the source of edge e (e < E): the wavefront
-// narrows [0, V) 64-fold per step.
-__device__ __forceinline__ uint32_t cc_row_near(const CcArgs &a, uint32_t e) {
-  uint32_t lo = 0, hi = a.V;
-  while (hi - lo > (uint32_t)kWave) {
-    const uint32_t step = (hi - lo + kWave - 1) / kWave;
-    const uint64_t i = lo + (uint64_t)lane_id() * step + step - 1;
-    const bool below = i < hi && glb(a.row_start)[i + 1] <= e;  // the source lies above vertex i
-    lo += (uint32_t)__builtin_popcountll(__ballot(below)) * step;
-    hi = min(hi, lo + step);
-  }
-  return lo;
-}
-
 // Joins the listed pairs, lane i's px and py for i < n.
 __device__ __forceinline__ void cc_join_listed(uint32_t *label, uint32_t n, uint32_t px, uint32_t py) {
   if (lane_id() >= n) px = py;
@@ -210,7 +196,7 @@ __device__ void cc_edge_pass(const CcArgs &a) {
     uint32_t e = t * kCcTile;
     const uint32_t left = a.E - e, tile_end = e + min(left, kCcTile);
     while (e < tile_end) {
-      const uint32_t u0 = cc_row_near(a, e);
+      const uint32_t u0 = wave_row_near(a.row_start, a.V, e);
       const uint32_t re = glb(a.row_start)[min(u0 + lane, a.V - 1) + 1];
       const uint32_t lab = glb(a.label)[min(u0 + lane, a.V - 1)];
       const uint32_t end = min(tile_end, readlane(re, kWave - 1));  // > e

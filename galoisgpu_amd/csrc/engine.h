@@ -238,6 +238,20 @@ __device__ __forceinline__ uint32_t wave_reserve(uint32_t n, uint32_t *tail) {
   return base + x - n;
 }
 
+// A vertex at most 63 below the source of CSR edge e (e < row_start[V]; e is
+// wave-uniform): the wavefront narrows [0, V) 64-fold per step.
+__device__ __forceinline__ uint32_t wave_row_near(const uint32_t *row_start, uint32_t V, uint32_t e) {
+  uint32_t lo = 0, hi = V;
+  while (hi - lo > (uint32_t)kWave) {
+    const uint32_t step = (hi - lo + kWave - 1) / kWave;
+    const uint64_t i = lo + (uint64_t)lane_id() * step + step - 1;
+    const bool below = i < hi && glb(row_start)[i + 1] <= e;  // the source lies above vertex i
+    lo += (uint32_t)__builtin_popcountll(__ballot(below)) * step;
+    hi = min(hi, lo + step);
+  }
+  return lo;
+}
+
 // ---- grid barrier ----------------------------------------------------------
 
 // One block's arrival (thread 0): true in the block that completes the barrier.
