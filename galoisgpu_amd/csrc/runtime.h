@@ -32,6 +32,7 @@ enum BufSlot {
   kBufLb,
   kBufValidate,
   kBufGraphPiles,
+  kBufWave,
   kBufCount
 };
 

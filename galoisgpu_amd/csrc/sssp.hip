@@ -1,5 +1,7 @@
 // Single-source traversal on gfx950: fixed-delta near/far SSSP and
-// level-synchronous BFS in one persistent, cooperatively launched kernel.
+// level-synchronous BFS in one persistent launch: the wavefront kernel
+// (wave.hip) where the options are the defaults', else persistent_kernel
+// (sssp_dev.h).
 //
 // Reference path: apps/sssp/kernel.cu (gg_main :455, persistent driver
 // gg_main_pipe_1_gpu_gb :355-391, relax operator sssp_kernel_dev :177-306,
@@ -29,6 +31,7 @@
 #include "runtime.h"
 #include "sched_mlp.h"
 #include "sssp_dev.h"
+#include "wave.h"
 
 namespace lsg {
 
@@ -55,38 +58,59 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
                     uint32_t *dist, bool graph_launch, lsg_stats *st, const Resume *resume = nullptr) {
   auto t0 = std::chrono::steady_clock::now();
   int bs, rc;
-  KArgs a;
+  WaveArgs a;
   void *seedbuf;
-  if ((rc = setup_single<A>(w, g, nseeds, o, dist, &a, &seedbuf, &bs))) return rc;
-  HIPCHK(hipMemcpyAsync(seedbuf, seeds, (size_t)nseeds * 4, hipMemcpyHostToDevice, w->stream));
+  // The wavefront kernel takes what a call asks for by default; the options
+  // that it does not have run in the persistent kernel.
+  const bool wave = o.expand_mode == LSG_EXPAND_LB && o.far_mode == LSG_FAR_REFERENCE && !o.sched && !o.trace;
+  lsg_opts ow = o;
+  if (wave) {
+    if (ow.block_size == 0) ow.block_size = kWaveBlock;
+    if (ow.heavy_deg <= 0) ow.heavy_deg = kWaveHeavyDeg;
+    ow.heavy_deg = std::min(ow.heavy_deg, 1 << 24);  // 64 lighter vertices' edges are counted in 32 bits
+  }
+  if ((rc = setup_single<A>(w, g, nseeds, ow, dist, &a, &seedbuf, &bs))) return rc;
+  if (wave) {
+    void *wbuf;
+    if ((rc = ws_buffer(w, kBufWave, sizeof(WaveCtrl), &wbuf))) return rc;
+    a.wc = (WaveCtrl *)wbuf;
+  }
+  // One seed of a plain launch goes to the wavefront kernel's initialisation as
+  // an argument; a captured launch must not depend on it.
+  const bool seed_arg = wave && nseeds == 1 && !graph_launch;
+  if (!seed_arg) HIPCHK(hipMemcpyAsync(seedbuf, seeds, (size_t)nseeds * 4, hipMemcpyHostToDevice, w->stream));
 
   KernelFn fn = A == Algo::SSSP ? pick_kernel<Algo::SSSP>(bs) : pick_kernel<Algo::BFS>(bs);
+  const void *fnp = wave ? wave_kernel_fn(A, bs) : (const void *)fn;
   int grid = 0;
-  if ((rc = resident_grid(w, (const void *)fn, bs, &grid))) return rc;
+  if ((rc = resident_grid(w, fnp, bs, &grid))) return rc;
   // Default: 2 blocks per CU at most for SSSP, 4 for BFS.  Fewer blocks per
   // grid barrier beat more parallel tiles (256-thread blocks; full resident
   // grid 1280 -> 512): RMAT-20 SSSP 2.24 -> 2.05 ms, road 2048^2 10.2 -> 8.3
   // ms, RMAT-22 6.31 -> 6.23 ms, grid 256^2 12.9 -> 12.8 ms; BFS levels are
   // wider and cheaper, RMAT-20 BFS 0.56 ms at 1280, 0.55 at 1024, 0.60 at 512.
   if (o.grid_blocks > 0) grid = std::min(o.grid_blocks, grid);
+  else if (wave) grid = std::min(grid, wave_blocks_per_cu(g.nnodes, g.nedges) * (int)w->cus);
   else grid = std::min(grid, (A == Algo::BFS ? 4 : 2) * (int)w->cus);
 
+  const KArgs &ka = a;
   Ctrl hc;
   float ms = 0;
   for (int attempt = 0;; ++attempt) {
     const uint32_t init_blocks = std::min<uint32_t>((g.nnodes + 255) / 256, 8u * w->cus);
     const uint32_t *sd = (const uint32_t *)seedbuf;
     auto enqueue = [&]() -> int {
+      if (wave) return wave_enqueue(A, bs, grid, a, seeds[0], seed_arg ? nullptr : sd, nseeds, resume, w->cus, w->stream);
       if (resume) {
-        hipLaunchKernelGGL(resume_init_kernel, dim3(init_blocks), dim3(256), 0, w->stream, a, a.delta,
+        hipLaunchKernelGGL(resume_init_kernel, dim3(init_blocks), dim3(256), 0, w->stream, ka, a.delta,
                            resume->curdelta);
-        hipLaunchKernelGGL(resume_seed_kernel, dim3(init_blocks), dim3(256), 0, w->stream, a, resume->lo,
+        hipLaunchKernelGGL(resume_seed_kernel, dim3(init_blocks), dim3(256), 0, w->stream, ka, resume->lo,
                            resume->hi);
       } else {
-        hipLaunchKernelGGL(init_kernel, dim3(init_blocks), dim3(256), 0, w->stream, a, a.delta);
-        hipLaunchKernelGGL(seed_kernel, dim3(1), dim3(256), 0, w->stream, a, sd, nseeds);
+        hipLaunchKernelGGL(init_kernel, dim3(init_blocks), dim3(256), 0, w->stream, ka, a.delta);
+        hipLaunchKernelGGL(seed_kernel, dim3(1), dim3(256), 0, w->stream, ka, sd, nseeds);
       }
-      hipLaunchKernelGGL(fn, dim3(grid), dim3(bs), 0, w->stream, a);
+      hipLaunchKernelGGL(fn, dim3(grid), dim3(bs), 0, w->stream, ka);
       HIPCHK(hipGetLastError());
       return LSG_OK;
     };
@@ -94,6 +118,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     if (graph_launch && !resume) {
       std::vector<uint8_t> key;
       key_append(key, (int)A);
+      key_append(key, wave);
       key_append(key, a);
       key_append(key, grid);
       key_append(key, bs);
@@ -113,7 +138,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
       return fail(LSG_ERR_HIP, "persistent grid of %d x %d blocks is not co-resident (%u were)", grid, bs,
                   hc.resident_seen);
     grid = (int)hc.resident_seen;
-    record_resident_grid(w, (const void *)fn, bs, grid);
+    record_resident_grid(w, fnp, bs, grid);
   }
   if (hc.abort == kAbortTimeout)
     return fail(LSG_ERR_TIMEOUT,

@@ -1,0 +1,54 @@
+// Single-source traversal by wavefronts (wave.hip): what its host side needs.
+#pragma once
+
+#include "sssp_dev.h"
+
+namespace lsg {
+
+constexpr int kWaveMsg = 5;
+
+// Words of the wavefront kernel beside the control block, each group of words
+// that one atomic unit serves on a line of its own.
+struct WaveCtrl {
+  // The state of the next round, published by the last block to reach the
+  // barrier: value << 32 | generation, so that a word is valid by itself and
+  // a waiting block needs no second load and the publisher no ordering.
+  // Items, heavy chunks, round, phase, roles and flags.
+  uint64_t msg[kWaveMsg];
+  uint64_t _p0[16 - kWaveMsg];
+  struct Line {
+    uint32_t n;
+    uint32_t _p[31];
+  } near_tail[3], heavy_tail[3],  // by generation mod 3: the leader of one round clears the words of the one after the next
+      far_tail[3],                // by queue
+      ticket[3][16];              // by generation mod 3 and group of blocks
+};
+
+struct WaveArgs : KArgs {
+  WaveCtrl *wc = nullptr;
+};
+
+// Blocks per CU, of 256 threads, where the call leaves the launch shape open.
+// Each block more makes a grid barrier dearer, each wavefront fewer the large
+// rounds longer; low-degree graphs have few of those.  Ms at 1 / 2 / 3 blocks:
+// RMAT-17 SSSP 0.50 / 0.53 / 0.54, RMAT-18 0.59 / 0.56 / 0.57, RMAT-20 1.33 /
+// 1.15 / 1.12, RMAT-21 2.31 / 1.78 / 1.71, RMAT-18 BFS 0.160 / 0.150 / 0.159,
+// RMAT-21 0.68 / 0.50 / 0.46; road-like 1000^2 SSSP 2.61 / 2.68 / 2.75, 2048^2
+// 3.76 / 3.87 / 3.99, BFS 1.54 / 1.64 / 1.70.  The same wavefronts in blocks of
+// 512: RMAT-18 0.73, RMAT-20 1.18, 2048^2 3.78; 1024 worse still.
+constexpr int kWaveBlock = 256;
+inline int wave_blocks_per_cu(uint64_t nnodes, uint64_t nedges) {
+  return nedges <= 6 * nnodes || nedges < 3u << 20 ? 1 : nedges < 1u << 25 ? 2 : 3;
+}
+// A chunk of a heavy vertex is the edges that a wavefront holds in flight
+// (kWaveU a lane); 512 and 1024: equal to 5 % slower on RMAT graphs.
+constexpr int kWaveHeavyDeg = 256;
+
+// Block sizes 256, 512 and 1024.
+const void *wave_kernel_fn(Algo algo, int bs);
+// Enqueues initialisation and traversal: from one seed (seeds null), from
+// several, or, with `resume`, from the distances in a.dist.
+int wave_enqueue(Algo algo, int bs, int grid, const WaveArgs &a, uint32_t seed, const uint32_t *seeds, uint32_t nseeds,
+                 const Resume *resume, int cus, hipStream_t stream);
+
+}  // namespace lsg

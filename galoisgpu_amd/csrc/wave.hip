@@ -1,0 +1,709 @@
+// Single-source SSSP and BFS in one persistent launch, by wavefronts.
+//
+// The rounds, piles and phases are the reference's (apps/sssp/kernel.cu:355-391
+// near/far piles, curdelta += DELTA per phase, the whole far pile becoming the
+// next phase; apps/bfs/kernel.cu:312-334 levels), as in persistent_kernel
+// (sssp_dev.h), which remains for what this kernel does not take: split and
+// bucket far piles, degree-binned expansion, the learned scheduler, round
+// traces, the -l sweep and the no-allocation entry point.
+//
+// What bounds a traversal differs: on a skewed graph (RMAT-20, ~20 rounds) the
+// random distance loads of some 65 M edge relaxations, on a road network or a
+// grid (hundreds of rounds of a few hundred to a few thousand vertices) the
+// chain of dependent round trips of a round.
+//
+//   - Work units belong to wavefronts: up to 64 in-queue items whose edges are
+//     flattened over the lanes, or one chunk of a heavy vertex.  No block
+//     barrier inside a round, and a wavefront goes on to its next unit while
+//     others wait for memory.  (Tiles of a block waited for their slowest
+//     wavefront at every ticket.)
+//   - Pushes and heavy items are staged per wavefront in LDS and placed with
+//     one atomic per pile and block at the end of the round.
+//   - The barrier's message is the round: the last block to arrive publishes
+//     the next round's counts and roles as words that carry the generation, so
+//     that the waiting blocks read everything with the poll that sees it, and
+//     nothing has to be ordered before it.  Tails and tickets are used in turn
+//     by generation and cleared two rounds ahead.
+//   - Small rounds (at most kLocalMax items, no heavy vertex) are run by the
+//     last block alone, with entries in LDS as in the one-workgroup kernel
+//     (block.hip): two round trips and two block barriers a round while the
+//     others stay parked.  Far pushes go to the far queue as usual.  The block
+//     leaves this mode when the round it would run next is too large, and hands
+//     the vertices over through the near queue.
+//
+// Ms in persistent_kernel -> here: SSSP RMAT-17 0.53 -> 0.50, RMAT-20 1.60 ->
+// 1.15, RMAT-22 5.1 -> 2.9, road-like 2048^2 4.69 -> 3.76, 1000^2 3.45 -> 2.61,
+// grid 256^2 (delta 32) 8.8 -> 5.7, 64^2 1.6 -> 0.85; BFS RMAT-17 0.162 ->
+// 0.128, RMAT-20 0.447 -> 0.299, road-like 1023 x 777 1.16 -> 0.87.
+
+#include <hip/hip_runtime.h>
+
+#include "wave.h"
+
+namespace lsg {
+
+// Largest round that one block runs alone, and the entries of a pile in LDS (a
+// round's pushes are not deduplicated in there).
+constexpr uint32_t kLocalMax = 512;
+constexpr uint32_t kLocalCap = 1024;
+constexpr uint32_t kWavePush = 256;   // staged items per wavefront and pile
+constexpr uint32_t kWaveHeavy = 32;   // staged heavy items per wavefront
+constexpr uint32_t kTicketGroups = 16;
+// In-queue items per unit: 64, or fewer where that leaves wavefronts idle, but
+// at least this many, so that a small round involves few blocks (each block
+// with pushes reserves queue space with an atomic of its own).
+constexpr uint32_t kUnitMin = 16;
+
+// Roles of the three queues and the state of a round.
+struct WaveRound {
+  uint32_t items, heavy, round, phase;
+  uint32_t roles;  // in | near << 2 | far << 4
+  uint32_t flags;
+  __device__ uint32_t in_q() const { return roles & 3u; }
+  __device__ uint32_t near_q() const { return roles >> 2 & 3u; }
+  __device__ uint32_t far_q() const { return roles >> 4 & 3u; }
+};
+constexpr uint32_t kWaveDone = 1, kWaveLead = 2, kWaveLocal = 4;
+__device__ __forceinline__ uint32_t wave_roles(uint32_t in, uint32_t near, uint32_t far) {
+  return in | near << 2 | far << 4;
+}
+
+struct WaveHeavy {
+  uint32_t u, nch;
+};
+
+template <int BS>
+struct WaveShared {
+  static constexpr int NW = BS / kWave;
+  uint32_t push[NW][2][kWavePush];  // near, far
+  WaveHeavy heavy[NW][kWaveHeavy];
+  uint32_t count[NW][3];            // end of a round: near, far, heavy chunks
+  uint32_t base[3];
+  WaveRound r;
+  // rounds of one block
+  Entry pile[2][kLocalCap];
+  uint32_t pile_n[2];
+  uint32_t far_n;    // the far queue's length
+  uint32_t spill_n;  // vertices handed to the near queue
+  uint32_t stop;     // a vertex too heavy for this mode was pushed
+  unsigned long long items;
+};
+
+// A wavefront's view of the round.
+struct WaveLane {
+  uint32_t near_stamp, far_stamp;  // this round's and phase's stamps
+  uint32_t thr;                    // a candidate is near iff it is at most this
+  uint32_t *nq, *fq, *ntail, *ftail;
+  uint64_t *hq;
+  uint32_t *htail;
+  uint32_t *pbuf[2];
+  WaveHeavy *hbuf;
+  uint32_t n[2], hn, hch;  // staged: items per pile, heavy items and their chunks (wave-uniform)
+};
+
+__device__ __forceinline__ uint32_t *wave_queue(const WaveArgs &a, uint32_t i) {
+  uint32_t *const q0 = a.q[0], *const q1 = a.q[1], *const q2 = a.q[2];
+  return i == 0 ? q0 : i == 1 ? q1 : q2;
+}
+
+// ---- pushes -------------------------------------------------------------------
+
+// Writes pile `which`'s staged items to its queue from `base` on.
+__device__ __forceinline__ void wave_store(const WaveArgs &a, WaveLane &w, int which, uint32_t base) {
+  uint32_t *const q = which ? w.fq : w.nq;
+  for (uint32_t i = lane_id(); i < w.n[which]; i += kWave) {
+    const uint32_t pos = base + i;
+    if (pos < a.qcap) st_coh(q + pos, w.pbuf[which][i]);
+    else st_coh(&a.ctrl->abort, kAbortCapacity);
+  }
+  w.n[which] = 0;
+}
+
+// Pushes `item` from every lane with `pred` (whole wavefront).
+__device__ __forceinline__ void wave_stage(const WaveArgs &a, WaveLane &w, int which, bool pred, uint32_t item) {
+  const uint64_t m = __ballot(pred);
+  if (m == 0) return;
+  const uint32_t c = (uint32_t)__builtin_popcountll(m);
+  if (w.n[which] + c > kWavePush) {
+    uint32_t base = 0;
+    if (lane_id() == 0) base = atomic_add(which ? w.ftail : w.ntail, w.n[which]);
+    wave_store(a, w, which, readlane(base, 0));
+  }
+  if (pred) w.pbuf[which][w.n[which] + lanes_below(m)] = item;
+  w.n[which] += c;
+}
+
+// Writes the staged heavy items' chunks from slot `base` on.
+__device__ __forceinline__ void wave_store_heavy(const WaveArgs &a, WaveLane &w, uint32_t base) {
+  for (uint32_t i = 0; i < w.hn; ++i) {
+    const uint32_t u = __builtin_amdgcn_readfirstlane(w.hbuf[i].u), nch = __builtin_amdgcn_readfirstlane(w.hbuf[i].nch);
+    for (uint32_t k = lane_id(); k < nch; k += kWave) {
+      const uint32_t pos = base + k;
+      if (pos < a.hcap) st_coh64(w.hq + pos, (uint64_t)k << 32 | u);
+      else st_coh(&a.ctrl->abort, kAbortCapacity);
+    }
+    base += nch;
+  }
+  w.hn = w.hch = 0;
+}
+
+// Queues the vertices u of the lanes with `heavy` (degree deg) as chunks of
+// heavy_deg edges, expanded in the next round.
+__device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool heavy, uint32_t u, uint32_t deg) {
+  for (uint64_t m = __ballot(heavy); m; m &= m - 1) {
+    const uint32_t l = (uint32_t)__builtin_ctzll(m);
+    if (w.hn == kWaveHeavy) {
+      uint32_t base = 0;
+      if (lane_id() == 0) base = atomic_add(w.htail, w.hch);
+      wave_store_heavy(a, w, readlane(base, 0));
+    }
+    const uint32_t nch = (readlane(deg, l) - 1) / a.heavy_deg + 1;
+    if (lane_id() == 0) w.hbuf[w.hn] = WaveHeavy{readlane(u, l), nch};
+    w.hn += 1;
+    w.hch += nch;
+  }
+}
+
+// ---- relaxation ----------------------------------------------------------------
+
+// Relaxes edges e[k], k < U, leaving vertices at distance du[k], of the lanes
+// with act[k] (e[k] names some edge in every lane): the tests, atomics and
+// pushes of relax_edges in sssp_dev.h.
+template <Algo A, int U>
+__device__ __forceinline__ void wave_relax(const WaveArgs &a, WaveLane &w, const uint32_t (&e)[U],
+                                           const uint32_t (&du)[U], const bool (&act)[U]) {
+  uint32_t v[U], nd[U], dv[U], old[U], seen[U], got[U];
+  bool near[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    v[k] = glb(a.edge_dst)[e[k]];
+    nd[k] = A == Algo::SSSP ? du[k] + glb(a.edge_data)[e[k]] : du[k] + 1u;
+  }
+  // through the caches: a stale distance is only ever larger
+#pragma unroll
+  for (int k = 0; k < U; ++k) dv[k] = glb(a.dist)[v[k]];
+  uint32_t *const ns = a.near_stamp, *const fs = a.far_stamp;
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    near[k] = A == Algo::BFS || nd[k] <= w.thr;
+    const bool cand = act[k] && nd[k] < dv[k];
+    seen[k] = glb(near[k] ? ns : fs)[cand ? v[k] : 0u];
+    old[k] = cand ? atomic_min(a.dist + v[k], nd[k]) : 0u;
+  }
+  // results are taken only here (left to itself the compiler tests each
+  // result inside its atomic's branch, waiting for the whole memory queue)
+#pragma unroll
+  for (int k = 0; k < U; ++k) asm volatile("" : "+v"(old[k]));
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const uint32_t stamp = near[k] ? w.near_stamp : w.far_stamp;
+    const bool want = nd[k] < old[k] && seen[k] != stamp;
+    got[k] = want ? atomic_exch((near[k] ? ns : fs) + v[k], stamp) : stamp;
+  }
+#pragma unroll
+  for (int k = 0; k < U; ++k) asm volatile("" : "+v"(got[k]));
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const bool push = nd[k] < old[k] && got[k] != (near[k] ? w.near_stamp : w.far_stamp);
+    wave_stage(a, w, 0, push && near[k], v[k]);
+    if (A == Algo::SSSP) wave_stage(a, w, 1, push && !near[k], v[k]);
+  }
+}
+
+constexpr int kWaveU = 4;
+
+// Up to 64 in-queue items, one per lane below n: heavy ones are queued as
+// chunks, the others' edges flattened over the wavefront.
+template <Algo A>
+__device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const uint32_t *in, uint32_t n) {
+  const uint32_t lane = lane_id();
+  const uint32_t u = lane < n ? ld_coh(in + lane) : 0u;
+  uint32_t du = kInf, rs = 0, deg = 0;
+  if (lane < n) {
+    du = ld_coh(a.dist + u);
+    rs = glb(a.row_start)[u];
+    deg = glb(a.row_start)[u + 1] - rs;
+  }
+  if (du == kInf) deg = 0;
+  const bool heavy = deg >= a.heavy_deg;
+  wave_heavy(a, w, heavy, u, deg);
+  if (heavy) deg = 0;
+  uint32_t end = deg;  // inclusive prefix over the lanes
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint32_t y = __shfl_up(end, d);
+    if (lane >= (uint32_t)d) end += y;
+  }
+  const uint32_t total = readlane(end, kWave - 1);
+  const uint32_t base = rs - (end - deg);
+  for (uint32_t b0 = 0; b0 < total; b0 += kWaveU * kWave) {
+    uint32_t e[kWaveU], d0[kWaveU];
+    bool act[kWaveU];
+#pragma unroll
+    for (int k = 0; k < kWaveU; ++k) {
+      const uint32_t f = min(b0 + k * kWave + lane, total - 1);
+      act[k] = b0 + k * kWave + lane < total;
+      uint32_t pos = 0;  // items that end at or before f
+#pragma unroll
+      for (uint32_t d = kWave / 2; d >= 1; d >>= 1)
+        if ((uint32_t)__shfl(end, pos + d - 1) <= f) pos += d;
+      e[k] = (uint32_t)__shfl(base, pos) + f;
+      d0[k] = (uint32_t)__shfl(du, pos);
+    }
+    wave_relax<A, kWaveU>(a, w, e, d0, act);
+  }
+}
+
+// One chunk of a heavy vertex.
+template <Algo A>
+__device__ __forceinline__ void wave_chunk(const WaveArgs &a, WaveLane &w, const uint64_t *ent) {
+  const uint32_t lane = lane_id();
+  const uint64_t x = ld_coh64(ent);
+  const uint32_t u = __builtin_amdgcn_readfirstlane((uint32_t)x), c = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+  if (u >= a.nnodes) return;
+  const uint32_t du = ld_coh(a.dist + u);
+  const uint32_t row = glb(a.row_start)[u], deg = glb(a.row_start)[u + 1] - row, skip = c * a.heavy_deg;
+  if (skip >= deg) return;
+  const uint32_t rs = row + skip, n = min(deg - skip, a.heavy_deg);
+  for (uint32_t b0 = 0; b0 < n; b0 += kWaveU * kWave) {
+    uint32_t e[kWaveU], d0[kWaveU];
+    bool act[kWaveU];
+#pragma unroll
+    for (int k = 0; k < kWaveU; ++k) {
+      const uint32_t f = b0 + k * kWave + lane;
+      act[k] = f < n;
+      e[k] = rs + min(f, n - 1);
+      d0[k] = du;
+    }
+    wave_relax<A, kWaveU>(a, w, e, d0, act);
+  }
+}
+
+// ---- rounds of one block --------------------------------------------------------
+
+// The relaxation of such a round: improved neighbours are appended to the next
+// pile in LDS with the row bounds loaded beside the atomicMin, or, beyond the
+// threshold, to the far queue.
+template <Algo A, int BS>
+struct LocalRelax {
+  const WaveArgs &a;
+  WaveShared<BS> &sh;
+  uint32_t nxt, thr, near_stamp, far_stamp;
+  uint32_t *nq, *fq;
+  __device__ __forceinline__ bool stopped() const { return false; }
+  __device__ __forceinline__ void operator()(const KArgs &, const uint32_t (&v)[kInFlight],
+                                             const uint32_t (&nd)[kInFlight], const bool (&act)[kInFlight]) const {
+    uint32_t old[kInFlight], seen[kInFlight], got[kInFlight];
+    uint64_t rb[kInFlight];
+    bool near[kInFlight];
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k) {
+      near[k] = A == Algo::BFS || nd[k] <= thr;
+      old[k] = act[k] ? atomic_min(a.dist + v[k], nd[k]) : 0u;
+      rb[k] = ld_pair(a.row_start + v[k]);
+      seen[k] = A == Algo::SSSP ? glb(a.far_stamp)[act[k] && !near[k] ? v[k] : 0u] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k) asm volatile("" : "+v"(old[k]));
+    if (A == Algo::SSSP) {
+#pragma unroll
+      for (int k = 0; k < kInFlight; ++k) {
+        const bool want = act[k] && nd[k] < old[k] && !near[k] && seen[k] != far_stamp;
+        got[k] = want ? atomic_exch(a.far_stamp + v[k], far_stamp) : far_stamp;
+      }
+    }
+    // near: one reservation per wavefront
+    uint64_t m[kInFlight];
+    uint32_t t = 0;
+#pragma unroll
+    for (int k = 0; k < kInFlight; ++k) {
+      m[k] = __ballot(act[k] && nd[k] < old[k] && near[k]);
+      t += (uint32_t)__builtin_popcountll(m[k]);
+    }
+    if (t) {
+      uint32_t pos = 0;
+      if (lane_id() == 0) pos = atomicAdd(&sh.pile_n[nxt], t);
+      pos = readlane(pos, 0);
+#pragma unroll
+      for (int k = 0; k < kInFlight; ++k) {
+        if ((m[k] >> lane_id()) & 1) {
+          const uint32_t p = pos + lanes_below(m[k]);
+          const uint32_t rs = (uint32_t)rb[k], re = (uint32_t)(rb[k] >> 32);
+          if (re - rs >= a.heavy_deg) sh.stop = 1;
+          if (p < kLocalCap) sh.pile[nxt][p] = Entry{v[k], nd[k], rs, re};
+          else spill(v[k]);
+        }
+        pos += (uint32_t)__builtin_popcountll(m[k]);
+      }
+    }
+    if (A == Algo::SSSP) {
+#pragma unroll
+      for (int k = 0; k < kInFlight; ++k) asm volatile("" : "+v"(got[k]));
+      t = 0;
+#pragma unroll
+      for (int k = 0; k < kInFlight; ++k) {
+        m[k] = __ballot(act[k] && nd[k] < old[k] && !near[k] && got[k] != far_stamp);
+        t += (uint32_t)__builtin_popcountll(m[k]);
+      }
+      if (t) {
+        uint32_t pos = 0;
+        if (lane_id() == 0) pos = atomicAdd(&sh.far_n, t);
+        pos = readlane(pos, 0);
+#pragma unroll
+        for (int k = 0; k < kInFlight; ++k) {
+          if ((m[k] >> lane_id()) & 1) put(fq, pos + lanes_below(m[k]), v[k]);
+          pos += (uint32_t)__builtin_popcountll(m[k]);
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void put(uint32_t *q, uint32_t pos, uint32_t v) const {
+    if (pos < a.qcap) st_coh(q + pos, v);
+    else st_coh(&a.ctrl->abort, kAbortCapacity);
+  }
+  // A vertex that this mode hands on: once to the near queue.
+  __device__ __forceinline__ void spill(uint32_t v) const {
+    if (atomic_exch(a.near_stamp + v, near_stamp) != near_stamp) put(nq, atomicAdd(&sh.spill_n, 1u), v);
+  }
+};
+
+__device__ __forceinline__ uint32_t wave_threshold(const WaveArgs &a, int64_t cd0, uint32_t phase) {
+  const int64_t cd = cd0 + (int64_t)phase * a.delta;
+  return (uint32_t)min(cd, (int64_t)0xFFFFFFFFll);
+}
+
+// Called by every thread of the block that leads, with the next round in sh.r
+// (at most kLocalMax items, no heavy chunks): runs it and the rounds that
+// follow for as long as they are small, and leaves in sh.r the round that the
+// whole grid runs next.  Every wavefront's memory operations are complete on
+// return.
+template <Algo A, int BS>
+__device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh, int64_t cd0) {
+  WaveRound r = sh.r;
+  const uint32_t far_in = A == Algo::SSSP ? ld_coh(&a.wc->far_tail[r.far_q()].n) : 0u;
+  if (threadIdx.x == 0) {
+    sh.far_n = far_in;
+    sh.stop = 0;
+    sh.items = 0;
+  }
+  uint32_t rounds = 0, cur = 0, n = r.items;
+  bool load = true;  // the round's items are still in queue in_q
+  unsigned long long popped = 0;
+  for (;;) {
+    if (load) {
+      const uint32_t *const in = wave_queue(a, r.in_q());
+      bool big = false;
+      for (uint32_t i = threadIdx.x; i < n; i += BS) {
+        const uint32_t v = ld_coh(in + i);
+        const uint32_t d = ld_coh(a.dist + v);
+        const uint64_t rb = ld_pair(a.row_start + v);
+        sh.pile[cur][i] = Entry{v, d, (uint32_t)rb, (uint32_t)(rb >> 32)};
+        big |= (uint32_t)(rb >> 32) - (uint32_t)rb >= a.heavy_deg;
+      }
+      // a heavy vertex among them: the grid runs this round
+      if (__syncthreads_or(big)) break;
+      load = false;
+    }
+    if (threadIdx.x == 0) {
+      sh.pile_n[cur ^ 1] = 0;
+      sh.spill_n = 0;
+    }
+    __syncthreads();
+    const LocalRelax<A, BS> relax{a,           sh, cur ^ 1, wave_threshold(a, cd0, r.phase), r.round + 1, r.phase + 1,
+                                  wave_queue(a, r.near_q()), wave_queue(a, r.far_q())};
+    expand_entries<A, kLdsAS, BS>(a, (EntryPtr<kLdsAS>)sh.pile[cur], n, relax, &sh.items);
+    __syncthreads();  // every push of the round is in
+    popped += n;
+    ++rounds;
+    r.round += 1;
+    const uint32_t near = sh.pile_n[cur ^ 1], far = sh.far_n;
+    if (threadIdx.x == 0) st_coh(&a.ctrl->progress, r.round);
+    if (near > kLocalMax || sh.stop) {
+      // hand over: what spilled already, and the pile
+      for (uint32_t i = threadIdx.x; i < min(near, kLocalCap); i += BS) relax.spill(sh.pile[cur ^ 1][i].v);
+      __syncthreads();
+      n = sh.spill_n;
+      r.roles = wave_roles(r.near_q(), r.in_q(), r.far_q());
+      break;
+    }
+    if (near) {
+      cur ^= 1;
+      n = near;
+    } else if (far) {
+      // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
+      r.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
+      r.phase += 1;
+      n = far;
+      order_release();  // this wavefront's far pushes have landed
+      __syncthreads();  // and every other's; far_n has been read
+      if (threadIdx.x == 0) sh.far_n = 0;
+      if (n > kLocalMax) break;
+      load = true;
+    } else {
+      r.flags |= kWaveDone;
+      n = 0;
+      break;
+    }
+    // (the next round's first barrier separates the reads of sh above from its writes)
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    r.items = n;
+    r.heavy = 0;
+    sh.r = r;
+    if (A == Algo::SSSP) {
+      st_coh(&a.wc->far_tail[r.far_q()].n, sh.far_n);
+      if (r.far_q() != 0) st_coh(&a.wc->far_tail[0].n, 0u);
+      if (r.far_q() != 1) st_coh(&a.wc->far_tail[1].n, 0u);
+      if (r.far_q() != 2) st_coh(&a.wc->far_tail[2].n, 0u);
+    }
+    __hip_atomic_fetch_add(&a.ctrl->stat_items, (uint64_t)popped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_fetch_add(&a.ctrl->stat_rounds, (uint64_t)rounds, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  order_release();
+  __syncthreads();
+}
+
+// ---- the kernel -------------------------------------------------------------------
+
+template <Algo A, int BS>
+__global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
+  constexpr uint32_t NW = BS / kWave;
+  __shared__ WaveShared<BS> sh;
+  Ctrl *const c = a.ctrl;
+  WaveCtrl *const wc = a.wc;
+  const uint32_t nb = gridDim.x, wv = threadIdx.x / kWave;
+  const uint32_t wave = blockIdx.x * NW + wv, nwaves = nb * NW;
+  const uint32_t ngroups = min(kTicketGroups, nb), g = blockIdx.x % ngroups;
+  const uint32_t gblocks = (nb + ngroups - 1 - g) / ngroups;  // blocks of this group
+  if (!residency_handshake(c, nb, a.residency_limit)) return;
+  const int64_t cd0 = c->s.curdelta();  // written before this launch, as is the first round
+  if (threadIdx.x == 0) {
+    sh.r.items = c->s.in_count;
+    sh.r.heavy = 0;
+    sh.r.round = 1;
+    sh.r.phase = 0;
+    sh.r.roles = wave_roles(0, 1, 2);
+    sh.r.flags = 0;
+  }
+  __syncthreads();
+  WaveLane w;
+  w.pbuf[0] = sh.push[wv][0];
+  w.pbuf[1] = sh.push[wv][1];
+  w.hbuf = sh.heavy[wv];
+  w.n[0] = w.n[1] = w.hn = w.hch = 0;
+  for (uint32_t gen = 0;; ++gen) {
+    const WaveRound r = sh.r;
+    if (r.flags & kWaveDone) break;
+    w.near_stamp = r.round + 1;
+    w.far_stamp = r.phase + 1;
+    w.thr = wave_threshold(a, cd0, r.phase);
+    w.nq = wave_queue(a, r.near_q());
+    w.fq = wave_queue(a, r.far_q());
+    w.ntail = &wc->near_tail[gen % 3].n;
+    w.ftail = &wc->far_tail[r.far_q()].n;
+    w.htail = &wc->heavy_tail[gen % 3].n;
+    w.hq = reinterpret_cast<uint64_t *>(gen & 1 ? a.hq[1] : a.hq[0]);
+    // Units: in-queue items, `per` at a time, then heavy chunks.  A wavefront
+    // takes the unit of its number; where there are more units than
+    // wavefronts, unit j * ngroups + g belongs to the blocks b with b % ngroups
+    // == g, whose wavefronts draw tickets of their group (one word for all
+    // wavefronts serialises, ~12 ns a ticket).
+    const uint32_t *const in = wave_queue(a, r.in_q());
+    const uint64_t *const hin = reinterpret_cast<const uint64_t *>(gen & 1 ? a.hq[0] : a.hq[1]);
+    const uint32_t per = min((uint32_t)kWave, max(kUnitMin, (r.items + nwaves - 1) / nwaves));
+    const uint32_t nitem = (r.items + per - 1) / per, nunits = nitem + r.heavy;
+    const bool many = nunits > nwaves;
+    uint32_t unit = many ? (blockIdx.x / ngroups * NW + wv) * ngroups + g : wave;
+    while (unit < nunits) {
+      uint32_t t = 0;
+      if (many && lane_id() == 0) t = atomic_add(&wc->ticket[gen % 3][g].n, 1u);
+      if (unit < nitem) wave_items<A>(a, w, in + (size_t)unit * per, min(per, r.items - unit * per));
+      else wave_chunk<A>(a, w, hin + (unit - nitem));
+      if (!many) break;
+      unit = (gblocks * NW + readlane(t, 0)) * ngroups + g;
+    }
+    // The block's pushes get their places with one atomic per pile.
+    order_release();
+    if (lane_id() == 0) {
+      sh.count[wv][0] = w.n[0];
+      sh.count[wv][1] = w.n[1];
+      sh.count[wv][2] = w.hch;
+    }
+    __syncthreads();
+    uint32_t tot[3] = {0, 0, 0}, off[3] = {0, 0, 0};
+#pragma unroll
+    for (uint32_t i = 0; i < NW; ++i)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        if (i < wv) off[p] += sh.count[i][p];
+        tot[p] += sh.count[i][p];
+      }
+    if (tot[0] | tot[1] | tot[2]) {
+      if (threadIdx.x < 3) {
+        const uint32_t n = threadIdx.x == 0 ? tot[0] : threadIdx.x == 1 ? tot[1] : tot[2];
+        uint32_t *const tail = threadIdx.x == 0 ? w.ntail : threadIdx.x == 1 ? w.ftail : w.htail;
+        sh.base[threadIdx.x] = n ? atomic_add(tail, n) : 0u;
+      }
+      __syncthreads();
+      if (w.n[0]) wave_store(a, w, 0, sh.base[0] + off[0]);
+      if (w.n[1]) wave_store(a, w, 1, sh.base[1] + off[1]);
+      if (w.hn) wave_store_heavy(a, w, sh.base[2] + off[2]);
+      order_release();
+      __syncthreads();
+    }
+    // The barrier.  The last block to arrive finds the next round.
+    if (threadIdx.x == 0) {
+      WaveRound x = r;
+      if (barrier_arrive(c, nb)) {
+        order_acquire();
+        const uint32_t nnear = ld_coh(&wc->near_tail[gen % 3].n), nheavy = ld_coh(&wc->heavy_tail[gen % 3].n);
+        const uint32_t nfar = ld_coh(&wc->far_tail[r.far_q()].n), ab = ld_coh(&c->abort);
+        __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(&c->stat_heavy, (uint64_t)r.heavy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(&c->stat_rounds, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        st_coh(&wc->near_tail[(gen + 2) % 3].n, 0u);
+        st_coh(&wc->heavy_tail[(gen + 2) % 3].n, 0u);
+        for (uint32_t i = 0; i < kTicketGroups; ++i) st_coh(&wc->ticket[(gen + 2) % 3][i].n, 0u);
+        x.flags = kWaveLead;
+        x.round = r.round + 1;
+        x.heavy = 0;
+        if (nnear > a.qcap || nfar > a.qcap || nheavy > a.hcap) {
+          st_coh(&c->abort, kAbortCapacity);
+          x.flags |= kWaveDone;
+        } else if (ab != kAbortNone) {
+          x.flags |= kWaveDone;
+        } else if (nnear > 0 || nheavy > 0) {
+          x.items = nnear;
+          x.heavy = nheavy;
+          x.roles = wave_roles(r.near_q(), r.in_q(), r.far_q());
+        } else if (A == Algo::SSSP && nfar > 0) {
+          // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
+          x.items = nfar;
+          x.phase = r.phase + 1;
+          x.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
+          st_coh(&wc->far_tail[r.far_q()].n, 0u);
+        } else {
+          x.flags |= kWaveDone;
+        }
+        if (!(x.flags & kWaveDone) && x.heavy == 0 && x.items <= kLocalMax) x.flags |= kWaveLocal;
+      } else {
+        uint64_t t0 = wall_clock64();
+        uint32_t seen = ld_coh(&c->progress);
+        for (;;) {
+          uint64_t m[kWaveMsg];
+#pragma unroll
+          for (int i = 0; i < kWaveMsg; ++i) m[i] = ld_coh64(&wc->msg[i]);
+          const uint32_t ab = ld_coh(&c->abort);
+          bool valid = true;
+#pragma unroll
+          for (int i = 0; i < kWaveMsg; ++i) valid &= (uint32_t)m[i] == gen + 1;
+          if (valid) {
+            x.items = (uint32_t)(m[0] >> 32);
+            x.heavy = (uint32_t)(m[1] >> 32);
+            x.round = (uint32_t)(m[2] >> 32);
+            x.phase = (uint32_t)(m[3] >> 32);
+            x.roles = (uint32_t)(m[4] >> 32) & 0x3fu;
+            x.flags = (uint32_t)(m[4] >> 38) & kWaveDone;
+            break;
+          }
+          if (ab != kAbortNone) {
+            x.flags = kWaveDone;
+            break;
+          }
+          if (wall_clock64() - t0 > a.spin_limit) {
+            // the leading block may be running rounds on its own
+            const uint32_t p = ld_coh(&c->progress);
+            if (p != seen) {
+              seen = p;
+              t0 = wall_clock64();
+              continue;
+            }
+            st_coh(&c->abort, kAbortTimeout);
+            x.flags = kWaveDone;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        order_acquire();
+      }
+      sh.r = x;
+    }
+    __syncthreads();
+    if (sh.r.flags & kWaveLead) {
+      if (sh.r.flags & kWaveLocal) wave_local<A, BS>(a, sh, cd0);
+      if (threadIdx.x == 0) {
+        const WaveRound x = sh.r;
+        const uint32_t done = x.flags & kWaveDone;
+        const uint32_t m[kWaveMsg] = {x.items, x.heavy, x.round, x.phase, x.roles | done << 6};
+#pragma unroll
+        for (int i = 0; i < kWaveMsg; ++i) st_coh64(&wc->msg[i], (uint64_t)m[i] << 32 | (gen + 1));
+        if (done) {
+          c->s.done = 1;
+          c->s.round = x.round;
+          c->s.phase = x.phase;
+          c->s.set_curdelta(cd0 + (int64_t)x.phase * a.delta);
+          c->stat_phases = x.phase + 1ull;
+        }
+      }
+    }
+  }
+}
+
+// ---- launch -------------------------------------------------------------------------
+
+__device__ __forceinline__ void wave_reset(WaveCtrl *wc, uint32_t tid, uint32_t nt) {
+  uint32_t *const p = reinterpret_cast<uint32_t *>(wc);
+  for (uint32_t i = tid; i < sizeof(WaveCtrl) / 4; i += nt) p[i] = 0;
+}
+__global__ void wave_reset_kernel(WaveCtrl *wc) { wave_reset(wc, threadIdx.x, blockDim.x); }
+
+// Distances, stamps, control words and the one seed (apps/sssp/kernel.cu:23-35,469,476-477).
+__global__ void wave_init_kernel(WaveArgs a, uint32_t seed) {
+  const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+  for (uint32_t v = tid; v < a.nnodes; v += nt) {
+    glb(a.dist)[v] = v == seed ? 0u : kInf;
+    glb(a.near_stamp)[v] = 0u;
+    glb(a.far_stamp)[v] = 0u;
+  }
+  ctrl_init(a, a.delta, 0, tid, nt);
+  if (blockIdx.x == 0) wave_reset(a.wc, threadIdx.x, blockDim.x);
+  if (tid == 0) {
+    a.q[0][0] = seed;
+    a.ctrl->s.in_count = 1;
+  }
+}
+
+using WaveFn = void (*)(WaveArgs);
+template <Algo A>
+static WaveFn pick_wave(int bs) {
+  return bs == 256 ? wave_kernel<A, 256> : bs == 1024 ? wave_kernel<A, 1024> : wave_kernel<A, 512>;
+}
+static WaveFn pick_wave(Algo algo, int bs) {
+  return algo == Algo::SSSP ? pick_wave<Algo::SSSP>(bs) : pick_wave<Algo::BFS>(bs);
+}
+
+const void *wave_kernel_fn(Algo algo, int bs) { return (const void *)pick_wave(algo, bs); }
+
+int wave_enqueue(Algo algo, int bs, int grid, const WaveArgs &a, uint32_t seed, const uint32_t *seeds, uint32_t nseeds,
+                 const Resume *resume, int cus, hipStream_t stream) {
+  const uint32_t blocks = std::min<uint32_t>((a.nnodes + 255) / 256, 8u * cus);
+  if (resume || seeds) {
+    const KArgs &k = a;
+    if (resume) {
+      hipLaunchKernelGGL(resume_init_kernel, dim3(blocks), dim3(256), 0, stream, k, a.delta, resume->curdelta);
+      hipLaunchKernelGGL(resume_seed_kernel, dim3(blocks), dim3(256), 0, stream, k, resume->lo, resume->hi);
+    } else {
+      hipLaunchKernelGGL(init_kernel, dim3(blocks), dim3(256), 0, stream, k, a.delta);
+      hipLaunchKernelGGL(seed_kernel, dim3(1), dim3(256), 0, stream, k, seeds, nseeds);
+    }
+    hipLaunchKernelGGL(wave_reset_kernel, dim3(1), dim3(256), 0, stream, a.wc);
+  } else {
+    hipLaunchKernelGGL(wave_init_kernel, dim3(blocks), dim3(256), 0, stream, a, seed);
+  }
+  hipLaunchKernelGGL(pick_wave(algo, bs), dim3(grid), dim3(bs), 0, stream, a);
+  HIPCHK(hipGetLastError());
+  return LSG_OK;
+}
+
+}  // namespace lsg

@@ -88,10 +88,11 @@ typedef struct lsg_opts {
   int32_t expand_mode; /* LSG_EXPAND_* */
   int32_t far_mode;    /* LSG_FAR_* */
   int32_t block_size;  /* threads per block: 256 (default), 512 or 1024 */
-  int32_t grid_blocks; /* persistent grid; 0 = every block the device can keep resident */
+  int32_t grid_blocks; /* persistent grid; 0 = chosen by the graph's size and mean degree */
   int32_t thread_deg;  /* TWB: degrees below this are expanded by one lane (default 8) */
   int32_t heavy_deg;   /* degrees >= this are split into chunks of heavy_deg edges, expanded by whole
-                          blocks in the next round (default 512; batched runs: by a wavefront,
+                          blocks in the next round (default 512; with the other options at their
+                          defaults by wavefronts, default 256; batched runs: by a wavefront,
                           default 64, or 256 from 2^24 edges, and >= 8) */
   int32_t sched;       /* 0 = fixed delta; 1 = the learned scheduler picks each phase's delta width
                           and mode (expansion mode for SSSP, far mode for batched runs) from the

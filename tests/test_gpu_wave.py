@@ -1,0 +1,93 @@
+"""The wavefront traversal kernel (default options of sssp/bfs) at the edges of
+its units, piles and modes, against the host oracle.  Distances are whole
+numbers: equality."""
+import numpy as np
+import pytest
+
+import oracle
+from galoisgpu_amd import CSRGraph, Options
+from galoisgpu_amd.apps import bfs_gg_main, sssp_gg_main
+
+pytestmark = pytest.mark.gpu
+
+
+def csr(n, edges):
+    """CSRGraph of (src, dst, weight) rows."""
+    e = np.asarray(edges, dtype=np.int64).reshape(-1, 3)
+    e = e[np.argsort(e[:, 0], kind="stable")]
+    row = np.zeros(n + 1, dtype=np.int64)
+    row[1:] = np.cumsum(np.bincount(e[:, 0], minlength=n))
+    return CSRGraph.from_arrays(row, e[:, 1], e[:, 2])
+
+
+def tree(*degrees):
+    """Every vertex of depth k has degrees[k] children; some cross edges."""
+    edges, level, n = [], [0], 1
+    rng = np.random.default_rng(sum(degrees))
+    for d in degrees:
+        nxt = []
+        for u in level:
+            for _ in range(d):
+                edges.append((u, n, int(rng.integers(1, 100))))
+                nxt.append(n)
+                n += 1
+        level = nxt
+    for _ in range(n // 2):
+        edges.append((int(rng.integers(n)), int(rng.integers(n)), int(rng.integers(1, 100))))
+    return csr(n, edges)
+
+
+def check(g, src, delta, **kw):
+    dev = g.copy_to_gpu()
+    print("wave", g.nnodes, g.nedges, src, delta, kw, flush=True)
+    sssp_gg_main(g, dev, Options(delta=delta, start_node=src, **kw))
+    dev.copy_to_cpu(g)
+    assert np.array_equal(g.node_data, oracle.dijkstra(g.row_start, g.edge_dst, g.edge_data, src))
+    bfs_gg_main(g, dev, Options(start_node=src, **kw))
+    dev.copy_to_cpu(g)
+    assert np.array_equal(g.node_data, oracle.bfs(g.row_start, g.edge_dst, src)[0])
+    dev.close()
+
+
+# Heavy threshold (256 edges by default), rounds of one block (512 items), its
+# piles (1024 entries), staged items (256 a wavefront) and heavy items (32).
+@pytest.mark.parametrize("degrees", [(1,), (255,), (256, 1, 1), (257,), (8, 64), (8, 64, 1, 1), (19, 27, 2), (4, 255, 1),
+                                     (4, 256, 1), (200, 6), (3, 2, 300), (40, 260, 1)])
+def test_trees(degrees):
+    g = tree(*degrees)
+    for delta in (1, 40, 10000):
+        check(g, 0, delta)
+
+
+@pytest.mark.parametrize("kw", [dict(block_size=b, grid_blocks=n) for b in (256, 512, 1024) for n in (1, 7, 16, 17, 300)]
+                         + [dict(heavy_deg=300), dict(heavy_deg=2**31 - 1), dict(graph_launch=True)])
+def test_launch_shapes(kw):
+    g = CSRGraph.rmat(13, 8, seed=3)
+    check(g, g.max_degree_vertex(), 32, **kw)
+    check(CSRGraph.grid(37, 53, seed=2), 5, 64, **kw)
+
+
+def test_captured_launch_takes_new_sources():
+    """Replays of one captured launch, each against the oracle, with plain launches between."""
+    g = CSRGraph.rmat(12, 8, seed=9)
+    dev = g.copy_to_gpu()
+    for src in (g.max_degree_vertex(), 1, 17, 4000):
+        for graph in (True, False, True):
+            print("captured", src, graph, flush=True)
+            sssp_gg_main(g, dev, Options(delta=64, start_node=src, graph_launch=graph))
+            dev.copy_to_cpu(g)
+            assert np.array_equal(g.node_data, oracle.dijkstra(g.row_start, g.edge_dst, g.edge_data, src))
+    dev.close()
+
+
+def test_large_weights():
+    """Distances near the end of the 31-bit range."""
+    w = 2**30 - 1
+    g = csr(6, [(0, 1, w), (1, 2, w), (0, 2, 2 * w), (2, 3, 1), (0, 4, 2**31 - 1), (4, 5, 7)])
+    dev = g.copy_to_gpu()
+    for delta in (1 << 20, 2**31 - 1):
+        print("large weights", delta, flush=True)
+        sssp_gg_main(g, dev, Options(delta=delta, start_node=0))
+        dev.copy_to_cpu(g)
+        assert np.array_equal(g.node_data, oracle.dijkstra(g.row_start, g.edge_dst, g.edge_data, 0))
+    dev.close()
