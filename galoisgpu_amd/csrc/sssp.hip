@@ -74,6 +74,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     void *wbuf;
     if ((rc = ws_buffer(w, kBufWave, sizeof(WaveCtrl), &wbuf))) return rc;
     a.wc = (WaveCtrl *)wbuf;
+    a.pace = g.nedges <= 6ull * g.nnodes;
   }
   // One seed of a plain launch goes to the wavefront kernel's initialisation as
   // an argument; a captured launch must not depend on it.

@@ -845,10 +845,11 @@ __device__ __forceinline__ void expand_light(const KArgs &a, const Entry &e, uin
 // wavefront.  relax(a, v, nd, act) relaxes kInFlight edges per lane (edge k:
 // to v[k] with candidate nd[k], where act[k]), called with the whole
 // wavefront; a heavy vertex's edges stop early once relax.stopped().  Adds
-// the live (not stale) entries to *items.  (Functors rather
+// the live (not stale) entries to *items.  kWg: the distances are this
+// workgroup's alone meanwhile (ld_wg).  (Functors rather
 // than lambdas: a lambda holding a reference to the kernel arguments made the
 // persistent kernel copy them to scratch.)
-template <Algo A, int AS, int NT, class Relax>
+template <Algo A, int AS, int NT, bool kWg = false, class Relax>
 __device__ __forceinline__ void expand_entries(const KArgs &a, EntryPtr<AS> in, uint32_t n, const Relax &relax,
                                                unsigned long long *items) {
   const uint32_t lane = lane_id();
@@ -862,7 +863,7 @@ __device__ __forceinline__ void expand_entries(const KArgs &a, EntryPtr<AS> in, 
     // compiler wait for it before the edge loads); d[0] for idle lanes.  A
     // BFS entry is never stale (its level is exact when it is pushed, and a
     // vertex is pushed once), so BFS takes the entry's level without a load.
-    const uint32_t du = A == Algo::BFS ? e.d : ld_coh(a.dist + e.v);
+    const uint32_t du = A == Algo::BFS ? e.d : kWg ? ld_wg(a.dist + e.v) : ld_coh(a.dist + e.v);
     const uint32_t deg = valid ? e.re - e.rs : 0u;
     const bool heavy = deg > kEntryHeavyDeg;
     const uint32_t ldeg = heavy ? 0u : deg;

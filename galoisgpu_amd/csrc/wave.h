@@ -5,7 +5,7 @@
 
 namespace lsg {
 
-constexpr int kWaveMsg = 5;
+constexpr int kWaveMsg = 6;
 
 // Words of the wavefront kernel beside the control block, each group of words
 // that one atomic unit serves on a line of its own.
@@ -13,9 +13,12 @@ struct WaveCtrl {
   // The state of the next round, published by the last block to reach the
   // barrier: value << 32 | generation, so that a word is valid by itself and
   // a waiting block needs no second load and the publisher no ordering.
-  // Items, heavy chunks, round, phase, roles and flags.
+  // Items, heavy chunks, round, phase, threshold steps, roles and flags.
   uint64_t msg[kWaveMsg];
   uint64_t _p0[16 - kWaveMsg];
+  // How far the next phase moves the threshold; between leading blocks only.
+  uint32_t pace[5];
+  uint32_t _p1[27];
   struct Line {
     uint32_t n;
     uint32_t _p[31];
@@ -26,6 +29,8 @@ struct WaveCtrl {
 
 struct WaveArgs : KArgs {
   WaveCtrl *wc = nullptr;
+  uint32_t pace = 0;  // the threshold's steps are paced (WavePace)
+  uint32_t _pad = 0;
 };
 
 // Blocks per CU, of 256 threads, where the call leaves the launch shape open.

@@ -1,8 +1,9 @@
 // Single-source SSSP and BFS in one persistent launch, by wavefronts.
 //
 // The rounds, piles and phases are the reference's (apps/sssp/kernel.cu:355-391
-// near/far piles, curdelta += DELTA per phase, the whole far pile becoming the
-// next phase; apps/bfs/kernel.cu:312-334 levels), as in persistent_kernel
+// near/far piles, curdelta += DELTA per phase -- here a multiple of it, see
+// WavePace -- the whole far pile becoming the next phase;
+// apps/bfs/kernel.cu:312-334 levels), as in persistent_kernel
 // (sssp_dev.h), which remains for what this kernel does not take: split and
 // bucket far piles, degree-binned expansion, the learned scheduler, round
 // traces, the -l sweep and the no-allocation entry point.
@@ -26,8 +27,9 @@
 //     by generation and cleared two rounds ahead.
 //   - Small rounds (at most kLocalMax items, no heavy vertex) are run by the
 //     last block alone, with entries in LDS as in the one-workgroup kernel
-//     (block.hip): two round trips and two block barriers a round while the
-//     others stay parked.  Far pushes go to the far queue as usual.  The block
+//     (block.hip): two or three round trips and two block barriers a round
+//     while the others stay parked.  What this block alone touches meanwhile is
+//     read at workgroup scope (64^2 grid 0.85 -> 0.79 ms).  The block
 //     leaves this mode when the round it would run next is too large, and hands
 //     the vertices over through the near queue.
 //
@@ -49,6 +51,7 @@ constexpr uint32_t kLocalCap = 1024;
 constexpr uint32_t kWavePush = 256;   // staged items per wavefront and pile
 constexpr uint32_t kWaveHeavy = 32;   // staged heavy items per wavefront
 constexpr uint32_t kTicketGroups = 16;
+constexpr uint32_t kMaxStep = 1u << 16;
 // In-queue items per unit: 64, or fewer where that leaves wavefronts idle, but
 // at least this many, so that a small round involves few blocks (each block
 // with pushes reserves queue space with an atomic of its own).
@@ -57,6 +60,7 @@ constexpr uint32_t kUnitMin = 16;
 // Roles of the three queues and the state of a round.
 struct WaveRound {
   uint32_t items, heavy, round, phase;
+  uint32_t steps;  // the near/far threshold, in steps of delta
   uint32_t roles;  // in | near << 2 | far << 4
   uint32_t flags;
   __device__ uint32_t in_q() const { return roles & 3u; }
@@ -72,6 +76,53 @@ struct WaveHeavy {
   uint32_t u, nch;
 };
 
+// Pace of the near/far threshold on graphs of low degree (the host decides:
+// at most 6 edges a vertex).  There nearly every round is bound by its fixed
+// cost, so a wider phase, with its fewer and larger rounds, is faster until
+// the vertices that are expanded more than once cost more than the rounds
+// saved; how wide depends on the graph, the weights and where the frontier is
+// (best multiple of the call's delta: 64^2 grid at 32: 64, 256^2: 16, road-like
+// 1000^2 at 10000: 16, 2048^2: 6).  So the threshold moves by `step` deltas,
+// and step is climbed: it is doubled while the threshold then moves further per
+// us of modelled round cost, or while rounds are nearly empty; else one step
+// back, and two phases later the next trial.  Distances do not depend on it.
+// Ms with step 1 -> here: grid 64^2 0.80 -> 0.50, 256^2 5.7 -> 3.8, 1000^2 30 ->
+// 20, road-like 1000^2 2.67 -> 1.90, 2048^2 3.83 -> 2.88, 2048^2 at delta 2000
+// 6.9 -> 3.0.  On RMAT graphs of 8 and more edges a vertex, whose rounds are
+// few and large, it gains nothing and loses up to 17 % from random sources.
+struct WavePace {
+  uint32_t step;    // deltas that the threshold moves by
+  uint32_t hold;    // phases until the next trial; 0: this phase is one
+  float best;       // deltas per us before the trial
+  float cost;       // of the phase so far, us: fitted to both kinds of rounds
+  uint32_t rounds;  // of the phase so far
+  __device__ void round(uint32_t items, bool local) {
+    cost += local ? 3.0f + (float)items * (1.0f / 80) : 6.0f + (float)items * (1.0f / 6000);
+    rounds += 1;
+  }
+  // The step to the threshold of the phase after `phase`.
+  __device__ uint32_t next(uint32_t phase) {
+    const float rate = (float)step / cost;
+    const bool empty = cost < 4.0f * (float)rounds;
+    cost = 0;
+    rounds = 0;
+    if (hold == 0 || empty) {
+      hold = 0;
+      if (rate > 1.02f * best || empty) {
+        if (phase > 0) best = rate;  // (phase 0 is the source alone)
+        step = min(step * 2, kMaxStep);
+      } else {
+        step = max(step / 2, 1u);
+        hold = 2;
+      }
+    } else if (--hold == 0) {
+      best = rate;
+      step = min(step * 2, kMaxStep);
+    }
+    return step;
+  }
+};
+
 template <int BS>
 struct WaveShared {
   static constexpr int NW = BS / kWave;
@@ -80,6 +131,7 @@ struct WaveShared {
   uint32_t count[NW][3];            // end of a round: near, far, heavy chunks
   uint32_t base[3];
   WaveRound r;
+  WavePace pace;
   // rounds of one block
   Entry pile[2][kLocalCap];
   uint32_t pile_n[2];
@@ -299,9 +351,9 @@ struct LocalRelax {
 #pragma unroll
     for (int k = 0; k < kInFlight; ++k) {
       near[k] = A == Algo::BFS || nd[k] <= thr;
-      old[k] = act[k] ? atomic_min(a.dist + v[k], nd[k]) : 0u;
+      old[k] = act[k] ? atomic_min_wg(a.dist + v[k], nd[k]) : 0u;
       rb[k] = ld_pair(a.row_start + v[k]);
-      seen[k] = A == Algo::SSSP ? glb(a.far_stamp)[act[k] && !near[k] ? v[k] : 0u] : 0u;
+      seen[k] = A == Algo::SSSP ? ld_wg(a.far_stamp + (act[k] && !near[k] ? v[k] : 0u)) : 0u;
     }
 #pragma unroll
     for (int k = 0; k < kInFlight; ++k) asm volatile("" : "+v"(old[k]));
@@ -309,7 +361,7 @@ struct LocalRelax {
 #pragma unroll
       for (int k = 0; k < kInFlight; ++k) {
         const bool want = act[k] && nd[k] < old[k] && !near[k] && seen[k] != far_stamp;
-        got[k] = want ? atomic_exch(a.far_stamp + v[k], far_stamp) : far_stamp;
+        got[k] = want ? atomic_exch_wg(a.far_stamp + v[k], far_stamp) : far_stamp;
       }
     }
     // near: one reservation per wavefront
@@ -358,17 +410,17 @@ struct LocalRelax {
     }
   }
   __device__ __forceinline__ void put(uint32_t *q, uint32_t pos, uint32_t v) const {
-    if (pos < a.qcap) st_coh(q + pos, v);
+    if (pos < a.qcap) st_wg(q + pos, v);
     else st_coh(&a.ctrl->abort, kAbortCapacity);
   }
   // A vertex that this mode hands on: once to the near queue.
   __device__ __forceinline__ void spill(uint32_t v) const {
-    if (atomic_exch(a.near_stamp + v, near_stamp) != near_stamp) put(nq, atomicAdd(&sh.spill_n, 1u), v);
+    if (atomic_exch_wg(a.near_stamp + v, near_stamp) != near_stamp) put(nq, atomicAdd(&sh.spill_n, 1u), v);
   }
 };
 
-__device__ __forceinline__ uint32_t wave_threshold(const WaveArgs &a, int64_t cd0, uint32_t phase) {
-  const int64_t cd = cd0 + (int64_t)phase * a.delta;
+__device__ __forceinline__ uint32_t wave_threshold(const WaveArgs &a, int64_t cd0, uint32_t steps) {
+  const int64_t cd = cd0 + (int64_t)steps * a.delta;
   return (uint32_t)min(cd, (int64_t)0xFFFFFFFFll);
 }
 
@@ -380,6 +432,8 @@ __device__ __forceinline__ uint32_t wave_threshold(const WaveArgs &a, int64_t cd
 template <Algo A, int BS>
 __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh, int64_t cd0) {
   WaveRound r = sh.r;
+  WavePace pace = sh.pace;
+  acquire_agent();
   const uint32_t far_in = A == Algo::SSSP ? ld_coh(&a.wc->far_tail[r.far_q()].n) : 0u;
   if (threadIdx.x == 0) {
     sh.far_n = far_in;
@@ -394,8 +448,8 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       const uint32_t *const in = wave_queue(a, r.in_q());
       bool big = false;
       for (uint32_t i = threadIdx.x; i < n; i += BS) {
-        const uint32_t v = ld_coh(in + i);
-        const uint32_t d = ld_coh(a.dist + v);
+        const uint32_t v = ld_wg(in + i);
+        const uint32_t d = ld_wg(a.dist + v);
         const uint64_t rb = ld_pair(a.row_start + v);
         sh.pile[cur][i] = Entry{v, d, (uint32_t)rb, (uint32_t)(rb >> 32)};
         big |= (uint32_t)(rb >> 32) - (uint32_t)rb >= a.heavy_deg;
@@ -409,12 +463,13 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       sh.spill_n = 0;
     }
     __syncthreads();
-    const LocalRelax<A, BS> relax{a,           sh, cur ^ 1, wave_threshold(a, cd0, r.phase), r.round + 1, r.phase + 1,
+    const LocalRelax<A, BS> relax{a,           sh, cur ^ 1, wave_threshold(a, cd0, r.steps), r.round + 1, r.phase + 1,
                                   wave_queue(a, r.near_q()), wave_queue(a, r.far_q())};
-    expand_entries<A, kLdsAS, BS>(a, (EntryPtr<kLdsAS>)sh.pile[cur], n, relax, &sh.items);
+    expand_entries<A, kLdsAS, BS, true>(a, (EntryPtr<kLdsAS>)sh.pile[cur], n, relax, &sh.items);
     __syncthreads();  // every push of the round is in
     popped += n;
     ++rounds;
+    if (A == Algo::SSSP) pace.round(n, true);
     r.round += 1;
     const uint32_t near = sh.pile_n[cur ^ 1], far = sh.far_n;
     if (threadIdx.x == 0) st_coh(&a.ctrl->progress, r.round);
@@ -433,6 +488,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
       r.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
       r.phase += 1;
+      r.steps += a.pace ? pace.next(r.phase - 1) : 1u;
       n = far;
       order_release();  // this wavefront's far pushes have landed
       __syncthreads();  // and every other's; far_n has been read
@@ -446,11 +502,14 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
     }
     // (the next round's first barrier separates the reads of sh above from its writes)
   }
+  order_release();
   __syncthreads();
   if (threadIdx.x == 0) {
+    release_agent();
     r.items = n;
     r.heavy = 0;
     sh.r = r;
+    sh.pace = pace;
     if (A == Algo::SSSP) {
       st_coh(&a.wc->far_tail[r.far_q()].n, sh.far_n);
       if (r.far_q() != 0) st_coh(&a.wc->far_tail[0].n, 0u);
@@ -483,6 +542,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     sh.r.heavy = 0;
     sh.r.round = 1;
     sh.r.phase = 0;
+    sh.r.steps = 0;
     sh.r.roles = wave_roles(0, 1, 2);
     sh.r.flags = 0;
   }
@@ -497,7 +557,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     if (r.flags & kWaveDone) break;
     w.near_stamp = r.round + 1;
     w.far_stamp = r.phase + 1;
-    w.thr = wave_threshold(a, cd0, r.phase);
+    w.thr = wave_threshold(a, cd0, r.steps);
     w.nq = wave_queue(a, r.near_q());
     w.fq = wave_queue(a, r.far_q());
     w.ntail = &wc->near_tail[gen % 3].n;
@@ -558,7 +618,15 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       if (barrier_arrive(c, nb)) {
         order_acquire();
         const uint32_t nnear = ld_coh(&wc->near_tail[gen % 3].n), nheavy = ld_coh(&wc->heavy_tail[gen % 3].n);
-        const uint32_t nfar = ld_coh(&wc->far_tail[r.far_q()].n), ab = ld_coh(&c->abort);
+        const uint32_t nfar = A == Algo::SSSP ? ld_coh(&wc->far_tail[r.far_q()].n) : 0u, ab = ld_coh(&c->abort);
+        WavePace pace{1, 0, 0, 0, 0};
+        if (A == Algo::SSSP) {
+          uint32_t p[5];
+#pragma unroll
+          for (int i = 0; i < 5; ++i) p[i] = ld_coh(&wc->pace[i]);
+          pace = WavePace{max(p[0], 1u), p[1], __uint_as_float(p[2]), __uint_as_float(p[3]), p[4]};
+          pace.round(r.items, false);
+        }
         __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_add(&c->stat_heavy, (uint64_t)r.heavy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_add(&c->stat_rounds, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -581,12 +649,14 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
           // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
           x.items = nfar;
           x.phase = r.phase + 1;
+          x.steps = r.steps + (a.pace ? pace.next(r.phase) : 1u);
           x.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
           st_coh(&wc->far_tail[r.far_q()].n, 0u);
         } else {
           x.flags |= kWaveDone;
         }
         if (!(x.flags & kWaveDone) && x.heavy == 0 && x.items <= kLocalMax) x.flags |= kWaveLocal;
+        sh.pace = pace;
       } else {
         uint64_t t0 = wall_clock64();
         uint32_t seen = ld_coh(&c->progress);
@@ -603,8 +673,9 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
             x.heavy = (uint32_t)(m[1] >> 32);
             x.round = (uint32_t)(m[2] >> 32);
             x.phase = (uint32_t)(m[3] >> 32);
-            x.roles = (uint32_t)(m[4] >> 32) & 0x3fu;
-            x.flags = (uint32_t)(m[4] >> 38) & kWaveDone;
+            x.steps = (uint32_t)(m[4] >> 32);
+            x.roles = (uint32_t)(m[5] >> 32) & 0x3fu;
+            x.flags = (uint32_t)(m[5] >> 38) & kWaveDone;
             break;
           }
           if (ab != kAbortNone) {
@@ -635,14 +706,21 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       if (threadIdx.x == 0) {
         const WaveRound x = sh.r;
         const uint32_t done = x.flags & kWaveDone;
-        const uint32_t m[kWaveMsg] = {x.items, x.heavy, x.round, x.phase, x.roles | done << 6};
+        const uint32_t m[kWaveMsg] = {x.items, x.heavy, x.round, x.phase, x.steps, x.roles | done << 6};
 #pragma unroll
         for (int i = 0; i < kWaveMsg; ++i) st_coh64(&wc->msg[i], (uint64_t)m[i] << 32 | (gen + 1));
+        if (A == Algo::SSSP) {
+          st_coh(&wc->pace[0], sh.pace.step);
+          st_coh(&wc->pace[1], sh.pace.hold);
+          st_coh(&wc->pace[2], __float_as_uint(sh.pace.best));
+          st_coh(&wc->pace[3], __float_as_uint(sh.pace.cost));
+          st_coh(&wc->pace[4], sh.pace.rounds);
+        }
         if (done) {
           c->s.done = 1;
           c->s.round = x.round;
           c->s.phase = x.phase;
-          c->s.set_curdelta(cd0 + (int64_t)x.phase * a.delta);
+          c->s.set_curdelta(cd0 + (int64_t)x.steps * a.delta);
           c->stat_phases = x.phase + 1ull;
         }
       }

@@ -67,6 +67,14 @@ def test_launch_shapes(kw):
     check(CSRGraph.grid(37, 53, seed=2), 5, 64, **kw)
 
 
+# Low-degree graphs, whose threshold moves in growing steps: up to one that passes every distance.
+@pytest.mark.parametrize("rows,cols,whi", [(1, 3000, 9), (64, 64, 100), (90, 131, 1 << 20), (300, 410, 60000)])
+def test_paced_threshold(rows, cols, whi):
+    g = CSRGraph.grid(rows, cols, 1, whi, seed=rows)
+    for delta in (1, 32, 5000, 1 << 30):
+        check(g, 7, delta)
+
+
 def test_captured_launch_takes_new_sources():
     """Replays of one captured launch, each against the oracle, with plain launches between."""
     g = CSRGraph.rmat(12, 8, seed=9)
