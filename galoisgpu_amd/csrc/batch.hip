@@ -64,8 +64,11 @@ constexpr int kMultiWaves = 4;
 //
 // The bounds come from up to kSweeps sweeps over D inside the launch, each
 // with the offsets of its time and into an array of its own, so that bounds
-// read through the caches are never of other offsets.  A sweep reads V rows
-// in order; it follows once E/2 edges were expanded since the last one.
+// read through the caches are never of other offsets; the arrays share no
+// cache line (the last bounds of one sweep read beside the first of the next
+// array would leave those in the caches as an earlier call left them).  A sweep
+// reads V rows in order; it follows once E/2 edges were expanded since the
+// last one.
 constexpr int kSweeps = 3;
 // The test needs a hub that most paths share: it is used where the largest
 // out-degree is at least kHubRatio times the mean.  Without / with the test
@@ -960,6 +963,7 @@ void multi_kernel(MArgs a) {
       if (s.aux[3]) {
         sweep_bounds(a, ls, bound, wave, nwaves);
         grid_barrier_block(c, nb, a.spin_limit, [] {});
+        acquire_agent();  // no line of the bounds that was read before is kept
       }
     }
     Pending p;
@@ -1201,6 +1205,9 @@ struct MultiRun {
   int grid = 0, bs = 0;
 };
 
+// Words of one sweep's bounds: whole wavefronts of a sweep, whole cache lines.
+static uint64_t bound_words(uint32_t V) { return ((uint64_t)V + kWave - 1) / kWave * kWave; }
+
 // Runs one vertex-major launch: S = nsrc <= 64 sources of `g` into D [V][S].
 static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host, uint32_t nsrc, const lsg_opts &o,
                      uint32_t *D, MultiRun *out) {
@@ -1219,7 +1226,7 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
   uint32_t hcap = (uint32_t)std::min<uint64_t>(hcap64, UINT32_MAX / 4);
   void *qbuf, *hbuf, *mbuf, *sbuf;
   if ((rc = ws_buffer(w, kBufQueues, 3ull * V * 4, &qbuf)) || (rc = ws_buffer(w, kBufHeavy, 2ull * hcap * 16, &hbuf)) ||
-      (rc = ws_buffer(w, kBufMasks, (4ull * 8 + 4 + 4 * kSweeps) * V + 16ull * w->cus * 8 + 256, &mbuf)) || (rc = ws_buffer(w, kBufSeeds, 2048 + kGroups * (sizeof(TicketGroup) + sizeof(MultiCounters)), &sbuf)))
+      (rc = ws_buffer(w, kBufMasks, (4ull * 8 + 4) * V + kSweeps * bound_words(V) * 4 + 16ull * w->cus * 8 + 512, &mbuf)) || (rc = ws_buffer(w, kBufSeeds, 2048 + kGroups * (sizeof(TicketGroup) + sizeof(MultiCounters)), &sbuf)))
     return rc;
   MArgs a;
   memset(&a, 0, sizeof a);
@@ -1233,8 +1240,9 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
   a.fmask[0] = masks + 2ull * V;
   a.fmask[1] = masks + 3ull * V;
   a.qstamp = (uint32_t *)(masks + 4ull * V);
-  for (int i = 0; i < kSweeps; ++i) a.bound[i] = (int32_t *)(masks + 4ull * V) + (1ull + i) * V;
-  a.hubs = (uint64_t *)(((uintptr_t)(a.bound[kSweeps - 1] + V) + 7) & ~(uintptr_t)7);
+  int32_t *const bounds = (int32_t *)(((uintptr_t)(a.qstamp + V) + 255) & ~(uintptr_t)255);
+  for (int i = 0; i < kSweeps; ++i) a.bound[i] = bounds + i * bound_words(V);
+  a.hubs = (uint64_t *)(bounds + kSweeps * bound_words(V));
   a.ninit = (uint32_t)std::min<uint64_t>(((uint64_t)V * nsrc + 255) / 256, 16ull * w->cus);
   for (int i = 0; i < 3; ++i) a.q[i] = (uint32_t *)qbuf + (size_t)i * V;
   a.hq[0] = (uint64_t *)hbuf;

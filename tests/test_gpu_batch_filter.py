@@ -73,3 +73,35 @@ def test_more_work_units_than_wavefronts():
     srcs = np.random.default_rng(1).integers(0, g.nnodes, 12)
     st = check(g, srcs, delta=1 << 30, block_size=256, heavy_deg=16)
     assert st["items"] > 4096 * 16
+
+
+@pytest.mark.parametrize("n", [1500, 3000, 3001, 3016, 5004, 20011])
+def test_bounds_of_an_earlier_call_are_not_seen(n):
+    """Vertices 0 to 15 lie beside the other arrays' last vertices in the bounds of the second and third
+    sweep.  Seen from `a` they are near and the hub is far, seen from the other sources the reverse:
+    a bound left over from the call before would cut them off."""
+    rng = np.random.default_rng(n)
+    hub, chain, first = 20, 60, 16
+    a = first + 4 + chain
+    core = np.arange(a + 1, n)
+    spokes = rng.choice(core, len(core) // 3, replace=False)
+    links = np.arange(first + 4, a)                        # hub+1 ... a: a chain that only ends at a
+    src = np.concatenate([np.full(len(spokes), hub), spokes, rng.choice(core, 8 * n),
+                          rng.choice(core, 9000), [core[5]], links[1:], [a - 1], np.full(16, a), [a]])
+    dst = np.concatenate([spokes, np.full(len(spokes), hub), rng.choice(core, 8 * n),
+                          rng.integers(n - 16, n, 9000), [links[1]], links[1:] + 1, [a], np.arange(16), [hub]])
+    w = rng.integers(1, 255, len(src))
+    w[-1] = 1000000
+    order = np.argsort(src, kind="stable")
+    row = np.zeros(n + 1, dtype=np.int64)
+    row[1:] = np.cumsum(np.bincount(src, minlength=n))
+    g = CSRGraph.from_arrays(row, dst[order], w[order])
+    dev = g.copy_to_gpu()
+    others = [int(x) for x in rng.choice(core, 4)]
+    ref = {s: oracle.dijkstra(g.row_start, g.edge_dst, g.edge_data, s) for s in [a] + others}
+    for s in others * 3:
+        for srcs in ([a], [s]):
+            print("bounds of an earlier call", n, srcs, flush=True)
+            d, _ = sssp_multi(dev, srcs, Options(delta=1 << 30))
+            assert np.array_equal(d[:, 0], ref[srcs[0]]), srcs
+    dev.close()
