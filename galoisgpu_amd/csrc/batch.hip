@@ -972,20 +972,22 @@ void multi_kernel(MArgs a) {
     DistSlots &dl = dls[threadIdx.x / kWave];
     // Work units: first the in-queue's items, `per` at a time (fewer than
     // kItems where that would leave wavefronts idle), then the heavy chunks.
-    // Unit j * kGroups + g belongs to group g; its wavefronts take one each,
-    // then kSpan per ticket (the next ticket is fetched while the last unit of
-    // the current one is processed), and at the end help other groups.
+    // Where each wavefront has one at most, the unit of its number; else unit j
+    // * kGroups + g belongs to group g, whose wavefronts take one each, then
+    // kSpan per ticket (the next ticket is fetched while the last unit of the
+    // current one is processed), and at the end help other groups.
     const uint32_t per = min((uint32_t)kItems, max(1u, (s.in_count + nwaves - 1) / nwaves));
     const uint32_t hper = min(min((uint32_t)kItems, max(1u, kChunkUnit / a.heavy_deg)),
                               max(1u, (s.heavy_count + nwaves - 1) / nwaves));
     const uint32_t nitems = (s.in_count + per - 1) / per;
     const uint32_t nunits = nitems + (s.heavy_count + hper - 1) / hper;
+    const bool few = nunits <= nwaves;
     uint32_t g = blockIdx.x % kGroups;
     uint32_t j = blockIdx.x / kGroups * wpb + threadIdx.x / kWave, jend = j + 1;
     for (;;) {
-      const uint32_t u = j * kGroups + g;
+      const uint32_t u = few ? wave : j * kGroups + g;
       if (u < nunits) {
-        const bool last = j + 1 >= jend && nunits > nwaves;
+        const bool last = j + 1 >= jend && !few;
         uint32_t t = 0;
         if (last && lane_id() == 0) t = atomic_add(&a.tickets[g].ticket, 1u);
         const bool chunks = u >= nitems;
@@ -997,11 +999,11 @@ void multi_kernel(MArgs a) {
           jend = j + kSpan;
         } else {
           ++j;
-          if (nunits <= nwaves) break;
+          if (few) break;
         }
         continue;
       }
-      if (nunits <= nwaves) break;
+      if (few) break;
       // this group's units are taken: the next group that has some left
       const uint32_t og = (g + 1 + lane_id()) % kGroups;
       const uint32_t oj = group_blocks(nb, og) * wpb + ld_coh(&a.tickets[og].ticket) * kSpan;

@@ -105,3 +105,14 @@ def test_bounds_of_an_earlier_call_are_not_seen(n):
             d, _ = sssp_multi(dev, srcs, Options(delta=1 << 30))
             assert np.array_equal(d[:, 0], ref[srcs[0]]), srcs
     dev.close()
+
+
+@pytest.mark.parametrize("blocks", [1, 3, 15, 16, 17, 31, 33, 250])
+def test_every_unit_is_taken(blocks):
+    """Grids that the ticket groups do not divide evenly, with fewer and more units than wavefronts."""
+    g = CSRGraph.rmat(12, 8, seed=4)
+    srcs = np.random.default_rng(blocks).integers(0, g.nnodes, 20)
+    for block_size in (256, 1024):
+        print("units", blocks, block_size, flush=True)
+        check(g, srcs, delta=40, grid_blocks=blocks, block_size=block_size)
+        check(CSRGraph.grid(40, 60, seed=blocks), [3, 700], delta=64, grid_blocks=blocks, block_size=block_size)
