@@ -72,25 +72,13 @@ __device__ __forceinline__ uint64_t atomic_exch64(uint64_t *p, uint64_t v) {
   return __hip_atomic_exchange(glb(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The same for words that only one workgroup reads and writes for a while:
-// executed in the L2 of its XCD, they take a fraction of the trip to the
-// coherence point.  Such a stretch begins with acquire_agent in every wave
-// (stale lines leave the caches) and ends with release_agent, after a barrier
-// behind every wave's order_release (its lines are written back).
+// A word that may be read from the caches of this XCD: as old as the last time
+// this wave acquired at agent scope.
 __device__ __forceinline__ uint32_t ld_wg(const uint32_t *p) {
   return __hip_atomic_load(glb(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ void st_wg(uint32_t *p, uint32_t v) {
-  __hip_atomic_store(glb(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ uint32_t atomic_min_wg(uint32_t *p, uint32_t v) {
-  return __hip_atomic_fetch_min(glb(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ uint32_t atomic_exch_wg(uint32_t *p, uint32_t v) {
-  return __hip_atomic_exchange(glb(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
+// Drops stale lines from this wave's caches.
 __device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
-__device__ __forceinline__ void release_agent() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
 
 // Orders this wave's earlier memory operations before its later ones: the
 // compiler may not move accesses across it and the wave waits until every

@@ -845,8 +845,8 @@ __device__ __forceinline__ void expand_light(const KArgs &a, const Entry &e, uin
 // wavefront.  relax(a, v, nd, act) relaxes kInFlight edges per lane (edge k:
 // to v[k] with candidate nd[k], where act[k]), called with the whole
 // wavefront; a heavy vertex's edges stop early once relax.stopped().  Adds
-// the live (not stale) entries to *items.  kWg: the distances are this
-// workgroup's alone meanwhile (ld_wg).  (Functors rather
+// the live (not stale) entries to *items.  kWg: d[u] is looked at through
+// ld_wg (an older one only keeps a stale entry).  (Functors rather
 // than lambdas: a lambda holding a reference to the kernel arguments made the
 // persistent kernel copy them to scratch.)
 template <Algo A, int AS, int NT, bool kWg = false, class Relax>

@@ -5,7 +5,8 @@
 
 namespace lsg {
 
-constexpr int kWaveMsg = 6;
+constexpr int kWaveMsg = 7;
+constexpr uint32_t kTicketGroups = 16;
 
 // Words of the wavefront kernel beside the control block, each group of words
 // that one atomic unit serves on a line of its own.
@@ -13,7 +14,6 @@ struct WaveCtrl {
   // The state of the next round, published by the last block to reach the
   // barrier: value << 32 | generation, so that a word is valid by itself and
   // a waiting block needs no second load and the publisher no ordering.
-  // Items, heavy chunks, round, phase, threshold steps, roles and flags.
   uint64_t msg[kWaveMsg];
   uint64_t _p0[16 - kWaveMsg];
   // How far the next phase moves the threshold; between leading blocks only.
@@ -22,15 +22,25 @@ struct WaveCtrl {
   struct Line {
     uint32_t n;
     uint32_t _p[31];
-  } near_tail[3], heavy_tail[3],  // by generation mod 3: the leader of one round clears the words of the one after the next
-      far_tail[3],                // by queue
-      ticket[3][16];              // by generation mod 3 and group of blocks
+  };
+  Line far_tail[3];  // by queue
+  // By generation mod 3: the leader of one round clears the words of the one
+  // after the next.
+  struct Slot {
+    Line near_tail, heavy_tail, ticket[kTicketGroups], top, arrive[kMaxBarGroups];
+  } slot[3];
+};
+
+// Up to heavy_deg edges of a heavy vertex: popped at distance d.
+struct WaveChunk {
+  uint32_t u, d, first, n;
 };
 
 struct WaveArgs : KArgs {
+  WaveChunk *chunk[2] = {nullptr, nullptr};  // in place of KArgs::hq
   WaveCtrl *wc = nullptr;
-  uint32_t pace = 0;  // the threshold's steps are paced (WavePace)
-  uint32_t _pad = 0;
+  uint32_t pace = 0;      // the threshold's steps are paced (WavePace)
+  uint32_t unit_min = 0;  // fewest items of a unit
 };
 
 // Blocks per CU, of 256 threads, where the call leaves the launch shape open.

@@ -20,23 +20,33 @@
 //     wavefront at every ticket.)
 //   - Pushes and heavy items are staged per wavefront in LDS and placed with
 //     one atomic per pile and block at the end of the round.
-//   - The barrier's message is the round: the last block to arrive publishes
-//     the next round's counts and roles as words that carry the generation, so
-//     that the waiting blocks read everything with the poll that sees it, and
-//     nothing has to be ordered before it.  Tails and tickets are used in turn
-//     by generation and cleared two rounds ahead.
+//   - Only blocks that had a unit arrive at the barrier (36 units: 9 blocks, one
+//     counter), and its message is the round: the last block to arrive
+//     publishes the next round's counts and roles as words that carry the
+//     generation, so that the waiting blocks read everything with the poll that
+//     sees it, and nothing has to be ordered before it.  Tails, tickets and
+//     arrival counts are used in turn by generation and cleared two rounds
+//     ahead.  A round of 600 low-degree items: 9.2 -> 7.5 us with the arrival
+//     of all 256 blocks and the look at d[v] before the atomicMin taken out.
+//   - What was expanded already is not expanded again: items of the far pile
+//     that came below the last threshold meanwhile were near items then
+//     (RMAT-20: most of 505,060, 145 -> 87 us), and chunks of a vertex that was
+//     lowered since it was popped are left to its next pop.
 //   - Small rounds (at most kLocalMax items, no heavy vertex) are run by the
 //     last block alone, with entries in LDS as in the one-workgroup kernel
 //     (block.hip): two or three round trips and two block barriers a round
-//     while the others stay parked.  What this block alone touches meanwhile is
-//     read at workgroup scope (64^2 grid 0.85 -> 0.79 ms).  The block
-//     leaves this mode when the round it would run next is too large, and hands
-//     the vertices over through the near queue.
+//     while the others stay parked.  The looks at d[v] and at stamps whose
+//     older value only costs work are at workgroup scope (64^2 grid 0.85 ->
+//     0.79 ms).  The block leaves
+//     this mode when the round it would run next is too large, and hands the
+//     vertices over through the near queue.  (Limits of 128 / 256 / 384 / 512
+//     items: 64^2 grid SSSP 0.62 / 0.53 / 0.52 / 0.49 ms, 256^2 3.7 / 3.4 / 3.5
+//     / 3.6, 512^2 BFS 6.0 / 5.2 / 4.9 / 4.8, road-like 1023 x 777 BFS 0.86 /
+//     0.85 / 0.84 / 0.84.)
 //
-// Ms in persistent_kernel -> here: SSSP RMAT-17 0.53 -> 0.50, RMAT-20 1.60 ->
-// 1.15, RMAT-22 5.1 -> 2.9, road-like 2048^2 4.69 -> 3.76, 1000^2 3.45 -> 2.61,
-// grid 256^2 (delta 32) 8.8 -> 5.7, 64^2 1.6 -> 0.85; BFS RMAT-17 0.162 ->
-// 0.128, RMAT-20 0.447 -> 0.299, road-like 1023 x 777 1.16 -> 0.87.
+// Ms in persistent_kernel -> here, at delta steps of 1 as in WavePace: SSSP
+// RMAT-17 0.53 -> 0.44, RMAT-20 1.60 -> 1.00, RMAT-22 5.1 -> 2.26; BFS RMAT-17
+// 0.162 -> 0.105, RMAT-20 0.447 -> 0.28, road-like 1023 x 777 1.16 -> 0.84.
 
 #include <hip/hip_runtime.h>
 
@@ -50,30 +60,32 @@ constexpr uint32_t kLocalMax = 512;
 constexpr uint32_t kLocalCap = 1024;
 constexpr uint32_t kWavePush = 256;   // staged items per wavefront and pile
 constexpr uint32_t kWaveHeavy = 32;   // staged heavy items per wavefront
-constexpr uint32_t kTicketGroups = 16;
 constexpr uint32_t kMaxStep = 1u << 16;
-// In-queue items per unit: 64, or fewer where that leaves wavefronts idle, but
-// at least this many, so that a small round involves few blocks (each block
-// with pushes reserves queue space with an atomic of its own).
-constexpr uint32_t kUnitMin = 16;
+// Rounds of at most this many items go straight to the atomicMins where a unit
+// has few edges: one round trip less, and few enough atomics.
+constexpr uint32_t kDirectMax = 4096;
 
 // Roles of the three queues and the state of a round.
 struct WaveRound {
   uint32_t items, heavy, round, phase;
   uint32_t steps;  // the near/far threshold, in steps of delta
+  uint32_t cut;    // kWaveCut: the previous phase's
+  uint32_t lead;   // the block that published the round
   uint32_t roles;  // in | near << 2 | far << 4
   uint32_t flags;
   __device__ uint32_t in_q() const { return roles & 3u; }
   __device__ uint32_t near_q() const { return roles >> 2 & 3u; }
   __device__ uint32_t far_q() const { return roles >> 4 & 3u; }
 };
-constexpr uint32_t kWaveDone = 1, kWaveLead = 2, kWaveLocal = 4;
+// kWaveCut: the round's input is the far pile; what has come below the previous
+// threshold since it was pushed has been expanded as a near item already.
+constexpr uint32_t kWaveDone = 1, kWaveCut = 2, kWaveLead = 4, kWaveLocal = 8;
 __device__ __forceinline__ uint32_t wave_roles(uint32_t in, uint32_t near, uint32_t far) {
   return in | near << 2 | far << 4;
 }
 
 struct WaveHeavy {
-  uint32_t u, nch;
+  uint32_t u, d, first, deg;
 };
 
 // Pace of the near/far threshold on graphs of low degree (the host decides:
@@ -131,6 +143,7 @@ struct WaveShared {
   uint32_t count[NW][3];            // end of a round: near, far, heavy chunks
   uint32_t base[3];
   WaveRound r;
+  uint32_t gen;
   WavePace pace;
   // rounds of one block
   Entry pile[2][kLocalCap];
@@ -145,8 +158,10 @@ struct WaveShared {
 struct WaveLane {
   uint32_t near_stamp, far_stamp;  // this round's and phase's stamps
   uint32_t thr;                    // a candidate is near iff it is at most this
+  int64_t cut;                     // items at most this far are skipped
+  bool direct;
   uint32_t *nq, *fq, *ntail, *ftail;
-  uint64_t *hq;
+  WaveChunk *hq;
   uint32_t *htail;
   uint32_t *pbuf[2];
   WaveHeavy *hbuf;
@@ -188,20 +203,28 @@ __device__ __forceinline__ void wave_stage(const WaveArgs &a, WaveLane &w, int w
 // Writes the staged heavy items' chunks from slot `base` on.
 __device__ __forceinline__ void wave_store_heavy(const WaveArgs &a, WaveLane &w, uint32_t base) {
   for (uint32_t i = 0; i < w.hn; ++i) {
-    const uint32_t u = __builtin_amdgcn_readfirstlane(w.hbuf[i].u), nch = __builtin_amdgcn_readfirstlane(w.hbuf[i].nch);
+    const uint32_t u = __builtin_amdgcn_readfirstlane(w.hbuf[i].u), d = __builtin_amdgcn_readfirstlane(w.hbuf[i].d);
+    const uint32_t first = __builtin_amdgcn_readfirstlane(w.hbuf[i].first);
+    const uint32_t deg = __builtin_amdgcn_readfirstlane(w.hbuf[i].deg), nch = (deg - 1) / a.heavy_deg + 1;
     for (uint32_t k = lane_id(); k < nch; k += kWave) {
-      const uint32_t pos = base + k;
-      if (pos < a.hcap) st_coh64(w.hq + pos, (uint64_t)k << 32 | u);
-      else st_coh(&a.ctrl->abort, kAbortCapacity);
+      const uint32_t pos = base + k, skip = k * a.heavy_deg;
+      if (pos < a.hcap) {
+        uint64_t *const p = reinterpret_cast<uint64_t *>(w.hq + pos);
+        st_coh64(p, (uint64_t)d << 32 | u);
+        st_coh64(p + 1, (uint64_t)min(deg - skip, a.heavy_deg) << 32 | (first + skip));
+      } else {
+        st_coh(&a.ctrl->abort, kAbortCapacity);
+      }
     }
     base += nch;
   }
   w.hn = w.hch = 0;
 }
 
-// Queues the vertices u of the lanes with `heavy` (degree deg) as chunks of
-// heavy_deg edges, expanded in the next round.
-__device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool heavy, uint32_t u, uint32_t deg) {
+// Queues the vertices u of the lanes with `heavy` (at distance d; edges first
+// to first + deg) as chunks of heavy_deg edges, expanded in the next round.
+__device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool heavy, uint32_t u, uint32_t d,
+                                           uint32_t first, uint32_t deg) {
   for (uint64_t m = __ballot(heavy); m; m &= m - 1) {
     const uint32_t l = (uint32_t)__builtin_ctzll(m);
     if (w.hn == kWaveHeavy) {
@@ -209,10 +232,9 @@ __device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool 
       if (lane_id() == 0) base = atomic_add(w.htail, w.hch);
       wave_store_heavy(a, w, readlane(base, 0));
     }
-    const uint32_t nch = (readlane(deg, l) - 1) / a.heavy_deg + 1;
-    if (lane_id() == 0) w.hbuf[w.hn] = WaveHeavy{readlane(u, l), nch};
+    if (lane_id() == l) w.hbuf[w.hn] = WaveHeavy{u, d, first, deg};
     w.hn += 1;
-    w.hch += nch;
+    w.hch += (readlane(deg, l) - 1) / a.heavy_deg + 1;
   }
 }
 
@@ -223,9 +245,9 @@ __device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool 
 // pushes of relax_edges in sssp_dev.h.
 template <Algo A, int U>
 __device__ __forceinline__ void wave_relax(const WaveArgs &a, WaveLane &w, const uint32_t (&e)[U],
-                                           const uint32_t (&du)[U], const bool (&act)[U]) {
+                                           const uint32_t (&du)[U], const bool (&act)[U], bool direct) {
   uint32_t v[U], nd[U], dv[U], old[U], seen[U], got[U];
-  bool near[U];
+  bool near[U], cand[U], any = false;
 #pragma unroll
   for (int k = 0; k < U; ++k) {
     v[k] = glb(a.edge_dst)[e[k]];
@@ -233,14 +255,23 @@ __device__ __forceinline__ void wave_relax(const WaveArgs &a, WaveLane &w, const
   }
   // through the caches: a stale distance is only ever larger
 #pragma unroll
-  for (int k = 0; k < U; ++k) dv[k] = glb(a.dist)[v[k]];
+  for (int k = 0; k < U; ++k) dv[k] = kInf;
+  if (!direct) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) dv[k] = glb(a.dist)[v[k]];
+  }
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    cand[k] = act[k] && nd[k] < dv[k];
+    any |= cand[k];
+  }
+  if (__ballot(any) == 0) return;
   uint32_t *const ns = a.near_stamp, *const fs = a.far_stamp;
 #pragma unroll
   for (int k = 0; k < U; ++k) {
     near[k] = A == Algo::BFS || nd[k] <= w.thr;
-    const bool cand = act[k] && nd[k] < dv[k];
-    seen[k] = glb(near[k] ? ns : fs)[cand ? v[k] : 0u];
-    old[k] = cand ? atomic_min(a.dist + v[k], nd[k]) : 0u;
+    seen[k] = glb(near[k] ? ns : fs)[cand[k] ? v[k] : 0u];
+    old[k] = cand[k] ? atomic_min(a.dist + v[k], nd[k]) : 0u;
   }
   // results are taken only here (left to itself the compiler tests each
   // result inside its atomic's branch, waiting for the whole memory queue)
@@ -276,9 +307,9 @@ __device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const
     rs = glb(a.row_start)[u];
     deg = glb(a.row_start)[u + 1] - rs;
   }
-  if (du == kInf) deg = 0;
+  if (du == kInf || (int64_t)du <= w.cut) deg = 0;
   const bool heavy = deg >= a.heavy_deg;
-  wave_heavy(a, w, heavy, u, deg);
+  wave_heavy(a, w, heavy, u, du, rs, deg);
   if (heavy) deg = 0;
   uint32_t end = deg;  // inclusive prefix over the lanes
 #pragma unroll
@@ -288,6 +319,7 @@ __device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const
   }
   const uint32_t total = readlane(end, kWave - 1);
   const uint32_t base = rs - (end - deg);
+  const bool direct = w.direct && total <= 2 * kWave;
   for (uint32_t b0 = 0; b0 < total; b0 += kWaveU * kWave) {
     uint32_t e[kWaveU], d0[kWaveU];
     bool act[kWaveU];
@@ -302,21 +334,21 @@ __device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const
       e[k] = (uint32_t)__shfl(base, pos) + f;
       d0[k] = (uint32_t)__shfl(du, pos);
     }
-    wave_relax<A, kWaveU>(a, w, e, d0, act);
+    wave_relax<A, kWaveU>(a, w, e, d0, act, direct);
   }
 }
 
-// One chunk of a heavy vertex.
+// One chunk of a heavy vertex.  Where the vertex has come nearer since it was
+// popped it is queued again, and the chunk is left to that.
 template <Algo A>
-__device__ __forceinline__ void wave_chunk(const WaveArgs &a, WaveLane &w, const uint64_t *ent) {
+__device__ __forceinline__ void wave_chunk(const WaveArgs &a, WaveLane &w, const WaveChunk *ent) {
   const uint32_t lane = lane_id();
-  const uint64_t x = ld_coh64(ent);
-  const uint32_t u = __builtin_amdgcn_readfirstlane((uint32_t)x), c = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
-  if (u >= a.nnodes) return;
-  const uint32_t du = ld_coh(a.dist + u);
-  const uint32_t row = glb(a.row_start)[u], deg = glb(a.row_start)[u + 1] - row, skip = c * a.heavy_deg;
-  if (skip >= deg) return;
-  const uint32_t rs = row + skip, n = min(deg - skip, a.heavy_deg);
+  const uint64_t *const p = reinterpret_cast<const uint64_t *>(ent);
+  const uint64_t x = ld_coh64(p), y = ld_coh64(p + 1);
+  const uint32_t u = __builtin_amdgcn_readfirstlane((uint32_t)x), d = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+  const uint32_t rs = __builtin_amdgcn_readfirstlane((uint32_t)y), n = __builtin_amdgcn_readfirstlane((uint32_t)(y >> 32));
+  if (u >= a.nnodes || n == 0 || (uint64_t)rs + n > a.nedges) return;
+  if (ld_coh(a.dist + u) < d) return;
   for (uint32_t b0 = 0; b0 < n; b0 += kWaveU * kWave) {
     uint32_t e[kWaveU], d0[kWaveU];
     bool act[kWaveU];
@@ -325,9 +357,9 @@ __device__ __forceinline__ void wave_chunk(const WaveArgs &a, WaveLane &w, const
       const uint32_t f = b0 + k * kWave + lane;
       act[k] = f < n;
       e[k] = rs + min(f, n - 1);
-      d0[k] = du;
+      d0[k] = d;
     }
-    wave_relax<A, kWaveU>(a, w, e, d0, act);
+    wave_relax<A, kWaveU>(a, w, e, d0, act, false);
   }
 }
 
@@ -351,7 +383,7 @@ struct LocalRelax {
 #pragma unroll
     for (int k = 0; k < kInFlight; ++k) {
       near[k] = A == Algo::BFS || nd[k] <= thr;
-      old[k] = act[k] ? atomic_min_wg(a.dist + v[k], nd[k]) : 0u;
+      old[k] = act[k] ? atomic_min(a.dist + v[k], nd[k]) : 0u;
       rb[k] = ld_pair(a.row_start + v[k]);
       seen[k] = A == Algo::SSSP ? ld_wg(a.far_stamp + (act[k] && !near[k] ? v[k] : 0u)) : 0u;
     }
@@ -361,7 +393,7 @@ struct LocalRelax {
 #pragma unroll
       for (int k = 0; k < kInFlight; ++k) {
         const bool want = act[k] && nd[k] < old[k] && !near[k] && seen[k] != far_stamp;
-        got[k] = want ? atomic_exch_wg(a.far_stamp + v[k], far_stamp) : far_stamp;
+        got[k] = want ? atomic_exch(a.far_stamp + v[k], far_stamp) : far_stamp;
       }
     }
     // near: one reservation per wavefront
@@ -410,12 +442,12 @@ struct LocalRelax {
     }
   }
   __device__ __forceinline__ void put(uint32_t *q, uint32_t pos, uint32_t v) const {
-    if (pos < a.qcap) st_wg(q + pos, v);
+    if (pos < a.qcap) st_coh(q + pos, v);
     else st_coh(&a.ctrl->abort, kAbortCapacity);
   }
   // A vertex that this mode hands on: once to the near queue.
   __device__ __forceinline__ void spill(uint32_t v) const {
-    if (atomic_exch_wg(a.near_stamp + v, near_stamp) != near_stamp) put(nq, atomicAdd(&sh.spill_n, 1u), v);
+    if (atomic_exch(a.near_stamp + v, near_stamp) != near_stamp) put(nq, atomicAdd(&sh.spill_n, 1u), v);
   }
 };
 
@@ -433,7 +465,6 @@ template <Algo A, int BS>
 __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh, int64_t cd0) {
   WaveRound r = sh.r;
   WavePace pace = sh.pace;
-  acquire_agent();
   const uint32_t far_in = A == Algo::SSSP ? ld_coh(&a.wc->far_tail[r.far_q()].n) : 0u;
   if (threadIdx.x == 0) {
     sh.far_n = far_in;
@@ -446,13 +477,15 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
   for (;;) {
     if (load) {
       const uint32_t *const in = wave_queue(a, r.in_q());
+      const int64_t cut = r.flags & kWaveCut ? (int64_t)wave_threshold(a, cd0, r.cut) : -1;
       bool big = false;
       for (uint32_t i = threadIdx.x; i < n; i += BS) {
-        const uint32_t v = ld_wg(in + i);
-        const uint32_t d = ld_wg(a.dist + v);
+        const uint32_t v = ld_coh(in + i);
+        const uint32_t d = ld_coh(a.dist + v);
         const uint64_t rb = ld_pair(a.row_start + v);
-        sh.pile[cur][i] = Entry{v, d, (uint32_t)rb, (uint32_t)(rb >> 32)};
-        big |= (uint32_t)(rb >> 32) - (uint32_t)rb >= a.heavy_deg;
+        const uint32_t rs = (uint32_t)rb, re = (int64_t)d <= cut ? rs : (uint32_t)(rb >> 32);
+        sh.pile[cur][i] = Entry{v, d, rs, re};
+        big |= re - rs >= a.heavy_deg;
       }
       // a heavy vertex among them: the grid runs this round
       if (__syncthreads_or(big)) break;
@@ -471,6 +504,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
     ++rounds;
     if (A == Algo::SSSP) pace.round(n, true);
     r.round += 1;
+    r.flags &= ~kWaveCut;
     const uint32_t near = sh.pile_n[cur ^ 1], far = sh.far_n;
     if (threadIdx.x == 0) st_coh(&a.ctrl->progress, r.round);
     if (near > kLocalMax || sh.stop) {
@@ -488,6 +522,8 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
       r.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
       r.phase += 1;
+      r.flags |= kWaveCut;
+      r.cut = r.steps;
       r.steps += a.pace ? pace.next(r.phase - 1) : 1u;
       n = far;
       order_release();  // this wavefront's far pushes have landed
@@ -505,7 +541,6 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
   order_release();
   __syncthreads();
   if (threadIdx.x == 0) {
-    release_agent();
     r.items = n;
     r.heavy = 0;
     sh.r = r;
@@ -523,6 +558,66 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
   __syncthreads();
 }
 
+// ---- between rounds -------------------------------------------------------------
+
+// Wavefront 0 of the block with number `seat` of `parties` arrives; true in the
+// last.  In groups of kBarGroup, as barrier_arrive; one level where one group
+// is enough.
+__device__ __forceinline__ bool wave_arrive(WaveCtrl::Slot *slot, uint32_t seat, uint32_t parties) {
+  uint32_t last = 0;
+  if (lane_id() == 0) {
+    const uint32_t grp = seat / kBarGroup, size = min(kBarGroup, parties - grp * kBarGroup);
+    last = atomic_add(&slot->arrive[grp].n, 1u) + 1 == size;
+    if (last && parties > kBarGroup)
+      last = atomic_add(&slot->top.n, 1u) + 1 == (parties + kBarGroup - 1) / kBarGroup;
+  }
+  return readlane(last, 0) != 0;
+}
+
+// Wavefront 0 waits for the message of a generation after `gen` (bounded by
+// spin_limit without progress): the round in x, and its generation.
+__device__ __forceinline__ uint32_t wave_wait(const WaveArgs &a, uint32_t gen, WaveRound &x) {
+  const uint32_t lane = lane_id();
+  const uint64_t *const p =
+      lane < kWaveMsg ? &a.wc->msg[lane] : reinterpret_cast<const uint64_t *>(&a.ctrl->abort);  // abort, checkin
+  uint64_t t0 = wall_clock64();
+  uint32_t seen = ld_coh(&a.ctrl->progress), tag;
+  uint32_t hi, flags = kWaveDone;
+  for (;;) {
+    const uint64_t m = ld_coh64(p);
+    const uint32_t lo = (uint32_t)m;
+    hi = (uint32_t)(m >> 32);
+    tag = readlane(lo, 0);
+    if (tag != gen && __ballot(lane < kWaveMsg && lo != tag) == 0) {
+      flags = readlane(hi, 6) >> 6 & (kWaveDone | kWaveCut);
+      break;
+    }
+    if (readlane(lo, kWaveMsg) != kAbortNone) break;
+    if (wall_clock64() - t0 > a.spin_limit) {
+      // the leading block may be running rounds on its own
+      const uint32_t now = ld_coh(&a.ctrl->progress);
+      if (now == seen) {
+        st_coh(&a.ctrl->abort, kAbortTimeout);
+        break;
+      }
+      seen = now;
+      t0 = wall_clock64();
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  x.items = readlane(hi, 0);
+  x.heavy = readlane(hi, 1);
+  x.round = readlane(hi, 2);
+  x.phase = readlane(hi, 3);
+  x.steps = readlane(hi, 4);
+  x.cut = readlane(hi, 5);
+  x.roles = readlane(hi, 6) & 0x3fu;
+  x.lead = readlane(hi, 6) >> 8;
+  x.flags = flags;
+  order_acquire();
+  return tag;
+}
+
 // ---- the kernel -------------------------------------------------------------------
 
 template <Algo A, int BS>
@@ -538,13 +633,13 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
   if (!residency_handshake(c, nb, a.residency_limit)) return;
   const int64_t cd0 = c->s.curdelta();  // written before this launch, as is the first round
   if (threadIdx.x == 0) {
-    sh.r.items = c->s.in_count;
-    sh.r.heavy = 0;
-    sh.r.round = 1;
-    sh.r.phase = 0;
-    sh.r.steps = 0;
-    sh.r.roles = wave_roles(0, 1, 2);
-    sh.r.flags = 0;
+    WaveRound x;
+    memset(&x, 0, sizeof x);
+    x.items = c->s.in_count;
+    x.round = 1;
+    x.roles = wave_roles(0, 1, 2);
+    sh.r = x;
+    sh.gen = 0;
   }
   __syncthreads();
   WaveLane w;
@@ -552,32 +647,36 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
   w.pbuf[1] = sh.push[wv][1];
   w.hbuf = sh.heavy[wv];
   w.n[0] = w.n[1] = w.hn = w.hch = 0;
-  for (uint32_t gen = 0;; ++gen) {
+  for (;;) {
     const WaveRound r = sh.r;
+    const uint32_t gen = sh.gen;
     if (r.flags & kWaveDone) break;
+    WaveCtrl::Slot *const slot = &wc->slot[gen % 3];
     w.near_stamp = r.round + 1;
     w.far_stamp = r.phase + 1;
     w.thr = wave_threshold(a, cd0, r.steps);
+    w.cut = r.flags & kWaveCut ? (int64_t)wave_threshold(a, cd0, r.cut) : -1;
+    w.direct = r.items <= kDirectMax;
     w.nq = wave_queue(a, r.near_q());
     w.fq = wave_queue(a, r.far_q());
-    w.ntail = &wc->near_tail[gen % 3].n;
+    w.ntail = &slot->near_tail.n;
     w.ftail = &wc->far_tail[r.far_q()].n;
-    w.htail = &wc->heavy_tail[gen % 3].n;
-    w.hq = reinterpret_cast<uint64_t *>(gen & 1 ? a.hq[1] : a.hq[0]);
+    w.htail = &slot->heavy_tail.n;
+    w.hq = gen & 1 ? a.chunk[1] : a.chunk[0];
     // Units: in-queue items, `per` at a time, then heavy chunks.  A wavefront
     // takes the unit of its number; where there are more units than
     // wavefronts, unit j * ngroups + g belongs to the blocks b with b % ngroups
     // == g, whose wavefronts draw tickets of their group (one word for all
     // wavefronts serialises, ~12 ns a ticket).
     const uint32_t *const in = wave_queue(a, r.in_q());
-    const uint64_t *const hin = reinterpret_cast<const uint64_t *>(gen & 1 ? a.hq[0] : a.hq[1]);
-    const uint32_t per = min((uint32_t)kWave, max(kUnitMin, (r.items + nwaves - 1) / nwaves));
+    const WaveChunk *const hin = gen & 1 ? a.chunk[0] : a.chunk[1];
+    const uint32_t per = min((uint32_t)kWave, max(a.unit_min, (r.items + nwaves - 1) / nwaves));
     const uint32_t nitem = (r.items + per - 1) / per, nunits = nitem + r.heavy;
     const bool many = nunits > nwaves;
     uint32_t unit = many ? (blockIdx.x / ngroups * NW + wv) * ngroups + g : wave;
     while (unit < nunits) {
       uint32_t t = 0;
-      if (many && lane_id() == 0) t = atomic_add(&wc->ticket[gen % 3][g].n, 1u);
+      if (many && lane_id() == 0) t = atomic_add(&slot->ticket[g].n, 1u);
       if (unit < nitem) wave_items<A>(a, w, in + (size_t)unit * per, min(per, r.items - unit * per));
       else wave_chunk<A>(a, w, hin + (unit - nitem));
       if (!many) break;
@@ -612,111 +711,86 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       order_release();
       __syncthreads();
     }
-    // The barrier.  The last block to arrive finds the next round.
-    if (threadIdx.x == 0) {
-      WaveRound x = r;
-      if (barrier_arrive(c, nb)) {
+    // The barrier: wavefront 0.  The blocks with a unit arrive, and the one that
+    // led the last round, so that what it cleared then is clear by now; the
+    // others only wait for a message of a later generation, and may miss rounds
+    // that they had no part in.  The last to arrive finds the next round.
+    if (wv == 0) {
+      const uint32_t active = many ? nb : (nunits + NW - 1) / NW;
+      const uint32_t parties = active + (r.lead >= active ? 1u : 0u);
+      const uint32_t seat = blockIdx.x < active ? blockIdx.x : blockIdx.x == r.lead ? active : parties;
+      if (seat < parties && wave_arrive(slot, seat, parties)) {
         order_acquire();
-        const uint32_t nnear = ld_coh(&wc->near_tail[gen % 3].n), nheavy = ld_coh(&wc->heavy_tail[gen % 3].n);
-        const uint32_t nfar = A == Algo::SSSP ? ld_coh(&wc->far_tail[r.far_q()].n) : 0u, ab = ld_coh(&c->abort);
-        WavePace pace{1, 0, 0, 0, 0};
-        if (A == Algo::SSSP) {
-          uint32_t p[5];
-#pragma unroll
-          for (int i = 0; i < 5; ++i) p[i] = ld_coh(&wc->pace[i]);
-          pace = WavePace{max(p[0], 1u), p[1], __uint_as_float(p[2]), __uint_as_float(p[3]), p[4]};
-          pace.round(r.items, false);
-        }
-        __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_fetch_add(&c->stat_heavy, (uint64_t)r.heavy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_fetch_add(&c->stat_rounds, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        st_coh(&wc->near_tail[(gen + 2) % 3].n, 0u);
-        st_coh(&wc->heavy_tail[(gen + 2) % 3].n, 0u);
-        for (uint32_t i = 0; i < kTicketGroups; ++i) st_coh(&wc->ticket[(gen + 2) % 3][i].n, 0u);
-        x.flags = kWaveLead;
+        WaveRound x = r;
+        // every word that the step needs in one load
+        const uint32_t lane = lane_id();
+        const uint32_t *p = lane == 0 ? &slot->near_tail.n : lane == 1 ? &slot->heavy_tail.n : lane == 2 ? &c->abort
+                            : lane < 8 ? &wc->pace[lane - 3] : &wc->far_tail[r.far_q()].n;
+        const uint32_t word = ld_coh(p);
+        const uint32_t nnear = readlane(word, 0), nheavy = readlane(word, 1), ab = readlane(word, 2);
+        const uint32_t nfar = A == Algo::SSSP ? readlane(word, 8) : 0u;
+        WavePace pace{max(readlane(word, 3), 1u), readlane(word, 4), __uint_as_float(readlane(word, 5)),
+                      __uint_as_float(readlane(word, 6)), readlane(word, 7)};
+        if (A == Algo::SSSP) pace.round(r.items, false);
+        // (the slot of the round before the last: no block reads it any more)
+        WaveCtrl::Slot *const next = &wc->slot[(gen + 2) % 3];
+        const uint32_t nclear = offsetof(WaveCtrl::Slot, arrive) / sizeof(WaveCtrl::Line) + (nb + kBarGroup - 1) / kBarGroup;
+        for (uint32_t i = lane; i < nclear; i += kWave) st_coh(&reinterpret_cast<WaveCtrl::Line *>(next)[i].n, 0u);
+        const bool full = nnear > a.qcap || nfar > a.qcap || nheavy > a.hcap;
+        if (full) st_coh(&c->abort, kAbortCapacity);
+        const bool within = nnear > 0 || nheavy > 0, phase = A == Algo::SSSP && !within && nfar > 0;
+        const bool done = full || ab != kAbortNone || !(within || phase);
         x.round = r.round + 1;
-        x.heavy = 0;
-        if (nnear > a.qcap || nfar > a.qcap || nheavy > a.hcap) {
-          st_coh(&c->abort, kAbortCapacity);
-          x.flags |= kWaveDone;
-        } else if (ab != kAbortNone) {
-          x.flags |= kWaveDone;
-        } else if (nnear > 0 || nheavy > 0) {
-          x.items = nnear;
-          x.heavy = nheavy;
-          x.roles = wave_roles(r.near_q(), r.in_q(), r.far_q());
-        } else if (A == Algo::SSSP && nfar > 0) {
+        x.lead = blockIdx.x;
+        x.heavy = nheavy;
+        x.items = phase ? nfar : nnear;
+        x.roles = wave_roles(r.near_q(), r.in_q(), r.far_q());
+        if (phase) {
           // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
-          x.items = nfar;
-          x.phase = r.phase + 1;
-          x.steps = r.steps + (a.pace ? pace.next(r.phase) : 1u);
           x.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
-          st_coh(&wc->far_tail[r.far_q()].n, 0u);
-        } else {
-          x.flags |= kWaveDone;
+          x.phase = r.phase + 1;
+          x.cut = r.steps;
+          x.steps = r.steps + (a.pace ? pace.next(r.phase) : 1u);
+          if (lane == 0) st_coh(&wc->far_tail[r.far_q()].n, 0u);
         }
-        if (!(x.flags & kWaveDone) && x.heavy == 0 && x.items <= kLocalMax) x.flags |= kWaveLocal;
-        sh.pace = pace;
+        x.flags = kWaveLead | (done ? kWaveDone : x.heavy == 0 && x.items <= kLocalMax ? kWaveLocal : 0u) |
+                  (phase ? kWaveCut : 0u);
+        if (lane == 0) {
+          __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_fetch_add(&c->stat_heavy, (uint64_t)r.heavy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_fetch_add(&c->stat_rounds, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          sh.pace = pace;
+          sh.r = x;
+          sh.gen = gen + 1;
+        }
       } else {
-        uint64_t t0 = wall_clock64();
-        uint32_t seen = ld_coh(&c->progress);
-        for (;;) {
-          uint64_t m[kWaveMsg];
-#pragma unroll
-          for (int i = 0; i < kWaveMsg; ++i) m[i] = ld_coh64(&wc->msg[i]);
-          const uint32_t ab = ld_coh(&c->abort);
-          bool valid = true;
-#pragma unroll
-          for (int i = 0; i < kWaveMsg; ++i) valid &= (uint32_t)m[i] == gen + 1;
-          if (valid) {
-            x.items = (uint32_t)(m[0] >> 32);
-            x.heavy = (uint32_t)(m[1] >> 32);
-            x.round = (uint32_t)(m[2] >> 32);
-            x.phase = (uint32_t)(m[3] >> 32);
-            x.steps = (uint32_t)(m[4] >> 32);
-            x.roles = (uint32_t)(m[5] >> 32) & 0x3fu;
-            x.flags = (uint32_t)(m[5] >> 38) & kWaveDone;
-            break;
-          }
-          if (ab != kAbortNone) {
-            x.flags = kWaveDone;
-            break;
-          }
-          if (wall_clock64() - t0 > a.spin_limit) {
-            // the leading block may be running rounds on its own
-            const uint32_t p = ld_coh(&c->progress);
-            if (p != seen) {
-              seen = p;
-              t0 = wall_clock64();
-              continue;
-            }
-            st_coh(&c->abort, kAbortTimeout);
-            x.flags = kWaveDone;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
+        WaveRound x = r;
+        const uint32_t tag = wave_wait(a, gen, x);
+        if (lane_id() == 0) {
+          sh.r = x;
+          sh.gen = tag;
         }
-        order_acquire();
       }
-      sh.r = x;
     }
     __syncthreads();
     if (sh.r.flags & kWaveLead) {
       if (sh.r.flags & kWaveLocal) wave_local<A, BS>(a, sh, cd0);
-      if (threadIdx.x == 0) {
+      if (wv == 0) {
+        const uint32_t lane = lane_id();
         const WaveRound x = sh.r;
-        const uint32_t done = x.flags & kWaveDone;
-        const uint32_t m[kWaveMsg] = {x.items, x.heavy, x.round, x.phase, x.steps, x.roles | done << 6};
+        const uint32_t m[kWaveMsg] = {x.items, x.heavy, x.round, x.phase, x.steps, x.cut,
+                                      x.lead << 8 | (x.flags & (kWaveDone | kWaveCut)) << 6 | x.roles};
+        uint32_t v = 0;
 #pragma unroll
-        for (int i = 0; i < kWaveMsg; ++i) st_coh64(&wc->msg[i], (uint64_t)m[i] << 32 | (gen + 1));
-        if (A == Algo::SSSP) {
-          st_coh(&wc->pace[0], sh.pace.step);
-          st_coh(&wc->pace[1], sh.pace.hold);
-          st_coh(&wc->pace[2], __float_as_uint(sh.pace.best));
-          st_coh(&wc->pace[3], __float_as_uint(sh.pace.cost));
-          st_coh(&wc->pace[4], sh.pace.rounds);
+        for (int i = 0; i < kWaveMsg; ++i)
+          if (lane == (uint32_t)i) v = m[i];
+        if (lane < kWaveMsg) st_coh64(&wc->msg[lane], (uint64_t)v << 32 | (gen + 1));
+        if (A == Algo::SSSP && lane < 5) {
+          const WavePace p = sh.pace;
+          st_coh(&wc->pace[lane], lane == 0 ? p.step : lane == 1 ? p.hold : lane == 2 ? __float_as_uint(p.best)
+                                  : lane == 3 ? __float_as_uint(p.cost) : p.rounds);
         }
-        if (done) {
+        if ((x.flags & kWaveDone) && lane == 0) {
           c->s.done = 1;
           c->s.round = x.round;
           c->s.phase = x.phase;
