@@ -79,6 +79,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     // (at 16 / 8 / 4: RMAT-17 SSSP 0.45 / 0.40 / 0.44 ms, RMAT-20 1.02 / 1.01 / 1.00).
     a.pace = g.nedges <= 6ull * g.nnodes;
     a.unit_min = a.pace ? 16 : 8;
+    a.local_max = wave_local_max(g.nnodes, g.nedges);
     void *chunks;
     if ((rc = ws_buffer(w, kBufHeavy, 2ull * a.hcap * sizeof(WaveChunk), &chunks))) return rc;
     a.chunk[0] = (WaveChunk *)chunks;

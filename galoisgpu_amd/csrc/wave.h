@@ -19,7 +19,7 @@ struct WaveCtrl {
   // How far the next phase moves the threshold; between leading blocks only.
   uint32_t pace[5];
   uint32_t _p1[27];
-  struct Line {
+  struct alignas(8) Line {
     uint32_t n;
     uint32_t _p[31];
   };
@@ -27,7 +27,9 @@ struct WaveCtrl {
   // By generation mod 3: the leader of one round clears the words of the one
   // after the next.
   struct Slot {
-    Line near_tail, heavy_tail, ticket[kTicketGroups], top, arrive[kMaxBarGroups];
+    Line near_tail, heavy_tail, ticket[kTicketGroups], top;
+    Line sum[kTicketGroups];  // u64: edges of the vertices found << 32 | vertices found (bfs_do.hip)
+    Line arrive[kMaxBarGroups];
   } slot[3];
 };
 
@@ -41,6 +43,8 @@ struct WaveArgs : KArgs {
   WaveCtrl *wc = nullptr;
   uint32_t pace = 0;      // the threshold's steps are paced (WavePace)
   uint32_t unit_min = 0;  // fewest items of a unit
+  uint32_t local_max = 0; // largest round that one block runs alone
+  uint32_t _pad = 0;
 };
 
 // Blocks per CU, of 256 threads, where the call leaves the launch shape open.
@@ -54,6 +58,11 @@ struct WaveArgs : KArgs {
 constexpr int kWaveBlock = 256;
 inline int wave_blocks_per_cu(uint64_t nnodes, uint64_t nedges) {
   return nedges <= 6 * nnodes || nedges < 3u << 20 ? 1 : nedges < 1u << 25 ? 2 : 3;
+}
+// Largest round, in items, that one block runs alone: some 2048 edges (limits
+// of 512 / 128 items on RMAT: 2^14 vertices 0.256 / 0.245 ms, 2^20 1.00 / 0.98).
+inline uint32_t wave_local_max(uint64_t nnodes, uint64_t nedges) {
+  return (uint32_t)(nedges <= 4 * nnodes ? 512 : 2048 * nnodes / nedges);
 }
 // A chunk of a heavy vertex is the edges that a wavefront holds in flight
 // (kWaveU a lane); 512 and 1024: equal to 5 % slower on RMAT graphs.

@@ -32,7 +32,7 @@
 //     that came below the last threshold meanwhile were near items then
 //     (RMAT-20: most of 505,060, 145 -> 87 us), and chunks of a vertex that was
 //     lowered since it was popped are left to its next pop.
-//   - Small rounds (at most kLocalMax items, no heavy vertex) are run by the
+//   - Small rounds (at most local_max items, no heavy vertex) are run by the
 //     last block alone, with entries in LDS as in the one-workgroup kernel
 //     (block.hip): two or three round trips and two block barriers a round
 //     while the others stay parked.  The looks at d[v] and at stamps whose
@@ -50,40 +50,16 @@
 
 #include <hip/hip_runtime.h>
 
-#include "wave.h"
+#include "wave_dev.h"
 
 namespace lsg {
 
-// Largest round that one block runs alone, and the entries of a pile in LDS (a
-// round's pushes are not deduplicated in there).
-constexpr uint32_t kLocalMax = 512;
+// The entries of a pile in LDS, of a round that one block runs alone (its pushes
+// are not deduplicated in there).
 constexpr uint32_t kLocalCap = 1024;
 constexpr uint32_t kWavePush = 256;   // staged items per wavefront and pile
-constexpr uint32_t kWaveHeavy = 32;   // staged heavy items per wavefront
+constexpr uint32_t kWaveHeavy = 64;   // staged heavy items per wavefront, one a lane
 constexpr uint32_t kMaxStep = 1u << 16;
-// Rounds of at most this many items go straight to the atomicMins where a unit
-// has few edges: one round trip less, and few enough atomics.
-constexpr uint32_t kDirectMax = 4096;
-
-// Roles of the three queues and the state of a round.
-struct WaveRound {
-  uint32_t items, heavy, round, phase;
-  uint32_t steps;  // the near/far threshold, in steps of delta
-  uint32_t cut;    // kWaveCut: the previous phase's
-  uint32_t lead;   // the block that published the round
-  uint32_t roles;  // in | near << 2 | far << 4
-  uint32_t flags;
-  __device__ uint32_t in_q() const { return roles & 3u; }
-  __device__ uint32_t near_q() const { return roles >> 2 & 3u; }
-  __device__ uint32_t far_q() const { return roles >> 4 & 3u; }
-};
-// kWaveCut: the round's input is the far pile; what has come below the previous
-// threshold since it was pushed has been expanded as a near item already.
-constexpr uint32_t kWaveDone = 1, kWaveCut = 2, kWaveLead = 4, kWaveLocal = 8;
-__device__ __forceinline__ uint32_t wave_roles(uint32_t in, uint32_t near, uint32_t far) {
-  return in | near << 2 | far << 4;
-}
-
 struct WaveHeavy {
   uint32_t u, d, first, deg;
 };
@@ -165,7 +141,7 @@ struct WaveLane {
   uint32_t *htail;
   uint32_t *pbuf[2];
   WaveHeavy *hbuf;
-  uint32_t n[2], hn, hch;  // staged: items per pile, heavy items and their chunks (wave-uniform)
+  uint32_t n[2], hn;  // staged: items per pile, heavy items (wave-uniform)
 };
 
 __device__ __forceinline__ uint32_t *wave_queue(const WaveArgs &a, uint32_t i) {
@@ -200,42 +176,40 @@ __device__ __forceinline__ void wave_stage(const WaveArgs &a, WaveLane &w, int w
   w.n[which] += c;
 }
 
-// Writes the staged heavy items' chunks from slot `base` on.
-__device__ __forceinline__ void wave_store_heavy(const WaveArgs &a, WaveLane &w, uint32_t base) {
-  for (uint32_t i = 0; i < w.hn; ++i) {
-    const uint32_t u = __builtin_amdgcn_readfirstlane(w.hbuf[i].u), d = __builtin_amdgcn_readfirstlane(w.hbuf[i].d);
-    const uint32_t first = __builtin_amdgcn_readfirstlane(w.hbuf[i].first);
-    const uint32_t deg = __builtin_amdgcn_readfirstlane(w.hbuf[i].deg), nch = (deg - 1) / a.heavy_deg + 1;
-    for (uint32_t k = lane_id(); k < nch; k += kWave) {
-      const uint32_t pos = base + k, skip = k * a.heavy_deg;
-      if (pos < a.hcap) {
-        uint64_t *const p = reinterpret_cast<uint64_t *>(w.hq + pos);
-        st_coh64(p, (uint64_t)d << 32 | u);
-        st_coh64(p + 1, (uint64_t)min(deg - skip, a.heavy_deg) << 32 | (first + skip));
-      } else {
-        st_coh(&a.ctrl->abort, kAbortCapacity);
-      }
+// Writes the staged heavy items' chunks, counted in `end`, from slot `base` on.
+__device__ __forceinline__ void wave_store_heavy(const WaveArgs &a, WaveLane &w, uint32_t end, uint32_t base) {
+  chunk_each(end, [&](uint32_t f, uint32_t item, uint32_t k) {
+    const uint32_t pos = base + f, skip = k * a.heavy_deg;
+    const WaveHeavy h = w.hbuf[item];
+    if (pos < a.hcap) {
+      uint64_t *const p = reinterpret_cast<uint64_t *>(w.hq + pos);
+      st_coh64(p, (uint64_t)h.d << 32 | h.u);
+      st_coh64(p + 1, (uint64_t)min(h.deg - skip, a.heavy_deg) << 32 | (h.first + skip));
+    } else {
+      st_coh(&a.ctrl->abort, kAbortCapacity);
     }
-    base += nch;
-  }
-  w.hn = w.hch = 0;
+  });
+  w.hn = 0;
+}
+__device__ __forceinline__ uint32_t wave_heavy_ends(const WaveArgs &a, const WaveLane &w) {
+  return chunk_ends(w.hn, lane_id() < w.hn ? w.hbuf[lane_id()].deg : 0u, a.heavy_deg);
 }
 
 // Queues the vertices u of the lanes with `heavy` (at distance d; edges first
 // to first + deg) as chunks of heavy_deg edges, expanded in the next round.
 __device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool heavy, uint32_t u, uint32_t d,
                                            uint32_t first, uint32_t deg) {
-  for (uint64_t m = __ballot(heavy); m; m &= m - 1) {
-    const uint32_t l = (uint32_t)__builtin_ctzll(m);
-    if (w.hn == kWaveHeavy) {
-      uint32_t base = 0;
-      if (lane_id() == 0) base = atomic_add(w.htail, w.hch);
-      wave_store_heavy(a, w, readlane(base, 0));
-    }
-    if (lane_id() == l) w.hbuf[w.hn] = WaveHeavy{u, d, first, deg};
-    w.hn += 1;
-    w.hch += (readlane(deg, l) - 1) / a.heavy_deg + 1;
+  const uint64_t m = __ballot(heavy);
+  if (m == 0) return;
+  const uint32_t c = (uint32_t)__builtin_popcountll(m);
+  if (w.hn + c > kWaveHeavy) {
+    const uint32_t end = wave_heavy_ends(a, w);
+    uint32_t base = 0;
+    if (lane_id() == 0) base = atomic_add(w.htail, readlane(end, kWave - 1));
+    wave_store_heavy(a, w, end, readlane(base, 0));
   }
+  if (heavy) w.hbuf[w.hn + lanes_below(m)] = WaveHeavy{u, d, first, deg};
+  w.hn += c;
 }
 
 // ---- relaxation ----------------------------------------------------------------
@@ -457,7 +431,7 @@ __device__ __forceinline__ uint32_t wave_threshold(const WaveArgs &a, int64_t cd
 }
 
 // Called by every thread of the block that leads, with the next round in sh.r
-// (at most kLocalMax items, no heavy chunks): runs it and the rounds that
+// (at most a.local_max items, no heavy chunks): runs it and the rounds that
 // follow for as long as they are small, and leaves in sh.r the round that the
 // whole grid runs next.  Every wavefront's memory operations are complete on
 // return.
@@ -507,7 +481,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
     r.flags &= ~kWaveCut;
     const uint32_t near = sh.pile_n[cur ^ 1], far = sh.far_n;
     if (threadIdx.x == 0) st_coh(&a.ctrl->progress, r.round);
-    if (near > kLocalMax || sh.stop) {
+    if (near > a.local_max || sh.stop) {
       // hand over: what spilled already, and the pile
       for (uint32_t i = threadIdx.x; i < min(near, kLocalCap); i += BS) relax.spill(sh.pile[cur ^ 1][i].v);
       __syncthreads();
@@ -529,7 +503,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       order_release();  // this wavefront's far pushes have landed
       __syncthreads();  // and every other's; far_n has been read
       if (threadIdx.x == 0) sh.far_n = 0;
-      if (n > kLocalMax) break;
+      if (n > a.local_max) break;
       load = true;
     } else {
       r.flags |= kWaveDone;
@@ -556,66 +530,6 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
   }
   order_release();
   __syncthreads();
-}
-
-// ---- between rounds -------------------------------------------------------------
-
-// Wavefront 0 of the block with number `seat` of `parties` arrives; true in the
-// last.  In groups of kBarGroup, as barrier_arrive; one level where one group
-// is enough.
-__device__ __forceinline__ bool wave_arrive(WaveCtrl::Slot *slot, uint32_t seat, uint32_t parties) {
-  uint32_t last = 0;
-  if (lane_id() == 0) {
-    const uint32_t grp = seat / kBarGroup, size = min(kBarGroup, parties - grp * kBarGroup);
-    last = atomic_add(&slot->arrive[grp].n, 1u) + 1 == size;
-    if (last && parties > kBarGroup)
-      last = atomic_add(&slot->top.n, 1u) + 1 == (parties + kBarGroup - 1) / kBarGroup;
-  }
-  return readlane(last, 0) != 0;
-}
-
-// Wavefront 0 waits for the message of a generation after `gen` (bounded by
-// spin_limit without progress): the round in x, and its generation.
-__device__ __forceinline__ uint32_t wave_wait(const WaveArgs &a, uint32_t gen, WaveRound &x) {
-  const uint32_t lane = lane_id();
-  const uint64_t *const p =
-      lane < kWaveMsg ? &a.wc->msg[lane] : reinterpret_cast<const uint64_t *>(&a.ctrl->abort);  // abort, checkin
-  uint64_t t0 = wall_clock64();
-  uint32_t seen = ld_coh(&a.ctrl->progress), tag;
-  uint32_t hi, flags = kWaveDone;
-  for (;;) {
-    const uint64_t m = ld_coh64(p);
-    const uint32_t lo = (uint32_t)m;
-    hi = (uint32_t)(m >> 32);
-    tag = readlane(lo, 0);
-    if (tag != gen && __ballot(lane < kWaveMsg && lo != tag) == 0) {
-      flags = readlane(hi, 6) >> 6 & (kWaveDone | kWaveCut);
-      break;
-    }
-    if (readlane(lo, kWaveMsg) != kAbortNone) break;
-    if (wall_clock64() - t0 > a.spin_limit) {
-      // the leading block may be running rounds on its own
-      const uint32_t now = ld_coh(&a.ctrl->progress);
-      if (now == seen) {
-        st_coh(&a.ctrl->abort, kAbortTimeout);
-        break;
-      }
-      seen = now;
-      t0 = wall_clock64();
-    }
-    __builtin_amdgcn_s_sleep(1);
-  }
-  x.items = readlane(hi, 0);
-  x.heavy = readlane(hi, 1);
-  x.round = readlane(hi, 2);
-  x.phase = readlane(hi, 3);
-  x.steps = readlane(hi, 4);
-  x.cut = readlane(hi, 5);
-  x.roles = readlane(hi, 6) & 0x3fu;
-  x.lead = readlane(hi, 6) >> 8;
-  x.flags = flags;
-  order_acquire();
-  return tag;
 }
 
 // ---- the kernel -------------------------------------------------------------------
@@ -646,7 +560,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
   w.pbuf[0] = sh.push[wv][0];
   w.pbuf[1] = sh.push[wv][1];
   w.hbuf = sh.heavy[wv];
-  w.n[0] = w.n[1] = w.hn = w.hch = 0;
+  w.n[0] = w.n[1] = w.hn = 0;
   for (;;) {
     const WaveRound r = sh.r;
     const uint32_t gen = sh.gen;
@@ -683,11 +597,12 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       unit = (gblocks * NW + readlane(t, 0)) * ngroups + g;
     }
     // The block's pushes get their places with one atomic per pile.
+    const uint32_t hend = w.hn ? wave_heavy_ends(a, w) : 0u;
     order_release();
-    if (lane_id() == 0) {
+    if (lane_id() == kWave - 1) {
       sh.count[wv][0] = w.n[0];
       sh.count[wv][1] = w.n[1];
-      sh.count[wv][2] = w.hch;
+      sh.count[wv][2] = hend;
     }
     __syncthreads();
     uint32_t tot[3] = {0, 0, 0}, off[3] = {0, 0, 0};
@@ -707,7 +622,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       __syncthreads();
       if (w.n[0]) wave_store(a, w, 0, sh.base[0] + off[0]);
       if (w.n[1]) wave_store(a, w, 1, sh.base[1] + off[1]);
-      if (w.hn) wave_store_heavy(a, w, sh.base[2] + off[2]);
+      if (w.hn) wave_store_heavy(a, w, hend, sh.base[2] + off[2]);
       order_release();
       __syncthreads();
     }
@@ -753,7 +668,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
           x.steps = r.steps + (a.pace ? pace.next(r.phase) : 1u);
           if (lane == 0) st_coh(&wc->far_tail[r.far_q()].n, 0u);
         }
-        x.flags = kWaveLead | (done ? kWaveDone : x.heavy == 0 && x.items <= kLocalMax ? kWaveLocal : 0u) |
+        x.flags = kWaveLead | (done ? kWaveDone : x.heavy == 0 && x.items <= a.local_max ? kWaveLocal : 0u) |
                   (phase ? kWaveCut : 0u);
         if (lane == 0) {
           __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -778,13 +693,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       if (wv == 0) {
         const uint32_t lane = lane_id();
         const WaveRound x = sh.r;
-        const uint32_t m[kWaveMsg] = {x.items, x.heavy, x.round, x.phase, x.steps, x.cut,
-                                      x.lead << 8 | (x.flags & (kWaveDone | kWaveCut)) << 6 | x.roles};
-        uint32_t v = 0;
-#pragma unroll
-        for (int i = 0; i < kWaveMsg; ++i)
-          if (lane == (uint32_t)i) v = m[i];
-        if (lane < kWaveMsg) st_coh64(&wc->msg[lane], (uint64_t)v << 32 | (gen + 1));
+        wave_publish(wc, gen + 1, x);
         if (A == Algo::SSSP && lane < 5) {
           const WavePace p = sh.pace;
           st_coh(&wc->pace[lane], lane == 0 ? p.step : lane == 1 ? p.hold : lane == 2 ? __float_as_uint(p.best)
@@ -804,10 +713,6 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
 
 // ---- launch -------------------------------------------------------------------------
 
-__device__ __forceinline__ void wave_reset(WaveCtrl *wc, uint32_t tid, uint32_t nt) {
-  uint32_t *const p = reinterpret_cast<uint32_t *>(wc);
-  for (uint32_t i = tid; i < sizeof(WaveCtrl) / 4; i += nt) p[i] = 0;
-}
 __global__ void wave_reset_kernel(WaveCtrl *wc) { wave_reset(wc, threadIdx.x, blockDim.x); }
 
 // Distances, stamps, control words and the one seed (apps/sssp/kernel.cu:23-35,469,476-477).

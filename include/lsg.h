@@ -266,8 +266,8 @@ int lsg_output_pr(const float *rank, uint32_t n, const char *file, int ids_only)
  * algorithm; the levels are apps/bfs's, as lsg_bfs_dist writes them).  `gt`
  * is the reverse of `g` (lsg_graph_transpose).  direction: 0 = per level by
  * frontier size (top-down, bottom-up once the frontier's edges exceed 1/14 of
- * the unexplored edges, top-down again below V/24 frontier vertices), 1 =
- * top-down only, 2 = bottom-up only.  level_dev is a device array of nnodes.
+ * the unexplored edges and 1/16 of all, top-down again below V/24 frontier
+ * vertices), 1 = top-down only, 2 = bottom-up only.  level_dev is a device array of nnodes.
  * stats: iterations = levels, near_iters = bottom-up levels. */
 int lsg_bfs_do(const lsg_graph *g, const lsg_graph *gt, uint32_t src, int direction, int32_t *level_dev,
                lsg_stats *stats);
