@@ -88,6 +88,28 @@ struct Filter {
   int32_t off[64];
 };
 
+// Pace of the near/far threshold (fixed delta, reference far pile): it moves by
+// `step` deltas.  A round of a batch costs some 20 us however small, and the far
+// pile, expanded as a whole every phase, is mostly work done again: with 64
+// sources the rounds of one wide phase expand a vertex for many of them at
+// once.  On graphs with a hub, of few hops, the step begins at kHubStep; it is
+// climbed from there while the threshold then moves further per us of modelled
+// cost, or while rounds are nearly empty; else one step back, and two phases
+// later the next trial.  Distances do not depend on it.
+// Ms at steps of 1 -> here (delta 32): RMAT of 16400 vertices x 5 sources 1.84 ->
+// 0.78, 100003 x 9 3.9 -> 1.37, 262900 x 64 12.0 -> 2.9 (at a delta that passes
+// every distance 2.7); grid 64^2 x 5 6.0 -> 2.6, road-like 300^2 x 64 at 10000
+// 13 -> 6.9.
+struct Pace {
+  uint32_t step;    // deltas that the threshold moves by
+  uint32_t hold;    // phases until the next trial; 0: this phase is one
+  float best;       // deltas per us before the trial
+  uint32_t rounds;  // before this phase
+  uint64_t edges;   // expanded before this phase
+};
+constexpr uint32_t kHubStep = 16, kMaxMultiStep = 1u << 16;
+constexpr float kRoundUs = 20, kEdgesPerUs = 30000;
+
 // Work tickets and round totals are kept per group of blocks (block b: group
 // b % kGroups), each on a line of its own: atomics on one word are performed
 // one at a time, ~12 ns each, and a word that all 4096 wavefronts share
@@ -132,6 +154,7 @@ struct MArgs {
   uint32_t *thr;        // [64] per-source near/far threshold of the current phase (bucket mode)
   uint32_t *qstamp;     // [V] last round whose in-queue holds the vertex
   Filter *flt;          // edge filter state
+  Pace *pace;           // threshold pace, or null (steps of delta)
   TicketGroup *tickets; // [kGroups]
   MultiCounters *tot;   // [kGroups]
   uint64_t *hubs;       // multi_init's largest (out-degree << 32 | ~vertex) of each block
@@ -862,6 +885,34 @@ __device__ __forceinline__ void multi_leader(const MArgs &a) {
   __shared__ int act_sh;
   int act = -1;
   if (a.sched) act = mlp_block_action(a.mlp, f, sc);
+  if (t == 0 && a.pace) {
+    Pace &p = *a.pace;  // touched by leaders only, ordered by the barrier
+    uint32_t step = ld_coh(&p.step), hold = ld_coh(&p.hold);
+    float best = __uint_as_float(ld_coh((uint32_t *)&p.best));
+    const float rounds = (float)(s.round - ld_coh(&p.rounds)), edges = (float)(edges_now - ld_coh64(&p.edges));
+    const float cost = kRoundUs * rounds + edges / kEdgesPerUs, rate = (float)step / cost;
+    if (s.phase == 0) {  // the sources alone
+      step = ld_coh(&a.flt->on) ? kHubStep : 1u;
+    } else if (hold == 0 || cost < 1.25f * kRoundUs * rounds) {
+      hold = 0;
+      if (rate > 1.02f * best || cost < 1.25f * kRoundUs * rounds) {
+        best = rate;
+        step = min(step * 2, kMaxMultiStep);
+      } else {
+        step = max(step / 2, 1u);
+        hold = 2;
+      }
+    } else if (--hold == 0) {
+      best = rate;
+      step = min(step * 2, kMaxMultiStep);
+    }
+    st_coh(&p.step, step);
+    st_coh(&p.hold, hold);
+    st_coh((uint32_t *)&p.best, __float_as_uint(best));
+    st_coh(&p.rounds, s.round);
+    st_coh64(&p.edges, edges_now);
+    s.delta = (uint32_t)min((uint64_t)step * a.delta, (uint64_t)kInf);
+  }
   if (t == 0) {
     if (act >= 0) {
       s.delta = action_delta(a.mlp, act, a.delta);
@@ -1126,6 +1177,7 @@ __global__ void multi_seed(MArgs a) {
     a.flt->hub = ~(uint32_t)hub;
     a.flt->on = (hub >> 32) * a.nnodes >= (uint64_t)kHubRatio * a.nedges && a.nedges;
     a.flt->incl = a.flt->last_edges = 0;
+    if (a.pace) *a.pace = Pace{1, 0, 0.0f, 0, 0};
     Ctrl *c = a.ctrl;
     c->qcount[0] = (uint32_t)__builtin_popcountll(pm);
     c->qcount[1] = 0;
@@ -1263,6 +1315,8 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
   a.fmin = (uint32_t *)((char *)sbuf + 512);
   a.thr = (uint32_t *)((char *)sbuf + 1024);
   a.flt = (Filter *)((char *)sbuf + 1280);
+  static_assert(1280 + sizeof(Filter) <= 1792 && 1792 + sizeof(Pace) <= 2048, "the words before the tickets");
+  if (!o.sched && !o.trace && o.far_mode == LSG_FAR_REFERENCE) a.pace = (Pace *)((char *)sbuf + 1792);
   a.tickets = (TicketGroup *)((char *)sbuf + 2048);
   a.tot = (MultiCounters *)(a.tickets + kGroups);
   if (o.sched) {

@@ -116,3 +116,12 @@ def test_every_unit_is_taken(blocks):
         print("units", blocks, block_size, flush=True)
         check(g, srcs, delta=40, grid_blocks=blocks, block_size=block_size)
         check(CSRGraph.grid(40, 60, seed=blocks), [3, 700], delta=64, grid_blocks=blocks, block_size=block_size)
+
+
+@pytest.mark.parametrize("whi", [1, 100, 60000, 1 << 24])
+@pytest.mark.parametrize("delta", [1, 32, 1 << 28])
+def test_paced_threshold(whi, delta):
+    """Steps of delta that grow from phase to phase, on graphs with and without a hub."""
+    print("paced", whi, delta, flush=True)
+    check(hub_graph(3001, whi, whi), [0, 1, 7, 2000, 2999], delta=delta)
+    check(CSRGraph.grid(60, 41, 1, whi, seed=3), [0, 17, 2459], delta=delta)
