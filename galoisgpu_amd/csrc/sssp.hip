@@ -48,6 +48,11 @@ static KernelFn pick_kernel(int bs) {
   }
 }
 
+// Whether a call asks for what the wavefront kernel has.
+static bool default_kernel(const lsg_opts &o) {
+  return o.expand_mode == LSG_EXPAND_LB && o.far_mode == LSG_FAR_REFERENCE && !o.sched && !o.trace;
+}
+
 // Runs one traversal from `nseeds` seeds (host array) into dist (device,
 // g.nnodes entries).  Synchronous.  With graph_launch the init, seed and
 // persistent kernels are replayed as one captured hipGraph.  With `resume`:
@@ -62,7 +67,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
   void *seedbuf;
   // The wavefront kernel takes what a call asks for by default; the options
   // that it does not have run in the persistent kernel.
-  const bool wave = o.expand_mode == LSG_EXPAND_LB && o.far_mode == LSG_FAR_REFERENCE && !o.sched && !o.trace;
+  const bool wave = default_kernel(o);
   lsg_opts ow = o;
   if (wave) {
     if (ow.block_size == 0) ow.block_size = kWaveBlock;
@@ -182,6 +187,12 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
   return LSG_OK;
 }
 
+// Small graphs of low degree, unless the call sets a launch shape of its own.
+static bool use_small(const CsrView &g, const lsg_opts &o) {
+  return default_kernel(o) && !o.enable_lb && !o.graph_launch && o.block_size == 0 && o.grid_blocks <= 0 &&
+         o.heavy_deg <= 0 && g.nnodes <= kSmallV && g.nedges <= 6ull * g.nnodes;
+}
+
 // One source on one device graph into dist (device array of g->nnodes).
 template <Algo A>
 static int run_single(const lsg_graph *g, const lsg_opts *o_in, uint32_t *dist, lsg_stats *st) {
@@ -218,6 +229,10 @@ static int run_single(const lsg_graph *g, const lsg_opts *o_in, uint32_t *dist, 
     } else if (rc == LSG_OK && st) {
       *st = bst;
     }
+  } else if (use_small(v, o)) {
+    int bs, expand;
+    if ((rc = check_single_opts(o, A == Algo::SSSP, &bs, &expand))) return rc;
+    rc = run_small_single((int)A, w, v, seed, o, dist, st);
   } else {
     rc = o.enable_lb ? run_lb_single((int)A, w, v, seed, o, dist, st)
                      : run_core<A>(w, v, &seed, 1, o, dist, o.graph_launch != 0, st);

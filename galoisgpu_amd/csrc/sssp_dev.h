@@ -1231,4 +1231,10 @@ int run_block_single(int algo, Workspace *w, const CsrView &g, uint32_t seed, co
 int run_graphs_block(Workspace *w, const lsg_graph *graphs, uint32_t ngraphs, const uint32_t *srcs,
                      int32_t *const *dist_out, const lsg_opts &o, lsg_batch_stats *stats);
 
+// Small low-degree graphs in one workgroup, distances in LDS (small.hip).  Takes
+// at most kSmallV vertices; options as the wavefront kernel's.
+constexpr uint32_t kSmallV = 32768;
+int run_small_single(int algo, Workspace *w, const CsrView &g, uint32_t seed, const lsg_opts &o, uint32_t *dist,
+                     lsg_stats *st);
+
 }  // namespace lsg

@@ -144,7 +144,7 @@ typedef struct lsg_round_trace {
 typedef struct lsg_stats {
   double ms_total;
   double ms_kernel;
-  uint64_t iterations;  /* sssp: delta phases ("iterations: %d", apps/sssp/kernel.cu:479);
+  uint64_t iterations;  /* sssp: phases ("iterations: %d", apps/sssp/kernel.cu:479), which may be several delta wide;
                            bfs: levels */
   uint64_t near_iters;  /* queue rounds over all phases */
   uint64_t items;       /* frontier items popped */

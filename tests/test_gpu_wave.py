@@ -56,7 +56,8 @@ def check(g, src, delta, **kw):
 def test_trees(degrees):
     g = tree(*degrees)
     for delta in (1, 40, 10000):
-        check(g, 0, delta)
+        check(g, 0, delta, block_size=256)
+        check(g, 0, delta)  # up to 32768 vertices: the one-workgroup kernel
 
 
 @pytest.mark.parametrize("kw", [dict(block_size=b, grid_blocks=n) for b in (256, 512, 1024) for n in (1, 7, 16, 17, 300)]
@@ -72,7 +73,27 @@ def test_launch_shapes(kw):
 def test_paced_threshold(rows, cols, whi):
     g = CSRGraph.grid(rows, cols, 1, whi, seed=rows)
     for delta in (1, 32, 5000, 1 << 30):
+        check(g, 7, delta, block_size=256)
         check(g, 7, delta)
+
+
+# The one-workgroup kernel: both sides of its largest size, rounds of more
+# vertices than it lists (4096), heavy vertices (32 edges), the array's last edges.
+@pytest.mark.parametrize("n,kind", [(32768, "grid"), (32769, "grid"), (32768, "star"), (32767, "star"), (30000, "random"),
+                                    (5, "star"), (2, "star"), (1, "star")])
+def test_one_workgroup(n, kind):
+    rng = np.random.default_rng(n)
+    if kind == "grid":
+        g = CSRGraph.grid(128, n // 128, 1, 1000, seed=1) if n % 128 == 0 else CSRGraph.grid(3, n // 3, 1, 1000, seed=1)
+    elif kind == "star":  # the hub's round pushes every other vertex at once
+        v = np.arange(1, n)
+        g = csr(n, np.stack([np.concatenate([v, np.zeros(n - 1, int)]), np.concatenate([np.zeros(n - 1, int), v]),
+                             rng.integers(1, 50, 2 * (n - 1))], axis=1))
+    else:
+        g = csr(n, np.stack([rng.integers(0, n, 5 * n), rng.integers(0, n, 5 * n), rng.integers(0, 100, 5 * n)], axis=1))
+    for delta in (1, 64, 1 << 30):
+        for src in (0, n // 2, n - 1):
+            check(g, min(src, g.nnodes - 1), delta)
 
 
 def test_captured_launch_takes_new_sources():
