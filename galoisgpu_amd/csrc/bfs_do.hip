@@ -893,7 +893,7 @@ __global__ __launch_bounds__(BS, 4) void do_kernel(DoArgs a) {
         x.items = up ? found : queued;
         x.heavy = next_up ? 0u : chunks;
         x.roles = (qi ^ 1) | (up ? bi ^ 1 : bi) << 1;
-        x.flags = kWaveLead | (done ? kWaveDone : x.phase == kDoQueue && small ? kWaveLocal : 0u);
+        x.flags = kWaveLead | (done ? kWaveDone : x.phase == kDoQueue && chunks == 0 && queued <= a.local_max / 2 ? kWaveLocal : 0u);
         if (lane == 0) {
           __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_fetch_add(&c->stat_rounds, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -39,7 +39,9 @@
 //     older value only costs work are at workgroup scope (64^2 grid 0.85 ->
 //     0.79 ms).  The block leaves
 //     this mode when the round it would run next is too large, and hands the
-//     vertices over through the near queue.  (Limits of 128 / 256 / 384 / 512
+//     vertices over through the near queue; it is entered at half that size (a
+//     pile counts a vertex as often as it is pushed: 256^2 grid 3.60 -> 3.37 ms,
+//     512^2 8.2 -> 7.8).  (Limits of 128 / 256 / 384 / 512
 //     items: 64^2 grid SSSP 0.62 / 0.53 / 0.52 / 0.49 ms, 256^2 3.7 / 3.4 / 3.5
 //     / 3.6, 512^2 BFS 6.0 / 5.2 / 4.9 / 4.8, road-like 1023 x 777 BFS 0.86 /
 //     0.85 / 0.84 / 0.84.)
@@ -668,7 +670,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
           x.steps = r.steps + (a.pace ? pace.next(r.phase) : 1u);
           if (lane == 0) st_coh(&wc->far_tail[r.far_q()].n, 0u);
         }
-        x.flags = kWaveLead | (done ? kWaveDone : x.heavy == 0 && x.items <= a.local_max ? kWaveLocal : 0u) |
+        x.flags = kWaveLead | (done ? kWaveDone : x.heavy == 0 && x.items <= a.local_max / 2 ? kWaveLocal : 0u) |
                   (phase ? kWaveCut : 0u);
         if (lane == 0) {
           __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
