@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <chrono>
 #include <climits>
 #include <cstring>
@@ -343,6 +344,14 @@ struct Pending {
   uint32_t v, nb_lo, nb_hi, fb_lo, fb_hi;
   uint32_t n;  // wave-uniform
 };
+// The same for packed rows: in LDS, 64 entries a wavefront.
+struct PackedEntry {
+  uint32_t v, nb, fb;
+};
+struct PackedPending {
+  PackedEntry *buf;
+  uint32_t n;  // wave-uniform
+};
 
 
 // Sets the pending destinations' mask bits; a destination whose mask was
@@ -553,13 +562,115 @@ __device__ __forceinline__ void flat_load(const MArgs &a, const Flat &t, uint32_
   x.k = item;
 }
 
+// ---- packed rows ------------------------------------------------------------
+//
+// With up to 32 (16) sources a row fills half (a quarter) of a wavefront or less:
+// P = 2 (4) edges are relaxed side by side, lanes sub * kWave / P on for the
+// sub-th.  A window is kSlots row accesses, P edges each, and its edges come from
+// the lanes: long items are flattened too.  Ms with one row an access -> packed
+// (learned schedule): RMAT of 16400 vertices x 5 sources 0.87 -> 0.70, 40000 x 20
+// 1.49 -> 1.14, 500000 x 12 2.79 -> 2.03, 2^20 x 20 3.52 -> 2.82, 2^22 x 16 9.2 ->
+// 7.7; fixed delta 100003 x 9 1.35 -> 1.28, 262900 x 3 1.85 -> 1.87.  (kSlots of 8 / 2:
+// 2^20 x 20 3.09 / 2.9 at P = 2; 8 spilled 109 registers.  P = 8 up to 8 sources: 4
+// to 8 % better with the learned schedule, 0 to 12 % worse without.)
+template <int P>
+struct Packing {
+  static constexpr uint32_t kRow = kWave / P;  // lanes of an edge
+  static constexpr int kSlots = 4;
+  static constexpr uint32_t kWindow = kSlots * P;
+};
+
+// The source of this lane's column.
+template <int P>
+__device__ __forceinline__ uint32_t lane_source() {
+  return P == 1 ? lane_id() : lane_id() % Packing<P>::kRow;
+}
+
+template <int P>
+__device__ __forceinline__ void flush_packed(const MArgs &a, const Sched &s, LaneSched &ls, PackedPending &p) {
+  if (p.n == 0) return;
+  order_release();
+  const bool in = lane_id() < p.n;
+  const PackedEntry e = p.buf[in ? lane_id() : 0u];
+  const bool act = in && has_edges(a, in ? e.v : 0u);
+  const bool pn = act && e.nb != 0 && atomic_or64(a.nmask[s.round & 1] + e.v, e.nb) == 0 && near_admit(a, s, e.v);
+  const bool pf = act && e.fb != 0 && atomic_or64(a.fmask[s.phase & 1] + e.v, e.fb) == 0;
+  pile_push(a, s, ls, 0, pn, e.v);
+  pile_push(a, s, ls, 1, pf, e.v);
+  p.n = 0;
+}
+
+// window_take for packed rows.
+template <int P, int N>
+__device__ __forceinline__ void packed_take(const MArgs &a, LaneSched &ls, const uint32_t (&v)[N], const uint32_t (&nd)[N],
+                                            const uint32_t (&val)[N], PackedPending &p, uint64_t &improved) {
+  constexpr uint32_t kRow = Packing<P>::kRow;
+  constexpr uint32_t kMask = (uint32_t)((1ull << kRow) - 1);
+  const uint32_t col = lane_id() % kRow, shift = lane_id() / kRow * kRow;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const bool imp = nd[k] < val[k];
+    const uint64_t im = __ballot(imp);
+    if (im == 0) continue;
+    if (imp) atomic_min(a.D + (size_t)v[k] * a.S + col, nd[k]);
+    const bool nearl = imp && nd[k] <= ls.thr32;
+    const uint64_t nb = __ballot(nearl);
+    if (imp && !nearl) ls.fmin = min(ls.fmin, nd[k]);
+    const uint32_t mine = (uint32_t)(im >> shift) & kMask, near = (uint32_t)(nb >> shift) & kMask;
+    const bool lead = col == 0 && mine != 0;
+    const uint64_t lm = __ballot(lead);
+    if (lead) p.buf[p.n + lanes_below(lm)] = PackedEntry{v[k], near, mine & ~near};
+    const uint32_t c = (uint32_t)__builtin_popcountll(lm);
+    p.n += c;
+    improved += c;
+  }
+}
+
+// relax_listed for packed rows.
+template <int P>
+__device__ __forceinline__ void relax_listed_packed(const MArgs &a, const Sched &s, LaneSched &ls, const DistSlots &dl,
+                                                    uint32_t pv, uint32_t pw, uint32_t pk, uint32_t n, PackedPending &p,
+                                                    uint64_t &improved) {
+  using K = Packing<P>;
+  const uint32_t col = lane_id() % K::kRow, sub = lane_id() / K::kRow, colc = min(col, a.S - 1);
+  for (uint32_t i = 0; i < n; i += K::kWindow) {
+    uint32_t v[K::kSlots], nd[K::kSlots], val[K::kSlots];
+#pragma unroll
+    for (int k = 0; k < K::kSlots; ++k) {
+      const uint32_t at = i + (uint32_t)k * P + sub, j = min(at, n - 1);
+      v[k] = (uint32_t)__shfl(pv, j);
+      const uint32_t wt = (uint32_t)__shfl(pw, j), item = (uint32_t)__shfl(pk, j);  // by every lane
+      val[k] = ld_coh(a.D + (size_t)v[k] * a.S + colc);
+      // (an edge past the list repeats its last one, with no candidate)
+      nd[k] = dl[item][col] + (at < n ? wt : 0x80000000u);
+    }
+    if (p.n > (uint32_t)kWave - K::kWindow) flush_packed<P>(a, s, ls, p);
+    packed_take<P, K::kSlots>(a, ls, v, nd, val, p, improved);
+  }
+}
+
+// A flattened list without the test: 64 edges at a time.
+template <int P>
+__device__ __forceinline__ void relax_packed(const MArgs &a, const Sched &s, LaneSched &ls, const DistSlots &dl,
+                                             const Flat &t, PackedPending &p, uint64_t &improved) {
+  if (t.total == 0) return;
+  FlatBatch x, y;
+  flat_load(a, t, 0, x);
+  for (uint32_t b0 = 0; b0 < t.total; b0 += kWave) {
+    flat_load(a, t, b0 + kWave, y);
+    relax_listed_packed<P>(a, s, ls, dl, x.v, x.w, x.k, min((uint32_t)kWave, t.total - b0), p, improved);
+    x = y;
+  }
+}
+
 // Relaxes a flattened list (total > 0).  The lanes take one edge each and test
 // it against its destination's bound; the edges that pass are collected in a
 // list of up to 64, one per lane, and relaxed from there.  Three batches of 64
 // are in flight: while one is tested and relaxed, the next one's bounds and
 // the edges of the one after it are being loaded.
+template <int P, class Pend>
 __device__ __forceinline__ void relax_filtered(const MArgs &a, const Sched &s, LaneSched &ls, const DistSlots &dl,
-                                               const Flat &t, Pending &p, uint64_t &improved) {
+                                               const Flat &t, Pend &p, uint64_t &improved) {
   const uint32_t lane = lane_id();
   uint32_t pv = 0, pw = 0, pk = 0, n = 0;
   FlatBatch x0, x1, x2;
@@ -578,7 +689,8 @@ __device__ __forceinline__ void relax_filtered(const MArgs &a, const Sched &s, L
       c = (uint32_t)__builtin_popcountll(m);
     }
     if (n && (b0 >= t.total || n + c > (uint32_t)kWave)) {
-      relax_listed(a, s, ls, dl, pv, pw, pk, n, p, improved);
+      if constexpr (P > 1) relax_listed_packed<P>(a, s, ls, dl, pv, pw, pk, n, p, improved);
+      else relax_listed(a, s, ls, dl, pv, pw, pk, n, p, improved);
       n = 0;
     }
     if (b0 >= t.total) break;
@@ -645,9 +757,9 @@ __device__ __forceinline__ void queue_heavy(const MArgs &a, const Sched &s, Lane
 // chunks for the next round; the others are relaxed (items of kLongDeg edges
 // and more one by one, the rest as one flattened list, 64 edges per batch) or,
 // with kFilter, returned as one flattened list.
-template <bool kFilter>
+template <bool kFilter, int P, class Pend>
 __device__ __forceinline__ Flat process_unit(const MArgs &a, const Sched &s, LaneSched &ls, bool chunks, uint32_t base,
-                                             uint32_t per, DistSlots &dl, RoundCounters &mc, Pending &p) {
+                                             uint32_t per, DistSlots &dl, RoundCounters &mc, Pend &p) {
   const uint32_t lane = lane_id();
   const uint32_t cnt = min(per, (chunks ? s.heavy_count : s.in_count) - base);
   uint32_t u = a.nnodes;
@@ -739,8 +851,8 @@ __device__ __forceinline__ Flat process_unit(const MArgs &a, const Sched &s, Lan
     mc.edges += now;
   }
   // items relaxed one by one (degree >= kLongDeg); the others as a flattened list
-  const uint32_t longm = kFilter ? 0u : (uint32_t)__ballot(now >= kLongDeg);
-  const uint32_t mydeg = kFilter || now < kLongDeg ? now : 0u;
+  const uint32_t longm = kFilter || P > 1 ? 0u : (uint32_t)__ballot(now >= kLongDeg);
+  const uint32_t mydeg = kFilter || P > 1 || now < kLongDeg ? now : 0u;
   // Inclusive prefix of the items' edge counts over lanes 0..kItems-1: item k
   // owns flattened edges [end_k - deg_k, end_k).
   uint32_t end = mydeg;
@@ -752,6 +864,9 @@ __device__ __forceinline__ Flat process_unit(const MArgs &a, const Sched &s, Lan
   const uint32_t total = readlane(end, kItems - 1);
   const uint32_t first = end - mydeg;
   if (kFilter) return Flat{total, end, rs - first, low};
+  if constexpr (P > 1) {
+    relax_packed<P>(a, s, ls, dl, Flat{total, end, rs - first, 0}, p, mc.improved);
+  } else {
   for (uint32_t b0 = 0; b0 < total; b0 += kWave) {
     const uint32_t f = b0 + lane;
     // the item holding flattened edge f is the number of items ending at or before f
@@ -769,6 +884,7 @@ __device__ __forceinline__ Flat process_unit(const MArgs &a, const Sched &s, Lan
   for (uint32_t lm = longm; lm; lm &= lm - 1) {
     const uint32_t k = (uint32_t)__builtin_ctz(lm);
     relax_edges(a, s, ls, dl[k][lane], readlane(rs, k), readlane(re, k), p, mc.improved);
+  }
   }
   return Flat{0, 0, 0, 0};
 }
@@ -966,7 +1082,7 @@ __device__ __forceinline__ uint32_t group_blocks(uint32_t nb, uint32_t g) { retu
 // against the bounds; the other variant runs the rounds before, and returns
 // when a sweep has been ordered.  (One kernel with both edge loops spilled
 // 170 VGPRs.)
-template <int BS, bool kFilter>
+template <int BS, bool kFilter, int P>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kMultiWaves, kMultiWaves)))
 void multi_kernel(MArgs a) {
   __shared__ Sched ss;
@@ -976,6 +1092,7 @@ void multi_kernel(MArgs a) {
   __shared__ uint32_t pushbuf[BS / kWave][2 * kPushBuf];
   __shared__ HeavyItem heavybuf[BS / kWave][kHeavyBuf];
   __shared__ uint32_t drain_n[BS / kWave][3], drain_base[3];  // near, far, heavy chunks
+  __shared__ PackedEntry pend[P > 1 ? BS / kWave : 1][P > 1 ? kWave : 1];
   Ctrl *c = a.ctrl;
   const uint32_t nb = gridDim.x;
   if (!residency_handshake(c, nb, a.residency_limit)) return;
@@ -996,7 +1113,7 @@ void multi_kernel(MArgs a) {
     RoundCounters mc = {0, 0, 0};
     LaneSched ls;
     ls.bucket = s.aux[1] == LSG_FAR_BUCKET;
-    ls.thr = ls.bucket && lane_id() < a.S ? ld_coh(a.thr + lane_id()) : 0u;
+    ls.thr = ls.bucket && lane_source<P>() < a.S ? ld_coh(a.thr + lane_source<P>()) : 0u;
     ls.thr32 = ls.bucket ? ls.thr : (uint32_t)min(s.curdelta(), (int64_t)UINT32_MAX);
     ls.fmin = kInf;
     ls.pb = &pushbuf[threadIdx.x / kWave][0];
@@ -1017,9 +1134,10 @@ void multi_kernel(MArgs a) {
         acquire_agent();  // no line of the bounds that was read before is kept
       }
     }
-    Pending p;
+    typename std::conditional<(P > 1), PackedPending, Pending>::type p;
     p.n = 0;
-    p.v = p.nb_lo = p.nb_hi = p.fb_lo = p.fb_hi = 0;
+    if constexpr (P > 1) p.buf = pend[threadIdx.x / kWave];
+    else p.v = p.nb_lo = p.nb_hi = p.fb_lo = p.fb_hi = 0;
     DistSlots &dl = dls[threadIdx.x / kWave];
     // Work units: first the in-queue's items, `per` at a time (fewer than
     // kItems where that would leave wavefronts idle), then the heavy chunks.
@@ -1042,9 +1160,9 @@ void multi_kernel(MArgs a) {
         uint32_t t = 0;
         if (last && lane_id() == 0) t = atomic_add(&a.tickets[g].ticket, 1u);
         const bool chunks = u >= nitems;
-        const Flat f = process_unit<kFilter>(a, s, ls, chunks, chunks ? (u - nitems) * hper : u * per,
+        const Flat f = process_unit<kFilter, P>(a, s, ls, chunks, chunks ? (u - nitems) * hper : u * per,
                                              chunks ? hper : per, dl, mc, p);
-        if (kFilter && f.total) relax_filtered(a, s, ls, dl, f, p, mc.improved);
+        if (kFilter && f.total) relax_filtered<P>(a, s, ls, dl, f, p, mc.improved);
         if (last) {
           j = group_blocks(nb, g) * wpb + readlane(t, 0) * kSpan;
           jend = j + kSpan;
@@ -1066,9 +1184,10 @@ void multi_kernel(MArgs a) {
       j = group_blocks(nb, g) * wpb + readlane(t, 0) * kSpan;
       jend = j + kSpan;
     }
-    flush_pending(a, s, ls, p);
+    if constexpr (P > 1) flush_packed<P>(a, s, ls, p);
+    else flush_pending(a, s, ls, p);
     // this wavefront's smallest far push per source -> phase minimum
-    if (__ballot(ls.fmin != kInf) && ls.fmin != kInf) atomic_min(a.fmin + (s.phase & 1) * 64 + lane_id(), ls.fmin);
+    if (__ballot(ls.fmin != kInf) && ls.fmin != kInf) atomic_min(a.fmin + (s.phase & 1) * 64 + lane_source<P>(), ls.fmin);
     const uint32_t wv = threadIdx.x / kWave;
     const uint64_t lane_items = wave_sum(mc.lane_items), edges = wave_sum(mc.edges);
     if (lane_id() == 0) {
@@ -1238,13 +1357,17 @@ __global__ void multi_expand(const uint32_t *Dc, uint32_t Sc, const int32_t *col
 
 using MultiFn = void (*)(MArgs);
 
-template <bool kFilter>
+template <bool kFilter, int P>
 static MultiFn pick_multi(int bs) {
   switch (bs) {
-    case 256: return multi_kernel<256, kFilter>;
-    case 1024: return multi_kernel<1024, kFilter>;
-    default: return multi_kernel<512, kFilter>;
+    case 256: return multi_kernel<256, kFilter, P>;
+    case 1024: return multi_kernel<1024, kFilter, P>;
+    default: return multi_kernel<512, kFilter, P>;
   }
+}
+template <bool kFilter>
+static MultiFn pick_multi(int bs, uint32_t nsrc) {
+  return nsrc <= 16 ? pick_multi<kFilter, 4>(bs) : nsrc <= 32 ? pick_multi<kFilter, 2>(bs) : pick_multi<kFilter, 1>(bs);
 }
 
 // Between the two kernels: the barrier and residency words start again.
@@ -1337,7 +1460,7 @@ static int run_multi(Workspace *w, const lsg_graph *g, const uint32_t *srcs_host
     a.feat = (float *)((char *)tbuf + tbytes);
   }
   HIPCHK(hipMemcpyAsync(sbuf, srcs_host, nsrc * 4, hipMemcpyHostToDevice, w->stream));
-  const MultiFn fn = pick_multi<false>(bs), ffn = pick_multi<true>(bs);
+  const MultiFn fn = pick_multi<false>(bs, nsrc), ffn = pick_multi<true>(bs, nsrc);
   int grid = 0, fgrid = 0;
   if ((rc = resident_grid(w, (const void *)fn, bs, &grid)) || (rc = resident_grid(w, (const void *)ffn, bs, &fgrid)))
     return rc;

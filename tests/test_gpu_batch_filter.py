@@ -125,3 +125,17 @@ def test_paced_threshold(whi, delta):
     print("paced", whi, delta, flush=True)
     check(hub_graph(3001, whi, whi), [0, 1, 7, 2000, 2999], delta=delta)
     check(CSRGraph.grid(60, 41, 1, whi, seed=3), [0, 17, 2459], delta=delta)
+
+
+@pytest.mark.parametrize("nsrc", [1, 2, 15, 16, 17, 31, 32, 33])
+def test_packed_rows(nsrc):
+    """Source counts on both sides of each row packing, every far mode, chunks and light items."""
+    g = CSRGraph.rmat(12, 10, seed=nsrc)
+    live = np.flatnonzero(np.diff(g.row_start.astype(np.int64)))  # each source keeps its column
+    srcs = np.random.default_rng(nsrc).choice(live, nsrc, replace=False)
+    for far_mode in (0, 1, 2):
+        for heavy_deg in (8, 64, 4000):
+            print("packed", nsrc, far_mode, heavy_deg, flush=True)
+            check(g, srcs, delta=40, far_mode=far_mode, heavy_deg=heavy_deg)
+    check(hub_graph(4001, nsrc, INT_MAX), srcs, delta=1 << 30)
+    check(CSRGraph.grid(50, 60, 1, 100, seed=nsrc), np.arange(nsrc) * 90, delta=64)
