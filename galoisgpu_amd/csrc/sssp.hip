@@ -85,6 +85,9 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     a.pace = g.nedges <= 6ull * g.nnodes;
     a.unit_min = a.pace ? 16 : 8;
     a.local_max = wave_local_max(g.nnodes, g.nedges);
+    a.split_deg = a.pace ? 0u : std::min(kWaveSplitDeg, a.heavy_deg);
+    // one chunk at least for each such vertex, and one per heavy_deg edges
+    if (a.split_deg) a.hcap = (uint32_t)std::min<uint64_t>(2ull * g.nedges / a.split_deg + 64, UINT32_MAX / 2);
     void *chunks;
     if ((rc = ws_buffer(w, kBufHeavy, 2ull * a.hcap * sizeof(WaveChunk), &chunks))) return rc;
     a.chunk[0] = (WaveChunk *)chunks;

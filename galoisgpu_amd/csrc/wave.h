@@ -33,7 +33,7 @@ struct WaveCtrl {
   } slot[3];
 };
 
-// Up to heavy_deg edges of a heavy vertex: popped at distance d.
+// Up to heavy_deg edges of a heavy vertex: popped at distance d, or INF.
 struct WaveChunk {
   uint32_t u, d, first, n;
 };
@@ -44,7 +44,7 @@ struct WaveArgs : KArgs {
   uint32_t pace = 0;      // the threshold's steps are paced (WavePace)
   uint32_t unit_min = 0;  // fewest items of a unit
   uint32_t local_max = 0; // largest round that one block runs alone
-  uint32_t _pad = 0;
+  uint32_t split_deg = 0; // edges from which a vertex is queued as chunks when it is pushed; 0: when it is popped
 };
 
 // Blocks per CU, of 256 threads, where the call leaves the launch shape open.
@@ -67,6 +67,17 @@ inline uint32_t wave_local_max(uint64_t nnodes, uint64_t nedges) {
 // A chunk of a heavy vertex is the edges that a wavefront holds in flight
 // (kWaveU a lane); 512 and 1024: equal to 5 % slower on RMAT graphs.
 constexpr int kWaveHeavyDeg = 256;
+// On graphs of more than 6 edges a vertex, vertices of this many edges are taken
+// apart when they are pushed: a round earlier than when they are popped, and no
+// item has many edges, so that the units of a round take alike.  The row bounds
+// are one more round trip, which the narrow rounds of low-degree graphs would
+// feel.  Ms when popped / at 128 / 64 / 32 edges: RMAT-14 (8 edges a vertex) SSSP
+// 0.25 / 0.21 / 0.19 / 0.18, RMAT-16 0.37 / 0.30 / 0.27 / 0.30, RMAT-18 0.50 / 0.45 /
+// 0.44 / 0.45, RMAT-20 0.97 / 0.86 / 0.88 / 0.90, RMAT-22 2.22 / 2.04 / 2.05 / 2.21;
+// BFS RMAT-14 0.072 / 0.069 / 0.067 / 0.067, RMAT-18 0.148 / 0.157 / 0.141 / 0.146,
+// RMAT-20 0.285 / 0.283 / 0.288 / 0.297, from random sources 0.340 / 0.286 / 0.303 /
+// 0.315.
+constexpr uint32_t kWaveSplitDeg = 64;
 
 // Block sizes 256, 512 and 1024.
 const void *wave_kernel_fn(Algo algo, int bs);

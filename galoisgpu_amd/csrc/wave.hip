@@ -47,8 +47,8 @@
 //     0.85 / 0.84 / 0.84.)
 //
 // Ms in persistent_kernel -> here, at delta steps of 1 as in WavePace: SSSP
-// RMAT-17 0.53 -> 0.44, RMAT-20 1.60 -> 1.00, RMAT-22 5.1 -> 2.26; BFS RMAT-17
-// 0.162 -> 0.105, RMAT-20 0.447 -> 0.28, road-like 1023 x 777 1.16 -> 0.84.
+// RMAT-18 0.72 -> 0.44, RMAT-20 1.60 -> 0.88, RMAT-22 5.1 -> 2.05; BFS RMAT-18
+// 0.205 -> 0.141, RMAT-20 0.447 -> 0.288, road-like 1023 x 777 1.16 -> 0.84.
 
 #include <hip/hip_runtime.h>
 
@@ -144,6 +144,7 @@ struct WaveLane {
   uint32_t *pbuf[2];
   WaveHeavy *hbuf;
   uint32_t n[2], hn;  // staged: items per pile, heavy items (wave-uniform)
+  uint32_t settled;   // see wave_settle
 };
 
 __device__ __forceinline__ uint32_t *wave_queue(const WaveArgs &a, uint32_t i) {
@@ -162,20 +163,7 @@ __device__ __forceinline__ void wave_store(const WaveArgs &a, WaveLane &w, int w
     else st_coh(&a.ctrl->abort, kAbortCapacity);
   }
   w.n[which] = 0;
-}
-
-// Pushes `item` from every lane with `pred` (whole wavefront).
-__device__ __forceinline__ void wave_stage(const WaveArgs &a, WaveLane &w, int which, bool pred, uint32_t item) {
-  const uint64_t m = __ballot(pred);
-  if (m == 0) return;
-  const uint32_t c = (uint32_t)__builtin_popcountll(m);
-  if (w.n[which] + c > kWavePush) {
-    uint32_t base = 0;
-    if (lane_id() == 0) base = atomic_add(which ? w.ftail : w.ntail, w.n[which]);
-    wave_store(a, w, which, readlane(base, 0));
-  }
-  if (pred) w.pbuf[which][w.n[which] + lanes_below(m)] = item;
-  w.n[which] += c;
+  if (which == 0) w.settled = 0;
 }
 
 // Writes the staged heavy items' chunks, counted in `end`, from slot `base` on.
@@ -212,6 +200,40 @@ __device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool 
   }
   if (heavy) w.hbuf[w.hn + lanes_below(m)] = WaveHeavy{u, d, first, deg};
   w.hn += c;
+}
+
+// The near items staged since the last call: those of split_deg edges and more
+// become chunks of the next round, read with the distance of that time; the
+// others close up.
+__device__ __forceinline__ void wave_settle(const WaveArgs &a, WaveLane &w) {
+  uint32_t out = w.settled;
+  for (uint32_t i0 = w.settled; i0 < w.n[0]; i0 += kWave) {
+    const bool valid = i0 + lane_id() < w.n[0];
+    const uint32_t v = valid ? w.pbuf[0][i0 + lane_id()] : 0u;
+    const uint64_t rb = ld_pair(a.row_start + v);
+    const uint32_t rs = (uint32_t)rb, deg = (uint32_t)(rb >> 32) - rs;
+    const bool split = valid && deg >= a.split_deg;
+    wave_heavy(a, w, split, v, kInf, rs, deg);
+    const uint64_t m = __ballot(valid && !split);
+    if (valid && !split) w.pbuf[0][out + lanes_below(m)] = v;
+    out += (uint32_t)__builtin_popcountll(m);
+  }
+  w.n[0] = w.settled = out;
+}
+
+// Pushes `item` from every lane with `pred` (whole wavefront).
+__device__ __forceinline__ void wave_stage(const WaveArgs &a, WaveLane &w, int which, bool pred, uint32_t item) {
+  const uint64_t m = __ballot(pred);
+  if (m == 0) return;
+  const uint32_t c = (uint32_t)__builtin_popcountll(m);
+  if (w.n[which] + c > kWavePush) {
+    if (which == 0 && a.split_deg) wave_settle(a, w);
+    uint32_t base = 0;
+    if (lane_id() == 0 && w.n[which]) base = atomic_add(which ? w.ftail : w.ntail, w.n[which]);
+    wave_store(a, w, which, readlane(base, 0));
+  }
+  if (pred) w.pbuf[which][w.n[which] + lanes_below(m)] = item;
+  w.n[which] += c;
 }
 
 // ---- relaxation ----------------------------------------------------------------
@@ -324,7 +346,8 @@ __device__ __forceinline__ void wave_chunk(const WaveArgs &a, WaveLane &w, const
   const uint32_t u = __builtin_amdgcn_readfirstlane((uint32_t)x), d = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
   const uint32_t rs = __builtin_amdgcn_readfirstlane((uint32_t)y), n = __builtin_amdgcn_readfirstlane((uint32_t)(y >> 32));
   if (u >= a.nnodes || n == 0 || (uint64_t)rs + n > a.nedges) return;
-  if (ld_coh(a.dist + u) < d) return;
+  const uint32_t du = ld_coh(a.dist + u);
+  if (d != kInf && du < d) return;
   for (uint32_t b0 = 0; b0 < n; b0 += kWaveU * kWave) {
     uint32_t e[kWaveU], d0[kWaveU];
     bool act[kWaveU];
@@ -333,7 +356,7 @@ __device__ __forceinline__ void wave_chunk(const WaveArgs &a, WaveLane &w, const
       const uint32_t f = b0 + k * kWave + lane;
       act[k] = f < n;
       e[k] = rs + min(f, n - 1);
-      d0[k] = d;
+      d0[k] = du;
     }
     wave_relax<A, kWaveU>(a, w, e, d0, act, false);
   }
@@ -562,7 +585,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
   w.pbuf[0] = sh.push[wv][0];
   w.pbuf[1] = sh.push[wv][1];
   w.hbuf = sh.heavy[wv];
-  w.n[0] = w.n[1] = w.hn = 0;
+  w.n[0] = w.n[1] = w.hn = w.settled = 0;
   for (;;) {
     const WaveRound r = sh.r;
     const uint32_t gen = sh.gen;
@@ -599,6 +622,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       unit = (gblocks * NW + readlane(t, 0)) * ngroups + g;
     }
     // The block's pushes get their places with one atomic per pile.
+    if (a.split_deg) wave_settle(a, w);
     const uint32_t hend = w.hn ? wave_heavy_ends(a, w) : 0u;
     order_release();
     if (lane_id() == kWave - 1) {

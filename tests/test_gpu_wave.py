@@ -96,6 +96,21 @@ def test_one_workgroup(n, kind):
             check(g, min(src, g.nnodes - 1), delta)
 
 
+# Vertices taken apart when they are pushed (64 edges, on graphs of more than 6
+# edges a vertex) or popped (256): degrees on both sides, many in one round.
+@pytest.mark.parametrize("kw", [dict(), dict(heavy_deg=40), dict(block_size=512), dict(graph_launch=True)])
+def test_split_when_pushed(kw):
+    rng = np.random.default_rng(5)
+    n = 6000
+    deg = rng.choice([0, 1, 8, 63, 64, 65, 255, 256, 257, 600], n, p=[.1, .3, .3, .05, .05, .05, .05, .04, .03, .03])
+    deg[0] = 3000
+    src = np.repeat(np.arange(n), deg)
+    g = csr(n, np.stack([src, rng.integers(0, n, len(src)), rng.integers(0, 60, len(src))], axis=1))
+    for delta in (1, 16, 1 << 20):
+        check(g, 0, delta, **kw)
+        check(g, 77, delta, **kw)
+
+
 def test_captured_launch_takes_new_sources():
     """Replays of one captured launch, each against the oracle, with plain launches between."""
     g = CSRGraph.rmat(12, 8, seed=9)
