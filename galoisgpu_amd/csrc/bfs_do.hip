@@ -1094,7 +1094,7 @@ int lsg_bfs_do(const lsg_graph *g, const lsg_graph *gt, uint32_t src, int direct
   // large graph many wavefronts (ms at 1 / 2 / 4: RMAT-16 0.061 / 0.068 / 0.087,
   // RMAT-18 0.070 / 0.076 / 0.097, RMAT-20 0.108 / 0.105 / 0.121, RMAT-22 0.247 /
   // 0.195 / 0.193; road-like 2048^2 1.58 / 1.65 / 1.77).
-  const int per_cu = g->nedges <= 6ull * V || g->nedges < (1u << 23) ? 1 : 2;
+  const int per_cu = low_degree(V, g->nedges) || g->nedges < (1u << 23) ? 1 : 2;
   grid = std::min<int>(grid, per_cu * (int)w->cus);
   void *qbuf, *hbuf, *bbuf, *wbuf;
   if ((rc = ws_buffer(w, kBufQueues, 2ull * V * 4, &qbuf)) || (rc = ws_buffer(w, kBufHeavy, 2ull * hcap * 8, &hbuf)) ||
@@ -1121,7 +1121,7 @@ int lsg_bfs_do(const lsg_graph *g, const lsg_graph *gt, uint32_t src, int direct
   a.hcap = hcap;
   a.heavy_deg = kDoHeavy;
   a.direction = (uint32_t)direction;
-  a.unit_min = g->nedges <= 6ull * V ? 16 : 8;
+  a.unit_min = low_degree(V, g->nedges) ? 16 : 8;
   a.local_max = direction == 2 ? 0 : wave_local_max(V, g->nedges);
   a.spin_limit = spin_limit_ticks(w);
   a.residency_limit = residency_limit_ticks(w);

@@ -15,8 +15,8 @@
 // beyond the workgroup's size halve it again.  Vertices whose distance came below
 // the last threshold since they were set were near vertices then, and are dropped.
 //
-// Used up to kSmallV vertices (128 KB of the CU's 160), and 6 edges a vertex: a
-// larger frontier's edges are faster over the whole GPU.  Kernel ms in wave.hip ->
+// Used up to kSmallV vertices (128 KB of the CU's 160) of low degree: a larger
+// frontier's edges are faster over the whole GPU.  Kernel ms in wave.hip ->
 // here: SSSP grid 64^2 0.50 -> 0.22, 100^2 0.89 -> 0.37, 181^2 2.2 -> 0.75, 40 x
 // 500 2.7 -> 1.3, road-like 181^2 0.80 -> 0.44; BFS grid 64^2 0.24 -> 0.16, 181^2
 // 0.86 -> 0.45, road-like 181^2 0.43 -> 0.19.

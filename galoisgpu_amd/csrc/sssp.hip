@@ -82,7 +82,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     // Low degrees: threshold paced, units of 16 items at least, so that a small
     // round involves few blocks; else of 8, as items may have 255 edges each
     // (at 16 / 8 / 4: RMAT-17 SSSP 0.45 / 0.40 / 0.44 ms, RMAT-20 1.02 / 1.01 / 1.00).
-    a.pace = g.nedges <= 6ull * g.nnodes;
+    a.pace = low_degree(g.nnodes, g.nedges);
     a.unit_min = a.pace ? 16 : 8;
     a.local_max = wave_local_max(g.nnodes, g.nedges);
     a.split_deg = a.pace ? 0u : std::min(kWaveSplitDeg, a.heavy_deg);
@@ -193,7 +193,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
 // Small graphs of low degree, unless the call sets a launch shape of its own.
 static bool use_small(const CsrView &g, const lsg_opts &o) {
   return default_kernel(o) && !o.enable_lb && !o.graph_launch && o.block_size == 0 && o.grid_blocks <= 0 &&
-         o.heavy_deg <= 0 && g.nnodes <= kSmallV && g.nedges <= 6ull * g.nnodes;
+         o.heavy_deg <= 0 && g.nnodes <= kSmallV && low_degree(g.nnodes, g.nedges);
 }
 
 // One source on one device graph into dist (device array of g->nnodes).

@@ -57,7 +57,7 @@ struct WaveArgs : KArgs {
 // 512: RMAT-18 0.73, RMAT-20 1.18, 2048^2 3.78; 1024 worse still.
 constexpr int kWaveBlock = 256;
 inline int wave_blocks_per_cu(uint64_t nnodes, uint64_t nedges) {
-  return nedges <= 6 * nnodes || nedges < 3u << 20 ? 1 : nedges < 1u << 25 ? 2 : 3;
+  return low_degree(nnodes, nedges) || nedges < 3u << 20 ? 1 : nedges < 1u << 25 ? 2 : 3;
 }
 // Largest round, in items, that one block runs alone: some 2048 edges (limits
 // of 512 / 128 items on RMAT: 2^14 vertices 0.256 / 0.245 ms, 2^20 1.00 / 0.98).
@@ -67,8 +67,8 @@ inline uint32_t wave_local_max(uint64_t nnodes, uint64_t nedges) {
 // A chunk of a heavy vertex is the edges that a wavefront holds in flight
 // (kWaveU a lane); 512 and 1024: equal to 5 % slower on RMAT graphs.
 constexpr int kWaveHeavyDeg = 256;
-// On graphs of more than 6 edges a vertex, vertices of this many edges are taken
-// apart when they are pushed: a round earlier than when they are popped, and no
+// On graphs that are not low_degree, vertices of this many edges are taken apart
+// when they are pushed: a round earlier than when they are popped, and no
 // item has many edges, so that the units of a round take alike.  The row bounds
 // are one more round trip, which the narrow rounds of low-degree graphs would
 // feel.  Ms when popped / at 128 / 64 / 32 edges: RMAT-14 (8 edges a vertex) SSSP

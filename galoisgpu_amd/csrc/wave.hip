@@ -66,8 +66,7 @@ struct WaveHeavy {
   uint32_t u, d, first, deg;
 };
 
-// Pace of the near/far threshold on graphs of low degree (the host decides:
-// at most 6 edges a vertex).  There nearly every round is bound by its fixed
+// Pace of the near/far threshold on graphs of low degree (low_degree).  There nearly every round is bound by its fixed
 // cost, so a wider phase, with its fewer and larger rounds, is faster until
 // the vertices that are expanded more than once cost more than the rounds
 // saved; how wide depends on the graph, the weights and where the frontier is

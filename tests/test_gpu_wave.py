@@ -96,7 +96,7 @@ def test_one_workgroup(n, kind):
             check(g, min(src, g.nnodes - 1), delta)
 
 
-# Vertices taken apart when they are pushed (64 edges, on graphs of more than 6
+# Vertices taken apart when they are pushed (64 edges, on graphs of more than 5
 # edges a vertex) or popped (256): degrees on both sides, many in one round.
 @pytest.mark.parametrize("kw", [dict(), dict(heavy_deg=40), dict(block_size=512), dict(graph_launch=True)])
 def test_split_when_pushed(kw):
