@@ -85,6 +85,8 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     a.pace = low_degree(g.nnodes, g.nedges);
     a.unit_min = a.pace ? 16 : 8;
     a.local_max = wave_local_max(g.nnodes, g.nedges);
+    // (a resumed BFS reports its own levels' rounds)
+    a.hops = a.pace && !(A == Algo::BFS && resume) ? kWaveHops : 0;
     a.split_deg = a.pace ? 0u : std::min(kWaveSplitDeg, a.heavy_deg);
     // one chunk at least for each such vertex, and one per heavy_deg edges
     if (a.split_deg) a.hcap = (uint32_t)std::min<uint64_t>(2ull * g.nedges / a.split_deg + 64, UINT32_MAX / 2);
@@ -175,6 +177,9 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     w->last_feat.resize((size_t)np * kFeatRec);
     if (np) HIPCHK(hipMemcpy(w->last_feat.data(), a.feat, w->last_feat.size() * sizeof(float), hipMemcpyDeviceToHost));
   }
+  // BFS in hops runs fewer rounds than there are levels: one a level, and the
+  // last, which finds nothing, are reported.
+  if (A == Algo::BFS && a.hops) hc.stat_rounds = hc.s.aux[3] + 1ull;
   if (st) {
     memset(st, 0, sizeof *st);
     st->ms_kernel = ms;

@@ -44,6 +44,8 @@ struct WaveArgs : KArgs {
   uint32_t pace = 0;      // the threshold's steps are paced (WavePace)
   uint32_t unit_min = 0;  // fewest items of a unit
   uint32_t local_max = 0; // largest round that one block runs alone
+  uint32_t hops = 0;      // times that a wavefront goes on with what it pushed near
+  uint32_t _pad = 0;
   uint32_t split_deg = 0; // edges from which a vertex is queued as chunks when it is pushed; 0: when it is popped
 };
 
@@ -78,6 +80,7 @@ constexpr int kWaveHeavyDeg = 256;
 // RMAT-20 0.285 / 0.283 / 0.288 / 0.297, from random sources 0.340 / 0.286 / 0.303 /
 // 0.315.
 constexpr uint32_t kWaveSplitDeg = 64;
+constexpr uint32_t kWaveHops = 4;  // on low-degree graphs
 
 // Block sizes 256, 512 and 1024.
 const void *wave_kernel_fn(Algo algo, int bs);

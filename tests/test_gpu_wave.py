@@ -77,6 +77,20 @@ def test_paced_threshold(rows, cols, whi):
         check(g, 7, delta)
 
 
+# Wavefronts that go on with what they pushed: levels are still reported one by one.
+@pytest.mark.parametrize("rows,cols", [(182, 182), (700, 90), (3, 30000)])
+def test_hops(rows, cols):
+    g = CSRGraph.roadlike(rows, cols, 0.1, 0.001, 1, 1000, seed=rows)
+    for delta in (20, 1000, 1 << 28):
+        check(g, 11, delta)
+    dev = g.copy_to_gpu()
+    st = bfs_gg_main(g, dev, Options(start_node=11))
+    dev.copy_to_cpu(g)
+    reached = g.node_data[g.node_data != 2**31 - 1]
+    assert st["iterations"] == st["near_iters"] == reached.max() + 1
+    dev.close()
+
+
 # The one-workgroup kernel: both sides of its largest size, rounds of more
 # vertices than it lists (4096), heavy vertices (32 edges), the array's last edges.
 @pytest.mark.parametrize("n,kind", [(32768, "grid"), (32769, "grid"), (32768, "star"), (32767, "star"), (30000, "random"),
