@@ -164,7 +164,7 @@ struct MArgs {
 };
 
 // Pushes are staged per wavefront in LDS, kPushBuf items per pile, and
-// written out with one queue-tail atomic per flush: one atomic per wave_push
+// written out with one queue-tail atomic per flush: one atomic per push
 // on a tail that every wavefront of the grid shares serialises at the
 // memory-side atomic unit (~12 ns each on gfx950).  512 entries measured
 // faster than 256 (26.0 vs 26.5 ms on RMAT-22 x 64 sources).

@@ -1,7 +1,7 @@
 // One-workgroup near/far traversals (lsg_opts.single_block).
 //
 // On a graph like a 256x256 grid a traversal is 1000+ near/far rounds of a
-// few hundred vertices each, and a round of the persistent kernel costs a
+// few hundred vertices each, and a round over the whole grid costs a
 // chain of dependent global round trips (in-queue load, d[u], row bounds,
 // edges, atomicMin, queue and count stores, the leader's schedule) of about
 // 8 us.  Here one workgroup of 1024 threads runs the same near/far rounds
@@ -25,8 +25,9 @@
 // Two kernels share the round code:
 //   block_kernel   one graph, one workgroup, the piles in LDS (kPileCap near
 //                  and kFarCap far entries); a traversal that would outgrow
-//                  them stops (kAbortCapacity) and the host runs the
-//                  persistent kernel instead;
+//                  them stops (kAbortCapacity) and the wavefront kernel
+//                  (or the persistent one, as the options say) goes on
+//                  from the distances reached;
 //   graphs_kernel  a batch of graphs (lsg_sssp_graphs), one workgroup per
 //                  graph, the piles in HBM, sized from the graph; no
 //                  workgroup waits for another, so no grid barrier and no
@@ -48,7 +49,7 @@ constexpr uint32_t kBlkThreads = 1024;
 constexpr uint32_t kPileCap = 2048;  // LDS: entries per round pile (two of them: 64 KB)
 constexpr uint32_t kFarCap = 4096;   // LDS: entries in the far pile (64 KB)
 constexpr uint32_t kFarPerThread = kFarCap / kBlkThreads;
-// A BFS level wider than this continues in the persistent kernel: such a
+// A BFS level wider than this continues over the whole grid: such a
 // level is faster over the whole GPU than in one CU, and levels only widen
 // on the graphs that reach it (BFS from source 0, road-like graphs of 256^2
 // to 2048^2, switch at 2048 / 1024 / 512 entries: 256^2 0.98 / 0.85 / 0.82

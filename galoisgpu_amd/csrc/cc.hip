@@ -7,14 +7,15 @@
 // (:630-723) iterates until no hook succeeds.  Edges are taken without
 // direction (weakly connected components of a directed graph).  The
 // reference's hooks are plain racing stores, so which id ends up as a
-// component's label depends on the schedule; here a hook is an atomicMin of
-// the larger root's parent to the smaller root, so every vertex ends labelled
+// component's label depends on the schedule; here a hook is a compare-and-swap
+// of the larger root's parent to the smaller root, so every vertex ends labelled
 // with the smallest id of its component -- the same partition, with one
 // deterministic label per component.
 //
 // Layout: label u32[V] (the parent pointer, node_data; a parent's id is never
-// above its child's) and one control word, the component count.  The reference repeats hook and
-// jump passes until no hook succeeds; here every edge is looked at once:
+// above its child's) and one control word, the component count.  The reference
+// repeats hook and jump passes until no hook succeeds; here every edge is
+// looked at once:
 //   cc_init_kernel      label[v] = v's first out-neighbour if that is smaller, else v;
 //   cc_flatten_kernel   every vertex to the root of that forest;
 //   cc_persistent_kernel  joins the trees of every edge's ends (compare-and-swap on

@@ -153,7 +153,7 @@ struct Ctrl {
   uint32_t bar_gen;   uint32_t _p1[31];
   uint32_t qcount[3]; uint32_t _p2[29];
   uint32_t hcount[2]; uint32_t _p3[30];
-  uint32_t ticket;    uint32_t ticket2; uint32_t _p4[30];
+  uint32_t ticket;    uint32_t _p4[31];
   uint32_t abort;     uint32_t checkin; uint32_t resident_seen; uint32_t progress; uint32_t _p5[28];
   Sched s;            uint32_t _p6[16];
   uint64_t stat_items, stat_rounds, stat_heavy, stat_phases, stat_edges;
@@ -207,26 +207,6 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
 
 __device__ __forceinline__ uint32_t readlane(uint32_t v, uint32_t l) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
-}
-
-// Wave-aggregated push: one atomicAdd per wave on the queue tail, every
-// active lane with `pred` writes its item at base + rank.  Replaces
-// Worklist::setup_push_warp_one + do_push (rt/include/worklist.h:348-368,414-420)
-// with 64-lane ballot/mbcnt.  Overflow raises kAbortCapacity instead of
-// asserting (worklist.h:356); nothing is silently dropped.
-__device__ __forceinline__ void wave_push(bool pred, uint32_t item, uint32_t *q, uint32_t *tail, uint32_t cap,
-                                          uint32_t *abort_flag) {
-  uint64_t m = __ballot(pred);
-  if (m == 0) return;
-  uint32_t leader = (uint32_t)__builtin_ctzll(m);
-  uint32_t base = 0;
-  if (lane_id() == leader) base = atomic_add(tail, (uint32_t)__builtin_popcountll(m));
-  base = readlane(base, leader);
-  if (pred) {
-    uint32_t pos = base + lanes_below(m);
-    if (pos < cap) st_coh(q + pos, item);
-    else st_coh(abort_flag, kAbortCapacity);
-  }
 }
 
 // Reserves `n` consecutive slots per lane (n may differ per lane); returns the

@@ -18,13 +18,12 @@
 // V floats, and at RMAT-22's 16 MB that array, four times an XCD's L2, bounds
 // them.  So a call first renumbers the vertices by in-degree, largest first
 // (a stable counting sort; in-degrees from kHeavyDeg on, or kWideDeg on small
-// graphs, are one class): the
-// contributions read most lie together, and vertices of one in-degree are
-// neighbours.  In that order
+// graphs, are one class): the contributions read most lie together, and
+// vertices of one in-degree are neighbours.  In that order
 //   positions [0, heavy)     in-degree >= kHeavyDeg: in-edges cut into chunks of
 //     kChunk; one wavefront sums a chunk, and where a vertex has several, one
-//     lane then adds their partials in chunk order (one wavefront per vertex left the
-//     sweep waiting on the largest in-degree, ~97 K edges on RMAT-22);
+//     lane then adds their partials in chunk order (one wavefront per vertex
+//     left the sweep waiting on the largest in-degree, ~97 K edges on RMAT-22);
 //   positions [heavy, live)  the others with in-edges, in slices of 64, one lane
 //     per vertex: a slice's sources are stored transposed, slot k of the 64
 //     lanes consecutive, as many slots as its largest vertex has in-edges;
@@ -40,8 +39,8 @@
 // degrees 146 -> 88, road-like 73 -> 60; preparing takes 1.0 ms on RMAT-22.
 //
 // The convergence test stays on the device: the host enqueues iterations in
-// batches of one or two launches each; a block in which some rank moved by more than
-// epsilon raises one of kFlags flags, and the iteration's last block
+// batches of one or two launches each; a block in which some rank moved by
+// more than epsilon raises one of kFlags flags, and the iteration's last block
 // counts the iteration and sets a done flag when none was raised; the kernels
 // of later iterations return at once when they find it set.  Iterations stay
 // separate launches: the launch boundary makes one iteration's contributions

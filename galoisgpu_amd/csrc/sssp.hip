@@ -55,7 +55,7 @@ static bool default_kernel(const lsg_opts &o) {
 
 // Runs one traversal from `nseeds` seeds (host array) into dist (device,
 // g.nnodes entries).  Synchronous.  With graph_launch the init, seed and
-// persistent kernels are replayed as one captured hipGraph.  With `resume`:
+// traversal kernels are replayed as one captured hipGraph.  With `resume`:
 // continue from the distances already in dist instead (resume_seed_kernel's
 // queue, curdelta resume->curdelta), not captured; the seeds are then not used.
 template <Algo A>
@@ -105,7 +105,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
   const void *fnp = wave ? wave_kernel_fn(A, bs) : (const void *)fn;
   int grid = 0;
   if ((rc = resident_grid(w, fnp, bs, &grid))) return rc;
-  // Default: 2 blocks per CU at most for SSSP, 4 for BFS.  Fewer blocks per
+  // The persistent kernel: 2 blocks per CU at most for SSSP, 4 for BFS.  Fewer blocks per
   // grid barrier beat more parallel tiles (256-thread blocks; full resident
   // grid 1280 -> 512): RMAT-20 SSSP 2.24 -> 2.05 ms, road 2048^2 10.2 -> 8.3
   // ms, RMAT-22 6.31 -> 6.23 ms, grid 256^2 12.9 -> 12.8 ms; BFS levels are
@@ -225,7 +225,7 @@ static int run_single(const lsg_graph *g, const lsg_opts *o_in, uint32_t *dist, 
     Resume res;
     rc = run_block_single((int)A, w, v, seed, o, dist, &bst, &res);
     if (rc == kBlockFallback) {
-      // The piles overflowed: the persistent kernel continues from the
+      // The piles overflowed: the whole grid continues from the
       // distances the workgroup reached (not captured: a one-off launch).
       rc = run_core<A>(w, v, &seed, 1, o, dist, false, st, &res);
       if (rc == LSG_OK && st) {

@@ -1,8 +1,10 @@
 // Device side of the single-source traversal: kernel arguments, the per-edge
 // operators, tile and heavy-chunk expansion, the leader step (pile rotation)
-// and block-local rounds.  Included by sssp.hip (the persistent launch) and
+// and block-local rounds.  Included by sssp.hip (the persistent launch of the
+// calls that ask for what the wavefront kernel does not have: degree-binned
+// expansion, other far modes, the learned schedule, a trace), noalloc.hip and
 // lb.hip (the host-driven edge-balanced -l loop), which share every operator
-// so that both compute exactly the same relaxations.
+// so that all compute exactly the same relaxations.
 //
 // Reference path: apps/sssp/kernel.cu (relax operator sssp_kernel_dev
 // :177-306, persistent driver :355-391) and apps/bfs/kernel.cu (operator
@@ -61,7 +63,7 @@ struct KArgs {
 
 // Pushes are staged per wavefront in LDS, kStage items per pile, and written
 // out with one queue-tail atomic per flush (and at the end of every round):
-// one atomic per wave_push on a tail that every wavefront of the grid shares
+// one atomic per push on a tail that every wavefront of the grid shares
 // serialises at the memory-side atomic unit (~12 ns each on gfx950).
 constexpr uint32_t kStage = 256;
 
@@ -1221,7 +1223,7 @@ int run_lb_single(int algo, Workspace *w, const CsrView &g, uint32_t seed, const
                   lsg_stats *st);
 
 // The one-workgroup near/far traversals (block.hip).  kBlockFallback: a pile
-// overflowed.  A single source then continues in the persistent kernel from
+// overflowed.  A single source then continues over the whole grid from
 // the distances left in dist, as *resume says (run_core's resume); a batch of
 // graphs runs the union launch instead.  *st holds the one-workgroup launch's
 // figures either way.
