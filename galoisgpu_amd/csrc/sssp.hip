@@ -260,48 +260,75 @@ struct UnionMember {
   uint64_t nedges, eoff;
 };
 
-__device__ __forceinline__ uint32_t member_of_vertex(const UnionMember *m, uint32_t n, uint32_t v) {
-  uint32_t lo = 0, hi = n;
-  while (hi - lo > 1) {
-    uint32_t mid = (lo + hi) >> 1;
-    if (m[mid].voff <= v) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
+// Packing and unpacking are bound by memory: a wavefront takes kPackTile
+// consecutive elements of the union, finds the member of the first by a binary
+// search and walks on from there, kPackFlight loads a lane in flight.  (With a
+// search for every element: 256 RMAT graphs of 35.8 M edges 438 + 33 us, now
+// 115, of 570 MB, + 15; 64 graphs 1187 -> 1139 us per call.)
+constexpr uint32_t kPackTile = 1024;
+constexpr int kPackFlight = 4;
 
-__device__ __forceinline__ uint32_t member_of_edge(const UnionMember *m, uint32_t n, uint64_t e) {
-  uint32_t lo = 0, hi = n;
-  while (hi - lo > 1) {
-    uint32_t mid = (lo + hi) >> 1;
-    if (m[mid].eoff <= e) lo = mid;
-    else hi = mid;
+// Calls f(member, first, end) for the runs of [0, n) that lie in one member and
+// one wavefront's tile; off: the first element of a member.
+template <class Off, class F>
+__device__ __forceinline__ void member_runs(const UnionMember *m, uint32_t nm, uint64_t n, Off off, F f) {
+  const uint32_t waves = gridDim.x * (blockDim.x / kWave);
+  const uint32_t w = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave);
+  for (uint64_t i = (uint64_t)w * kPackTile; i < n; i += (uint64_t)waves * kPackTile) {
+    const uint64_t end = min(i + kPackTile, n);
+    uint32_t lo = 0, hi = nm;  // the last member that begins at or before i
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (off(m[mid]) <= i) lo = mid;
+      else hi = mid;
+    }
+    for (uint64_t at = i; at < end; ++lo) {
+      const uint64_t to = lo + 1 < nm ? min<uint64_t>(end, off(m[lo + 1])) : end;
+      f(m[lo], at, to);
+      at = to;
+    }
   }
-  return lo;
 }
 
 // Disjoint union: vertex ids shifted by voff, edge offsets by eoff.
-__global__ void pack_union_kernel(const UnionMember *m, uint32_t n, uint32_t *urow, uint32_t *udst, uint32_t *uw,
-                                  uint32_t V, uint64_t E) {
-  size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
-  for (size_t v = tid; v < V; v += nt) {
-    const UnionMember &g = m[member_of_vertex(m, n, (uint32_t)v)];
-    urow[v] = (uint32_t)(g.row[v - g.voff] + g.eoff);
-  }
-  if (tid == 0) urow[V] = (uint32_t)E;
-  for (size_t e = tid; e < E; e += nt) {
-    const UnionMember &g = m[member_of_edge(m, n, e)];
-    udst[e] = g.dst[e - g.eoff] + g.voff;
-    uw[e] = g.w[e - g.eoff];
-  }
+__global__ __launch_bounds__(256) void pack_union_kernel(const UnionMember *m, uint32_t n, uint32_t *urow,
+                                                         uint32_t *udst, uint32_t *uw, uint32_t V, uint64_t E) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) urow[V] = (uint32_t)E;
+  member_runs(m, n, E, [](const UnionMember &g) { return g.eoff; }, [&](const UnionMember &g, uint64_t at, uint64_t to) {
+    const uint32_t *dst = g.dst, *wt = g.w;
+    const uint64_t eoff = g.eoff;
+    const uint32_t voff = g.voff;
+    for (uint64_t i = at + lane_id(); i < to; i += kPackFlight * kWave) {
+      uint32_t d[kPackFlight], x[kPackFlight];
+#pragma unroll
+      for (int k = 0; k < kPackFlight; ++k) {
+        const uint64_t e = min(i + (uint64_t)k * kWave, to - 1) - eoff;
+        d[k] = glb(dst)[e];
+        x[k] = glb(wt)[e];
+      }
+#pragma unroll
+      for (int k = 0; k < kPackFlight; ++k) {
+        const uint64_t e = i + (uint64_t)k * kWave;
+        if (e >= to) break;
+        glb(udst)[e] = d[k] + voff;
+        glb(uw)[e] = x[k];
+      }
+    }
+  });
+  member_runs(m, n, V, [](const UnionMember &g) { return (uint64_t)g.voff; }, [&](const UnionMember &g, uint64_t at, uint64_t to) {
+    const uint32_t *row = g.row;
+    const uint64_t voff = g.voff, eoff = g.eoff;
+    for (uint64_t v = at + lane_id(); v < to; v += kWave) glb(urow)[v] = (uint32_t)(glb(row)[v - voff] + eoff);
+  });
 }
 
-__global__ void unpack_union_kernel(const UnionMember *m, uint32_t n, const uint32_t *udist, uint32_t V) {
-  size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x, nt = (size_t)gridDim.x * blockDim.x;
-  for (size_t v = tid; v < V; v += nt) {
-    const UnionMember &g = m[member_of_vertex(m, n, (uint32_t)v)];
-    g.out[v - g.voff] = (int32_t)udist[v];
-  }
+__global__ __launch_bounds__(256) void unpack_union_kernel(const UnionMember *m, uint32_t n, const uint32_t *udist,
+                                                           uint32_t V) {
+  member_runs(m, n, V, [](const UnionMember &g) { return (uint64_t)g.voff; }, [&](const UnionMember &g, uint64_t at, uint64_t to) {
+    int32_t *out = g.out;
+    const uint64_t voff = g.voff;
+    for (uint64_t v = at + lane_id(); v < to; v += kWave) glb(out)[v - voff] = (int32_t)glb(udist)[v];
+  });
 }
 
 // Checks a device CSR in place: row_start[0] == 0, offsets never decrease,

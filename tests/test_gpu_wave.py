@@ -149,3 +149,25 @@ def test_large_weights():
         dev.copy_to_cpu(g)
         assert np.array_equal(g.node_data, oracle.dijkstra(g.row_start, g.edge_dst, g.edge_data, 0))
     dev.close()
+
+
+# A batch of graphs is packed and unpacked in tiles of 1024 edges or vertices of
+# one wavefront each: members that end at and beside a tile's end, members
+# without edges (first, last, in a row), many in one tile.
+@pytest.mark.parametrize("members", [
+    [(1, 0)], [(1, 0), (3, 1024), (1, 0)], [(1023, 1023), (1, 1), (1024, 1025), (1025, 1024)],
+    [(2, 0), (5, 0), (700, 3000), (9, 0), (9, 0), (40, 255), (2500, 9000), (1, 0)], [(3, 7)] * 300 + [(1, 0)] * 3,
+])
+def test_union_of_members(members):
+    from galoisgpu_amd.batch import sssp_graphs
+
+    rng = np.random.default_rng(len(members))
+    gs = [csr(n, np.stack([rng.integers(0, n, e), rng.integers(0, n, e), rng.integers(1, 50, e)], 1)) for n, e in members]
+    srcs = [int(rng.integers(n)) for n, _ in members]
+    devs = [g.copy_to_gpu() for g in gs]
+    print("union", members[:8], flush=True)
+    outs, _ = sssp_graphs(devs, srcs, Options(delta=20))
+    for g, s, out in zip(gs, srcs, outs):
+        assert np.array_equal(out, oracle.dijkstra(g.row_start, g.edge_dst, g.edge_data, s))
+    for d in devs:
+        d.close()
