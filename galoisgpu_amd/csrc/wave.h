@@ -50,16 +50,20 @@ struct WaveArgs : KArgs {
 };
 
 // Blocks per CU, of 256 threads, where the call leaves the launch shape open.
-// Each block more makes a grid barrier dearer, each wavefront fewer the large
-// rounds longer; low-degree graphs have few of those.  Ms at 1 / 2 / 3 blocks:
-// RMAT-17 SSSP 0.50 / 0.53 / 0.54, RMAT-18 0.59 / 0.56 / 0.57, RMAT-20 1.33 /
-// 1.15 / 1.12, RMAT-21 2.31 / 1.78 / 1.71, RMAT-18 BFS 0.160 / 0.150 / 0.159,
-// RMAT-21 0.68 / 0.50 / 0.46; road-like 1000^2 SSSP 2.61 / 2.68 / 2.75, 2048^2
-// 3.76 / 3.87 / 3.99, BFS 1.54 / 1.64 / 1.70.  The same wavefronts in blocks of
-// 512: RMAT-18 0.73, RMAT-20 1.18, 2048^2 3.78; 1024 worse still.
+// Blocks without a unit stay out of a round's barrier, so more of them cost a
+// small round little; each wavefront fewer makes the large rounds longer, and a
+// graph has to be large to have such rounds.  Ms at 1 / 2 / 3 blocks: RMAT-17
+// SSSP 0.358 / 0.359 / 0.369, RMAT-18 0.464 / 0.448 / 0.463, RMAT-19 0.67 / 0.62
+// / 0.63, RMAT-20 1.10 / 0.90 / 0.87, RMAT-21 1.81 / 1.35 / 1.26, RMAT-22 3.1 /
+// 2.3 / 2.1; BFS RMAT-17 0.117 / 0.117 / 0.132, RMAT-19 0.223 / 0.198 / 0.202, RMAT-20 0.385 /
+// 0.293 / 0.278; road-like SSSP 1000^2 1.18 / 1.14 / 1.15, 1500^2 1.77 / 1.73 /
+// 1.77, 2048^2 2.17 / 2.05 / 2.03, BFS 0.62 / 0.63 / 0.64, 0.88 / 0.84 / 0.86, 1.13 /
+// 1.12 / 1.10; grid 1500^2 SSSP 18.65 / 18.74 / 18.80.  The same wavefronts in blocks
+// of 512: RMAT-19 0.71, RMAT-20 0.98, 2048^2 2.08; 1024 worse still.
 constexpr int kWaveBlock = 256;
 inline int wave_blocks_per_cu(uint64_t nnodes, uint64_t nedges) {
-  return low_degree(nnodes, nedges) || nedges < 3u << 20 ? 1 : nedges < 1u << 25 ? 2 : 3;
+  if (low_degree(nnodes, nedges)) return nedges < 6'000'000 ? 1 : 2;
+  return nedges < 3'000'000 ? 1 : nedges < 12'000'000 ? 2 : 3;
 }
 // Largest round, in items, that one block runs alone: some 2048 edges (limits
 // of 512 / 128 items on RMAT: 2^14 vertices 0.256 / 0.245 ms, 2^20 1.00 / 0.98).
