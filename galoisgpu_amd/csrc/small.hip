@@ -17,9 +17,9 @@
 //
 // Used up to kSmallV vertices (128 KB of the CU's 160) of low degree: a larger
 // frontier's edges are faster over the whole GPU.  Kernel ms in wave.hip ->
-// here: SSSP grid 64^2 0.50 -> 0.22, 100^2 0.89 -> 0.37, 181^2 2.2 -> 0.75, 40 x
-// 500 2.7 -> 1.3, road-like 181^2 0.80 -> 0.44; BFS grid 64^2 0.24 -> 0.16, 181^2
-// 0.86 -> 0.45, road-like 181^2 0.43 -> 0.19.
+// here: SSSP grid 64^2 0.52 -> 0.22, 100^2 0.93 -> 0.36, 181^2 1.74 -> 0.75, 40 x
+// 500 2.7 -> 1.3, road-like 181^2 0.63 -> 0.44; BFS grid 64^2 0.26 -> 0.16, 181^2
+// 0.90 -> 0.45, road-like 181^2 0.39 -> 0.19.
 //
 // There are no spin waits: every wait is a workgroup barrier.
 

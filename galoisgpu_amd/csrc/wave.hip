@@ -46,9 +46,10 @@
 //     / 3.6, 512^2 BFS 6.0 / 5.2 / 4.9 / 4.8, road-like 1023 x 777 BFS 0.86 /
 //     0.85 / 0.84 / 0.84.)
 //
-// Ms in persistent_kernel -> here, at delta steps of 1 as in WavePace: SSSP
-// RMAT-18 0.72 -> 0.44, RMAT-20 1.60 -> 0.88, RMAT-22 5.1 -> 2.05; BFS RMAT-18
-// 0.205 -> 0.141, RMAT-20 0.447 -> 0.288, road-like 1023 x 777 1.16 -> 0.84.
+// Ms in persistent_kernel -> here: SSSP RMAT-18 0.72 -> 0.45, RMAT-20 1.60 ->
+// 0.87, RMAT-22 5.1 -> 2.07, grid 256^2 8.2 -> 2.57, road-like 2048^2 4.4 -> 2.04;
+// BFS RMAT-18 0.205 -> 0.143, RMAT-20 0.447 -> 0.278, road-like 2048^2 1.99 ->
+// 1.11.
 
 #include <hip/hip_runtime.h>
 

@@ -104,12 +104,12 @@ typedef struct lsg_opts {
                           thread count, the reference's DEGREE_LIMIT (rt/include/ggcuda.h:19-22) */
   int32_t single_block; /* 1 = the near/far rounds run in one workgroup with the piles in LDS and
                            a workgroup barrier between rounds (same distances), for small sparse
-                           high-diameter graphs, where a round of the persistent kernel is a chain
-                           of global round trips: SSSP on the 256x256 grid 8.0 -> 4.2 ms at delta
-                           32, 2.5 ms at delta 256; BFS 3.6 -> 1.5 ms.  When the piles outgrow
+                           high-diameter graphs, where a round is a chain of global round trips: SSSP
+                           on the 256x256 grid 4.3 ms at delta 32, 2.56 ms at delta 256, BFS 1.42
+                           (the default 2.5 ms at delta 32, BFS 1.48).  When the piles outgrow
                            LDS (SSSP: 2048 entries per round, 4096 far; BFS levels wider than
-                           1024 vertices) the persistent kernel continues from the distances
-                           reached (road-like 1024x1024 at delta 10000: 3.4 -> 3.0 ms); a
+                           1024 vertices) the whole grid continues from the distances reached
+                           (road-like 2048x2048 at delta 10000: 2.19 ms, default 2.22); a
                            frontier that explodes at once (RMAT BFS from a hub) costs that launch
                            extra.  stats then add both launches' rounds, items and kernel time;
                            a trace holds the persistent kernel's rounds only.  Single-source
