@@ -294,17 +294,14 @@ __device__ __forceinline__ void wave_relax(const WaveArgs &a, WaveLane &w, const
 
 constexpr int kWaveU = 4;
 
-// Up to 64 vertices u, one per lane below n: heavy ones are queued as chunks, the
-// others' edges flattened over the wavefront.  Returns their number.
+// The vertices u of the lanes below n, with `deg` edges from rs on (0: none to
+// expand): heavy ones are queued as chunks, the others' edges flattened over the
+// wavefront.  Returns their number.
 template <Algo A>
-__device__ __forceinline__ uint32_t wave_vertices(const WaveArgs &a, WaveLane &w, int64_t cut, uint32_t u, uint32_t n) {
+__device__ __forceinline__ uint32_t wave_vertices(const WaveArgs &a, WaveLane &w, int64_t cut, uint32_t u, uint32_t n,
+                                                  uint32_t rs, uint32_t deg) {
   const uint32_t lane = lane_id();
-  uint32_t du = kInf, rs = 0, deg = 0;
-  if (lane < n) {
-    du = ld_coh(a.dist + u);
-    rs = glb(a.row_start)[u];
-    deg = glb(a.row_start)[u + 1] - rs;
-  }
+  const uint32_t du = lane < n ? ld_coh(a.dist + u) : kInf;
   if (du == kInf || (int64_t)du <= cut) deg = 0;
   const bool heavy = deg >= a.heavy_deg;
   wave_heavy(a, w, heavy, u, du, rs, deg);
@@ -341,7 +338,13 @@ __device__ __forceinline__ uint32_t wave_vertices(const WaveArgs &a, WaveLane &w
 // just pushed near (64 at most), without waiting for the round's end.  A vertex
 // taken so loses its stamp before its distance is read, and pushes go by the
 // exchange alone (a stamp read ahead of it may be gone): whoever lowers the vertex
-// later queues it again.  Distances and levels are lowered until nothing changes,
+// later queues it again.  A heavy vertex is not taken: the chunk queue holds one
+// set of chunks per vertex and round (in-queue items are distinct: at most 2 E /
+// heavy_deg chunks), and a hub that many light vertices lower within a round would
+// be taken apart each time (1000 vertices of 257 edges with a leaf an edge, 16
+// blocks: 6440 chunks in a round, room for 4079).  It gets its stamp again and
+// stays among the pushes, unless it was pushed by another wavefront meanwhile.
+// Distances and levels are lowered until nothing changes,
 // so the order is free; a hop costs three round trips, a round ten.  Not for units
 // of more than kHopEdges edges, where what the other wavefronts would have lowered
 // meanwhile is expanded twice: skewed graphs (RMAT of 2^18 vertices and 4 edges
@@ -354,17 +357,28 @@ template <Algo A>
 __device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const uint32_t *in, uint32_t n) {
   const uint32_t lane = lane_id();
   uint32_t kept = w.n[0], u = lane < n ? ld_coh(in + lane) : 0u;
+  uint64_t rb = ld_pair(a.row_start + u);
   int64_t cut = w.cut;
   for (uint32_t h = 0;; ++h) {
-    const uint32_t total = wave_vertices<A>(a, w, cut, u, n);
+    const uint32_t rs = (uint32_t)rb, deg = lane < n ? (uint32_t)(rb >> 32) - rs : 0u;
+    const uint32_t total = wave_vertices<A>(a, w, cut, u, n, rs, deg);
     if (h == a.hops || total > kHopEdges) break;
     if (w.n[0] < kept) kept = 0;  // written out meanwhile
     n = min((uint32_t)kWave, w.n[0] - kept);
     if (n == 0) break;
     w.n[0] = kept = w.n[0] - n;
     u = lane < n ? w.pbuf[0][kept + lane] : 0u;
+    rb = ld_pair(a.row_start + u);
     if (lane < n) (void)atomic_exch(a.near_stamp + u, 0u);
     order_release();  // the stamp is gone before the distance is read
+    const bool heavy = lane < n && (uint32_t)(rb >> 32) - (uint32_t)rb >= a.heavy_deg;
+    if (__ballot(heavy)) {
+      const bool back = heavy && atomic_exch(a.near_stamp + u, w.near_stamp) != w.near_stamp;
+      const uint64_t m = __ballot(back);
+      if (back) w.pbuf[0][kept + lanes_below(m)] = u;
+      w.n[0] = kept = kept + (uint32_t)__builtin_popcountll(m);
+      if (heavy) rb = 0;
+    }
     cut = -1;
   }
 }
