@@ -185,6 +185,8 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
   // BFS in hops runs fewer rounds than there are levels: one a level, and the
   // last, which finds nothing, are reported.
   if (A == Algo::BFS && a.hops) hc.stat_rounds = hc.s.aux[3] + 1ull;
+  if (a.hops)
+    for (const auto &h : hc.hop_items) hc.stat_items += h[0];
   if (st) {
     memset(st, 0, sizeof *st);
     st->ms_kernel = ms;

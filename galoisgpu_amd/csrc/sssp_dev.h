@@ -1019,6 +1019,7 @@ __global__ __launch_bounds__(BS, 4) void persistent_kernel(KArgs a) {
 // grid calls it (the barrier words are cleared grid-strided).
 __device__ __forceinline__ void ctrl_init(const KArgs &a, uint32_t delta, int64_t cd0, uint32_t tid, uint32_t nt) {
   ctrl_reset_barrier(a.ctrl, tid, nt);
+  if (tid < kHopGroups) a.ctrl->hop_items[tid][0] = 0;
   if (tid == 0) {
     Ctrl *c = a.ctrl;
     c->qcount[0] = 0;

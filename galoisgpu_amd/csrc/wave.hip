@@ -146,6 +146,7 @@ struct WaveLane {
   WaveHeavy *hbuf;
   uint32_t n[2], hn;  // staged: items per pile, heavy items (wave-uniform)
   uint32_t settled;   // see wave_settle
+  uint32_t hopped;    // vertices popped in hops
 };
 
 __device__ __forceinline__ uint32_t *wave_queue(const WaveArgs &a, uint32_t i) {
@@ -372,7 +373,9 @@ __device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const
     if (lane < n) (void)atomic_exch(a.near_stamp + u, 0u);
     order_release();  // the stamp is gone before the distance is read
     const bool heavy = lane < n && (uint32_t)(rb >> 32) - (uint32_t)rb >= a.heavy_deg;
-    if (__ballot(heavy)) {
+    const uint64_t hm = __ballot(heavy);
+    w.hopped += n - (uint32_t)__builtin_popcountll(hm);
+    if (hm) {
       const bool back = heavy && atomic_exch(a.near_stamp + u, w.near_stamp) != w.near_stamp;
       const uint64_t m = __ballot(back);
       if (back) w.pbuf[0][kept + lanes_below(m)] = u;
@@ -632,7 +635,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
   w.pbuf[0] = sh.push[wv][0];
   w.pbuf[1] = sh.push[wv][1];
   w.hbuf = sh.heavy[wv];
-  w.n[0] = w.n[1] = w.hn = w.settled = 0;
+  w.n[0] = w.n[1] = w.hn = w.settled = w.hopped = 0;
   for (;;) {
     const WaveRound r = sh.r;
     const uint32_t gen = sh.gen;
@@ -781,6 +784,14 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
         }
       }
     }
+  }
+  if (!a.hops) return;
+  if (lane_id() == 0) sh.count[wv][0] = w.hopped;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint64_t n = 0;
+    for (uint32_t i = 0; i < NW; ++i) n += sh.count[i][0];
+    if (n) __hip_atomic_fetch_add(&c->hop_items[blockIdx.x % kHopGroups][0], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 

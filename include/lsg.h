@@ -147,7 +147,7 @@ typedef struct lsg_stats {
   uint64_t iterations;  /* sssp: phases ("iterations: %d", apps/sssp/kernel.cu:479), which may be several delta wide;
                            bfs: levels */
   uint64_t near_iters;  /* queue rounds over all phases */
-  uint64_t items;       /* frontier items popped */
+  uint64_t items;       /* frontier items popped (a vertex as often as it is expanded) */
   uint64_t heavy_chunks;
   int32_t last_delta;   /* curdelta at exit */
   int32_t grid_blocks;
