@@ -242,12 +242,23 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs a) {
       ++phases;
     }
   }
-  for (uint32_t v = tid; v < a.nnodes; v += kSmallThreads) glb(a.dist)[v] = sh.dist[v];
+  if (tid == 0) sh.left = 0;
+  __syncthreads();
+  uint32_t deep = 0;
+  for (uint32_t v = tid; v < a.nnodes; v += kSmallThreads) {
+    const uint32_t d = sh.dist[v];
+    glb(a.dist)[v] = d;
+    if (A == Algo::BFS && d != kInf) deep = max(deep, d);
+  }
+  // BFS: one round a level and the last, which finds nothing (a round that takes its
+  // vertices from the bitmap goes on with what it finds, and saves some)
+  if (A == Algo::BFS && deep) atomicMax(&sh.left, deep);
+  __syncthreads();
   if (tid == 0) {
     Ctrl *c = a.ctrl;
     c->abort = kAbortNone;
     c->stat_items = items;
-    c->stat_rounds = rounds;
+    c->stat_rounds = A == Algo::BFS ? sh.left + 1 : rounds;
     c->stat_heavy = 0;
     c->stat_phases = phases + 1ull;
     c->s.set_curdelta(cd);
