@@ -146,7 +146,7 @@ constexpr uint32_t kBarGroup = 32;
 constexpr uint32_t kMaxBarGroups = 128;
 constexpr uint32_t kMaxGridBlocks = kBarGroup * kMaxBarGroups;
 
-constexpr uint32_t kHopGroups = 8;
+constexpr uint32_t kHopGroups = 32;
 
 // Device control block.  Each hot word sits on its own 128-byte line.  The
 // host copies back the part before bar_grp (kCtrlHostBytes) after a launch.
@@ -161,7 +161,7 @@ struct Ctrl {
   uint64_t stat_items, stat_rounds, stat_heavy, stat_phases, stat_edges;
   uint32_t _p7[22];
   uint32_t far_min;   uint32_t _p8[31];  // bucket far mode: smallest distance sent to the far pile this phase
-  uint64_t hop_items[kHopGroups][16];    // popped without a round of their own (wave.hip), by groups of blocks
+  uint64_t hop_items[kHopGroups][16];    // popped without a round of their own (wave.hip), by groups of wavefronts
   uint32_t bar_grp[kMaxBarGroups][32];  // group arrival counters, one line each
 };
 constexpr size_t kCtrlHostBytes = offsetof(Ctrl, bar_grp);

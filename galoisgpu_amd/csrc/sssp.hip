@@ -87,14 +87,14 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     a.local_max = wave_local_max(g.nnodes, g.nedges);
     // (a resumed BFS reports its own levels' rounds)
     a.hops = a.pace && !(A == Algo::BFS && resume) ? kWaveHops : 0;
-    a.split_deg = a.pace ? 0u : std::min(kWaveSplitDeg, a.heavy_deg);
+    a.split = !a.pace;
     // Chunks of one round, each of up to heavy_deg edges (at least 256).  Taken apart
     // when they are popped, once a round at most (wave_items): ceil(d / heavy_deg)
-    // for a vertex of d >= heavy_deg edges, 2 E / heavy_deg in all.  With
-    // split_deg a vertex may be popped from the far pile and pushed near in one
-    // round: 1 chunk from 64 edges on, 2 ceil(d / heavy_deg) <= d / 64 from heavy_deg
-    // on, so half of this.
-    if (a.split_deg) a.hcap = (uint32_t)std::min<uint64_t>(2ull * g.nedges / a.split_deg + 64, UINT32_MAX / 2);
+    // for a vertex of d >= heavy_deg edges, 2 E / heavy_deg in all.  Where vertices
+    // are split when they are pushed (a.split, or WaveGrowth's wide rounds), one
+    // may be popped from the far pile and pushed near in one round: 1 chunk from 64
+    // edges on, 2 ceil(d / heavy_deg) <= d / 64 from heavy_deg on, so half of this.
+    a.hcap = (uint32_t)std::min<uint64_t>(2ull * g.nedges / kWaveSplitDeg + 64, UINT32_MAX / 2);
     void *chunks;
     if ((rc = ws_buffer(w, kBufHeavy, 2ull * a.hcap * sizeof(WaveChunk), &chunks))) return rc;
     a.chunk[0] = (WaveChunk *)chunks;

@@ -16,9 +16,10 @@ struct WaveCtrl {
   // a waiting block needs no second load and the publisher no ordering.
   uint64_t msg[kWaveMsg];
   uint64_t _p0[16 - kWaveMsg];
-  // How far the next phase moves the threshold; between leading blocks only.
-  uint32_t pace[5];
-  uint32_t _p1[27];
+  // How far the next phase moves the threshold, and how the rounds grow (WavePace,
+  // WaveGrowth); between leading blocks only.
+  uint32_t pace[7];
+  uint32_t _p1[25];
   struct alignas(8) Line {
     uint32_t n;
     uint32_t _p[31];
@@ -46,7 +47,7 @@ struct WaveArgs : KArgs {
   uint32_t local_max = 0; // largest round that one block runs alone
   uint32_t hops = 0;      // times that a wavefront goes on with what it pushed near
   uint32_t _pad = 0;
-  uint32_t split_deg = 0; // edges from which a vertex is queued as chunks when it is pushed; 0: when it is popped
+  uint32_t split = 0;     // vertices of kWaveSplitDeg edges are queued as chunks when they are pushed, else of heavy_deg when popped
 };
 
 // Blocks per CU, of 256 threads, where the call leaves the launch shape open.

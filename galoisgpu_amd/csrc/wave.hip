@@ -92,7 +92,14 @@ struct WavePace {
     rounds += 1;
   }
   // The step to the threshold of the phase after `phase`.
-  __device__ uint32_t next(uint32_t phase) {
+  __device__ uint32_t next(uint32_t phase, uint32_t flags, bool forest) {
+    // (see WaveGrowth)
+    if (flags & kWaveSplit || (flags & kWaveWide && forest)) {
+      cost = 0;
+      rounds = 0;
+      step = 1;
+      return flags & kWaveSplit ? 1u : kMaxStep;
+    }
     const float rate = (float)step / cost;
     const bool empty = cost < 4.0f * (float)rounds;
     cost = 0;
@@ -114,6 +121,44 @@ struct WavePace {
   }
 };
 
+// Growth of the rounds on graphs of low degree.  Few edges a vertex do not make a
+// graph deep: on a random graph or an RMAT graph of 4 edges a vertex the frontier
+// grows by factors, the traversal is a few dozen rounds, and what pays on a grid
+// does not.  From a round of more than kWideItems items that is more than three times
+// the largest so far (a grid's frontier, which grows by a ring a round, never is;
+// at twice road-like 2048^2 took 2.55 ms, with it or without the rule 2.03)
+// the next kWideRounds rounds -- all that such a graph has -- are wide:
+//   - wavefronts go on with what they pushed only in rounds of at most kWideHops
+//     items: larger ones are bound by work, and what is expanded at a distance that
+//     falls later is work done twice;
+//   - units are smaller (kWideUnit items at least): a vertex may have many edges;
+//   - where vertices of heavy_deg edges are found too (kWaveSplit), the rounds are
+//     those of skewed graphs: no going on, vertices of kWaveSplitDeg edges split
+//     when they are pushed, the threshold moved by the call's delta;
+//   - on graphs of at most 2 edges a vertex (forests: one way to each vertex) the
+//     next phase is all that is left.
+// A chunk counts as heavy_deg items: it may push so many.
+// Kernel us without / with, delta 10000 where the delta is not said: 5 edges a vertex
+// RMAT-like, 32,000 vertices 347 / 207, 100,000 455 / 248, 10^6 1040 / 679, delta 32
+// 916 / 612; uniform out-degree 4, 10^6 1028 / 865, BFS 451 / 340, 4 x 10^6 2734 /
+// 2405, BFS 1250 / 908; random trees of 10^5 delta 32 388 / 289; 4 x 10^6 leaves of
+// 1000 hubs, delta 32 1576 / 1150.  Grids and road-like graphs alike.
+constexpr uint32_t kWideItems = 512, kWideRounds = 48, kWideUnit = 4;
+template <Algo A>
+constexpr uint32_t kWideHops = A == Algo::SSSP ? 16384 : 8192;
+constexpr uint32_t kWideChunks = 4;  // chunks of a round that say that the graph is skewed
+struct WaveGrowth {
+  uint32_t peak;   // items of the largest round so far
+  uint32_t until;  // rounds before this one are wide
+  // The flags of round `round`, of n items, after a round with flags `before`;
+  // `heavy`: it took vertices apart.
+  __device__ uint32_t flags(uint32_t round, uint32_t n, bool heavy, uint32_t before) {
+    if (n > kWideItems && n / 3 > peak) until = round + kWideRounds;
+    peak = max(peak, n);
+    return round >= until ? 0u : heavy ? kWaveWide | kWaveSplit : kWaveWide | (before & kWaveSplit);
+  }
+};
+
 template <int BS>
 struct WaveShared {
   static constexpr int NW = BS / kWave;
@@ -124,6 +169,7 @@ struct WaveShared {
   WaveRound r;
   uint32_t gen;
   WavePace pace;
+  WaveGrowth growth;
   // rounds of one block
   Entry pile[2][kLocalCap];
   uint32_t pile_n[2];
@@ -146,7 +192,9 @@ struct WaveLane {
   WaveHeavy *hbuf;
   uint32_t n[2], hn;  // staged: items per pile, heavy items (wave-uniform)
   uint32_t settled;   // see wave_settle
-  uint32_t hopped;    // vertices popped in hops
+  uint32_t hopped;    // vertices popped in hops, per lane
+  uint32_t hops;      // this round's WaveArgs::hops
+  bool split;         // vertices of kWaveSplitDeg edges are taken apart when they are pushed
 };
 
 __device__ __forceinline__ uint32_t *wave_queue(const WaveArgs &a, uint32_t i) {
@@ -204,7 +252,7 @@ __device__ __forceinline__ void wave_heavy(const WaveArgs &a, WaveLane &w, bool 
   w.hn += c;
 }
 
-// The near items staged since the last call: those of split_deg edges and more
+// The near items staged since the last call: those of kWaveSplitDeg edges and more
 // become chunks of the next round, read with the distance of that time; the
 // others close up.
 __device__ __forceinline__ void wave_settle(const WaveArgs &a, WaveLane &w) {
@@ -214,7 +262,7 @@ __device__ __forceinline__ void wave_settle(const WaveArgs &a, WaveLane &w) {
     const uint32_t v = valid ? w.pbuf[0][i0 + lane_id()] : 0u;
     const uint64_t rb = ld_pair(a.row_start + v);
     const uint32_t rs = (uint32_t)rb, deg = (uint32_t)(rb >> 32) - rs;
-    const bool split = valid && deg >= a.split_deg;
+    const bool split = valid && deg >= kWaveSplitDeg;
     wave_heavy(a, w, split, v, kInf, rs, deg);
     const uint64_t m = __ballot(valid && !split);
     if (valid && !split) w.pbuf[0][out + lanes_below(m)] = v;
@@ -229,7 +277,7 @@ __device__ __forceinline__ void wave_stage(const WaveArgs &a, WaveLane &w, int w
   if (m == 0) return;
   const uint32_t c = (uint32_t)__builtin_popcountll(m);
   if (w.n[which] + c > kWavePush) {
-    if (which == 0 && a.split_deg) wave_settle(a, w);
+    if (which == 0 && w.split) wave_settle(a, w);
     uint32_t base = 0;
     if (lane_id() == 0 && w.n[which]) base = atomic_add(which ? w.ftail : w.ntail, w.n[which]);
     wave_store(a, w, which, readlane(base, 0));
@@ -280,7 +328,7 @@ __device__ __forceinline__ void wave_relax(const WaveArgs &a, WaveLane &w, const
 #pragma unroll
   for (int k = 0; k < U; ++k) {
     const uint32_t stamp = near[k] ? w.near_stamp : w.far_stamp;
-    const bool want = nd[k] < old[k] && (seen[k] != stamp || (a.hops && near[k]));
+    const bool want = nd[k] < old[k] && (seen[k] != stamp || (w.hops && near[k]));
     got[k] = want ? atomic_exch((near[k] ? ns : fs) + v[k], stamp) : stamp;
   }
 #pragma unroll
@@ -335,7 +383,7 @@ __device__ __forceinline__ uint32_t wave_vertices(const WaveArgs &a, WaveLane &w
   return total;
 }
 
-// A unit of n in-queue items, and then, a.hops times, what the wavefront itself has
+// A unit of n in-queue items, and then, w.hops times, what the wavefront itself has
 // just pushed near (64 at most), without waiting for the round's end.  A vertex
 // taken so loses its stamp before its distance is read, and pushes go by the
 // exchange alone (a stamp read ahead of it may be gone): whoever lowers the vertex
@@ -363,7 +411,7 @@ __device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const
   for (uint32_t h = 0;; ++h) {
     const uint32_t rs = (uint32_t)rb, deg = lane < n ? (uint32_t)(rb >> 32) - rs : 0u;
     const uint32_t total = wave_vertices<A>(a, w, cut, u, n, rs, deg);
-    if (h == a.hops || total > kHopEdges) break;
+    if (h == w.hops || total > kHopEdges) break;
     if (w.n[0] < kept) kept = 0;  // written out meanwhile
     n = min((uint32_t)kWave, w.n[0] - kept);
     if (n == 0) break;
@@ -373,9 +421,8 @@ __device__ __forceinline__ void wave_items(const WaveArgs &a, WaveLane &w, const
     if (lane < n) (void)atomic_exch(a.near_stamp + u, 0u);
     order_release();  // the stamp is gone before the distance is read
     const bool heavy = lane < n && (uint32_t)(rb >> 32) - (uint32_t)rb >= a.heavy_deg;
-    const uint64_t hm = __ballot(heavy);
-    w.hopped += n - (uint32_t)__builtin_popcountll(hm);
-    if (hm) {
+    w.hopped += lane < n && !heavy ? 1u : 0u;
+    if (__ballot(heavy)) {
       const bool back = heavy && atomic_exch(a.near_stamp + u, w.near_stamp) != w.near_stamp;
       const uint64_t m = __ballot(back);
       if (back) w.pbuf[0][kept + lanes_below(m)] = u;
@@ -514,6 +561,7 @@ template <Algo A, int BS>
 __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh, int64_t cd0) {
   WaveRound r = sh.r;
   WavePace pace = sh.pace;
+  WaveGrowth growth = sh.growth;
   const uint32_t far_in = A == Algo::SSSP ? ld_coh(&a.wc->far_tail[r.far_q()].n) : 0u;
   if (threadIdx.x == 0) {
     sh.far_n = far_in;
@@ -523,6 +571,10 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
   uint32_t rounds = 0, cur = 0, n = r.items;
   bool load = true;  // the round's items are still in queue in_q
   unsigned long long popped = 0;
+  const auto grow = [&]() {
+    const uint32_t f = growth.flags(r.round, n, false, r.flags);
+    r.flags = (r.flags & ~(kWaveWide | kWaveSplit)) | f;
+  };
   for (;;) {
     if (load) {
       const uint32_t *const in = wave_queue(a, r.in_q());
@@ -562,19 +614,22 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       __syncthreads();
       n = sh.spill_n;
       r.roles = wave_roles(r.near_q(), r.in_q(), r.far_q());
+      if (a.hops) grow();
       break;
     }
     if (near) {
       cur ^= 1;
       n = near;
+      if (a.hops) grow();
     } else if (far) {
       // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
       r.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
       r.phase += 1;
       r.flags |= kWaveCut;
       r.cut = r.steps;
-      r.steps += a.pace ? pace.next(r.phase - 1) : 1u;
+      r.steps += a.pace ? pace.next(r.phase - 1, r.flags, a.nedges <= 2ull * a.nnodes) : 1u;
       n = far;
+      if (a.hops) grow();
       order_release();  // this wavefront's far pushes have landed
       __syncthreads();  // and every other's; far_n has been read
       if (threadIdx.x == 0) sh.far_n = 0;
@@ -594,6 +649,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
     r.heavy = 0;
     sh.r = r;
     sh.pace = pace;
+    sh.growth = growth;
     if (A == Algo::SSSP) {
       st_coh(&a.wc->far_tail[r.far_q()].n, sh.far_n);
       if (r.far_q() != 0) st_coh(&a.wc->far_tail[0].n, 0u);
@@ -652,6 +708,12 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     w.ftail = &wc->far_tail[r.far_q()].n;
     w.htail = &slot->heavy_tail.n;
     w.hq = gen & 1 ? a.chunk[1] : a.chunk[0];
+    // (BFS's first round stays one level: levels that mix there mix in every round)
+    w.hops = (A == Algo::BFS && r.round == 1) || r.flags & kWaveSplit ||
+                     (r.flags & kWaveWide && r.items > kWideHops<A>)
+                 ? 0u
+                 : a.hops;
+    w.split = a.split || r.flags & kWaveSplit;
     // Units: in-queue items, `per` at a time, then heavy chunks.  A wavefront
     // takes the unit of its number; where there are more units than
     // wavefronts, unit j * ngroups + g belongs to the blocks b with b % ngroups
@@ -659,7 +721,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     // wavefronts serialises, ~12 ns a ticket).
     const uint32_t *const in = wave_queue(a, r.in_q());
     const WaveChunk *const hin = gen & 1 ? a.chunk[0] : a.chunk[1];
-    const uint32_t per = min((uint32_t)kWave, max(a.unit_min, (r.items + nwaves - 1) / nwaves));
+    const uint32_t per = min((uint32_t)kWave, max(r.flags & kWaveWide ? kWideUnit : a.unit_min, (r.items + nwaves - 1) / nwaves));
     const uint32_t nitem = (r.items + per - 1) / per, nunits = nitem + r.heavy;
     const bool many = nunits > nwaves;
     uint32_t unit = many ? (blockIdx.x / ngroups * NW + wv) * ngroups + g : wave;
@@ -672,7 +734,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
       unit = (gblocks * NW + readlane(t, 0)) * ngroups + g;
     }
     // The block's pushes get their places with one atomic per pile.
-    if (a.split_deg) wave_settle(a, w);
+    if (w.split) wave_settle(a, w);
     const uint32_t hend = w.hn ? wave_heavy_ends(a, w) : 0u;
     order_release();
     if (lane_id() == kWave - 1) {
@@ -716,12 +778,13 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
         // every word that the step needs in one load
         const uint32_t lane = lane_id();
         const uint32_t *p = lane == 0 ? &slot->near_tail.n : lane == 1 ? &slot->heavy_tail.n : lane == 2 ? &c->abort
-                            : lane < 8 ? &wc->pace[lane - 3] : &wc->far_tail[r.far_q()].n;
+                            : lane < 10 ? &wc->pace[lane - 3] : &wc->far_tail[r.far_q()].n;
         const uint32_t word = ld_coh(p);
         const uint32_t nnear = readlane(word, 0), nheavy = readlane(word, 1), ab = readlane(word, 2);
-        const uint32_t nfar = A == Algo::SSSP ? readlane(word, 8) : 0u;
+        const uint32_t nfar = A == Algo::SSSP ? readlane(word, 10) : 0u;
         WavePace pace{max(readlane(word, 3), 1u), readlane(word, 4), __uint_as_float(readlane(word, 5)),
                       __uint_as_float(readlane(word, 6)), readlane(word, 7)};
+        WaveGrowth growth{max(readlane(word, 8), r.items), readlane(word, 9)};
         if (A == Algo::SSSP) pace.round(r.items, false);
         // (the slot of the round before the last: no block reads it any more)
         WaveCtrl::Slot *const next = &wc->slot[(gen + 2) % 3];
@@ -741,16 +804,17 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
           x.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
           x.phase = r.phase + 1;
           x.cut = r.steps;
-          x.steps = r.steps + (a.pace ? pace.next(r.phase) : 1u);
+          x.steps = r.steps + (a.pace ? pace.next(r.phase, r.flags, a.nedges <= 2ull * a.nnodes) : 1u);
           if (lane == 0) st_coh(&wc->far_tail[r.far_q()].n, 0u);
         }
         x.flags = kWaveLead | (done ? kWaveDone : x.heavy == 0 && x.items <= a.local_max / 2 ? kWaveLocal : 0u) |
-                  (phase ? kWaveCut : 0u);
+                  (phase ? kWaveCut : 0u) | (a.hops ? growth.flags(x.round, x.items + a.heavy_deg * nheavy, nheavy >= kWideChunks, r.flags) : 0u);
         if (lane == 0) {
           __hip_atomic_fetch_add(&c->stat_items, (uint64_t)r.items, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_fetch_add(&c->stat_heavy, (uint64_t)r.heavy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_fetch_add(&c->stat_rounds, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           sh.pace = pace;
+          sh.growth = growth;
           sh.r = x;
           sh.gen = gen + 1;
         }
@@ -770,10 +834,11 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
         const uint32_t lane = lane_id();
         const WaveRound x = sh.r;
         wave_publish(wc, gen + 1, x);
-        if (A == Algo::SSSP && lane < 5) {
+        if (a.hops && lane < 7) {
           const WavePace p = sh.pace;
           st_coh(&wc->pace[lane], lane == 0 ? p.step : lane == 1 ? p.hold : lane == 2 ? __float_as_uint(p.best)
-                                  : lane == 3 ? __float_as_uint(p.cost) : p.rounds);
+                                  : lane == 3 ? __float_as_uint(p.cost) : lane == 4 ? p.rounds
+                                  : lane == 5 ? sh.growth.peak : sh.growth.until);
         }
         if ((x.flags & kWaveDone) && lane == 0) {
           c->s.done = 1;
@@ -786,13 +851,11 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     }
   }
   if (!a.hops) return;
-  if (lane_id() == 0) sh.count[wv][0] = w.hopped;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t n = 0;
-    for (uint32_t i = 0; i < NW; ++i) n += sh.count[i][0];
-    if (n) __hip_atomic_fetch_add(&c->hop_items[blockIdx.x % kHopGroups][0], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  uint32_t hopped = w.hopped;
+#pragma unroll
+  for (int d = kWave / 2; d >= 1; d >>= 1) hopped += __shfl_xor(hopped, d);
+  if (lane_id() == 0 && hopped)
+    __hip_atomic_fetch_add(&c->hop_items[wave % kHopGroups][0], (uint64_t)hopped, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- launch -------------------------------------------------------------------------

@@ -24,7 +24,8 @@ struct WaveRound {
 };
 // kWaveCut: the round's input is the far pile; what has come below the previous
 // threshold since it was pushed has been expanded as a near item already.
-constexpr uint32_t kWaveDone = 1, kWaveCut = 2, kWaveLead = 4, kWaveLocal = 8;
+// kWaveWide, kWaveSplit: see WaveGrowth.
+constexpr uint32_t kWaveDone = 1, kWaveCut = 2, kWaveLead = 4, kWaveLocal = 8, kWaveWide = 16, kWaveSplit = 32;
 __device__ __forceinline__ uint32_t wave_roles(uint32_t in, uint32_t near, uint32_t far) {
   return in | near << 2 | far << 4;
 }
@@ -94,7 +95,7 @@ __device__ __forceinline__ uint32_t wave_wait(const WaveArgs &a, uint32_t gen, W
     hi = (uint32_t)(m >> 32);
     tag = readlane(lo, 0);
     if (tag != gen && __ballot(lane < kWaveMsg && lo != tag) == 0) {
-      flags = readlane(hi, 6) >> 6 & (kWaveDone | kWaveCut);
+      flags = (readlane(hi, 6) >> 6 & (kWaveDone | kWaveCut)) | (readlane(hi, 6) >> 26 & (kWaveWide | kWaveSplit));
       break;
     }
     if (readlane(lo, kWaveMsg) != kAbortNone) break;
@@ -117,7 +118,7 @@ __device__ __forceinline__ uint32_t wave_wait(const WaveArgs &a, uint32_t gen, W
   x.steps = readlane(hi, 4);
   x.cut = readlane(hi, 5);
   x.roles = readlane(hi, 6) & 0x3fu;
-  x.lead = readlane(hi, 6) >> 8;
+  x.lead = readlane(hi, 6) >> 8 & 0x3fffffu;
   x.flags = flags;
   order_acquire();
   return tag;
@@ -126,7 +127,8 @@ __device__ __forceinline__ uint32_t wave_wait(const WaveArgs &a, uint32_t gen, W
 // Wavefront 0 publishes round x as generation `tag`.
 __device__ __forceinline__ void wave_publish(WaveCtrl *wc, uint32_t tag, const WaveRound &x) {
   const uint32_t m[kWaveMsg] = {x.items, x.heavy, x.round, x.phase, x.steps, x.cut,
-                                x.lead << 8 | (x.flags & (kWaveDone | kWaveCut)) << 6 | x.roles};
+                                (x.flags & (kWaveWide | kWaveSplit)) << 26 | x.lead << 8 |
+                                    (x.flags & (kWaveDone | kWaveCut)) << 6 | x.roles};
   uint32_t v = 0;
 #pragma unroll
   for (int i = 0; i < kWaveMsg; ++i)
