@@ -15,8 +15,15 @@
 // beyond the workgroup's size halve it again.  Vertices whose distance came below
 // the last threshold since they were set were near vertices then, and are dropped.
 //
-// Used up to kSmallV vertices (128 KB of the CU's 160) of low degree: a larger
-// frontier's edges are faster over the whole GPU.  Kernel ms in wave.hip ->
+// Used up to kSmallV vertices (128 KB of the CU's 160) of low degree.  A frontier
+// of many vertices is faster over the whole GPU: a round of more than kSmallList,
+// or, above kSmallSkewV vertices, one that met a vertex of kSmallHub edges (the
+// mark of a skewed graph) is left to the wavefront kernel, which goes on from the
+// distances reached.  Call us with the persistent kernel / with all rounds here /
+// now, delta 10000: uniform out-degree 4, 16384 vertices 260 / 271 / 190, 32768 260 /
+// 352 / 194; RMAT-like of 5 edges, 32768 vertices 267 / 857 / 240; 50 hubs and 32768
+// vertices 171 / 597 / 198; a tree of degree 16 111 / 260 / 133.  At most 8192
+// vertices of a hub's are as fast here.  Kernel ms in wave.hip ->
 // here: SSSP grid 64^2 0.52 -> 0.22, 100^2 0.93 -> 0.36, 181^2 1.74 -> 0.75, 40 x
 // 500 2.7 -> 1.3, road-like 181^2 0.63 -> 0.44; BFS grid 64^2 0.26 -> 0.16, 181^2
 // 0.90 -> 0.45, road-like 181^2 0.39 -> 0.19.
@@ -32,17 +39,28 @@
 namespace lsg {
 
 constexpr uint32_t kSmallThreads = 1024;  // (512 / 256: road-like 181^2 0.44 -> 0.53 / 0.77 ms, grids alike)
-constexpr uint32_t kSmallList = 4096;    // listed vertices of a round; more are taken from the bitmap
+constexpr uint32_t kSmallList = 4096;    // listed vertices of a round; with more, the whole grid goes on
 constexpr uint32_t kSmallTarget = 256;   // vertices that a phase begins with, if there are so many
 constexpr uint32_t kSmallHeavy = 32;     // vertices of more edges are expanded by their wavefront
+constexpr uint32_t kSmallHub = 256, kSmallSkewV = 8192;
 constexpr uint32_t kSmallWords = kSmallV / 32;
+
+// What the host reads at the end: written to host memory, as a copy back after
+// the kernel costs some 8 us of a call.
+struct SmallResult {
+  uint64_t items, rounds, phases;
+  int64_t curdelta;
+  uint32_t handed;  // the rounds go on over the whole grid
+};
+static_assert(sizeof(SmallResult) <= 256, "the workspace's pinned words");
 
 struct SmallArgs {
   const uint32_t *row_start, *edge_dst, *edge_data;
   uint32_t *dist;
-  Ctrl *ctrl;
+  SmallResult *res;
   uint64_t nedges;
   uint32_t nnodes, seed, delta;
+  uint32_t hub;  // edges from which a vertex ends the rounds here
 };
 
 struct SmallShared {
@@ -141,6 +159,7 @@ __device__ __forceinline__ void small_expand(const SmallArgs &a, SmallShared &sh
   for (uint64_t hm = __ballot(heavy); hm; hm &= hm - 1) {
     const uint32_t l = (uint32_t)__builtin_ctzll(hm);
     const uint32_t hd = readlane(d, l), hrs = readlane(rs, l), hre = hrs + readlane(deg, l);
+    if (hre - hrs >= a.hub && lane_id() == 0) atomicAdd(count, kSmallV);  // more than a list holds
     for (uint32_t j = hrs; j < hre; j += kWave * kInFlight) {
       uint32_t u[kInFlight], nd[kInFlight];
       bool act[kInFlight];
@@ -165,34 +184,29 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs a) {
     sh.queued[i] = i == a.seed / 32 ? 1u << (a.seed % 32) : 0u;
     sh.far[i] = 0;
   }
+  const uint64_t seed_row = ld_pair(a.row_start + a.seed);
   if (tid == 0) {
+    const uint32_t deg = (uint32_t)(seed_row >> 32) - (uint32_t)seed_row;
     sh.list[0][0] = (uint16_t)a.seed;
     sh.n[1] = sh.n[2] = 0;
+    sh.n[0] = deg >= a.hub || deg > kSmallList ? kSmallV : 1u;
   }
   // list cur, count of the round to come in n[slot], of the one after in n[slot + 1]
-  uint32_t cur = 0, slot = 0, n = 1, rounds = 0, phases = 0, in_phase = 0, since = 0;
+  uint32_t cur = 0, slot = 0, n, rounds = 0, phases = 0, in_phase = 0, since = 0;
   int64_t cd = 0, step = a.delta;
   unsigned long long items = 0;
+  bool handed = false;
   __syncthreads();
+  n = *(volatile uint32_t *)&sh.n[0];
   for (;;) {
+    handed = n > kSmallList;
+    if (handed) break;
     const uint32_t thr = (uint32_t)min(cd, (int64_t)0xFFFFFFFFll);
     slot = slot == 2 ? 0 : slot + 1;
     uint32_t *const count = &sh.n[slot];
-    if (n <= kSmallList) {
-      for (uint32_t i0 = 0; i0 < n; i0 += kSmallThreads) {
-        const uint32_t i = i0 + tid;
-        if (__ballot(i < n)) small_expand<A>(a, sh, cur ^ 1, count, thr, i < n, i < n ? sh.list[cur][i] : 0u);
-      }
-    } else {
-      for (uint32_t i = tid; __ballot(i < words); i += kSmallThreads) {
-        uint32_t w = i < words ? *(volatile uint32_t *)&sh.queued[i] : 0u;
-        while (__ballot(w != 0)) {
-          const bool valid = w != 0;
-          const uint32_t v = valid ? i * 32 + (uint32_t)__builtin_ctz(w) : 0u;
-          w &= w - 1;
-          small_expand<A>(a, sh, cur ^ 1, count, thr, valid, v);
-        }
-      }
+    for (uint32_t i0 = 0; i0 < n; i0 += kSmallThreads) {
+      const uint32_t i = i0 + tid;
+      if (__ballot(i < n)) small_expand<A>(a, sh, cur ^ 1, count, thr, i < n, i < n ? sh.list[cur][i] : 0u);
     }
     ++rounds;
     ++since;
@@ -242,58 +256,51 @@ __global__ __launch_bounds__(kSmallThreads) void small_kernel(SmallArgs a) {
       ++phases;
     }
   }
-  if (tid == 0) sh.left = 0;
-  __syncthreads();
-  uint32_t deep = 0;
-  for (uint32_t v = tid; v < a.nnodes; v += kSmallThreads) {
-    const uint32_t d = sh.dist[v];
-    glb(a.dist)[v] = d;
-    if (A == Algo::BFS && d != kInf) deep = max(deep, d);
-  }
-  // BFS: one round a level and the last, which finds nothing (a round that takes its
-  // vertices from the bitmap goes on with what it finds, and saves some)
-  if (A == Algo::BFS && deep) atomicMax(&sh.left, deep);
-  __syncthreads();
+  for (uint32_t v = tid; v < a.nnodes; v += kSmallThreads) glb(a.dist)[v] = sh.dist[v];
   if (tid == 0) {
-    Ctrl *c = a.ctrl;
-    c->abort = kAbortNone;
-    c->stat_items = items;
-    c->stat_rounds = A == Algo::BFS ? sh.left + 1 : rounds;
-    c->stat_heavy = 0;
-    c->stat_phases = phases + 1ull;
-    c->s.set_curdelta(cd);
+    SmallResult *r = a.res;
+    r->items = items;
+    r->rounds = rounds;
+    r->phases = phases + 1ull;
+    r->curdelta = cd;
+    r->handed = handed;
   }
 }
 
 template <Algo A>
-static int run_small(Workspace *w, const CsrView &g, uint32_t seed, const lsg_opts &o, uint32_t *dist, lsg_stats *st) {
-  const SmallArgs a{g.row, g.dst, g.w, dist, w->ctrl, g.nedges, g.nnodes, seed, A == Algo::SSSP ? (uint32_t)o.delta : 1u};
+static int run_small(Workspace *w, const CsrView &g, uint32_t seed, const lsg_opts &o, uint32_t *dist, lsg_stats *st,
+                     Resume *resume) {
+  const SmallArgs a{g.row, g.dst, g.w, dist, (SmallResult *)w->pinned, g.nedges, g.nnodes, seed, A == Algo::SSSP ? (uint32_t)o.delta : 1u,
+                    g.nnodes > kSmallSkewV ? kSmallHub : UINT32_MAX};
   HIPCHK(hipEventRecord(w->ev0, w->stream));
   hipLaunchKernelGGL(small_kernel<A>, dim3(1), dim3(kSmallThreads), 0, w->stream, a);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(w->ev1, w->stream));
-  Ctrl hc;
-  HIPCHK(hipMemcpyAsync(&hc, w->ctrl, kCtrlHostBytes, hipMemcpyDeviceToHost, w->stream));
   HIPCHK(hipStreamSynchronize(w->stream));
+  const SmallResult r = *(const SmallResult *)w->pinned;
   float ms = 0;
   HIPCHK(hipEventElapsedTime(&ms, w->ev0, w->ev1));
   if (st) {
     memset(st, 0, sizeof *st);
     st->ms_kernel = ms;
-    st->items = hc.stat_items;
-    st->near_iters = hc.stat_rounds;
-    st->iterations = A == Algo::SSSP ? hc.stat_phases : hc.stat_rounds;
-    st->last_delta = (int32_t)std::min<int64_t>(hc.s.curdelta(), INT32_MAX);
+    st->items = r.items;
+    st->near_iters = r.rounds;
+    st->iterations = A == Algo::SSSP ? r.phases : r.rounds;
+    st->last_delta = (int32_t)std::min<int64_t>(r.curdelta, INT32_MAX);
     st->grid_blocks = 1;
     st->block_size = (int32_t)kSmallThreads;
   }
-  return LSG_OK;
+  // (BFS's rounds are its levels: the next one's vertices are of that level)
+  const uint32_t level = (uint32_t)r.rounds;
+  if (A == Algo::SSSP) *resume = Resume{r.curdelta, 0u, kInf - 1u, true};
+  else *resume = Resume{0, level, level, true};
+  return r.handed ? kBlockFallback : LSG_OK;
 }
 
 int run_small_single(int algo, Workspace *w, const CsrView &g, uint32_t seed, const lsg_opts &o, uint32_t *dist,
-                     lsg_stats *st) {
-  return algo == (int)Algo::SSSP ? run_small<Algo::SSSP>(w, g, seed, o, dist, st)
-                                 : run_small<Algo::BFS>(w, g, seed, o, dist, st);
+                     lsg_stats *st, Resume *resume) {
+  return algo == (int)Algo::SSSP ? run_small<Algo::SSSP>(w, g, seed, o, dist, st, resume)
+                                 : run_small<Algo::BFS>(w, g, seed, o, dist, st, resume);
 }
 
 }  // namespace lsg

@@ -85,8 +85,10 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     a.pace = low_degree(g.nnodes, g.nedges);
     a.unit_min = a.pace ? 16 : 8;
     a.local_max = wave_local_max(g.nnodes, g.nedges);
+    a.wide = resume && resume->wide;
     // (a resumed BFS reports its own levels' rounds)
     a.hops = a.pace && !(A == Algo::BFS && resume) ? kWaveHops : 0;
+    a.levels = A == Algo::BFS && (a.hops || a.wide);
     a.split = !a.pace;
     // Chunks of one round, each of up to heavy_deg edges (at least 256).  Taken apart
     // when they are popped, once a round at most (wave_items): ceil(d / heavy_deg)
@@ -182,9 +184,9 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     w->last_feat.resize((size_t)np * kFeatRec);
     if (np) HIPCHK(hipMemcpy(w->last_feat.data(), a.feat, w->last_feat.size() * sizeof(float), hipMemcpyDeviceToHost));
   }
-  // BFS in hops runs fewer rounds than there are levels: one a level, and the
-  // last, which finds nothing, are reported.
-  if (A == Algo::BFS && a.hops) hc.stat_rounds = hc.s.aux[3] + 1ull;
+  // BFS on these graphs may run fewer rounds than there are levels, or more where
+  // hubs are taken apart: one a level, and the last, which finds nothing, are reported.
+  if (A == Algo::BFS && a.levels) hc.stat_rounds = hc.s.aux[3] + 1ull - (resume ? resume->lo : 0u);
   if (a.hops)
     for (const auto &h : hc.hop_items) hc.stat_items += h[0];
   if (st) {
@@ -227,10 +229,14 @@ static int run_single(const lsg_graph *g, const lsg_opts *o_in, uint32_t *dist, 
   CsrView v{g->row_start, g->edge_dst, (const uint32_t *)g->edge_data, g->nnodes, g->nedges};
   uint32_t seed = (uint32_t)o.start_node;
   if (o.single_block && o.enable_lb) return fail(LSG_ERR_ARG, "single_block and enable_lb (-l) exclude each other");
-  if (o.single_block) {
+  const bool small = !o.single_block && use_small(v, o);
+  if (o.single_block || small) {
     lsg_stats bst;
     Resume res;
-    rc = run_block_single((int)A, w, v, seed, o, dist, &bst, &res);
+    int bs, expand;
+    if (small && (rc = check_single_opts(o, A == Algo::SSSP, &bs, &expand))) return rc;
+    rc = small ? run_small_single((int)A, w, v, seed, o, dist, &bst, &res)
+               : run_block_single((int)A, w, v, seed, o, dist, &bst, &res);
     if (rc == kBlockFallback) {
       // The piles overflowed: the whole grid continues from the
       // distances the workgroup reached (not captured: a one-off launch).
@@ -244,10 +250,6 @@ static int run_single(const lsg_graph *g, const lsg_opts *o_in, uint32_t *dist, 
     } else if (rc == LSG_OK && st) {
       *st = bst;
     }
-  } else if (use_small(v, o)) {
-    int bs, expand;
-    if ((rc = check_single_opts(o, A == Algo::SSSP, &bs, &expand))) return rc;
-    rc = run_small_single((int)A, w, v, seed, o, dist, st);
   } else {
     rc = o.enable_lb ? run_lb_single((int)A, w, v, seed, o, dist, st)
                      : run_core<A>(w, v, &seed, 1, o, dist, o.graph_launch != 0, st);

@@ -1087,6 +1087,7 @@ static __global__ void resume_init_kernel(KArgs a, uint32_t delta, int64_t cd0) 
 struct Resume {
   int64_t curdelta;
   uint32_t lo, hi;
+  bool wide = false;  // the wavefront kernel's first rounds are wide (WaveGrowth)
 };
 
 // The queue order is unspecified; the distances do not depend on it.
@@ -1235,9 +1236,10 @@ int run_graphs_block(Workspace *w, const lsg_graph *graphs, uint32_t ngraphs, co
                      int32_t *const *dist_out, const lsg_opts &o, lsg_batch_stats *stats);
 
 // Small low-degree graphs in one workgroup, distances in LDS (small.hip).  Takes
-// at most kSmallV vertices; options as the wavefront kernel's.
+// at most kSmallV vertices; options as the wavefront kernel's.  kBlockFallback: the
+// frontier grew too wide, and the whole grid goes on as *resume says.
 constexpr uint32_t kSmallV = 32768;
 int run_small_single(int algo, Workspace *w, const CsrView &g, uint32_t seed, const lsg_opts &o, uint32_t *dist,
-                     lsg_stats *st);
+                     lsg_stats *st, Resume *resume);
 
 }  // namespace lsg

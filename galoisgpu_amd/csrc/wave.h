@@ -46,6 +46,8 @@ struct WaveArgs : KArgs {
   uint32_t unit_min = 0;  // fewest items of a unit
   uint32_t local_max = 0; // largest round that one block runs alone
   uint32_t hops = 0;      // times that a wavefront goes on with what it pushed near
+  uint32_t wide = 0;      // the first rounds are wide (WaveGrowth)
+  uint32_t levels = 0;    // BFS: the deepest level is looked up at the end
   uint32_t _pad = 0;
   uint32_t split = 0;     // vertices of kWaveSplitDeg edges are queued as chunks when they are pushed, else of heavy_deg when popped
 };

@@ -683,6 +683,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     x.items = c->s.in_count;
     x.round = 1;
     x.roles = wave_roles(0, 1, 2);
+    x.flags = a.wide ? kWaveWide : 0u;
     sh.r = x;
     sh.gen = 0;
   }
@@ -860,7 +861,11 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
 
 // ---- launch -------------------------------------------------------------------------
 
-__global__ void wave_reset_kernel(WaveCtrl *wc) { wave_reset(wc, threadIdx.x, blockDim.x); }
+__global__ void wave_reset_kernel(WaveCtrl *wc, uint32_t wide) {
+  wave_reset(wc, threadIdx.x, blockDim.x);
+  __syncthreads();
+  if (threadIdx.x == 0 && wide) wc->pace[6] = kWideRounds;  // WaveGrowth::until
+}
 
 // Distances, stamps, control words and the one seed (apps/sssp/kernel.cu:23-35,469,476-477).
 __global__ void wave_init_kernel(WaveArgs a, uint32_t seed) {
@@ -913,12 +918,12 @@ int wave_enqueue(Algo algo, int bs, int grid, const WaveArgs &a, uint32_t seed, 
       hipLaunchKernelGGL(init_kernel, dim3(blocks), dim3(256), 0, stream, k, a.delta);
       hipLaunchKernelGGL(seed_kernel, dim3(1), dim3(256), 0, stream, k, seeds, nseeds);
     }
-    hipLaunchKernelGGL(wave_reset_kernel, dim3(1), dim3(256), 0, stream, a.wc);
+    hipLaunchKernelGGL(wave_reset_kernel, dim3(1), dim3(256), 0, stream, a.wc, a.wide);
   } else {
     hipLaunchKernelGGL(wave_init_kernel, dim3(blocks), dim3(256), 0, stream, a, seed);
   }
   hipLaunchKernelGGL(pick_wave(algo, bs), dim3(grid), dim3(bs), 0, stream, a);
-  if (algo == Algo::BFS && a.hops)
+  if (a.levels)
     hipLaunchKernelGGL(wave_levels_kernel, dim3(std::min<uint32_t>(blocks, (uint32_t)cus)), dim3(256), 0, stream,
                        (const uint32_t *)a.dist, a.nnodes, a.ctrl);
   HIPCHK(hipGetLastError());
