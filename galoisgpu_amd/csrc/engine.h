@@ -146,7 +146,7 @@ constexpr uint32_t kBarGroup = 32;
 constexpr uint32_t kMaxBarGroups = 128;
 constexpr uint32_t kMaxGridBlocks = kBarGroup * kMaxBarGroups;
 
-constexpr uint32_t kHopGroups = 32;
+constexpr uint32_t kHopGroups = 16;
 
 // Device control block.  Each hot word sits on its own 128-byte line.  The
 // host copies back the part before bar_grp (kCtrlHostBytes) after a launch.

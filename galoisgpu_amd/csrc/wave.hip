@@ -620,7 +620,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
     if (near) {
       cur ^= 1;
       n = near;
-      if (a.hops) grow();
+      growth.peak = max(growth.peak, n);
     } else if (far) {
       // the whole far pile is the next phase's input (apps/sssp/kernel.cu:374-383)
       r.roles = wave_roles(r.far_q(), r.near_q(), r.in_q());
@@ -629,11 +629,14 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       r.cut = r.steps;
       r.steps += a.pace ? pace.next(r.phase - 1, r.flags, a.nedges <= 2ull * a.nnodes) : 1u;
       n = far;
-      if (a.hops) grow();
       order_release();  // this wavefront's far pushes have landed
       __syncthreads();  // and every other's; far_n has been read
       if (threadIdx.x == 0) sh.far_n = 0;
-      if (n > a.local_max) break;
+      if (n > a.local_max) {
+        if (a.hops) grow();
+        break;
+      }
+      growth.peak = max(growth.peak, n);
       load = true;
     } else {
       r.flags |= kWaveDone;
