@@ -251,6 +251,9 @@ __global__ void row_bounds_kernel(const uint32_t *dst, uint32_t E, uint32_t V, u
 //     unvisited vertices of a few words are dealt one to a lane, 64 a step; when
 //     few lanes still search, the wavefront takes their long rows in turn.
 //     (64 consecutive vertices a step, visited or not: RMAT-22 0.33 ms, now 0.20.)
+//     The words of a unit lie as far apart as there are units: hubs that follow
+//     each other are many wavefronts' (10^6 leaves of 1000 hubs, words in a row /
+//     apart: 0.85 / 0.40 ms, bottom-up only 10.6 / 1.2; RMAT-22 so 1.84 / 1.63).
 //   - The first top-down level after those reads its frontier from the bitmaps.
 //   - Small top-down levels are run by one block, as in wave.hip.
 // Kernel ms (with a bitmap per level in place of queues, read through to the
@@ -520,17 +523,18 @@ __device__ __forceinline__ uint32_t nth_bit(uint64_t x, uint32_t n) {
   return pos;
 }
 
-// Bottom-up: the unvisited vertices with in-edges of nwords <= kDoWords words,
-// one per lane and step.
+// Bottom-up: the unvisited vertices with in-edges of up to kDoWords words (word0
+// and every stride-th after it), one per lane and step.
 __device__ __forceinline__ void do_up(const DoArgs &a, DoLane &w, const uint64_t *prev, uint64_t *next, uint32_t word0,
-                                      uint32_t nwords, uint64_t *hits) {
+                                      uint32_t stride, uint64_t *hits) {
   const uint32_t lane = lane_id();
   const uint32_t *const prev32 = (const uint32_t *)prev;
-  const bool mine = lane < nwords && word0 + lane < a.words;
+  const uint32_t own_word = word0 + lane * stride;
+  const bool mine = lane < kDoWords && own_word < a.words;
   uint64_t seen = 0, open = 0;
   if (mine) {
-    seen = ((const LSG_GLOBAL uint64_t *)prev)[word0 + lane];
-    open = ((const LSG_GLOBAL uint64_t *)a.in_any)[word0 + lane] & ~seen;
+    seen = ((const LSG_GLOBAL uint64_t *)prev)[own_word];
+    open = ((const LSG_GLOBAL uint64_t *)a.in_any)[own_word] & ~seen;
   }
   uint32_t end = (uint32_t)__builtin_popcountll(open);  // inclusive prefix over the words
   const uint32_t own = end;
@@ -552,7 +556,7 @@ __device__ __forceinline__ void do_up(const DoArgs &a, DoLane &w, const uint64_t
     const uint32_t before = (uint32_t)__shfl(end - own, wd);
     const bool valid = f < total;
     const uint32_t bit = valid ? nth_bit(bits, f - before) : 0u;
-    const uint32_t v = valid ? (word0 + wd) * kWave + bit : 0u;
+    const uint32_t v = valid ? (word0 + wd * stride) * kWave + bit : 0u;
     const uint64_t in = ld_pair(a.in_row + v), rb = ld_pair(a.row_start + v);
     uint32_t e = (uint32_t)in, e1 = valid ? (uint32_t)(in >> 32) : e;
     bool found = false;
@@ -601,7 +605,7 @@ __device__ __forceinline__ void do_up(const DoArgs &a, DoLane &w, const uint64_t
     }
     if (__ballot(found)) do_found(a, w, found, (uint32_t)rb, (uint32_t)(rb >> 32) - (uint32_t)rb);
   }
-  if (mine) st_coh64(next + word0 + lane, seen | hits[lane]);
+  if (mine) st_coh64(next + own_word, seen | hits[lane]);
 }
 
 // Bottom-up once the frontier's edges exceed 1/kAlpha of the unexplored ones,
@@ -800,7 +804,7 @@ __global__ __launch_bounds__(BS, 4) void do_kernel(DoArgs a) {
     const uint32_t nunits = nitem + (up ? 0u : r.heavy);
     const bool many = nunits > nwaves;
     if (up) {
-      for (uint32_t i = wave; i < nunits; i += nwaves) do_up(a, w, now, other, i * upw, upw, sh.hits[wv]);
+      for (uint32_t i = wave; i < nunits; i += nwaves) do_up(a, w, now, other, i, nunits, sh.hits[wv]);
     } else {
       const uint32_t *const in = qi ? a.q[1] : a.q[0];
       const uint64_t *const hin = gen & 1 ? a.hchunk[0] : a.hchunk[1];
@@ -1093,8 +1097,11 @@ int lsg_bfs_do(const lsg_graph *g, const lsg_graph *gt, uint32_t src, int direct
   // Blocks per CU: small levels want few at the barrier, the large ones of a
   // large graph many wavefronts (ms at 1 / 2 / 4: RMAT-16 0.061 / 0.068 / 0.087,
   // RMAT-18 0.070 / 0.076 / 0.097, RMAT-20 0.108 / 0.105 / 0.121, RMAT-22 0.247 /
-  // 0.195 / 0.193; road-like 2048^2 1.58 / 1.65 / 1.77).
-  const int per_cu = low_degree(V, g->nedges) || g->nedges < (1u << 23) ? 1 : 2;
+  // 0.195 / 0.193; road-like 2048^2 1.58 / 1.65 / 1.77).  Bottom-up only, every level
+  // looks at every word (10^6 vertices: uniform out-degree 4 0.48 / 0.38 / 0.42, a
+  // random tree 0.58 / 0.51 / 0.60, 100^3 grid 6.7 / 5.5 / 5.8; RMAT-18 0.116 / 0.103 /
+  // 0.122, uniform of 10^5 0.136 / 0.148 / 0.201).
+  const int per_cu = direction == 2 ? (V < (1u << 18) ? 1 : 2) : low_degree(V, g->nedges) || g->nedges < (1u << 23) ? 1 : 2;
   grid = std::min<int>(grid, per_cu * (int)w->cus);
   void *qbuf, *hbuf, *bbuf, *wbuf;
   if ((rc = ws_buffer(w, kBufQueues, 2ull * V * 4, &qbuf)) || (rc = ws_buffer(w, kBufHeavy, 2ull * hcap * 8, &hbuf)) ||
