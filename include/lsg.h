@@ -264,7 +264,9 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
 int lsg_output_pr(const float *rank, uint32_t n, const char *file, int ids_only);
 /* Direction-optimising BFS from `src` (no reference counterpart as an
  * algorithm; the levels are apps/bfs's, as lsg_bfs_dist writes them).  `gt`
- * is the reverse of `g` (lsg_graph_transpose).  direction: 0 = per level by
+ * is the exact reverse of `g` (lsg_graph_transpose): a bottom-up level takes any
+ * visited in-neighbour for one of the level before, so with another `gt` the
+ * levels are wrong (its sources beyond the vertices count as not visited).  direction: 0 = per level by
  * frontier size (top-down, bottom-up once the frontier's edges exceed 1/14 of
  * the unexplored edges and 1/16 of all, top-down again below V/24 frontier
  * vertices), 1 = top-down only, 2 = bottom-up only.  level_dev is a device array of nnodes.
