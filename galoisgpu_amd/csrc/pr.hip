@@ -133,7 +133,7 @@ struct PrArgs {
 // control words; the flags of an iteration are those of its parity, so that
 // the next iteration's can be cleared while they are read
 constexpr int kCtlMax = 0, kCtlDone = 1, kCtlIters = 2, kCtlArrive = 3, kCtlHeavy = 4, kCtlWide = 5, kCtlLive = 6,
-              kCtlChunks = 7, kCtlEdges = 8, kCtlHot = 9, kCtlFlags = 16, kCtlTickets = kCtlFlags + 2 * (int)kFlags + 16, kCtlWords = kCtlTickets + 32 * (int)kPrGroups;
+              kCtlChunks = 7, kCtlEdges = 8, kCtlHot = 9, kCtlFlags = 32, kCtlTickets = kCtlFlags + 2 * 32 * (int)kFlags, kCtlWords = kCtlTickets + 32 * (int)kPrGroups;
 
 __device__ __forceinline__ uint32_t pr_class(const PrArgs &a, uint32_t indeg) { return a.hdeg - min(indeg, a.hdeg); }
 
@@ -320,9 +320,16 @@ __device__ __forceinline__ bool pr_store(const PrArgs &a, float *c_next, size_t 
   return fabsf(pn - pc) / pn > a.epsilon;  // pn >= 1 - alpha > 0
 }
 
+// Flag f of iteration `it`, on a line of its own: stores to one line from all
+// XCDs are performed one at a time (2500 blocks, 10,000 vertices of in-degree 300:
+// 36 us an iteration, now 18).
+__device__ __forceinline__ uint32_t *pr_flag(const PrArgs &a, uint32_t it, uint32_t f) {
+  return a.ctl + kCtlFlags + ((it & 1) * kFlags + f) * 32;
+}
+
 // Raises the block's flag if some lane's rank moved.
 __device__ __forceinline__ void pr_raise(const PrArgs &a, uint32_t it, bool moved) {
-  if (__syncthreads_or(moved) && threadIdx.x == 0) st_coh(a.ctl + kCtlFlags + (it & 1) * kFlags + blockIdx.x % kFlags, 1u);
+  if (__syncthreads_or(moved) && threadIdx.x == 0) st_coh(pr_flag(a, it, blockIdx.x % kFlags), 1u);
 }
 
 // A contribution.  kTab: those of the first kTabSize positions are in LDS, and
@@ -345,9 +352,8 @@ __device__ __forceinline__ void pr_end(const PrArgs &a, uint32_t it) {
   }
   __syncthreads();
   if (!last) return;
-  uint32_t *const flags = a.ctl + kCtlFlags;
-  const bool some = threadIdx.x < kFlags && ld_coh(flags + (it & 1) * kFlags + threadIdx.x) != 0;
-  if (threadIdx.x < kFlags) flags[((it + 1) & 1) * kFlags + threadIdx.x] = 0;
+  const bool some = threadIdx.x < kFlags && ld_coh(pr_flag(a, it, threadIdx.x)) != 0;
+  if (threadIdx.x < kFlags) *pr_flag(a, it + 1, threadIdx.x) = 0;
   if (threadIdx.x < kPrGroups) a.ctl[kCtlTickets + threadIdx.x * 32] = 0;
   const bool go_on = __syncthreads_or(some);
   if (threadIdx.x == 0) {
