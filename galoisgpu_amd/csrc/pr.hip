@@ -95,7 +95,10 @@ constexpr uint32_t kSmallEdges = 200000;
 constexpr uint32_t kChunk = 4096;    // in-edges per wavefront-sized partial sum
 constexpr int kUnrollPr = 8;         // in-edges per lane in flight
 constexpr uint32_t kPrBlock = 256;
-constexpr uint32_t kPrTile = 4096;   // vertices per block of the counting sort
+// Vertices per block of the counting sort, which takes them 256 at a time (4096 /
+// 512, whole call: 20,000 vertices of out-degree 4 0.89 / 0.83 ms, 4 x 10^6 18.3 /
+// 16.7, small world of 10^6 1.87 / 1.58, road-like 2048^2 2.61 / 2.55, RMAT-22 alike).
+constexpr uint32_t kPrTile = 512;
 // Sweeps of at most this many blocks end the iteration themselves (every block
 // arrives on one word, ~12 ns each); larger ones leave it to pr_finish_kernel's
 // launch, ~5 us (road-like 128^2, whole call: 0.88 -> 0.75 ms).
@@ -133,7 +136,7 @@ struct PrArgs {
 // control words; the flags of an iteration are those of its parity, so that
 // the next iteration's can be cleared while they are read
 constexpr int kCtlMax = 0, kCtlDone = 1, kCtlIters = 2, kCtlArrive = 3, kCtlHeavy = 4, kCtlWide = 5, kCtlLive = 6,
-              kCtlChunks = 7, kCtlEdges = 8, kCtlHot = 9, kCtlFlags = 32, kCtlTickets = kCtlFlags + 2 * 32 * (int)kFlags, kCtlWords = kCtlTickets + 32 * (int)kPrGroups;
+              kCtlChunks = 7, kCtlEdges = 8, kCtlHot = 9, kCtlSlots = 10, kCtlFlags = 32, kCtlTickets = kCtlFlags + 2 * 32 * (int)kFlags, kCtlWords = kCtlTickets + 32 * (int)kPrGroups;
 
 __device__ __forceinline__ uint32_t pr_class(const PrArgs &a, uint32_t indeg) { return a.hdeg - min(indeg, a.hdeg); }
 
@@ -283,6 +286,7 @@ __global__ void pr_chunks_kernel(PrArgs a) {
   if (tid == 0) {
     a.ctl[kCtlChunks] = a.hbase[heavy] = pr_shape_at(a, c0 + heavy) - first;
     a.ctl[kCtlEdges] = pr_shape_at(a, heavy);
+    a.ctl[kCtlSlots] = pr_shape_at(a, s0 + nsl) - first_slot;
   }
 }
 
@@ -607,11 +611,6 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
   const uint32_t maxdeg = hc[kCtlMax];
   a.local = maxdeg < kWideDeg;
   a.hdeg = E < kSmallEdges ? kWideDeg : kHeavyDeg;
-  // slots: every in-edge, and empty ones where a slice's vertices differ (the
-  // widths of a tile's slices, or of all, never rise: less than 64 x the first)
-  const uint64_t nidx = E + (uint64_t)kWave * (std::min(maxdeg, kHeavyDeg) + 1ull) * (a.local ? tiles : 1u);
-  if ((rc = ws_buffer(w, kBufUnion, nidx * 4, &ibuf))) return rc;
-  a.idx = (uint32_t *)ibuf;
   hipLaunchKernelGGL(pr_hist_kernel, dim3(tiles), dim3(kPrBlock), 0, w->stream, a);
   hipLaunchKernelGGL(scan_tile_kernel, dim3((uint32_t)hscan), dim3(kScanBlock), 0, w->stream, a.hist, (uint32_t)nhist,
                      a.hist, hist_tiles);
@@ -621,7 +620,9 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
   hipLaunchKernelGGL(scan_tile_kernel, dim3((uint32_t)sscan), dim3(kScanBlock), 0, w->stream, a.shape,
                      (uint32_t)nshape, a.shape, shape_tiles);
   hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kScanBlock), 0, w->stream, shape_tiles, (uint32_t)sscan, total);
-  hipLaunchKernelGGL(pr_chunks_kernel, dim3(vgrid), dim3(256), 0, w->stream, a);
+  // (a wavefront per heavy vertex: 10,000 of them over 160 wavefronts took 39 us)
+  const uint32_t kgrid = std::max(vgrid, (uint32_t)std::min<uint64_t>(a.nh / 4 + 1ull, 8ull * w->cus));
+  hipLaunchKernelGGL(pr_chunks_kernel, dim3(kgrid), dim3(256), 0, w->stream, a);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(hc, a.ctl, 16 * 4, hipMemcpyDeviceToHost, w->stream));
   HIPCHK(hipStreamSynchronize(w->stream));
@@ -632,8 +633,11 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
   a.nslices = (a.live - a.heavy + kWave - 1) / kWave;
   a.wide = std::min(a.nslices, (hc[kCtlWide] - nheavy * (a.local ? 0u : 1u) + kWave - 1) / kWave);
   a.slots = ((size_t)hc[kCtlEdges] + kWave - 1) / kWave * kWave;
+  const uint64_t nidx = a.slots + (uint64_t)kWave * hc[kCtlSlots];
   if (nheavy > a.nh || a.nchunks > maxchunks || a.nslices > a.ns)
     return fail(LSG_ERR_CAPACITY, "pagerank: the reverse graph's degrees exceed its edge count");
+  if ((rc = ws_buffer(w, kBufUnion, std::max<uint64_t>(nidx, 1) * 4, &ibuf))) return rc;
+  a.idx = (uint32_t *)ibuf;
   hipLaunchKernelGGL(pr_layout_kernel, dim3(8u * w->cus), dim3(kPrBlock), 0, w->stream, a);
   a.units = (uint32_t)((uint64_t)a.nchunks + a.wide + (a.nslices - a.wide + kSlices - 1) / kSlices);
   const bool tab = V >= kTabSize && E >= kTabEdges && hc[kCtlHot] >= E / kTabShare;
