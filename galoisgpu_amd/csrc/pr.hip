@@ -17,7 +17,7 @@
 // Layout.  The iterations gather one contribution per in-edge from an array of
 // V floats, and at RMAT-22's 16 MB that array, four times an XCD's L2, bounds
 // them.  So a call first renumbers the vertices by in-degree, largest first
-// (a stable counting sort; in-degrees from kHeavyDeg on, or kWideDeg on small
+// (a stable counting sort; in-degrees from kHeavyDeg on, or less on small
 // graphs, are one class): the contributions read most lie together, and
 // vertices of one in-degree are neighbours.  In that order
 //   positions [0, heavy)     in-degree >= kHeavyDeg: in-edges cut into chunks of
@@ -79,6 +79,9 @@ constexpr int kSlices = 4;
 // us per iteration without / with it: RMAT-22 (56% of the edges) 400 / 261, of
 // ef 8 221 / 141, RMAT-21 179 / 107, RMAT-20 88 / 67, 8 M edges 47 / 49, 4 M 28 / 43.
 // 16384 entries and twice the wavefronts: 320 on RMAT-22; 32768: 273.
+// Without skew -- the positions' share of the edges less than twice their share of
+// the vertices -- the L2 answers as well (100,000 vertices of in-degree 300 11.4 ms with,
+// 10.0 without).
 constexpr uint32_t kTabSize = 40448, kTabBlock = 1024, kTabEdges = 10000000, kTabShare = 4;
 // Index arrays of this many edges and more outgrow the memory-side cache
 // (256 MB), which then holds nothing of the last iteration when the next one
@@ -92,6 +95,11 @@ constexpr uint32_t kPrGroups = 16;  // groups of blocks with work tickets of the
 // behind (whole call, kHeavyDeg / kWideDeg: 120 K edges 1.58 / 1.12 ms, 228 K
 // 1.29 / 1.30, 679 K 1.74 / 2.27, 3.9 M 2.8 / 5.5).
 constexpr uint32_t kSmallEdges = 200000;
+// So are those of kMidDeg on graphs of few slices or where nearly every vertex is
+// heavy: the slices' chains would be what an iteration waits for (kHeavyDeg /
+// kMidDeg: 10,000 vertices of in-degree 200 2.03 / 1.24 ms, 20,000 2.08 / 1.77, of 300
+// 30,000 4.27 / 3.20, 100,000 12.4 / 11.4; 40,000 of 200 2.49 / 3.20, RMAT-22 19.2 / 23.5).
+constexpr uint32_t kMidDeg = 128, kMidV = 32768;
 constexpr uint32_t kChunk = 4096;    // in-edges per wavefront-sized partial sum
 constexpr int kUnrollPr = 8;         // in-edges per lane in flight
 constexpr uint32_t kPrBlock = 256;
@@ -610,7 +618,7 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
   HIPCHK(hipStreamSynchronize(w->stream));
   const uint32_t maxdeg = hc[kCtlMax];
   a.local = maxdeg < kWideDeg;
-  a.hdeg = E < kSmallEdges ? kWideDeg : kHeavyDeg;
+  a.hdeg = E < kSmallEdges ? kWideDeg : V <= kMidV || E >= (uint64_t)kHeavyDeg * V ? kMidDeg : kHeavyDeg;
   hipLaunchKernelGGL(pr_hist_kernel, dim3(tiles), dim3(kPrBlock), 0, w->stream, a);
   hipLaunchKernelGGL(scan_tile_kernel, dim3((uint32_t)hscan), dim3(kScanBlock), 0, w->stream, a.hist, (uint32_t)nhist,
                      a.hist, hist_tiles);
@@ -640,7 +648,8 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
   a.idx = (uint32_t *)ibuf;
   hipLaunchKernelGGL(pr_layout_kernel, dim3(8u * w->cus), dim3(kPrBlock), 0, w->stream, a);
   a.units = (uint32_t)((uint64_t)a.nchunks + a.wide + (a.nslices - a.wide + kSlices - 1) / kSlices);
-  const bool tab = V >= kTabSize && E >= kTabEdges && hc[kCtlHot] >= E / kTabShare;
+  const bool tab = V >= kTabSize && E >= kTabEdges && hc[kCtlHot] >= E / kTabShare &&
+                   (uint64_t)hc[kCtlHot] * V >= 2 * E * kTabSize;
   a.turn = E >= kTurnEdges;
   const uint32_t sgrid = tab ? (uint32_t)w->cus : ((a.units + kPrBlock / kWave - 1) / (kPrBlock / kWave) + 7) / 8 * 8;
   a.fused = maxdeg <= kChunk && !tab && sgrid && sgrid <= kFusedBlocks;
