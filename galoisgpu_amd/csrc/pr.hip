@@ -679,7 +679,7 @@ int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float eps
     stats->iterations = (uint64_t)iters;
     stats->items = nheavy;
     stats->grid_blocks = (int32_t)sgrid;
-    stats->block_size = 256;
+    stats->block_size = (int32_t)(tab ? kTabBlock : kPrBlock);
     stats->ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   }
   return LSG_OK;

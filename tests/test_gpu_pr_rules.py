@@ -68,5 +68,5 @@ def test_tiles(n):
 
 def test_table_needs_skew():
     n = 100000
-    check(with_in_degrees(n, np.full(n, 101), 3))  # 40 % of the edges leave the table's vertices
-    check(CSRGraph.rmat(20, 11, seed=4))
+    check(with_in_degrees(n, np.full(n, 101), 3), 256)  # 40 % of the edges leave the table's vertices
+    check(CSRGraph.rmat(20, 11, seed=4), 1024)
