@@ -1186,8 +1186,7 @@ void multi_kernel(MArgs a) {
     }
     if constexpr (P > 1) flush_packed<P>(a, s, ls, p);
     else flush_pending(a, s, ls, p);
-    // this wavefront's smallest far push per source -> phase minimum
-    if (__ballot(ls.fmin != kInf) && ls.fmin != kInf) atomic_min(a.fmin + (s.phase & 1) * 64 + lane_source<P>(), ls.fmin);
+    dl[0][lane_id()] = ls.fmin;  // (the items' distances are no longer needed)
     const uint32_t wv = threadIdx.x / kWave;
     const uint64_t lane_items = wave_sum(mc.lane_items), edges = wave_sum(mc.edges);
     if (lane_id() == 0) {
@@ -1214,6 +1213,19 @@ void multi_kernel(MArgs a) {
       }
       uint32_t *const tail = which == 2 ? &c->hcount[1u - s.heavy_in] : &c->qcount[which ? s.far_q : s.near_q];
       drain_base[which] = tot_n ? atomic_add(tail, tot_n) : 0u;
+    }
+    // The block's smallest far push per source -> phase minimum.  One atomic per
+    // wavefront and lane, 64 words that every wavefront meets at (with packed rows
+    // the same word 2 or 4 times over), took most of a wide round that defers: ms, 16
+    // sources, 300,000 vertices of out-degree 4 6.4 -> 2.0, grid 500^2 at 1000 28.7
+    // -> 23.6; RMAT of 2^18 vertices, weights to 10000, x 24 19.0 -> 9.9; smallest
+    // distances as thresholds, road-like 300^2 x 16 at 32 1905 -> 843.
+    if (threadIdx.x >= BS - kWave) {
+      uint32_t m = kInf;
+      for (uint32_t w = 0; w < BS / kWave; ++w) m = min(m, dls[w][0][lane_id()]);
+#pragma unroll
+      for (uint32_t d = kWave / P; d < kWave; d *= 2) m = min(m, (uint32_t)__shfl_xor(m, d));
+      if (m != kInf && lane_id() < kWave / P) atomic_min(a.fmin + (s.phase & 1) * 64 + lane_id(), m);
     }
     if (threadIdx.x == 0 && (blk[0] | blk[1])) {
       MultiCounters *const tot = a.tot + blockIdx.x % kGroups;
