@@ -93,14 +93,20 @@ struct Filter {
 // `step` deltas.  A round of a batch costs some 20 us however small, and the far
 // pile, expanded as a whole every phase, is mostly work done again: with 64
 // sources the rounds of one wide phase expand a vertex for many of them at
-// once.  On graphs with a hub, of few hops, the step begins at kHubStep; it is
-// climbed from there while the threshold then moves further per us of modelled
-// cost, or while rounds are nearly empty; else one step back, and two phases
-// later the next trial.  Distances do not depend on it.
-// Ms at steps of 1 -> here (delta 32): RMAT of 16400 vertices x 5 sources 1.84 ->
-// 0.78, 100003 x 9 3.9 -> 1.37, 262900 x 64 12.0 -> 2.9 (at a delta that passes
-// every distance 2.7); grid 64^2 x 5 6.0 -> 2.6, road-like 300^2 x 64 at 10000
-// 13 -> 6.9.
+// once.  On graphs with a hub, of few hops, the step begins at kHubStep: at 16 and
+// less the cost of the first phases, whose frontiers grow by factors, says that
+// a wider step does not pay, and the climb stays where vertices are expanded most
+// often.  It is climbed from there, or from 1 on other graphs, while the threshold
+// then moves further per us of modelled cost, or while rounds are nearly empty;
+// else one step back, and two phases later the next trial.  Distances do not
+// depend on it.
+// Ms at steps of 1 -> from 16 on hubs, 1 elsewhere (delta 32): RMAT of 16400 vertices
+// x 5 sources 1.84 -> 0.78, 100003 x 9 3.9 -> 1.37, 262900 x 64 12.0 -> 2.9; grid
+// 64^2 x 5 6.0 -> 2.6, road-like 300^2 x 64 at 10000 13 -> 6.9.  Hubs from 16 -> from
+// kHubStep: RMAT of 2^20 x 64 at 1 15.4 -> 4.6 (steps of 1: 8.6), 2^18, weights to
+// 10000, x 64 at 32 22.0 -> 4.4 (19.9), x 24 9.9 -> 2.8 (13.5), 2^16 of 32 edges x 64
+// at 1 9.3 -> 2.7 (5.1); slower only where the hub is no way across: grid 300^2 with
+// 1000 edges more at a corner, x 64 at 32, 21.4 -> 28.8 (101).
 struct Pace {
   uint32_t step;    // deltas that the threshold moves by
   uint32_t hold;    // phases until the next trial; 0: this phase is one
@@ -108,7 +114,7 @@ struct Pace {
   uint32_t rounds;  // before this phase
   uint64_t edges;   // expanded before this phase
 };
-constexpr uint32_t kHubStep = 16, kMaxMultiStep = 1u << 16;
+constexpr uint32_t kMaxMultiStep = 1u << 16, kHubStep = kMaxMultiStep;
 constexpr float kRoundUs = 20, kEdgesPerUs = 30000;
 
 // Work tickets and round totals are kept per group of blocks (block b: group
