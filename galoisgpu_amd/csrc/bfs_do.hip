@@ -1157,7 +1157,7 @@ int lsg_bfs_do(const lsg_graph *g, const lsg_graph *gt, uint32_t src, int direct
     record_resident_grid(w, fn, kBs, grid);
   }
   if (hc.abort == kAbortTimeout)
-    return fail(LSG_ERR_TIMEOUT, "bfs_do: grid barrier timed out at level %u; levels are incomplete", hc.s.round);
+    return fail(LSG_ERR_TIMEOUT, "bfs_do: grid barrier timed out at level %u; levels are incomplete", wave_last(a.wc).round);
   if (hc.abort == kAbortCapacity) return fail(LSG_ERR_CAPACITY, "bfs_do: chunk queue capacity exceeded");
   if (stats) {
     memset(stats, 0, sizeof *stats);

@@ -168,6 +168,13 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
     grid = (int)hc.resident_seen;
     record_resident_grid(w, fnp, bs, grid);
   }
+  if (hc.abort == kAbortTimeout && wave) {
+    const WaveLast l = wave_last(a.wc);
+    return fail(LSG_ERR_TIMEOUT,
+                "grid barrier timed out (grid %d x %d) after round %u phase %u was published, generation %u; "
+                "distances are incomplete",
+                grid, bs, l.round, l.phase, l.generation);
+  }
   if (hc.abort == kAbortTimeout)
     return fail(LSG_ERR_TIMEOUT,
                 "grid barrier timed out (grid %d x %d) at round %u phase %u done %u with %u of %u arrival "

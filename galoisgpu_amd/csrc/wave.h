@@ -96,4 +96,19 @@ const void *wave_kernel_fn(Algo algo, int bs);
 int wave_enqueue(Algo algo, int bs, int grid, const WaveArgs &a, uint32_t seed, const uint32_t *seeds, uint32_t nseeds,
                  const Resume *resume, int cus, hipStream_t stream);
 
+// The last round that was published, for the text of an error: the control block
+// does not follow the rounds.  (A launch starts with round 1, unpublished.)
+struct WaveLast {
+  uint32_t round = 1, phase = 0, generation = 0;
+};
+inline WaveLast wave_last(const WaveCtrl *wc) {
+  uint64_t m[kWaveMsg];
+  WaveLast l;
+  if (hipMemcpy(m, wc->msg, sizeof m, hipMemcpyDeviceToHost) != hipSuccess || m[0] == 0) return l;
+  l.round = (uint32_t)(m[2] >> 32);
+  l.phase = (uint32_t)(m[3] >> 32);
+  l.generation = (uint32_t)m[0];
+  return l;
+}
+
 }  // namespace lsg
