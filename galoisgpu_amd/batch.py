@@ -99,7 +99,10 @@ def sssp_batch(dev: DeviceGraph, srcs: Sequence[int], opts: Optional[Options] = 
 
 def sssp_graphs(devs: Sequence[DeviceGraph], srcs: Sequence[int], opts: Optional[Options] = None
                 ) -> Tuple[List[np.ndarray], dict]:
-    """Many graphs, one source each, in one persistent launch (disjoint-union multi-seed run)."""
+    """Many graphs, one source each, in one persistent launch (disjoint-union multi-seed run).
+
+    The distances are views of one array: keeping one graph's keeps all of them.
+    """
     opts = opts or Options()
     n = len(devs)
     if len(srcs) != n:

@@ -93,7 +93,8 @@ typedef struct lsg_opts {
   int32_t heavy_deg;   /* degrees >= this are split into chunks of heavy_deg edges, expanded by whole
                           blocks in the next round (default 512; with the other options at their
                           defaults by wavefronts, default 256; batched runs: by a wavefront,
-                          default 64, or 256 from 2^24 edges, and >= 8) */
+                          default 64, or 256 from 2^24 edges, and >= 8).  Single source: values
+                          below the block size are raised to it */
   int32_t sched;       /* 0 = fixed delta; 1 = the learned scheduler picks each phase's delta width
                           and mode (expansion mode for SSSP, far mode for batched runs) from the
                           model loaded with lsg_sched_set_model */
@@ -255,7 +256,9 @@ int lsg_output_cc(const lsg_graph *host_g, const char *file);
  * itself or max_iterations pass.  The reference uses alpha 0.85, epsilon 1e-6
  * (apps/pr/kernel.cu:19-20) and pushes residuals instead; both reach the same
  * fixpoint, within float rounding.  rank_dev is a device array of nnodes
- * floats.  stats: iterations. */
+ * floats.  Each call sorts the in-edges' sources into the device's workspace: 4
+ * bytes an edge and some 32 a vertex, kept until lsg_workspace_release.  stats:
+ * iterations. */
 int lsg_pagerank(const lsg_graph *g, const lsg_graph *gt, float alpha, float epsilon, int32_t max_iterations,
                  float *rank_dev, lsg_stats *stats);
 /* apps/pr/support.cu:45-97 output: prints "sum: %f (%d)" (float sum of the
