@@ -73,6 +73,14 @@ inline int wave_blocks_per_cu(uint64_t nnodes, uint64_t nedges) {
 inline uint32_t wave_local_max(uint64_t nnodes, uint64_t nedges) {
   return (uint32_t)(nedges <= 4 * nnodes ? 512 : 2048 * nnodes / nedges);
 }
+// On low-degree graphs a round with a vertex of this many edges is the whole grid's,
+// one item a unit: in a round of one block a lane has its edges four at a time, or a
+// wavefront several such vertices one after another, and of units of 16 items as few
+// wavefronts would have any.  BFS kernel us where it is left at 256 (heavy_deg) / 32 /
+// 16 edges: 100,000 vertices of 1000 hubs 391 / 122 / 124, a tree of degree 64 224 / 86
+// / 86, of degree 30 117 / 105 / 99, a random tree 202 / 205 / 188; grids and road-like
+// graphs alike, also with vertices of 20 and 40 edges among them.
+constexpr uint32_t kLocalDeg = 16;
 // A chunk of a heavy vertex is the edges that a wavefront holds in flight
 // (kWaveU a lane); 512 and 1024: equal to 5 % slower on RMAT graphs.
 constexpr int kWaveHeavyDeg = 256;

@@ -128,22 +128,25 @@ struct WavePace {
 // the largest so far (a grid's frontier, which grows by a ring a round, never is;
 // at twice road-like 2048^2 took 2.55 ms, with it or without the rule 2.03)
 // the next kWideRounds rounds -- all that such a graph has -- are wide:
-//   - wavefronts go on with what they pushed only in rounds of at most kWideHops
-//     items: larger ones are bound by work, and what is expanded at a distance that
-//     falls later is work done twice;
-//   - units are smaller (kWideUnit items at least): a vertex may have many edges;
+//   - wavefronts go on with what they pushed only in rounds of more than kWideItems
+//     and at most kWideHops items: larger ones are bound by work, and what is
+//     expanded at a distance that falls later is work done twice; in smaller ones
+//     few wavefronts would go on with what all can take;
+//   - units are of one item where there are wavefronts enough: a vertex may have many
+//     edges;
 //   - where vertices of heavy_deg edges are found too (kWaveSplit), the rounds are
 //     those of skewed graphs: no going on, vertices of kWaveSplitDeg edges split
 //     when they are pushed, the threshold moved by the call's delta;
 //   - on graphs of at most 2 edges a vertex (forests: one way to each vertex) the
 //     next phase is all that is left.
-// A chunk counts as heavy_deg items: it may push so many.
+// A chunk counts as heavy_deg items: it may push so many.  A round that one block
+// leaves to the grid because of a vertex's edges (kLocalDeg) is wide by itself.
 // Kernel us without / with, delta 10000 where the delta is not said: 5 edges a vertex
 // RMAT-like, 32,000 vertices 347 / 207, 100,000 455 / 248, 10^6 1040 / 679, delta 32
 // 916 / 612; uniform out-degree 4, 10^6 1028 / 865, BFS 451 / 340, 4 x 10^6 2734 /
 // 2405, BFS 1250 / 908; random trees of 10^5 delta 32 388 / 289; 4 x 10^6 leaves of
 // 1000 hubs, delta 32 1576 / 1150.  Grids and road-like graphs alike.
-constexpr uint32_t kWideItems = 512, kWideRounds = 48, kWideUnit = 4;
+constexpr uint32_t kWideItems = 512, kWideRounds = 48;
 template <Algo A>
 constexpr uint32_t kWideHops = A == Algo::SSSP ? 16384 : 8192;
 constexpr uint32_t kWideChunks = 4;  // chunks of a round that say that the graph is skewed
@@ -175,7 +178,7 @@ struct WaveShared {
   uint32_t pile_n[2];
   uint32_t far_n;    // the far queue's length
   uint32_t spill_n;  // vertices handed to the near queue
-  uint32_t stop;     // a vertex too heavy for this mode was pushed
+  uint32_t stop;     // a vertex of too many edges for this mode was pushed
   unsigned long long items;
 };
 
@@ -509,7 +512,7 @@ struct LocalRelax {
         if ((m[k] >> lane_id()) & 1) {
           const uint32_t p = pos + lanes_below(m[k]);
           const uint32_t rs = (uint32_t)rb[k], re = (uint32_t)(rb[k] >> 32);
-          if (re - rs >= a.heavy_deg) sh.stop = 1;
+          if (re - rs >= (a.pace ? kLocalDeg : a.heavy_deg)) sh.stop = 1;
           if (p < kLocalCap) sh.pile[nxt][p] = Entry{v[k], nd[k], rs, re};
           else spill(v[k]);
         }
@@ -586,10 +589,13 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
         const uint64_t rb = ld_pair(a.row_start + v);
         const uint32_t rs = (uint32_t)rb, re = (int64_t)d <= cut ? rs : (uint32_t)(rb >> 32);
         sh.pile[cur][i] = Entry{v, d, rs, re};
-        big |= re - rs >= a.heavy_deg;
+        big |= re - rs >= (a.pace ? kLocalDeg : a.heavy_deg);
       }
-      // a heavy vertex among them: the grid runs this round
-      if (__syncthreads_or(big)) break;
+      // a vertex of many edges among them: the grid runs this round, as a wide one
+      if (__syncthreads_or(big)) {
+        if (a.hops) r.flags |= kWaveWide;
+        break;
+      }
       load = false;
     }
     if (threadIdx.x == 0) {
@@ -615,6 +621,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
       n = sh.spill_n;
       r.roles = wave_roles(r.near_q(), r.in_q(), r.far_q());
       if (a.hops) grow();
+      if (a.hops && sh.stop) r.flags |= kWaveWide;
       break;
     }
     if (near) {
@@ -714,7 +721,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     w.hq = gen & 1 ? a.chunk[1] : a.chunk[0];
     // (BFS's first round stays one level: levels that mix there mix in every round)
     w.hops = (A == Algo::BFS && r.round == 1) || r.flags & kWaveSplit ||
-                     (r.flags & kWaveWide && r.items > kWideHops<A>)
+                     (r.flags & kWaveWide && (r.items > kWideHops<A> || r.items <= kWideItems))
                  ? 0u
                  : a.hops;
     w.split = a.split || r.flags & kWaveSplit;
@@ -725,7 +732,7 @@ __global__ __launch_bounds__(BS, 4) void wave_kernel(WaveArgs a) {
     // wavefronts serialises, ~12 ns a ticket).
     const uint32_t *const in = wave_queue(a, r.in_q());
     const WaveChunk *const hin = gen & 1 ? a.chunk[0] : a.chunk[1];
-    const uint32_t per = min((uint32_t)kWave, max(r.flags & kWaveWide ? kWideUnit : a.unit_min, (r.items + nwaves - 1) / nwaves));
+    const uint32_t per = min((uint32_t)kWave, max(r.flags & kWaveWide ? 1u : a.unit_min, (r.items + nwaves - 1) / nwaves));
     const uint32_t nitem = (r.items + per - 1) / per, nunits = nitem + r.heavy;
     const bool many = nunits > nwaves;
     uint32_t unit = many ? (blockIdx.x / ngroups * NW + wv) * ngroups + g : wave;
