@@ -73,12 +73,15 @@ inline int wave_blocks_per_cu(uint64_t nnodes, uint64_t nedges) {
 inline uint32_t wave_local_max(uint64_t nnodes, uint64_t nedges) {
   return (uint32_t)(nedges <= 4 * nnodes ? 512 : 2048 * nnodes / nedges);
 }
-// On low-degree graphs a round with a vertex of this many edges is the whole grid's,
+// A round with a vertex of this many edges is the whole grid's, on low-degree graphs
 // one item a unit: in a round of one block a lane has its edges four at a time, or a
 // wavefront several such vertices one after another, and of units of 16 items as few
 // wavefronts would have any.  BFS kernel us where it is left at 256 (heavy_deg) / 32 /
 // 16 edges: 100,000 vertices of 1000 hubs 391 / 122 / 124, a tree of degree 64 224 / 86
-// / 86, of degree 30 117 / 105 / 99, a random tree 202 / 205 / 188; grids and road-like
+// / 86, of degree 30 117 / 105 / 99, a random tree 202 / 205 / 188; SSSP delta 32 at 256
+// / 32 / 16 / 8: uniform out-degree 32, 1000 vertices 259 / 186 / 185 / 186, 10,000 484 /
+// 334 / 324 / 327, out-degree 16 378 / 377 / 339 / 335, out-degree 7 280 / 282 / 280 /
+// 293, RMAT of 16,384 vertices and 8 edges 196 / 192 / 191 / 197; grids and road-like
 // graphs alike, also with vertices of 20 and 40 edges among them.
 constexpr uint32_t kLocalDeg = 16;
 // A chunk of a heavy vertex is the edges that a wavefront holds in flight

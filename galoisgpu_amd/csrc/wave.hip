@@ -512,7 +512,7 @@ struct LocalRelax {
         if ((m[k] >> lane_id()) & 1) {
           const uint32_t p = pos + lanes_below(m[k]);
           const uint32_t rs = (uint32_t)rb[k], re = (uint32_t)(rb[k] >> 32);
-          if (re - rs >= (a.pace ? kLocalDeg : a.heavy_deg)) sh.stop = 1;
+          if (re - rs >= kLocalDeg) sh.stop = 1;
           if (p < kLocalCap) sh.pile[nxt][p] = Entry{v[k], nd[k], rs, re};
           else spill(v[k]);
         }
@@ -589,7 +589,7 @@ __device__ __forceinline__ void wave_local(const WaveArgs &a, WaveShared<BS> &sh
         const uint64_t rb = ld_pair(a.row_start + v);
         const uint32_t rs = (uint32_t)rb, re = (int64_t)d <= cut ? rs : (uint32_t)(rb >> 32);
         sh.pile[cur][i] = Entry{v, d, rs, re};
-        big |= re - rs >= (a.pace ? kLocalDeg : a.heavy_deg);
+        big |= re - rs >= kLocalDeg;
       }
       // a vertex of many edges among them: the grid runs this round, as a wide one
       if (__syncthreads_or(big)) {

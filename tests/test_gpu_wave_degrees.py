@@ -1,9 +1,10 @@
-"""Low-degree graphs with vertices of more edges than a round of one block takes.
+"""Graphs with vertices of more edges than a round of one block takes.
 
-From 16 edges on such a vertex sends its round to the whole grid, one item a unit.  The
-cases have degrees on both sides of that, in the first rounds and in the middle of a
-traversal, more than 32,768 vertices (fewer run in one workgroup), and rounds of every
-size between the block's and the grid's.  Against the oracle, exact.
+From 16 edges on such a vertex sends its round to the whole grid, on low-degree graphs
+one item a unit.  The cases have degrees on both sides of that, in the first rounds and in
+the middle of a traversal, rounds of every size between the block's and the grid's, and,
+on low-degree graphs, more than 32,768 vertices (fewer run in one workgroup).  Against
+the oracle, exact.
 """
 import numpy as np
 import pytest
@@ -71,3 +72,12 @@ def test_leaves_of_two_hubs(k):
 def test_bushes_on_a_path(deg):
     print("comb", deg, flush=True)
     check(comb(deg), 3)
+
+
+@pytest.mark.parametrize("n", [300, 3000])
+@pytest.mark.parametrize("deg", [8, 15, 16, 17, 40])
+def test_every_vertex_of_one_degree(n, deg):
+    rng = np.random.default_rng(deg)
+    g = CSRGraph.from_arrays(np.arange(n + 1) * deg, rng.integers(0, n, n * deg), rng.integers(0, 100, n * deg))
+    print("uniform", n, deg, flush=True)
+    check(g, 5)
