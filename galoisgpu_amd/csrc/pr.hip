@@ -32,11 +32,11 @@
 // Without heavy vertices the sort is by in-degree within tiles of kPrTile
 // vertices only (heavy = 0, live = V): there is no hub to bring together, and
 // neighbours of a road network stay near (2048^2 road-like: 60 us per
-// iteration, sorted as a whole 187).
+// iteration, sorted as a whole 187; with flags on lines of their own 29).
 // Ranks, out-degrees and both contribution arrays are kept in that order and
 // the ranks put back at the end.  Per iteration, against lanes that walked the
-// reverse CSR in vertex order: RMAT-22 513 -> 242 us, 2^20 vertices of uniform
-// degrees 146 -> 88, road-like 73 -> 60; preparing takes 1.0 ms on RMAT-22.
+// reverse CSR in vertex order: RMAT-22 514 -> 245 us, 2^20 vertices of uniform
+// degrees 145 -> 88, road-like 74 -> 29; preparing takes 1.1 ms on RMAT-22.
 //
 // The convergence test stays on the device: the host enqueues iterations in
 // batches of one or two launches each; a block in which some rank moved by

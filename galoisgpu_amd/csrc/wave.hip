@@ -142,10 +142,10 @@ struct WavePace {
 // A chunk counts as heavy_deg items: it may push so many.  A round that one block
 // leaves to the grid because of a vertex's edges (kLocalDeg) is wide by itself.
 // Kernel us without / with, delta 10000 where the delta is not said: 5 edges a vertex
-// RMAT-like, 32,000 vertices 347 / 207, 100,000 455 / 248, 10^6 1040 / 679, delta 32
-// 916 / 612; uniform out-degree 4, 10^6 1028 / 865, BFS 451 / 340, 4 x 10^6 2734 /
-// 2405, BFS 1250 / 908; random trees of 10^5 delta 32 388 / 289; 4 x 10^6 leaves of
-// 1000 hubs, delta 32 1576 / 1150.  Grids and road-like graphs alike.
+// RMAT-like, 32,000 vertices 347 / 207, 100,000 455 / 255, 10^6 1040 / 700, delta 32
+// 916 / 622; uniform out-degree 4, 10^6 1028 / 853, BFS 451 / 311, 4 x 10^6 2734 /
+// 2381, BFS 1250 / 897; random trees of 10^5 delta 32 388 / 260; 4 x 10^6 leaves of
+// 1000 hubs, delta 32 1576 / 1158.  Grids and road-like graphs alike.
 constexpr uint32_t kWideItems = 512, kWideRounds = 48;
 template <Algo A>
 constexpr uint32_t kWideHops = A == Algo::SSSP ? 16384 : 8192;
