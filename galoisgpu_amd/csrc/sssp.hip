@@ -150,6 +150,7 @@ static int run_core(Workspace *w, const CsrView &g, const uint32_t *seeds, uint3
       key_append(key, a);
       key_append(key, grid);
       key_append(key, bs);
+      key_append(key, sd);  // (another call's use of the buffer may have moved it)
       key_append(key, nseeds);
       if ((rc = launch_captured(w, key, enqueue))) return rc;
     } else if ((rc = enqueue())) {
